@@ -18,8 +18,11 @@
 // COMP: sums of up to kSmallBlock sources are Kahan-added per lane (as the
 // 64-source partials of the other kernels) and the lanes and waves are
 // combined in FP64; otherwise plain FP32 throughout (the plain FP32 path).
-// Pair arithmetic as in stream_sources: 12 VALU slots per ordered pair plus
-// one LDS read per source shared by the lane's A targets.
+// Pair arithmetic as in stream_sources: 12 VALU instructions and a root per
+// ordered pair, the roots of 8 pairs together (rsq_group.h), plus one LDS read
+// per source shared by the lane's A targets.  Per step, mixed: N = 8192 23.3 us
+// (27.3 with a root per pair), 6001 18.3 (21.2), 4096 8.9 (9.6); below that the
+// launch and the copy into LDS bound it (N = 1024: 4.0 us either way).
 #pragma once
 
 #include <type_traits>
@@ -58,7 +61,7 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
     __syncthreads();
 
     const int split = wave * G + g;
-    const int iters = n_pad / SPL;  // n_pad is a multiple of 1024 and SPL divides 1024
+    const int iters = n_pad / SPL;  // n_pad is a multiple of 1024 and SPL divides 128: a multiple of 8
     for (int b0 = 0; b0 < iters; b0 += kSmallBlock) {
         const int b1 = b0 + kSmallBlock < iters ? b0 + kSmallBlock : iters;
         float ax[A], ay[A], az[A];
@@ -70,18 +73,33 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
                 ax[a] = hx[a]; ay[a] = hy[a]; az[a] = hz[a];
             }
         }
-#pragma unroll 8
-        for (int i = b0; i < b1; ++i) {
-            const float4 b = sh[split + i * SPL];
+        constexpr int J = A >= 4 ? 2 : 8 / A;  // sources per group of reciprocal roots; divides kSmallBlock and iters
+#pragma unroll 1
+        for (int i = b0; i < b1; i += J) {
+            float rx[J * A], ry[J * A], rz[J * A], d2[J * A], y[J * A], m[J];
 #pragma unroll
-            for (int a = 0; a < A; ++a) {
-                const float rx = b.x - px[a], ry = b.y - py[a], rz = b.z - pz[a];
-                const float d2 = __builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, __builtin_fmaf(rz, rz, eps2)));
-                const float s = pair_scale<NEWTON>(d2, b.w);
-                ax[a] = __builtin_fmaf(rx, s, ax[a]);
-                ay[a] = __builtin_fmaf(ry, s, ay[a]);
-                az[a] = __builtin_fmaf(rz, s, az[a]);
+            for (int u = 0; u < J; ++u) {
+                const float4 b = sh[split + (i + u) * SPL];
+                m[u] = b.w;
+#pragma unroll
+                for (int a = 0; a < A; ++a) {
+                    const int q = u * A + a;
+                    rx[q] = b.x - px[a]; ry[q] = b.y - py[a]; rz[q] = b.z - pz[a];
+                    d2[q] = __builtin_fmaf(rx[q], rx[q],
+                                           __builtin_fmaf(ry[q], ry[q], __builtin_fmaf(rz[q], rz[q], eps2)));
+                }
             }
+            rsq_group<J * A>(d2, y);
+#pragma unroll
+            for (int u = 0; u < J; ++u)
+#pragma unroll
+                for (int a = 0; a < A; ++a) {
+                    const int q = u * A + a;
+                    const float s = pair_scale<NEWTON>(d2[q], y[q], m[u]);
+                    ax[a] = __builtin_fmaf(rx[q], s, ax[a]);
+                    ay[a] = __builtin_fmaf(ry[q], s, ay[a]);
+                    az[a] = __builtin_fmaf(rz[q], s, az[a]);
+                }
         }
 #pragma unroll
         for (int a = 0; a < A; ++a) {
@@ -145,7 +163,7 @@ template <int A, int TL, int W, int CAP, bool COMP, bool NEWTON, class Epi>
 hipError_t launch_small_tile(const float4* src, int i0, int nt, int n_pad, float eps2, const Epi& epi,
                              hipStream_t st)
 {
-    static_assert(64 % TL == 0 && 1024 % ((64 / TL) * W) == 0, "source splits must divide kPadJ");
+    static_assert(64 % TL == 0 && kPadJ / 8 % ((64 / TL) * W) == 0, "each split takes a multiple of 8 sources");
     if (n_pad > CAP || n_pad % kPadJ != 0)
         return hipErrorInvalidValue;
     constexpr int TW = TL * A;

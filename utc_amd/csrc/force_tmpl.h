@@ -10,11 +10,11 @@
 //
 // Arithmetic per pair (the reference's pair, benchapps/nbody/seq/bodysystem.h:70-96,
 // rewritten for the VALU): r = pj - pi (3 sub), d2 = r.r + eps2 (3 fma),
-// y = v_rsq_f32(d2) (transcendental; it co-issues with the FMA pipe),
-// s = mj*y*y*y (3 mul), acc += r*s (3 fma): 12 VALU issue slots per pair.
-// Measured on MI355X this runs at ~99% of the non-packed FP32 VALU issue
-// rate; replacing y^3 by rsq(d2)*rcp(d2) (11 slots, two transcendentals) is
-// slower because the second transcendental does not co-issue.  The NEWTON
+// y = v_rsq_f32(d2) (transcendental), s = mj*y*y*y (3 mul), acc += r*s
+// (3 fma): 12 VALU instructions and a root per pair.  The roots of 8 pairs are
+// taken together (rsq_group.h): k2s8 at N = 262144 18.6 ms/step, 20.8 with a
+// root per pair; k2s16 20.8, was 23.7.  Replacing y^3 by rsq(d2)*rcp(d2) (11
+// instructions, two transcendentals) is slower.  The NEWTON
 // variant applies one Newton-Raphson step to y, carried into the cube: with
 // e = 1 - d2*y^2 the refined y1 = y (1 + e/2) has y1^3 = y^3 (1 + 3e/2) +
 // O(e^2) y^3, and |e| ~ 2^-22 leaves the e^2 terms far below FP32 rounding,
@@ -28,24 +28,28 @@
 #pragma once
 
 #include "internal.h"
+#include "rsq_group.h"
 
 namespace utcnb {
 
-__device__ __forceinline__ float rsq_f32(float x) { return __builtin_amdgcn_rsqf(x); }
-
+// m d2^{-3/2} from d2 and y = rsq(d2).
 template <bool NEWTON>
-__device__ __forceinline__ float pair_scale(float d2, float m)
+__device__ __forceinline__ float pair_scale(float d2, float y, float m)
 {
     if constexpr (NEWTON) {
-        const float y = rsq_f32(d2);
         const float y2 = y * y;
         const float e = __builtin_fmaf(-d2, y2, 1.0f);
         const float y3 = y2 * y;
         return m * __builtin_fmaf(y3 * e, 1.5f, y3);
     } else {
-        float y = rsq_f32(d2);
         return m * y * y * y;
     }
+}
+
+template <bool NEWTON>
+__device__ __forceinline__ float pair_scale(float d2, float m)
+{
+    return pair_scale<NEWTON>(d2, __builtin_amdgcn_rsqf(d2), m);
 }
 
 // Kahan step: add partial p into (s, c).
@@ -75,20 +79,34 @@ __device__ __forceinline__ void stream_sources(const float4* __restrict__ src, i
                 ax[k] = hx[k]; ay[k] = hy[k]; az[k] = hz[k];
             }
         }
-#pragma unroll 4
-        for (int j = jc; j < jc + kChunk; ++j) {
-            const float4 b = src[j];
+        constexpr int J = K >= 4 ? 4 : 8 / K;  // sources (one or two scalar loads) per group of roots
+#pragma unroll 1
+        for (int j = jc; j < jc + kChunk; j += J) {
+            float rx[J][K], ry[J][K], rz[J][K], d2[J * K], y[J * K], bw[J];
 #pragma unroll
-            for (int k = 0; k < K; ++k) {
-                float rx = b.x - px[k];
-                float ry = b.y - py[k];
-                float rz = b.z - pz[k];
-                float d2 = __builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, __builtin_fmaf(rz, rz, eps2)));
-                float s = pair_scale<NEWTON>(d2, b.w);
-                ax[k] = __builtin_fmaf(rx, s, ax[k]);
-                ay[k] = __builtin_fmaf(ry, s, ay[k]);
-                az[k] = __builtin_fmaf(rz, s, az[k]);
+            for (int u = 0; u < J; ++u) {
+                const float4 b = src[j + u];
+                bw[u] = b.w;
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    rx[u][k] = b.x - px[k];
+                    ry[u][k] = b.y - py[k];
+                    rz[u][k] = b.z - pz[k];
+                    d2[u * K + k] = __builtin_fmaf(rx[u][k], rx[u][k],
+                                                   __builtin_fmaf(ry[u][k], ry[u][k],
+                                                                  __builtin_fmaf(rz[u][k], rz[u][k], eps2)));
+                }
             }
+            rsq_group<J * K>(d2, y);
+#pragma unroll
+            for (int u = 0; u < J; ++u)
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    const float s = pair_scale<NEWTON>(d2[u * K + k], y[u * K + k], bw[u]);
+                    ax[k] = __builtin_fmaf(rx[u][k], s, ax[k]);
+                    ay[k] = __builtin_fmaf(ry[u][k], s, ay[k]);
+                    az[k] = __builtin_fmaf(rz[u][k], s, az[k]);
+                }
         }
 #pragma unroll
         for (int k = 0; k < K; ++k) {
