@@ -46,12 +46,6 @@ __device__ __forceinline__ float pair_scale(float d2, float y, float m)
     }
 }
 
-template <bool NEWTON>
-__device__ __forceinline__ float pair_scale(float d2, float m)
-{
-    return pair_scale<NEWTON>(d2, __builtin_amdgcn_rsqf(d2), m);
-}
-
 // Kahan step: add partial p into (s, c).
 __device__ __forceinline__ void kahan_add(float& s, float& c, float p)
 {

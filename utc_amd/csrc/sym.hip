@@ -2,16 +2,15 @@
 //
 // The field on body i from body j and the reaction on j from i share r, d^2
 // and y^3 = (|r|^2 + eps2)^{-3/2}: a_i += m_j y^3 r, a_j -= m_i y^3 r.  The
-// one-pass kernels (force_tmpl.h) spend 12 VALU issue slots per ordered pair;
-// here an unordered pair costs 16 (3 sub, 3 fma, 2 mul for y^3, 2 mul for the
-// two mass factors, 6 fma for the two accumulations) plus, per 64-source
-// rotation step, 7 wave-wide DPP moves shared by the K targets of a lane:
-// (16 + 7/K)/2 slots per ordered pair, 8.4 at K = 8.  When the wave's targets
-// and the block's sources all have one mass m (the reference's initial
-// conditions give every body mass 1), both sides use y^3 r directly and the
-// block partials are scaled by m once: 14 slots and 6 DPP moves, (14 + 6/K)/2
-// = 7.4 per ordered pair.  For m a power of two the two forms are bitwise
-// equal; otherwise they differ by the rounding of one product per partial.
+// one-pass kernels (force_tmpl.h) spend 12 VALU instructions and a root per
+// ordered pair; here an unordered pair costs 16 (3 sub, 3 fma, 2 mul for y^3,
+// 2 mul for the two mass factors, 6 fma for the two accumulations) and a
+// root, 8 and half a root per ordered pair.  When the wave's targets and the
+// block's sources all have one mass m (the reference's initial conditions
+// give every body mass 1), both sides use y^3 r directly and the block
+// partials are scaled by m once: 14 instructions.  For m a power of two the
+// two forms are bitwise equal; otherwise they differ by the rounding of one
+// product per partial.
 //
 // Mapping.  Bodies form wave blocks of 64*K (lane l holds K targets).  Wave
 // block w takes (a) its own K blocks of 64 sources: block kb both sides
@@ -20,9 +19,12 @@
 // of wave blocks v = w+1 .. w+NW/2 (mod NW), both sides; for even NW the
 // block half way round is taken by the lower half only, so every unordered
 // pair of wave blocks is visited exactly once.  A block of 64
-// sources sits one per lane and rotates around the wave with DPP wave_ror:1
-// for 64 steps, carrying its reaction accumulator, so after 64 steps every
-// target has met every source and each reaction sum is back in its home lane.
+// sources lies in the wave's own LDS, twice in a row; at step t = 0 .. 63 lane
+// l meets source (l + t) mod 64, at slot l + t, and adds its K reactions to
+// the source's sum in LDS at the same slot (slots s and s + 64 are one source
+// and meet at the end), so after 64 steps every target has met every source.
+// No two lanes touch one slot in a step and the steps of a wave run in order,
+// so the sums need no atomics and are the same on every run.
 // R waves split a wave block's work into sub-units (u, kb): source block kb of
 // unit u, where unit 0 is the wave block's own sources and unit 1 + d the wave
 // block d + 1 places round; wave r takes sub-units [Q*r/R, Q*(r+1)/R) of
@@ -33,29 +35,25 @@
 // one wave alone on a SIMD waits on its own dependent instructions.  Tiles
 // with a rotation split RS (SPLIT kernels) cut each sub-unit's 64 rotation
 // steps into RS chunks of 64/RS steps, and the R waves of a wave block share
-// its Q * RS chunks: chunk c starts with the source block already rotated by
-// 64c/RS lanes (lane l loads source (l - 64c/RS) mod 64) and leaves the
-// reaction sums rotated by 64(c+1)/RS, so each chunk stores its reactions to
-// the source lane they belong to, in a reaction record of its own.
+// its Q * RS chunks, each with a reaction record of its own.
+//
+// What bounds it: FP32 issue and, at large N, the power the FMAs draw.  A step
+// issues one 16-byte and three 4-byte LDS reads and three LDS writes beside
+// its K pairs; carrying the source and its sums round the wave in registers
+// instead (7 DPP moves per step, which pair with nothing) and taking each
+// root as it comes cost 55 cycles per pair and wave where this takes 44
+// (N = 262144, equal masses: 23.2e6 clocks for 28.9e6; the clock drops from
+// 2383 to 2113 MHz meanwhile, so the time falls less).  Per step, mixed, same
+// device: N = 262144 10.7-10.9 ms (12.3 before), log-uniform masses 11.8
+// (14.0), N = 65536 0.716 ms (0.829), plain FP32 0.700 (0.819), N = 16384
+// (sym4r64) 68 us (75).  The roots are taken 4 at a time: with 8 the K = 8
+// kernel needs 202 VGPRs (two waves per SIMD) and runs 3-10% slower; held to
+// 128 VGPRs it spills and runs 8-10% slower.
 #include "force_tmpl.h"
 #include "sym_items.h"
 #include "sym_reduce.h"
 
 namespace utcnb {
-
-// Lane l receives lane l-1's value (lane 0 lane 63's).  Every lane has a
-// source under wave_ror:1, so the "old" operand is never used.  Passing v as
-// "old" lets the compiler rotate in place, without a v_mov that first zeroes
-// a new register; which form is faster depends on K (same-device A/B runs on
-// MI355X, equal masses): in place is 7.7% faster at K = 2 (N = 4096, sym2r32)
-// but 3% slower at K = 8 (N = 262144, sym8r64) and 3.4% slower for the
-// batched K = 4 kernel, and the same within noise for the K = 4 tiles.
-template <int K>
-__device__ __forceinline__ float wave_ror1(float v)
-{
-    const int x = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(K <= 2 ? x : 0, x, 0x13C /* wave_ror:1 */, 0xF, 0xF, false));
-}
 
 // Adds a block partial p into the running target sum: Kahan-compensated
 // (COMP) or plain FP32.
@@ -68,64 +66,107 @@ __device__ __forceinline__ void block_add(float& a, float& c, float p)
         a += p;
 }
 
-// One rotation step of sym_block (statement macro: the same code in the
-// fixed 64-step loop and in the chunked loop).
-#define SYM_BLOCK_STEP()                                                                               \
-    _Pragma("unroll")                                                                                  \
-    for (int k = 0; k < K; ++k) {                                                                      \
-        const float rx = sx - xi[k], ry = sy - yi[k], rz = sz - zi[k];                                 \
-        const float d2 = __builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, __builtin_fmaf(rz, rz, eps2))); \
-        const float y3 = pair_scale<NEWTON>(d2, 1.0f);                                                 \
-        const float si = UNI ? y3 : sm * y3;                                                           \
-        const float cj = UNI ? y3 : mi[k] * y3;                                                        \
-        px[k] = __builtin_fmaf(rx, si, px[k]);                                                         \
-        py[k] = __builtin_fmaf(ry, si, py[k]);                                                         \
-        pz[k] = __builtin_fmaf(rz, si, pz[k]);                                                         \
-        gx = __builtin_fmaf(-rx, cj, gx);                                                              \
-        gy = __builtin_fmaf(-ry, cj, gy);                                                              \
-        gz = __builtin_fmaf(-rz, cj, gz);                                                              \
-    }                                                                                                  \
-    sx = wave_ror1<K>(sx); sy = wave_ror1<K>(sy); sz = wave_ror1<K>(sz);                               \
-    if constexpr (!UNI)                                                                                \
-        sm = wave_ror1<K>(sm);                                                                         \
-    gx = wave_ror1<K>(gx); gy = wave_ror1<K>(gy); gz = wave_ror1<K>(gz);
+// A wave's source block and its reaction sums in LDS (wave private).  Slots are
+// read and written up to 127 = 63 + 64.
+struct SymLds {
+    float4 s[128];    // the block's 64 sources, twice
+    float g[3][128];  // reaction sums of source (slot mod 64)
+};
 
-// A block of 64 sources (one per lane, s) against the K targets of each lane,
-// both sides: the target-side block partials are added into (a, c) by
-// block_add<COMP>, the reaction sums of the lane's source come back in g after
-// 64 rotations.
-// UNI: every target mass mi[k] and source mass equals m, so the pair terms
-// drop the mass factors and the block sums are scaled by m at the end.
-// SPLIT: `steps` rotation steps (a chunk of the rotation), else all 64.
-template <int K, bool NEWTON, bool COMP, bool UNI, bool SPLIT = false>
-__device__ __forceinline__ void sym_block(float4 s, const float (&xi)[K], const float (&yi)[K],
-                                          const float (&zi)[K], const float (&mi)[K], float m, float eps2,
-                                          float (&ax)[K], float (&ay)[K], float (&az)[K], float (&cx)[K],
-                                          float (&cy)[K], float (&cz)[K], float& gx, float& gy, float& gz,
-                                          int steps = 64)
+// LDS written by other lanes of the wave is read after this (the wave's LDS
+// operations run in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_fence()
 {
-    float sx = s.x, sy = s.y, sz = s.z, sm = s.w;
-    float px[K], py[K], pz[K];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Rotation steps [t0, t0 + steps) of a block of 64 sources (lane l's source
+// s; wave private LDS L) against target slots 0 .. N-1 of each lane: at step
+// t lane l meets source (l + t) mod 64.  Slots k < N2 are two-sided; the
+// others collect the target side only.  Target-side sums are added to p; the
+// reaction sums of lane l's own source come back in g (N2 > 0).
+// UNI: every target mass mi[k] and source mass is the same, and p and g lack
+// that factor.
+template <int K, int N, int N2, bool NEWTON, bool UNI>
+__device__ __forceinline__ void sym_rotate(SymLds& L, int lane, int t0, int steps, float4 s, const float (&xi)[K],
+                                           const float (&yi)[K], const float (&zi)[K], const float (&mi)[K],
+                                           float eps2, float (&px)[N], float (&py)[N], float (&pz)[N], float (&g)[3])
+{
+    wave_lds_fence();
+    L.s[lane] = s;
+    L.s[lane + 64] = s;
+    if constexpr (N2 > 0) {
 #pragma unroll
-    for (int k = 0; k < K; ++k)
-        px[k] = py[k] = pz[k] = 0.f;
-    gx = gy = gz = 0.f;
-    if constexpr (SPLIT) {
-        // a chunk's `steps` (a multiple of 4) in unrolled groups of 4: a loop
-        // of DPP steps with a run-time trip count is not unrolled otherwise
-        for (int t = 0; t < steps; t += 4)
-#pragma unroll
-            for (int t4 = 0; t4 < 4; ++t4) {
-                SYM_BLOCK_STEP();
-            }
-    } else {
-#pragma unroll 4
-        for (int t = 0; t < 64; ++t) {
-            SYM_BLOCK_STEP();
-        }
+        for (int c = 0; c < 3; ++c)
+            L.g[c][lane] = L.g[c][lane + 64] = 0.f;
     }
+    wave_lds_fence();
+    const float4* sp = &L.s[lane + t0];
+    float* gp = &L.g[0][lane + t0];
+    float4 cur = *sp;
+#pragma unroll 4
+    for (int t = 0; t < steps; ++t) {
+        const float4 nxt = sp[t + 1];  // the next step's source: at most L.s[127]
+        float gx = 0.f, gy = 0.f, gz = 0.f;
+        if constexpr (N2 > 0) {
+            gx = gp[t]; gy = gp[128 + t]; gz = gp[256 + t];
+        }
+        constexpr int GK = N < 4 ? N : 4;  // pairs per group of reciprocal roots
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
+        for (int k0 = 0; k0 < N; k0 += GK) {
+            float rx[GK], ry[GK], rz[GK], d2[GK], y[GK];
+#pragma unroll
+            for (int q = 0; q < GK; ++q) {
+                const int k = k0 + q;
+                rx[q] = cur.x - xi[k]; ry[q] = cur.y - yi[k]; rz[q] = cur.z - zi[k];
+                d2[q] = __builtin_fmaf(rx[q], rx[q], __builtin_fmaf(ry[q], ry[q], __builtin_fmaf(rz[q], rz[q], eps2)));
+            }
+            rsq_group<GK>(d2, y);
+#pragma unroll
+            for (int q = 0; q < GK; ++q) {
+                const int k = k0 + q;
+                const float y3 = pair_scale<NEWTON>(d2[q], y[q], 1.0f);
+                const float si = UNI ? y3 : cur.w * y3;
+                px[k] = __builtin_fmaf(rx[q], si, px[k]);
+                py[k] = __builtin_fmaf(ry[q], si, py[k]);
+                pz[k] = __builtin_fmaf(rz[q], si, pz[k]);
+                if (k < N2) {
+                    const float cj = UNI ? y3 : mi[k] * y3;
+                    gx = __builtin_fmaf(-rx[q], cj, gx);
+                    gy = __builtin_fmaf(-ry[q], cj, gy);
+                    gz = __builtin_fmaf(-rz[q], cj, gz);
+                }
+            }
+        }
+        if constexpr (N2 > 0) {
+            gp[t] = gx; gp[128 + t] = gy; gp[256 + t] = gz;
+        }
+        wave_lds_fence();
+        cur = nxt;
+    }
+    if constexpr (N2 > 0) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            g[c] = L.g[c][lane] + L.g[c][lane + 64];
+    }
+}
+
+// sym_rotate with the block's target-side partials added into (a, c) by
+// block_add<COMP> and everything scaled by the mass m (UNI).
+template <int K, int N, int N2, bool NEWTON, bool COMP, bool UNI>
+__device__ __forceinline__ void sym_block(SymLds& L, int lane, int t0, int steps, float4 s, const float (&xi)[K],
+                                          const float (&yi)[K], const float (&zi)[K], const float (&mi)[K], float m,
+                                          float eps2, float (&ax)[K], float (&ay)[K], float (&az)[K], float (&cx)[K],
+                                          float (&cy)[K], float (&cz)[K], float (&g)[3])
+{
+    float px[N], py[N], pz[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        px[k] = py[k] = pz[k] = 0.f;
+    sym_rotate<K, N, N2, NEWTON, UNI>(L, lane, t0, steps, s, xi, yi, zi, mi, eps2, px, py, pz, g);
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
         if constexpr (UNI) {
             px[k] *= m; py[k] *= m; pz[k] *= m;
         }
@@ -133,118 +174,43 @@ __device__ __forceinline__ void sym_block(float4 s, const float (&xi)[K], const 
         block_add<COMP>(ay[k], cy[k], py[k]);
         block_add<COMP>(az[k], cz[k], pz[k]);
     }
-    if constexpr (UNI) {
-        gx *= m; gy *= m; gz *= m;
+    if constexpr (UNI && N2 > 0) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            g[c] *= m;
     }
 }
-
-// One rotation step of sym_own.
-#define SYM_OWN_STEP()                                                                                 \
-    _Pragma("unroll")                                                                                  \
-    for (int k = 0; k < KB; ++k) {                                                                     \
-        const float rx = sx - xi[k], ry = sy - yi[k], rz = sz - zi[k];                                 \
-        const float d2 = __builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, __builtin_fmaf(rz, rz, eps2))); \
-        const float y3 = pair_scale<NEWTON>(d2, 1.0f);                                                 \
-        const float si = UNI ? y3 : sm * y3;                                                           \
-        const float cj = UNI ? y3 : mi[k] * y3;                                                        \
-        px[k] = __builtin_fmaf(rx, si, px[k]);                                                         \
-        py[k] = __builtin_fmaf(ry, si, py[k]);                                                         \
-        pz[k] = __builtin_fmaf(rz, si, pz[k]);                                                         \
-        gx = __builtin_fmaf(-rx, cj, gx);                                                              \
-        gy = __builtin_fmaf(-ry, cj, gy);                                                              \
-        gz = __builtin_fmaf(-rz, cj, gz);                                                              \
-    }                                                                                                  \
-    {                                                                                                  \
-        const float rx = sx - xi[KB], ry = sy - yi[KB], rz = sz - zi[KB];                              \
-        const float d2 = __builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, __builtin_fmaf(rz, rz, eps2))); \
-        const float si = pair_scale<NEWTON>(d2, UNI ? 1.0f : sm);                                      \
-        px[KB] = __builtin_fmaf(rx, si, px[KB]);                                                       \
-        py[KB] = __builtin_fmaf(ry, si, py[KB]);                                                       \
-        pz[KB] = __builtin_fmaf(rz, si, pz[KB]);                                                       \
-    }                                                                                                  \
-    sx = wave_ror1<K>(sx); sy = wave_ror1<K>(sy); sz = wave_ror1<K>(sz);                               \
-    if constexpr (!UNI)                                                                                \
-        sm = wave_ror1<K>(sm);                                                                         \
-    if constexpr (KB > 0) {                                                                            \
-        gx = wave_ror1<K>(gx); gy = wave_ror1<K>(gy); gz = wave_ror1<K>(gz);                           \
-    }
 
 // Own source block KB of the wave's block (K <= 4): target slots k < KB meet
 // it two-sided (the pairs of blocks k and KB, each unordered pair once), slot
 // KB one-sided (the block with itself: each ordered pair once, the self pair
 // adds r = 0); slots k > KB take these sources when their own block is the
-// source.  The reaction sums come home to slot KB after 64 rotations.  UNI as
-// in sym_block.  SPLIT: a chunk of `steps` rotation steps that ends `rot`
-// lanes short of home (lane l then holds the reactions of lane l - rot's
-// body); the sums are moved home by a lane shuffle.
-template <int K, bool NEWTON, bool COMP, bool UNI, int KB, bool SPLIT = false>
-__device__ __forceinline__ void sym_own(float4 s, const float (&xi)[K], const float (&yi)[K],
-                                        const float (&zi)[K], const float (&mi)[K], float m, float eps2,
-                                        float (&ax)[K], float (&ay)[K], float (&az)[K], float (&cx)[K],
-                                        float (&cy)[K], float (&cz)[K], int steps = 64, int rot = 0,
-                                        int lane = 0)
-{
-    float sx = s.x, sy = s.y, sz = s.z, sm = s.w;
-    float px[KB + 1], py[KB + 1], pz[KB + 1];
-#pragma unroll
-    for (int k = 0; k <= KB; ++k)
-        px[k] = py[k] = pz[k] = 0.f;
-    float gx = 0.f, gy = 0.f, gz = 0.f;
-    if constexpr (SPLIT) {
-        for (int t = 0; t < steps; t += 4)  // in unrolled groups of 4, as in sym_block
-#pragma unroll
-            for (int t4 = 0; t4 < 4; ++t4) {
-                SYM_OWN_STEP();
-            }
-    } else {
-#pragma unroll 4
-        for (int t = 0; t < 64; ++t) {
-            SYM_OWN_STEP();
-        }
-    }
-#pragma unroll
-    for (int k = 0; k <= KB; ++k) {
-        if constexpr (UNI) {
-            px[k] *= m; py[k] *= m; pz[k] *= m;
-        }
-        block_add<COMP>(ax[k], cx[k], px[k]);
-        block_add<COMP>(ay[k], cy[k], py[k]);
-        block_add<COMP>(az[k], cz[k], pz[k]);
-    }
-    if constexpr (KB > 0) {
-        if constexpr (SPLIT) {
-            if (rot != 0) {  // wave-uniform
-                const int from = (lane + rot) & 63;
-                gx = __shfl(gx, from, 64); gy = __shfl(gy, from, 64); gz = __shfl(gz, from, 64);
-            }
-        }
-        if constexpr (UNI) {
-            gx *= m; gy *= m; gz *= m;
-        }
-        block_add<COMP>(ax[KB], cx[KB], gx);
-        block_add<COMP>(ay[KB], cy[KB], gy);
-        block_add<COMP>(az[KB], cz[KB], gz);
-    }
-}
-
-// sym_own for the wave-uniform block index kb, 0 <= kb < K.
-template <int K, bool NEWTON, bool COMP, bool SPLIT = false, int KB = 0>
-__device__ __forceinline__ void sym_own_at(int kb, bool uni, float4 s, const float (&xi)[K], const float (&yi)[K],
-                                           const float (&zi)[K], const float (&mi)[K], float m, float eps2,
-                                           float (&ax)[K], float (&ay)[K], float (&az)[K], float (&cx)[K],
-                                           float (&cy)[K], float (&cz)[K], int steps = 64, int rot = 0,
-                                           int lane = 0)
+// source.  The reaction sums belong to slot KB.
+template <int K, bool NEWTON, bool COMP, int KB = 0>
+__device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane, int t0, int steps, float4 s,
+                                           const float (&xi)[K], const float (&yi)[K], const float (&zi)[K],
+                                           const float (&mi)[K], float m, float eps2, float (&ax)[K], float (&ay)[K],
+                                           float (&az)[K], float (&cx)[K], float (&cy)[K], float (&cz)[K])
 {
     if (kb == KB) {
+        float g[3];
         if (uni)
-            sym_own<K, NEWTON, COMP, true, KB, SPLIT>(s, xi, yi, zi, mi, m, eps2, ax, ay, az, cx, cy, cz, steps,
-                                                      rot, lane);
+            sym_block<K, KB + 1, KB, NEWTON, COMP, true>(L, lane, t0, steps, s, xi, yi, zi, mi, m, eps2, ax, ay, az,
+                                                         cx, cy, cz, g);
         else
-            sym_own<K, NEWTON, COMP, false, KB, SPLIT>(s, xi, yi, zi, mi, m, eps2, ax, ay, az, cx, cy, cz, steps,
-                                                       rot, lane);
+            sym_block<K, KB + 1, KB, NEWTON, COMP, false>(L, lane, t0, steps, s, xi, yi, zi, mi, m, eps2, ax, ay, az,
+                                                          cx, cy, cz, g);
+        if constexpr (KB > 0) {
+            block_add<COMP>(ax[KB], cx[KB], g[0]);
+            block_add<COMP>(ay[KB], cy[KB], g[1]);
+            block_add<COMP>(az[KB], cz[KB], g[2]);
+            // keeps the compiler from merging the K branches' adds into one
+            // through a pointer to slot KB, which would put the sums in memory
+            asm volatile("; own block %0" : : "n"(KB));
+        }
     } else if constexpr (KB + 1 < K) {
-        sym_own_at<K, NEWTON, COMP, SPLIT, KB + 1>(kb, uni, s, xi, yi, zi, mi, m, eps2, ax, ay, az, cx, cy, cz,
-                                                   steps, rot, lane);
+        sym_own_at<K, NEWTON, COMP, KB + 1>(kb, uni, L, lane, t0, steps, s, xi, yi, zi, mi, m, eps2, ax, ay, az, cx,
+                                            cy, cz);
     }
 }
 
@@ -261,7 +227,7 @@ __device__ __forceinline__ void sym_own_at(int kb, bool uni, float4 s, const flo
 template <int K, bool NEWTON, bool COMP, bool SPLIT = false>
 __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW, int R, int w, int r,
                                          float eps2, float* __restrict__ ipart,
-                                         float* __restrict__ jpart, int lane, int jbase = 0,
+                                         float* __restrict__ jpart, SymLds& L, int lane, int jbase = 0,
                                          long long istride = -1, int ibody0 = 0, int rs = 1)
 {
     const int half = NW / 2;
@@ -292,54 +258,23 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
             c = qs - q * rs;
         }
         const int u = q / K, kb = q - u * K;
-        // chunk c runs rotation steps [t0, t0 + steps): lane l starts with
-        // source (l - t0) mod 64 and ends holding source (l - t0 - steps) mod 64
-        const int t0 = c * steps;
-        const int sl = SPLIT ? ((lane - t0) & 63) : lane;
-        const int el = SPLIT ? ((lane - t0 - steps) & 63) : lane;
-        if constexpr (K <= 4) {
-            if (u == 0) {
+        const int t0 = c * steps;  // chunk c: rotation steps [t0, t0 + steps)
+        if (u == 0) {
+            const float4 s = src[w * 64 * K + kb * 64 + lane];
+            const bool uni = __ballot(tuni && s.w == m0) == ~0ull;
+            if constexpr (K <= 4) {
                 // own block kb: two-sided against the lower target slots
-                const float4 s = src[w * 64 * K + kb * 64 + sl];
-                const bool uni = __ballot(tuni && s.w == m0) == ~0ull;
-                sym_own_at<K, NEWTON, COMP, SPLIT>(kb, uni, s, xi, yi, zi, mi, m0, eps2, ax, ay, az, cx, cy, cz,
-                                                   steps, (t0 + steps) & 63, lane);
-                continue;
-            }
-        }
-        if constexpr (K > 4) {
-            if (u == 0) {
+                sym_own_at<K, NEWTON, COMP>(kb, uni, L, lane, t0, steps, s, xi, yi, zi, mi, m0, eps2, ax, ay, az, cx,
+                                            cy, cz);
+            } else {
                 // own block kb (K = 8, where own blocks are a small share and
-                // eight variants of sym_own would crowd the instruction cache):
+                // eight variants of sym_own_at would crowd the instruction cache):
                 // target side only (each ordered pair once, self pair gives 0)
-                static_assert(!SPLIT, "rotation chunks need K <= 4");
-                const float4 s = src[w * 64 * K + kb * 64 + lane];
-                float sx = s.x, sy = s.y, sz = s.z, sm = s.w;
-                float px[K], py[K], pz[K];
-#pragma unroll
-                for (int k = 0; k < K; ++k)
-                    px[k] = py[k] = pz[k] = 0.f;
-#pragma unroll 4
-                for (int t = 0; t < 64; ++t) {
-#pragma unroll
-                    for (int k = 0; k < K; ++k) {
-                        const float rx = sx - xi[k], ry = sy - yi[k], rz = sz - zi[k];
-                        const float d2 = __builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, __builtin_fmaf(rz, rz, eps2)));
-                        const float si = pair_scale<NEWTON>(d2, sm);
-                        px[k] = __builtin_fmaf(rx, si, px[k]);
-                        py[k] = __builtin_fmaf(ry, si, py[k]);
-                        pz[k] = __builtin_fmaf(rz, si, pz[k]);
-                    }
-                    sx = wave_ror1<K>(sx); sy = wave_ror1<K>(sy); sz = wave_ror1<K>(sz); sm = wave_ror1<K>(sm);
-                }
-#pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    block_add<COMP>(ax[k], cx[k], px[k]);
-                    block_add<COMP>(ay[k], cy[k], py[k]);
-                    block_add<COMP>(az[k], cz[k], pz[k]);
-                }
-                continue;
+                float g[3];
+                sym_block<K, K, 0, NEWTON, COMP, false>(L, lane, t0, steps, s, xi, yi, zi, mi, m0, eps2, ax, ay, az,
+                                                        cx, cy, cz, g);
             }
+            continue;
         }
         const int d = u - 1;
         if (2 * (d + 1) == NW && w >= half)
@@ -347,18 +282,18 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
         int v = w + 1 + d;
         if (v >= NW)
             v -= NW;
-        const float4 s = src[v * 64 * K + kb * 64 + sl];
-        float gx, gy, gz;
+        const float4 s = src[v * 64 * K + kb * 64 + lane];
+        float g[3];
         if (__ballot(tuni && s.w == m0) == ~0ull)
-            sym_block<K, NEWTON, COMP, true, SPLIT>(s, xi, yi, zi, mi, m0, eps2, ax, ay, az, cx, cy, cz, gx, gy, gz,
-                                                    steps);
+            sym_block<K, K, K, NEWTON, COMP, true>(L, lane, t0, steps, s, xi, yi, zi, mi, m0, eps2, ax, ay, az, cx,
+                                                   cy, cz, g);
         else
-            sym_block<K, NEWTON, COMP, false, SPLIT>(s, xi, yi, zi, mi, m0, eps2, ax, ay, az, cx, cy, cz, gx, gy,
-                                                     gz, steps);
-        const size_t o = ((((size_t)(w - jbase) * half + d) * (SPLIT ? rs : 1) + c) * (64 * K) + kb * 64 + el) * 3;
-        jpart[o + 0] = gx;
-        jpart[o + 1] = gy;
-        jpart[o + 2] = gz;
+            sym_block<K, K, K, NEWTON, COMP, false>(L, lane, t0, steps, s, xi, yi, zi, mi, m0, eps2, ax, ay, az, cx,
+                                                    cy, cz, g);
+        const size_t o = ((((size_t)(w - jbase) * half + d) * (SPLIT ? rs : 1) + c) * (64 * K) + kb * 64 + lane) * 3;
+        jpart[o + 0] = g[0];
+        jpart[o + 1] = g[1];
+        jpart[o + 2] = g[2];
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -372,15 +307,16 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
 
 // One system: wave gw = w * R + r.  SPLIT: rs rotation chunks per sub-unit.
 template <int K, bool NEWTON, bool COMP, bool SPLIT>
-__global__ __launch_bounds__(256) void sym_force_kernel(const float4* __restrict__ src, int NW, int R,
+__global__ __launch_bounds__(256, 2) void sym_force_kernel(const float4* __restrict__ src, int NW, int R,
                                                         float eps2, float* __restrict__ ipart,
                                                         float* __restrict__ jpart, int rs)
 {
+    __shared__ SymLds lds[4];
     const int gw = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     if (gw >= NW * R)
         return;  // whole waves only
-    sym_wave<K, NEWTON, COMP, SPLIT>(src, NW, R, gw / R, gw % R, eps2, ipart, jpart, threadIdx.x & 63, 0, -1, 0,
-                                     rs);
+    sym_wave<K, NEWTON, COMP, SPLIT>(src, NW, R, gw / R, gw % R, eps2, ipart, jpart, lds[threadIdx.x >> 6],
+                                     threadIdx.x & 63, 0, -1, 0, rs);
 }
 
 // Batched systems: each wave runs items (system, wave block, split), a system
@@ -390,6 +326,7 @@ __global__ __launch_bounds__(256) void batch_sym_kernel(BatchSymGeom g, int nwav
                                                         float eps2, float* __restrict__ ipart,
                                                         float* __restrict__ jpart)
 {
+    __shared__ SymLds lds[4];
     const int gw = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     if (gw >= nwaves)
         return;  // whole waves only
@@ -399,7 +336,7 @@ __global__ __launch_bounds__(256) void batch_sym_kernel(BatchSymGeom g, int nwav
         const int4 item = g.items[it];  // (system, wave block, split, splits)
         const int s = item.x;
         sym_wave<K, false, true>(snap + g.off[s], g.nw[s], item.w, item.y, item.z, eps2, ipart + g.ipo[s],
-                           jpart + g.jpo[s], lane);
+                           jpart + g.jpo[s], lds[threadIdx.x >> 6], lane);
     }
 }
 
@@ -577,11 +514,12 @@ __global__ __launch_bounds__(256) void sym_share_kernel(const float4* __restrict
                                                         float* __restrict__ jpart, int jbase, long long istride,
                                                         int ibody0)
 {
+    __shared__ SymLds lds[4];
     const int gw = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     if (gw >= nwaves)
         return;  // whole waves only
-    sym_wave<K, NEWTON, true>(src, NW, R, w0 + gw / R, gw % R, eps2, ipart, jpart, threadIdx.x & 63, jbase,
-                              istride, ibody0);
+    sym_wave<K, NEWTON, true>(src, NW, R, w0 + gw / R, gw % R, eps2, ipart, jpart, lds[threadIdx.x >> 6],
+                              threadIdx.x & 63, jbase, istride, ibody0);
 }
 
 // react3[b] (FP64, bodies b < n) = the reactions on body b from the wave
