@@ -36,29 +36,28 @@ int tile_count() { return (int)(sizeof(kTiles) / sizeof(kTiles[0])); }
 const Tile& tile_get(int id) { return kTiles[id]; }
 
 // Default tile, from sweeps of every tile on MI355X (mixed precision, time per
-// step, best three; Plummer spheres, equal masses; log-uniform masses rank
+// step, best three; equal masses; log-uniform masses and plain FP32 rank
 // alike):
-//   N = 262144: sym8r64 12.29, sym8r48 12.34, sym8r32 12.34 ms  (k2s8, one-pass: 20.7)
-//   N = 131072: sym8r48 3.139, sym8r64 3.143, sym8r32 3.160 ms
-//   N =  65536: sym8r64 0.830, sym8r48 0.830, sym8r32 0.871 ms
-//   N =  32768: sym8r64 0.235, sym8r48 0.239, sym8r32 0.240 ms
-//   N =  24576: sym8r64 148.0, sym4r32 150.9, sym4r64 152.5 us
-//   N =  16384: sym4r64x2 75.9, sym4r64 77.5, sym4r128x2 79.3 us
-//   N =  12288: sym2r32 51.8, sym4r64x2 51.8, sym4r128x2 52.4 us
-//   N =   8192: sm2t16w16n8k 28.4, sm1t16w16n8k 29.0, sm4t8w16n8k 29.5 us  (sym2r32 29.7)
-//   N =   6144: sm2t16w16n8k 21.4, sm1t8w16n8k 21.8, sm1t16w16n8k 22.4 us  (sym2r64x2 23.2)
-//   N =   4096: sm1t16w16n4k 9.57, sm1t16w16n8k 9.59, sm2t8w16n8k 10.2 us  (sym2r32 16.0)
-//   N =   3072: sm1t16w16n4k 7.88, sm1t16w16n8k 7.91, sm2t8w16n8k 8.42 us  (sym2r32 12.1)
-//   N =   2048: sm1t8w16n8k 5.11, sm1t8w16n4k 5.44, sm1t8w8n2k 5.48 us  (sym2r32 10.9)
-//   N =   1024: sm1t4w8n2k 3.94, sm1t8w8n2k 4.01, sm1t8w16n8k 4.17 us  (k1s16 10.1)
-// (sym8r48, sym8r24 and several other small-system shapes were swept and
-// are not in the table.)  Up to 8192 bodies the small-system kernels win:
+//   N = 131072: sym8r64 2.660, sym8r32 2.686, sym8r128 2.714 ms  (sym4r64 2.778)
+//   N =  65536: sym8r64 0.710, sym4r64 0.725, sym4r32 0.726 ms
+//   N =  32768: sym4r64 205.8, sym4r32 205.9, sym8r32 206.4 us   (sym8r64 211.7)
+//   N =  24576: sym4r64 126.8, sym4r32 127.9, sym8r64 129.5 us
+//   N =  16384: sym4r64 65.6, sym4r32 67.5, sym4r64x2 68.3 us    (sym8r128 76)
+//   N =  12288: sym4r64 43.7, sym4r128 43.9, sym2r64 45.1 us
+//   N =   8192: sm2t16w16n8k 23.3, sm1t16w16n8k 26.4, sym4r128 27.9 us
+//   N =   6144: sm2t16w16n8k 18.3, sym2r64 20.7, sm1t8w16n8k 20.7 us
+//   N =   4096: sm1t16w16n8k 8.80, sm1t16w16n4k 8.84, sm1t8w16n8k 11.3 us  (sym2r64 16.4)
+//   N =   2048: sm1t8w16n8k 5.12, sm1t8w8n2k 5.16, sm1t4w8n2k 5.67 us  (sym2r64x2 12.5)
+//   N =   1024: sm1t4w8n2k 4.04, sm1t8w8n2k 4.10, sm1t8w16n8k 4.15 us  (sym2r128x4 12.1)
+// (sym8r48, sym8r24 and several other small-system shapes were swept earlier
+// and are not in the table.)  Up to 8192 bodies the small-system kernels win:
 // one launch per step against two, and their one-pass pair sums fill the
 // chip where the symmetric kernels' 64-step rotations leave it waiting.  The
-// symmetric tiles need enough wave blocks to fill the chip (K = 8 from 96
-// bodies per CU, K = 4 from 64), and their partial sums must fit the
-// device's budget (sym_partial_budget); above it the best one-pass tile
-// (k2s8) is used.
+// symmetric tiles need enough wave blocks to fill the chip: K = 4 above 8192
+// bodies, K = 8, which has the less LDS traffic and reaction partials per
+// pair, from 160 bodies per CU.  Their partial sums must fit the device's
+// budget (sym_partial_budget; K = 8 needs half the reaction partials of K =
+// 4); above it the best one-pass tile (k2s8) is used.
 size_t sym_partial_budget(size_t device_bytes)
 {
     if (device_bytes == 0)
@@ -84,10 +83,12 @@ int tile_default(int64_t n, int cu_count, size_t partial_budget)
         return 31;  // sm1t16w16n4k
     if (n <= 8192)
         return 33;  // sm2t16w16n8k
-    if (n >= 96 * cus && fits(8))
+    if (n >= 160 * cus && fits(8))
         return 22;  // sym8r64
-    if (n >= 64 * cus && fits(4))
-        return 25;  // sym4r64x2
+    if (n >= 8 * cus && fits(4))
+        return 18;  // sym4r64
+    if (n >= 96 * cus && fits(8))
+        return 22;
     if (n >= 8 * cus && fits(2))
         return 20;  // sym2r32
     if ((n + 127) / 128 * 8 >= cus * 16)
