@@ -8,15 +8,23 @@
 // so both bodies' terms come from one evaluation.  Written as
 // J w = y^3 (w - 3 y^2 (r.w) r) with r.w = m_i (a_j.r) - m_j (a_i.r), reusing
 // the two dot products the mass terms need, an unordered pair costs 36 VALU
-// slots (3 sub, 3 fma for d^2, rsq, 2 mul for y^2 and y^3, 6 for the two dot
+// instructions (3 sub, 3 fma for d^2, 2 mul for y^2 and y^3, 6 for the two dot
 // products, 2 for r.w, 2 mul for -3 y^2 r.w, 6 for w, 3 fma for the bracket,
-// 6 fma for the two position terms, 2 fma for the two mass terms) against 31
-// per ordered pair in the one-pass VJP, plus 11 DPP moves per 64-source
-// rotation step shared by the K targets of a lane.  When the targets of the
+// 6 fma for the two position terms, 2 fma for the two mass terms) and a root,
+// against 31 per ordered pair in the one-pass VJP.  When the targets of the
 // wave and the sources of a block all have one mass m, w = m (alpha_j -
 // alpha_i) and r.w = m (a_j.r - a_i.r): the pair works with the differences
-// alone and the block's position partials are scaled by m once (31 slots, 10
-// DPP moves).
+// alone and the block's position partials are scaled by m once (31).
+//
+// As in the force kernel a source block and its reaction sums rotate through
+// the wave's LDS and the roots of a step's 4 pairs are taken together.  FP32
+// issue bounds it: per VJP step (pair sum, reduction and the adjoint's
+// per-body work), same device, N = 65536 1.59 ms (2.09 with the block carried
+// round the wave in 10 DPP moves per step and one root at a time), N = 16384
+// with log-uniform masses 162 us (200); 96 systems of 256 to 8192 bodies, 20
+// steps forward and adjoint 16.7 ms (20.9).  Roots 2 at a time, an unroll of 4
+// and 128 VGPRs (four waves per SIMD, for 143 and three) are the same within
+// 1%; without unrolling it is 8% slower at N = 65536.
 //
 // The mapping is the symmetric force kernel's (sym.hip): wave blocks of 64*K
 // bodies, unit 0 = own blocks (source block kb two-sided against target slots
@@ -26,6 +34,7 @@
 // Partials go to HBM (float4 per body: x, y, z, m) and a second kernel adds
 // them per body in FP64, in a fixed order, into xbar and mbar.
 #include "internal.h"
+#include "rsq_group.h"
 #include "sym_items.h"
 #include "sym_reduce.h"
 #include "vjp_pair.h"
@@ -33,17 +42,6 @@
 namespace utcnb {
 
 namespace {
-
-// Lane l receives lane l-1's value (lane 0 lane 63's).  Every lane has a
-// source under wave_ror:1, so the "old" operand is never used; passing v lets
-// the compiler rotate in place, without a v_mov that first zeroes a new
-// register: 8% faster VJP steps at N = 262144 on MI355X than "old" = 0 (a
-// same-device A/B; the force kernel measured the other way, see sym.hip).
-__device__ __forceinline__ float ror1(float v)
-{
-    const int x = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(x, x, 0x13C /* wave_ror:1 */, 0xF, 0xF, false));
-}
 
 __device__ __forceinline__ void kahan1(float& s, float& c, float p)
 {
@@ -55,151 +53,113 @@ __device__ __forceinline__ void kahan1(float& s, float& c, float p)
 
 }  // namespace
 
-// A block of 64 sources (one per lane: position/mass sp, alpha sa) against
-// the K targets of each lane, both sides: the target-side block partials are
-// Kahan-added into (g, c); h receives the source's reaction sums after 64
-// rotations.  UNI: every target mass mi[k] and source mass equals m.
-template <int K, bool UNI>
-__device__ __forceinline__ void sym_vjp_block(float4 sp, float4 sa, const float (&xi)[K], const float (&yi)[K],
-                                              const float (&zi)[K], const float (&mi)[K], const float (&bx)[K],
-                                              const float (&by)[K], const float (&bz)[K], float m, float eps2,
-                                              float (&g)[K][4], float (&c)[K][4], float4& h)
+// A wave's source block and its reaction sums in LDS (wave private), as in
+// sym.hip: source s in slots s and s + 64.
+struct SymVjpLds {
+    float4 p[128], a[128];
+    float h[4][128];
+};
+
+__device__ __forceinline__ void vjp_lds_fence()
 {
-    float sx = sp.x, sy = sp.y, sz = sp.z, sm = sp.w, ax = sa.x, ay = sa.y, az = sa.z;
-    float hx = 0.f, hy = 0.f, hz = 0.f, hm = 0.f;  // reaction on the source body
-    float p[K][4];
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-        p[k][0] = p[k][1] = p[k][2] = p[k][3] = 0.f;
-#pragma unroll 2
-    for (int t = 0; t < 64; ++t) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const float rx = sx - xi[k], ry = sy - yi[k], rz = sz - zi[k];
-            const float d2 = __builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, __builtin_fmaf(rz, rz, eps2)));
-            const float y = __builtin_amdgcn_rsqf(d2);
-            const float y2 = y * y, y3 = y2 * y;
-            // J w = y^3 (w - 3 y^2 (r.w) r), r.w = m_i (a_j.r) - m_j (a_i.r)
-            const float arj = __builtin_fmaf(ax, rx, __builtin_fmaf(ay, ry, az * rz));
-            const float ari = __builtin_fmaf(bx[k], rx, __builtin_fmaf(by[k], ry, bz[k] * rz));
-            float s3, wx, wy, wz;
-            if constexpr (UNI) {  // w / m and r.w / m
-                s3 = (-3.f * y2) * (arj - ari);
-                wx = ax - bx[k]; wy = ay - by[k]; wz = az - bz[k];
-            } else {
-                s3 = (-3.f * y2) * __builtin_fmaf(mi[k], arj, -(sm * ari));
-                wx = w_fast(mi[k], ax, sm, bx[k]);
-                wy = w_fast(mi[k], ay, sm, by[k]);
-                wz = w_fast(mi[k], az, sm, bz[k]);
-            }
-            const float tx = __builtin_fmaf(s3, rx, wx);
-            const float ty = __builtin_fmaf(s3, ry, wy);
-            const float tz = __builtin_fmaf(s3, rz, wz);
-            p[k][0] = __builtin_fmaf(y3, tx, p[k][0]);
-            p[k][1] = __builtin_fmaf(y3, ty, p[k][1]);
-            p[k][2] = __builtin_fmaf(y3, tz, p[k][2]);
-            hx = __builtin_fmaf(-y3, tx, hx);
-            hy = __builtin_fmaf(-y3, ty, hy);
-            hz = __builtin_fmaf(-y3, tz, hz);
-            p[k][3] = __builtin_fmaf(-y3, arj, p[k][3]);
-            hm = __builtin_fmaf(y3, ari, hm);
-        }
-        sx = ror1(sx); sy = ror1(sy); sz = ror1(sz);
-        if constexpr (!UNI)
-            sm = ror1(sm);
-        ax = ror1(ax); ay = ror1(ay); az = ror1(az);
-        hx = ror1(hx); hy = ror1(hy); hz = ror1(hz); hm = ror1(hm);
-    }
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        if constexpr (UNI) {
-            p[k][0] *= m; p[k][1] *= m; p[k][2] *= m;
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            kahan1(g[k][q], c[k][q], p[k][q]);
-    }
-    if constexpr (UNI) {
-        hx *= m; hy *= m; hz *= m;
-    }
-    h = make_float4(hx, hy, hz, hm);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-// Own source block KB of the wave's block: target slots k < KB meet it
-// two-sided (as sym_vjp_block; no self pairs), slot KB one-sided (the block
-// with itself, self pairs included, so w is exact: vjp_pair.h); slots k > KB
-// take these sources when their own block is the source.  The reaction sums
-// come home to slot KB after 64 rotations.  UNI applies to the two-sided
-// pairs.
-template <int K, bool UNI, int KB>
-__device__ __forceinline__ void sym_vjp_own(float4 sp, float4 sa, const float (&xi)[K], const float (&yi)[K],
-                                            const float (&zi)[K], const float (&mi)[K], const float (&bx)[K],
-                                            const float (&by)[K], const float (&bz)[K], float m, float eps2,
-                                            float (&g)[K][4], float (&c)[K][4])
+// A block of 64 sources (lane l's source: position/mass sp, alpha sa; wave
+// private LDS L) against target slots 0 .. N-1 of each lane: at step t lane l
+// meets source (l + t) mod 64.  Slots k < N2 are two-sided; slot N2 < N is the
+// block with itself (self pairs included, so w is exact: vjp_pair.h), target
+// side only.  The target-side block partials are Kahan-added into (g, c); the
+// reaction sums of lane l's own source come back in h (N2 > 0).
+// UNI: every target mass mi[k] and source mass equals m (two-sided slots).
+template <int K, int N, int N2, bool UNI>
+__device__ __forceinline__ void sym_vjp_block(SymVjpLds& L, int lane, float4 sp, float4 sa, const float (&xi)[K],
+                                              const float (&yi)[K], const float (&zi)[K], const float (&mi)[K],
+                                              const float (&bx)[K], const float (&by)[K], const float (&bz)[K],
+                                              float m, float eps2, float (&g)[K][4], float (&c)[K][4], float4& h)
 {
-    float sx = sp.x, sy = sp.y, sz = sp.z, sm = sp.w, ax = sa.x, ay = sa.y, az = sa.z;
-    float hx = 0.f, hy = 0.f, hz = 0.f, hm = 0.f;  // reaction on the source body
-    float p[KB + 1][4];
+    float p[N][4];
 #pragma unroll
-    for (int k = 0; k <= KB; ++k)
+    for (int k = 0; k < N; ++k)
         p[k][0] = p[k][1] = p[k][2] = p[k][3] = 0.f;
+    vjp_lds_fence();
+    L.p[lane] = L.p[lane + 64] = sp;
+    L.a[lane] = L.a[lane + 64] = sa;
+    if constexpr (N2 > 0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            L.h[q][lane] = L.h[q][lane + 64] = 0.f;
+    }
+    vjp_lds_fence();
+    const float4* pp = &L.p[lane];
+    const float4* pa = &L.a[lane];
+    float* ph = &L.h[0][lane];
+    float4 cp = *pp, ca = *pa;
 #pragma unroll 2
     for (int t = 0; t < 64; ++t) {
+        const float4 np = pp[t + 1], na = pa[t + 1];  // the next step's source: at most slot 127
+        float hx = 0.f, hy = 0.f, hz = 0.f, hm = 0.f;
+        if constexpr (N2 > 0) {
+            hx = ph[t]; hy = ph[128 + t]; hz = ph[256 + t]; hm = ph[384 + t];
+        }
+        float rx[N], ry[N], rz[N], d2[N], yy[N];
 #pragma unroll
-        for (int k = 0; k < KB; ++k) {
-            const float rx = sx - xi[k], ry = sy - yi[k], rz = sz - zi[k];
-            const float d2 = __builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, __builtin_fmaf(rz, rz, eps2)));
-            const float y = __builtin_amdgcn_rsqf(d2);
-            const float y2 = y * y, y3 = y2 * y;
-            const float arj = __builtin_fmaf(ax, rx, __builtin_fmaf(ay, ry, az * rz));
-            const float ari = __builtin_fmaf(bx[k], rx, __builtin_fmaf(by[k], ry, bz[k] * rz));
-            float s3, wx, wy, wz;
-            if constexpr (UNI) {
-                s3 = (-3.f * y2) * (arj - ari);
-                wx = ax - bx[k]; wy = ay - by[k]; wz = az - bz[k];
+        for (int k = 0; k < N; ++k) {
+            rx[k] = cp.x - xi[k]; ry[k] = cp.y - yi[k]; rz[k] = cp.z - zi[k];
+            d2[k] = __builtin_fmaf(rx[k], rx[k], __builtin_fmaf(ry[k], ry[k], __builtin_fmaf(rz[k], rz[k], eps2)));
+        }
+        rsq_group<N>(d2, yy);
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const float y = yy[k], y2 = y * y, y3 = y2 * y;
+            const float arj = __builtin_fmaf(ca.x, rx[k], __builtin_fmaf(ca.y, ry[k], ca.z * rz[k]));
+            if (k < N2) {
+                // J w = y^3 (w - 3 y^2 (r.w) r), r.w = m_i (a_j.r) - m_j (a_i.r)
+                const float ari = __builtin_fmaf(bx[k], rx[k], __builtin_fmaf(by[k], ry[k], bz[k] * rz[k]));
+                float s3, wx, wy, wz;
+                if constexpr (UNI) {  // w / m and r.w / m
+                    s3 = (-3.f * y2) * (arj - ari);
+                    wx = ca.x - bx[k]; wy = ca.y - by[k]; wz = ca.z - bz[k];
+                } else {
+                    s3 = (-3.f * y2) * __builtin_fmaf(mi[k], arj, -(cp.w * ari));
+                    wx = w_fast(mi[k], ca.x, cp.w, bx[k]);
+                    wy = w_fast(mi[k], ca.y, cp.w, by[k]);
+                    wz = w_fast(mi[k], ca.z, cp.w, bz[k]);
+                }
+                const float tx = __builtin_fmaf(s3, rx[k], wx);
+                const float ty = __builtin_fmaf(s3, ry[k], wy);
+                const float tz = __builtin_fmaf(s3, rz[k], wz);
+                p[k][0] = __builtin_fmaf(y3, tx, p[k][0]);
+                p[k][1] = __builtin_fmaf(y3, ty, p[k][1]);
+                p[k][2] = __builtin_fmaf(y3, tz, p[k][2]);
+                hx = __builtin_fmaf(-y3, tx, hx);
+                hy = __builtin_fmaf(-y3, ty, hy);
+                hz = __builtin_fmaf(-y3, tz, hz);
+                hm = __builtin_fmaf(y3, ari, hm);
             } else {
-                s3 = (-3.f * y2) * __builtin_fmaf(mi[k], arj, -(sm * ari));
-                wx = w_fast(mi[k], ax, sm, bx[k]);
-                wy = w_fast(mi[k], ay, sm, by[k]);
-                wz = w_fast(mi[k], az, sm, bz[k]);
+                const float y5m3 = (-3.f * y2) * y3;
+                const float wx = w_exact(mi[k], ca.x, cp.w, bx[k]);
+                const float wy = w_exact(mi[k], ca.y, cp.w, by[k]);
+                const float wz = w_exact(mi[k], ca.z, cp.w, bz[k]);
+                const float e = y5m3 * __builtin_fmaf(rx[k], wx, __builtin_fmaf(ry[k], wy, rz[k] * wz));
+                p[k][0] = __builtin_fmaf(e, rx[k], __builtin_fmaf(y3, wx, p[k][0]));
+                p[k][1] = __builtin_fmaf(e, ry[k], __builtin_fmaf(y3, wy, p[k][1]));
+                p[k][2] = __builtin_fmaf(e, rz[k], __builtin_fmaf(y3, wz, p[k][2]));
             }
-            const float tx = __builtin_fmaf(s3, rx, wx);
-            const float ty = __builtin_fmaf(s3, ry, wy);
-            const float tz = __builtin_fmaf(s3, rz, wz);
-            p[k][0] = __builtin_fmaf(y3, tx, p[k][0]);
-            p[k][1] = __builtin_fmaf(y3, ty, p[k][1]);
-            p[k][2] = __builtin_fmaf(y3, tz, p[k][2]);
-            hx = __builtin_fmaf(-y3, tx, hx);
-            hy = __builtin_fmaf(-y3, ty, hy);
-            hz = __builtin_fmaf(-y3, tz, hz);
             p[k][3] = __builtin_fmaf(-y3, arj, p[k][3]);
-            hm = __builtin_fmaf(y3, ari, hm);
         }
-        {
-            const float rx = sx - xi[KB], ry = sy - yi[KB], rz = sz - zi[KB];
-            const float d2 = __builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, __builtin_fmaf(rz, rz, eps2)));
-            const float y = __builtin_amdgcn_rsqf(d2);
-            const float y2 = y * y, y3 = y2 * y, y5m3 = (-3.f * y2) * y3;
-            const float wx = w_exact(mi[KB], ax, sm, bx[KB]);
-            const float wy = w_exact(mi[KB], ay, sm, by[KB]);
-            const float wz = w_exact(mi[KB], az, sm, bz[KB]);
-            const float q = y5m3 * __builtin_fmaf(rx, wx, __builtin_fmaf(ry, wy, rz * wz));
-            p[KB][0] = __builtin_fmaf(q, rx, __builtin_fmaf(y3, wx, p[KB][0]));
-            p[KB][1] = __builtin_fmaf(q, ry, __builtin_fmaf(y3, wy, p[KB][1]));
-            p[KB][2] = __builtin_fmaf(q, rz, __builtin_fmaf(y3, wz, p[KB][2]));
-            const float arj = __builtin_fmaf(ax, rx, __builtin_fmaf(ay, ry, az * rz));
-            p[KB][3] = __builtin_fmaf(-y3, arj, p[KB][3]);
+        if constexpr (N2 > 0) {
+            ph[t] = hx; ph[128 + t] = hy; ph[256 + t] = hz; ph[384 + t] = hm;
         }
-        sx = ror1(sx); sy = ror1(sy); sz = ror1(sz); sm = ror1(sm);
-        ax = ror1(ax); ay = ror1(ay); az = ror1(az);
-        if constexpr (KB > 0) {
-            hx = ror1(hx); hy = ror1(hy); hz = ror1(hz); hm = ror1(hm);
-        }
+        vjp_lds_fence();
+        cp = np;
+        ca = na;
     }
 #pragma unroll
-    for (int k = 0; k <= KB; ++k) {
+    for (int k = 0; k < N; ++k) {
         if constexpr (UNI) {
-            if (k < KB) {
+            if (k < N2) {
                 p[k][0] *= m; p[k][1] *= m; p[k][2] *= m;
             }
         }
@@ -207,31 +167,43 @@ __device__ __forceinline__ void sym_vjp_own(float4 sp, float4 sa, const float (&
         for (int q = 0; q < 4; ++q)
             kahan1(g[k][q], c[k][q], p[k][q]);
     }
-    if constexpr (KB > 0) {
+    if constexpr (N2 > 0) {
+        h = make_float4(L.h[0][lane] + L.h[0][lane + 64], L.h[1][lane] + L.h[1][lane + 64],
+                        L.h[2][lane] + L.h[2][lane + 64], L.h[3][lane] + L.h[3][lane + 64]);
         if constexpr (UNI) {
-            hx *= m; hy *= m; hz *= m;
+            h.x *= m; h.y *= m; h.z *= m;
         }
-        kahan1(g[KB][0], c[KB][0], hx);
-        kahan1(g[KB][1], c[KB][1], hy);
-        kahan1(g[KB][2], c[KB][2], hz);
-        kahan1(g[KB][3], c[KB][3], hm);
     }
 }
 
-// sym_vjp_own for the wave-uniform block index kb, 0 <= kb < K.
+// Own source block KB of the wave's block, for the wave-uniform kb: target
+// slots k < KB meet it two-sided, slot KB one-sided (the block with itself);
+// slots k > KB take these sources when their own block is the source.  The
+// reaction sums belong to slot KB.
 template <int K, int KB = 0>
-__device__ __forceinline__ void sym_vjp_own_at(int kb, bool uni, float4 sp, float4 sa, const float (&xi)[K],
-                                               const float (&yi)[K], const float (&zi)[K], const float (&mi)[K],
-                                               const float (&bx)[K], const float (&by)[K], const float (&bz)[K],
-                                               float m, float eps2, float (&g)[K][4], float (&c)[K][4])
+__device__ __forceinline__ void sym_vjp_own_at(int kb, bool uni, SymVjpLds& L, int lane, float4 sp, float4 sa,
+                                               const float (&xi)[K], const float (&yi)[K], const float (&zi)[K],
+                                               const float (&mi)[K], const float (&bx)[K], const float (&by)[K],
+                                               const float (&bz)[K], float m, float eps2, float (&g)[K][4],
+                                               float (&c)[K][4])
 {
     if (kb == KB) {
+        float4 h;
         if (uni)
-            sym_vjp_own<K, true, KB>(sp, sa, xi, yi, zi, mi, bx, by, bz, m, eps2, g, c);
+            sym_vjp_block<K, KB + 1, KB, true>(L, lane, sp, sa, xi, yi, zi, mi, bx, by, bz, m, eps2, g, c, h);
         else
-            sym_vjp_own<K, false, KB>(sp, sa, xi, yi, zi, mi, bx, by, bz, m, eps2, g, c);
+            sym_vjp_block<K, KB + 1, KB, false>(L, lane, sp, sa, xi, yi, zi, mi, bx, by, bz, m, eps2, g, c, h);
+        if constexpr (KB > 0) {
+            kahan1(g[KB][0], c[KB][0], h.x);
+            kahan1(g[KB][1], c[KB][1], h.y);
+            kahan1(g[KB][2], c[KB][2], h.z);
+            kahan1(g[KB][3], c[KB][3], h.w);
+        }
+        // keeps the compiler from merging the K branches' adds into one
+        // through a pointer to slot KB, which would put the sums in memory
+        asm volatile("; own block %0" : : "n"(KB));
     } else if constexpr (KB + 1 < K) {
-        sym_vjp_own_at<K, KB + 1>(kb, uni, sp, sa, xi, yi, zi, mi, bx, by, bz, m, eps2, g, c);
+        sym_vjp_own_at<K, KB + 1>(kb, uni, L, lane, sp, sa, xi, yi, zi, mi, bx, by, bz, m, eps2, g, c);
     }
 }
 
@@ -241,7 +213,7 @@ __device__ __forceinline__ void sym_vjp_own_at(int kb, bool uni, float4 sp, floa
 template <int K>
 __device__ __forceinline__ void sym_vjp_wave(const float4* __restrict__ jrec, int NW, int R, int w, int r,
                                              float eps2, float4* __restrict__ ipart,
-                                             float4* __restrict__ jpart, int lane)
+                                             float4* __restrict__ jpart, SymVjpLds& L, int lane)
 {
     const int half = NW / 2;
     const int n_pad = NW * 64 * K;
@@ -274,7 +246,7 @@ __device__ __forceinline__ void sym_vjp_wave(const float4* __restrict__ jrec, in
             const int b = w * 64 * K + kb * 64 + lane;
             const float4 sp = jrec[2 * b], sa = jrec[2 * b + 1];
             const bool uni = __ballot(tuni && sp.w == m0) == ~0ull;
-            sym_vjp_own_at<K>(kb, uni, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c);
+            sym_vjp_own_at<K>(kb, uni, L, lane, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c);
             continue;
         }
         const int d = u - 1;
@@ -287,9 +259,9 @@ __device__ __forceinline__ void sym_vjp_wave(const float4* __restrict__ jrec, in
         const float4 sp = jrec[2 * b], sa = jrec[2 * b + 1];
         float4 h;
         if (__ballot(tuni && sp.w == m0) == ~0ull)
-            sym_vjp_block<K, true>(sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c, h);
+            sym_vjp_block<K, K, K, true>(L, lane, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c, h);
         else
-            sym_vjp_block<K, false>(sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c, h);
+            sym_vjp_block<K, K, K, false>(L, lane, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c, h);
         jpart[((size_t)w * half + d) * (64 * K) + kb * 64 + lane] = h;
     }
 #pragma unroll
@@ -300,24 +272,26 @@ __device__ __forceinline__ void sym_vjp_wave(const float4* __restrict__ jrec, in
 
 // One system: wave gw = w * R + r.
 template <int K>
-__global__ __launch_bounds__(256) void sym_vjp_kernel(const float4* __restrict__ jrec, int NW, int R,
+__global__ __launch_bounds__(256, 2) void sym_vjp_kernel(const float4* __restrict__ jrec, int NW, int R,
                                                       float eps2, float4* __restrict__ ipart,
                                                       float4* __restrict__ jpart)
 {
+    __shared__ SymVjpLds lds[4];
     const int gw = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     if (gw >= NW * R)
         return;  // whole waves only
-    sym_vjp_wave<K>(jrec, NW, R, gw / R, gw % R, eps2, ipart, jpart, threadIdx.x & 63);
+    sym_vjp_wave<K>(jrec, NW, R, gw / R, gw % R, eps2, ipart, jpart, lds[threadIdx.x >> 6], threadIdx.x & 63);
 }
 
 // Batched systems: each wave runs items in the schedule of batch_next_item
 // (sym_items.h).
 template <int K>
-__global__ __launch_bounds__(256) void batch_sym_vjp_kernel(BatchSymGeom g, int nwaves,
+__global__ __launch_bounds__(256, 2) void batch_sym_vjp_kernel(BatchSymGeom g, int nwaves,
                                                             const float4* __restrict__ jrec, float eps2,
                                                             float4* __restrict__ ipart,
                                                             float4* __restrict__ jpart)
 {
+    __shared__ SymVjpLds lds[4];
     const int gw = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     if (gw >= nwaves)
         return;  // whole waves only
@@ -327,7 +301,7 @@ __global__ __launch_bounds__(256) void batch_sym_vjp_kernel(BatchSymGeom g, int 
         const int4 item = g.items[it];  // (system, wave block, split, splits)
         const int s = item.x;
         sym_vjp_wave<K>(jrec + 2 * (size_t)g.off[s], g.nw[s], item.w, item.y, item.z, eps2,
-                        ipart + g.vipo[s], jpart + g.vjpo[s], lane);
+                        ipart + g.vipo[s], jpart + g.vjpo[s], lds[threadIdx.x >> 6], lane);
     }
 }
 
