@@ -484,6 +484,8 @@ int utcnb_create(const utcnb_config* cfg, void* stream, utcnb_system** out)
                     s->args.cipart = s->cipart;
                     s->args.cjpart = s->cjpart;
                     s->args.react = s->react;
+                    s->args.part_ws = s->cipart;
+                    s->args.part_ws_floats = cif;
                 }
             } else if (!full_fits) {
                 rc = fail(UTCNB_EINVAL, "utcnb_create: N too large for a symmetric tile (partial sums "
@@ -491,10 +493,23 @@ int utcnb_create(const utcnb_config* cfg, void* stream, utcnb_system** out)
                                         "(or MIXED, which evaluates the symmetric step in chunks)");
             } else {
                 rc = dalloc(&s->ipart, jif) || dalloc(&s->jpart, jf);
+                s->args.part_ws = s->ipart;
+                s->args.part_ws_floats = jif;
             }
         }
         s->args.ipart = s->ipart;
         s->args.jpart = s->jpart;
+    }
+    if (!rc && (c.precision == UTCNB_PREC_FP32 || c.precision == UTCNB_PREC_MIXED) &&
+        tile_get(s->args.tile).parts > 0) {
+        const size_t pf = part_floats(s->args.tile, c.n);
+        if (pf * sizeof(float) > s->partial_budget)
+            rc = fail(UTCNB_EINVAL, "utcnb_create: N too large for a tile with source parts (partial sums above a "
+                                    "quarter of the device, at most 64 GiB); use another one-pass tile");
+        else
+            rc = dalloc(&s->ipart, pf);
+        s->args.ipart = s->args.part_ws = s->ipart;
+        s->args.part_ws_floats = pf;
     }
     if (!rc) {
         s->scratch_bytes = sizeof(double) * (3 * n + 5 + 5 * ((n + 255) / 256));
@@ -706,7 +721,9 @@ static int slice_tile_of(const utcnb_system* s, int count)
 {
     if (s->cfg.precision != UTCNB_PREC_FP32 && s->cfg.precision != UTCNB_PREC_MIXED)
         return -1;
-    return tile_get(s->args.tile).sym ? slice_tile_default(count, s->cu_count) : s->args.tile;
+    // a symmetric tile's target-side partials are free between its own steps:
+    // the slices' workspace
+    return tile_get(s->args.tile).sym ? slice_tile_default(count, s->cu_count, s->args.part_ws_floats) : s->args.tile;
 }
 
 int utcnb_slice_tile(const utcnb_system* s, int count, int* tile)

@@ -29,8 +29,13 @@ const Tile kTiles[] = {
     {1, 16, "sm1t16w16n8k", false, 1, 16, 8192}, {2, 16, "sm2t16w16n8k", false, 1, 16, 8192},
     // more one-pass tiles (appended: ids are stable)
     {2, 16, "k2s16", false}, {4, 8, "k4s8", false}, {4, 16, "k4s16", false},
+    // one-pass, the sources in P parts over separate waves (force_part.h): kKpP
+    {1, 1, "k1p128", false, 1, 0, 0, 128}, {2, 1, "k2p64", false, 1, 0, 0, 64},
 };
 }  // namespace
+
+constexpr int kTilePart128 = 37, kTilePart64 = 38;  // k1p128, k2p64
+size_t part_floats(int tile, int64_t nt) { return (size_t)kTiles[tile].parts * nt * 3; }
 
 int tile_count() { return (int)(sizeof(kTiles) / sizeof(kTiles[0])); }
 const Tile& tile_get(int id) { return kTiles[id]; }
@@ -57,7 +62,8 @@ const Tile& tile_get(int id) { return kTiles[id]; }
 // bodies, K = 8, which has the less LDS traffic and reaction partials per
 // pair, from 160 bodies per CU.  Their partial sums must fit the device's
 // budget (sym_partial_budget; K = 8 needs half the reaction partials of K =
-// 4); above it the best one-pass tile (k2s8) is used.
+// 4); above it the best one-pass tile whose partial sums do is used (N =
+// 262144: k2p64 15.99, k1p128 16.18, k2s8 19.03, k2s16 20.95 ms).
 size_t sym_partial_budget(size_t device_bytes)
 {
     if (device_bytes == 0)
@@ -91,6 +97,8 @@ int tile_default(int64_t n, int cu_count, size_t partial_budget)
         return 22;
     if (n >= 8 * cus && fits(2))
         return 20;  // sym2r32
+    if (part_floats(kTilePart64, n) * sizeof(float) <= partial_budget)
+        return kTilePart64;
     if ((n + 127) / 128 * 8 >= cus * 16)
         return 8;   // k2s8
     return 9;       // k1s16
@@ -112,8 +120,8 @@ hipError_t launch_fp32_step(const StepArgs& a, const float4* pos_old, float4* po
         return launch_sym(tile_get(a.tile), a.newton, false, pos_old, a.n, a.n_pad, a.eps2f, a.ipart,
                           a.jpart, epi, st);
     if (a.newton)
-        return launch_force<false, true>(a.tile, pos_old, a.n, a.n_pad, a.eps2f, epi, st);
-    return launch_force<false, false>(a.tile, pos_old, a.n, a.n_pad, a.eps2f, epi, st);
+        return launch_force<false, true>(a.tile, pos_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+    return launch_force<false, false>(a.tile, pos_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
 }
 
 hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* snap_new,
@@ -127,23 +135,31 @@ hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* 
         return launch_sym(tile_get(a.tile), a.newton, true, snap_old, a.n, a.n_pad, a.eps2f, a.ipart,
                           a.jpart, epi, st);
     if (a.newton)
-        return launch_force<true, true>(a.tile, snap_old, a.n, a.n_pad, a.eps2f, epi, st);
-    return launch_force<true, false>(a.tile, snap_old, a.n, a.n_pad, a.eps2f, epi, st);
+        return launch_force<true, true>(a.tile, snap_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+    return launch_force<true, false>(a.tile, snap_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
 }
 
 // One-pass tile for a slice of nt targets against all sources (the
 // symmetric tiles evaluate unordered pairs of the whole system and do not
-// split by target).  From a sweep on MI355X, slices of N = 262144, ms per
-// step (best three):
-//   nt =   8192: k1s16 1.81, k1s8 1.98, k2s16 2.86
-//   nt =  16384: k1s16 1.81, k1s8 2.12, k2s16 2.86
-//   nt =  32768: k2s16 2.89, k2s8 3.22, k1s16 3.59
-//   nt =  65536: k2s8 5.73, k2s16 5.84, k4s16 5.96   (k1s16 7.19)
-//   nt = 131072: k2s8 10.76, k2s16 11.74, k4s16 11.89 (k1s16 14.59)
-//   nt = 262144: k2s8 20.72, k2s16 23.65, k4s16 23.76
-// The fewer the targets per CU, the more source splits keep the waves busy.
-int slice_tile_default(int64_t nt, int cu_count)
+// split by target); part_ws: floats of workspace for the tiles with source
+// parts.  From sweeps on MI355X, ms per step:
+//   N = 262145: nt = 32769 k1p256 2.106, k1p128 2.109, k2p128 2.168, k2p64
+//               2.322   (k2s8 5.19, k2s16 5.50, k1s16 5.86)
+//   N = 262144: nt =   8192 k1p256 0.545, k1p128 0.561, k2p64 0.683 (k1s16 1.97)
+//               nt =  32768 k1p128 2.090, k1p256 2.108, k2p64 2.220 (k2s16 2.63)
+//               nt = 131072 k2p64 8.057, k2p128 8.060, k1p128 8.122 (k2s8 10.0)
+//   N =  32768: nt =   4096 k1p128 0.051, k2p64 0.056               (k1s16 0.237)
+// Many small waves fill the chip whatever the number of targets; 256 parts
+// gain at most 3% more and take twice the workspace, K = 4 (k4p32 ... k4p128)
+// is slower throughout.
+int slice_tile_default(int64_t nt, int cu_count, size_t part_ws)
 {
+    if (part_floats(kTilePart128, nt) <= part_ws)
+        return kTilePart128;
+    if (part_floats(kTilePart64, nt) <= part_ws)
+        return kTilePart64;
+    // without the workspace: the fewer the targets per CU, the more source
+    // splits keep the waves busy
     const int64_t cus = cu_count > 0 ? cu_count : 256;
     if (nt <= 64 * cus)
         return 9;   // k1s16
@@ -159,8 +175,8 @@ hipError_t launch_fp32_step_slice(const StepArgs& a, int tile, int i0, int nt, c
         return hipErrorInvalidValue;
     EpiFP32 epi{pos_old, pos_new, vel, (float)a.dt, (float)a.damping, a.kick};
     if (a.newton)
-        return launch_force_range<false, true>(tile, pos_old, i0, nt, a.n_pad, a.eps2f, epi, st);
-    return launch_force_range<false, false>(tile, pos_old, i0, nt, a.n_pad, a.eps2f, epi, st);
+        return launch_force_range<false, true>(tile, pos_old, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st);
+    return launch_force_range<false, false>(tile, pos_old, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st);
 }
 
 hipError_t launch_mixed_step_slice(const StepArgs& a, int tile, int i0, int nt, const float4* snap_old,
@@ -170,8 +186,8 @@ hipError_t launch_mixed_step_slice(const StepArgs& a, int tile, int i0, int nt, 
         return hipErrorInvalidValue;
     EpiMixed epi{pos, vel, snap_new, a.dt, a.damping, a.kick};
     if (a.newton)
-        return launch_force_range<true, true>(tile, snap_old, i0, nt, a.n_pad, a.eps2f, epi, st);
-    return launch_force_range<true, false>(tile, snap_old, i0, nt, a.n_pad, a.eps2f, epi, st);
+        return launch_force_range<true, true>(tile, snap_old, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st);
+    return launch_force_range<true, false>(tile, snap_old, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st);
 }
 
 hipError_t launch_fp32_accel_slice(const StepArgs& a, int tile, int i0, int nt, const float4* src,
@@ -181,10 +197,10 @@ hipError_t launch_fp32_accel_slice(const StepArgs& a, int tile, int i0, int nt, 
         return hipErrorInvalidValue;
     EpiAccel epi{acc3, i0};
     if (compensated)
-        return a.newton ? launch_force_range<true, true>(tile, src, i0, nt, a.n_pad, a.eps2f, epi, st)
-                        : launch_force_range<true, false>(tile, src, i0, nt, a.n_pad, a.eps2f, epi, st);
-    return a.newton ? launch_force_range<false, true>(tile, src, i0, nt, a.n_pad, a.eps2f, epi, st)
-                    : launch_force_range<false, false>(tile, src, i0, nt, a.n_pad, a.eps2f, epi, st);
+        return a.newton ? launch_force_range<true, true>(tile, src, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st)
+                        : launch_force_range<true, false>(tile, src, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st);
+    return a.newton ? launch_force_range<false, true>(tile, src, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st)
+                    : launch_force_range<false, false>(tile, src, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st);
 }
 
 hipError_t launch_fp32_accel(const StepArgs& a, const float4* src, bool compensated,
@@ -202,12 +218,12 @@ hipError_t launch_fp32_accel(const StepArgs& a, const float4* src, bool compensa
                           a.jpart, epi, st);
     if (compensated) {
         if (a.newton)
-            return launch_force<true, true>(a.tile, src, a.n, a.n_pad, a.eps2f, epi, st);
-        return launch_force<true, false>(a.tile, src, a.n, a.n_pad, a.eps2f, epi, st);
+            return launch_force<true, true>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+        return launch_force<true, false>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
     }
     if (a.newton)
-        return launch_force<false, true>(a.tile, src, a.n, a.n_pad, a.eps2f, epi, st);
-    return launch_force<false, false>(a.tile, src, a.n, a.n_pad, a.eps2f, epi, st);
+        return launch_force<false, true>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+    return launch_force<false, false>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
 }
 
 }  // namespace utcnb

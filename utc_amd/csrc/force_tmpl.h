@@ -215,9 +215,25 @@ struct EpiAccel {
     }
 };
 
+// The epilogues take (hi, c) with value hi - c; split an FP64 sum exactly.
+template <class Epi>
+__device__ __forceinline__ void sum_epilogue(const Epi& epi, int i, const double (&s)[3])
+{
+    const float h0 = (float)s[0], h1 = (float)s[1], h2 = (float)s[2];
+    epi(i, h0, h1, h2, (float)((double)h0 - s[0]), (float)((double)h1 - s[1]), (float)((double)h2 - s[2]));
+}
+
+// Plain FP32 sums go to the epilogue as they are (no compensation term).
+template <class Epi>
+__device__ __forceinline__ void sum_epilogue(const Epi& epi, int i, const float (&s)[3])
+{
+    epi(i, s[0], s[1], s[2], 0.f, 0.f, 0.f);
+}
+
 }  // namespace utcnb
 
-#include "force_small.h"  // uses pair_scale and kahan_add above
+#include "force_part.h"   // use the pieces above
+#include "force_small.h"
 
 namespace utcnb {
 
@@ -306,12 +322,18 @@ hipError_t launch_force_tile(const float4* src, int i0, int nt, int n_pad, float
 }
 
 // Dispatch over the tile table (must match tile_get()); targets [i0, i0 + nt).
+// part: workspace of the tiles with source parts ([parts][nt][3] floats).
 template <bool COMP, bool NEWTON, class Epi>
-hipError_t launch_force_range(int tile, const float4* src, int i0, int nt, int n_pad, float eps2,
+hipError_t launch_force_range(int tile, const float4* src, int i0, int nt, int n_pad, float eps2, float* part,
                               const Epi& epi, hipStream_t st)
 {
     if (nt < 1)
         return hipErrorInvalidValue;
+    if (const int P = tile_get(tile).parts) {
+        if (tile_get(tile).k == 1)
+            return launch_part_tile<1, COMP, NEWTON>(P, src, i0, nt, n_pad, eps2, part, epi, st);
+        return launch_part_tile<2, COMP, NEWTON>(P, src, i0, nt, n_pad, eps2, part, epi, st);
+    }
     switch (tile) {
     case 0: return launch_force_tile<1, 1, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
     case 1: return launch_force_tile<2, 1, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
@@ -338,10 +360,10 @@ hipError_t launch_force_range(int tile, const float4* src, int i0, int nt, int n
 
 // All n bodies as targets.
 template <bool COMP, bool NEWTON, class Epi>
-hipError_t launch_force(int tile, const float4* src, int n, int n_pad, float eps2,
+hipError_t launch_force(int tile, const float4* src, int n, int n_pad, float eps2, float* part,
                         const Epi& epi, hipStream_t st)
 {
-    return launch_force_range<COMP, NEWTON>(tile, src, 0, n, n_pad, eps2, epi, st);
+    return launch_force_range<COMP, NEWTON>(tile, src, 0, n, n_pad, eps2, part, epi, st);
 }
 
 }  // namespace utcnb

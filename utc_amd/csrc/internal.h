@@ -41,6 +41,7 @@ struct Tile {
     int rs = 1;  // symmetric tiles: rotation chunks per sub-unit (1, 2, 4, 8 or 16; K <= 4 when > 1)
     int tl = 0;  // small-system tiles (force_small.h): target lanes per wave; 0 for the other tiles
     int cap = 0; // small-system tiles: the most bodies (padded) their LDS holds
+    int parts = 0; // one-pass tiles with the sources split over separate waves (force_part.h): the parts; else 0
 };
 int tile_count();
 const Tile& tile_get(int id);
@@ -61,8 +62,11 @@ struct StepArgs {
     int kick;       // UTCNB_KICK_*
     bool newton;
     int tile;       // tile id
-    float* ipart;   // symmetric tiles: target-side partials [R][n_pad][3]
+    float* ipart;   // symmetric tiles: target-side partials [R][n_pad][3]; tiles
+                    // with source parts: [parts][n][3]
     float* jpart;   // symmetric tiles: reaction partials
+    float* part_ws;        // slices: workspace of the tiles with source parts
+    size_t part_ws_floats; //   and its size
     // symmetric tiles evaluated in chunks of wave blocks (0: one launch)
     int chunks;
     int chunk_r;    // waves per wave block in a chunk
@@ -117,7 +121,9 @@ hipError_t launch_ref_accel_slice_f64(const double4* src, int n, int i0, int nt,
                                       hipStream_t st);
 // Fast paths on one-pass tiles (`tile`; the symmetric ones do not split by
 // target): full-size state arrays, updated for the slice only.
-int slice_tile_default(int64_t nt, int cu_count);
+int slice_tile_default(int64_t nt, int cu_count, size_t part_ws);
+// Workspace of a tile with source parts for nt targets (floats; 0 for others).
+size_t part_floats(int tile, int64_t nt);
 hipError_t launch_fp32_step_slice(const StepArgs& a, int tile, int i0, int nt, const float4* pos_old,
                                   float4* pos_new, float4* vel, hipStream_t st);
 hipError_t launch_mixed_step_slice(const StepArgs& a, int tile, int i0, int nt, const float4* snap_old,

@@ -119,6 +119,9 @@ extern "C" int utcnb_accel_noalloc(const float* pos4, int n, double eps2, int pr
             need += round256(sym_ipart_floats((int)n_pad, tl.k, sym_tile_r(tl, (int)n_pad)) * sizeof(float));
             jpart_off = need;
             need += round256(sym_jpart_floats((int)n_pad, tl.k, tl.rs) * sizeof(float));
+        } else if (tl.parts > 0) {
+            ipart_off = need;
+            need += round256(part_floats(t, n) * sizeof(float));
         }
         return need;
     };
@@ -151,7 +154,7 @@ extern "C" int utcnb_accel_noalloc(const float* pos4, int n, double eps2, int pr
     a.eps2f = (float)eps2;
     a.newton = (flags & UTCNB_FLAG_NO_NEWTON) == 0;
     a.tile = t;
-    a.ipart = tl.sym ? (float*)(base + ipart_off) : nullptr;
+    a.ipart = tl.sym || tl.parts > 0 ? (float*)(base + ipart_off) : nullptr;
     a.jpart = tl.sym ? (float*)(base + jpart_off) : nullptr;
     e = launch_fp32_accel(a, src, precision == UTCNB_PREC_MIXED, acc3, st);
     if (e != hipSuccess)

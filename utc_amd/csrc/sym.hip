@@ -348,21 +348,6 @@ __global__ void batch_counter_reset_kernel(int* counter)
         *counter = 0;
 }
 
-// The epilogues take (hi, c) with value hi - c; split an FP64 sum exactly.
-template <class Epi>
-__device__ __forceinline__ void sym_epilogue(const Epi& epi, int i, const double (&s)[3])
-{
-    const float h0 = (float)s[0], h1 = (float)s[1], h2 = (float)s[2];
-    epi(i, h0, h1, h2, (float)((double)h0 - s[0]), (float)((double)h1 - s[1]), (float)((double)h2 - s[2]));
-}
-
-// Plain FP32 sums go to the epilogue as they are (no compensation term).
-template <class Epi>
-__device__ __forceinline__ void sym_epilogue(const Epi& epi, int i, const float (&s)[3])
-{
-    epi(i, s[0], s[1], s[2], 0.f, 0.f, 0.f);
-}
-
 // Body b's partials summed by T lanes (sym_reduce.h) in FP64 (Acc = double,
 // the compensated paths) or plain FP32 (Acc = float), then the epilogue.
 template <int T, typename Acc, class Epi>
@@ -375,7 +360,7 @@ __global__ __launch_bounds__(256) void sym_reduce_kernel(const float* __restrict
     Acc s[3];
     sym_split_sum<T>((const Part3*)ipart, (const Part3*)jpart, b < n ? b : n - 1, NW, R, K, t, s, rsl);
     if (b < n && t == 0)
-        sym_epilogue(epi, b, s);
+        sum_epilogue(epi, b, s);
 }
 
 // Batched systems: body b of the concatenated padded layout (systems start on
@@ -394,7 +379,7 @@ __global__ __launch_bounds__(256) void batch_sym_reduce_kernel(BatchSymGeom g, i
     sym_split_sum<T>((const Part3*)(ipart + g.ipo[s]), (const Part3*)(jpart + g.jpo[s]), loc, g.nw[s], g.rs[s],
                      K, t, sum);
     if (j < total && loc < g.n[s] && t == 0)
-        sym_epilogue(epi, b, sum);  // padding bodies keep their far-away zero-mass records
+        sum_epilogue(epi, b, sum);  // padding bodies keep their far-away zero-mass records
 }
 
 int sym_tile_r(const Tile& t, int n_pad)
@@ -584,7 +569,7 @@ __global__ __launch_bounds__(256) void sym_share_finish_kernel(const float* __re
         s[0] += react_sum3[3 * (size_t)j + 0];
         s[1] += react_sum3[3 * (size_t)j + 1];
         s[2] += react_sum3[3 * (size_t)j + 2];
-        sym_epilogue(epi, b, s);
+        sum_epilogue(epi, b, s);
     }
 }
 
