@@ -36,6 +36,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "rsq_group.h"
+
 namespace utcnb {
 
 // Smallest d2 for which ref_inv_dist is exact.
@@ -65,6 +67,46 @@ __device__ __forceinline__ float ref_recip_rn(float s)
 __device__ __forceinline__ float ref_inv_dist(float d2)
 {
     return ref_recip_rn(ref_sqrt_rn(d2));
+}
+
+// ref_inv_dist of G pairs with one approximation for both steps: y =
+// v_rsq_f32(x); s = s0 + (x - s0^2) y/2 with s0 = x y is the correctly rounded
+// root, and y + y (1 - s y) the correctly rounded 1/s, except where 1 - s y =
+// 2^-24 and y is a power of two (then the tie goes the wrong way; two
+// significands of x, just below a power of four) and at x = inf (s0 = NaN).
+// In both y has an all-zero significand: if any of the wave's G pairs has such
+// a y, the group takes ref_inv_dist (exact powers of four, which need not,
+// among them).  6 instructions and the check against 11 and a second
+// transcendental.  tests/device/probe_invdist_group.hip compares it with the
+// compiler's correctly rounded sqrtf and division for every float d2 in
+// [2^-96, inf] and NaN on the device.
+__device__ __forceinline__ float ref_inv_dist_y(float x, float y)
+{
+    const float s0 = x * y;
+    const float s = __builtin_fmaf(__builtin_fmaf(-s0, s0, x), 0.5f * y, s0);
+    return __builtin_fmaf(y, __builtin_fmaf(-s, y, 1.0f), y);
+}
+
+template <int G>
+__device__ __forceinline__ void ref_inv_dist_group(const float (&x)[G], float (&inv)[G])
+{
+    float y[G];
+    rsq_group<G>(x, y);
+    unsigned low = ~0u;  // the smallest significand of y
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+        const unsigned f = __float_as_uint(y[k]) << 9;
+        low = f < low ? f : low;
+    }
+    if (__ballot(low == 0) == 0) {
+#pragma unroll
+        for (int k = 0; k < G; ++k)
+            inv[k] = ref_inv_dist_y(x[k], y[k]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < G; ++k)
+            inv[k] = ref_inv_dist(x[k]);
+    }
 }
 
 // FP64: 1.0 / sqrt(d2) (benchapps/nbody/seq/bodysystem.h:86 for T = double)
