@@ -31,6 +31,8 @@ const Tile kTiles[] = {
     {2, 16, "k2s16", false}, {4, 8, "k4s8", false}, {4, 16, "k4s16", false},
     // one-pass, the sources in P parts over separate waves (force_part.h): kKpP
     {1, 1, "k1p128", false, 1, 0, 0, 128}, {2, 1, "k2p64", false, 1, 0, 0, 64},
+    // 24 targets per workgroup
+    {3, 16, "sm3t8w16n8k", false, 1, 8, 8192},
 };
 }  // namespace
 
@@ -50,12 +52,15 @@ const Tile& tile_get(int id) { return kTiles[id]; }
 //   N =  16384: sym4r64 65.6, sym4r32 67.5, sym4r64x2 68.3 us    (sym8r128 76)
 //   N =  12288: sym4r64 43.7, sym4r128 43.9, sym2r64 45.1 us
 //   N =   8192: sm2t16w16n8k 23.3, sm1t16w16n8k 26.4, sym4r128 27.9 us
-//   N =   6144: sm2t16w16n8k 18.3, sym2r64 20.7, sm1t8w16n8k 20.7 us
+//   N =   7168: sm2t16w16n8k 20.9, sm4t8w16n8k 23.1, sm1t16w16n8k 23.9 us
+//   N =   6144: sm3t8w16n8k 16.6, sm2t16w16n8k 18.3, sm6t4w16n8k 19.4 us  (sym2r64 20.7)
+//   N =   5120: sm3t8w16n8k 14.5, sm5t4w16n8k 15.3, sm2t16w16n8k 15.8 us
 //   N =   4096: sm1t16w16n8k 8.80, sm1t16w16n4k 8.84, sm1t8w16n8k 11.3 us  (sym2r64 16.4)
 //   N =   2048: sm1t8w16n8k 5.12, sm1t8w8n2k 5.16, sm1t4w8n2k 5.67 us  (sym2r64x2 12.5)
 //   N =   1024: sm1t4w8n2k 4.04, sm1t8w8n2k 4.10, sm1t8w16n8k 4.15 us  (sym2r128x4 12.1)
-// (sym8r48, sym8r24 and several other small-system shapes were swept earlier
-// and are not in the table.)  Up to 8192 bodies the small-system kernels win:
+// (sym8r48, sym8r24 and several other small-system shapes were swept and are
+// not in the table: 4 to 8 targets per lane, 4 target lanes with 16 waves, 8
+// waves per workgroup.)  Up to 8192 bodies the small-system kernels win:
 // one launch per step against two, and their one-pass pair sums fill the
 // chip where the symmetric kernels' 64-step rotations leave it waiting.  The
 // symmetric tiles need enough wave blocks to fill the chip: K = 4 above 8192
@@ -87,6 +92,8 @@ int tile_default(int64_t n, int cu_count, size_t partial_budget)
         return 30;  // sm1t8w16n8k
     if (n <= 4096)
         return 31;  // sm1t16w16n4k
+    if (n <= 6144)
+        return 39;  // sm3t8w16n8k: 24 targets for each of the 256 CUs at 6144
     if (n <= 8192)
         return 33;  // sm2t16w16n8k
     if (n >= 160 * cus && fits(8))

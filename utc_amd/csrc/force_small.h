@@ -21,8 +21,9 @@
 // Pair arithmetic as in stream_sources: 12 VALU instructions and a root per
 // ordered pair, the roots of 8 pairs together (rsq_group.h), plus one LDS read
 // per source shared by the lane's A targets.  Per step, mixed: N = 8192 23.3 us
-// (27.3 with a root per pair), 6001 18.3 (21.2), 4096 8.9 (9.6); below that the
-// launch and the copy into LDS bound it (N = 1024: 4.0 us either way).
+// (27.3 with a root per pair), 6001 16.5 (21.2; 18.3 with 32 targets per
+// workgroup instead of 24), 4096 8.9 (9.6); below that the launch and the copy
+// into LDS bound it (N = 1024: 4.0 us either way).
 #pragma once
 
 #include <type_traits>
@@ -73,7 +74,7 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
                 ax[a] = hx[a]; ay[a] = hy[a]; az[a] = hz[a];
             }
         }
-        constexpr int J = A >= 4 ? 2 : 8 / A;  // sources per group of reciprocal roots; divides kSmallBlock and iters
+        constexpr int J = A == 1 ? 8 : A == 2 ? 4 : 2;  // sources per group of reciprocal roots
 #pragma unroll 1
         for (int i = b0; i < b1; i += J) {
             float rx[J * A], ry[J * A], rz[J * A], d2[J * A], y[J * A], m[J];
@@ -163,7 +164,9 @@ template <int A, int TL, int W, int CAP, bool COMP, bool NEWTON, class Epi>
 hipError_t launch_small_tile(const float4* src, int i0, int nt, int n_pad, float eps2, const Epi& epi,
                              hipStream_t st)
 {
-    static_assert(64 % TL == 0 && kPadJ / 8 % ((64 / TL) * W) == 0, "each split takes a multiple of 8 sources");
+    static_assert(A <= 3 && 64 % TL == 0 && kPadJ / 8 % ((64 / TL) * W) == 0,
+                  "each split takes a multiple of 8 sources, in groups of 8 / A");
+
     if (n_pad > CAP || n_pad % kPadJ != 0)
         return hipErrorInvalidValue;
     constexpr int TW = TL * A;
