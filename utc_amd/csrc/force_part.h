@@ -52,7 +52,7 @@ __global__ __launch_bounds__(256) void part_force_kernel(const float4* __restric
 }
 
 // Target j's P records summed by T lanes (lane t takes records t, t + T, ...;
-// a fixed butterfly combines them, as in sym_reduce.h), then the epilogue.
+// lane_sum.h combines them, as in sym_reduce.h), then the epilogue.
 template <int T, typename Acc, class Epi>
 __global__ __launch_bounds__(256) void part_reduce_kernel(const float* __restrict__ part, int i0, int nt, int P,
                                                           Epi epi)
@@ -65,10 +65,8 @@ __global__ __launch_bounds__(256) void part_reduce_kernel(const float* __restric
     for (int p = t; p < P; p += T)
         part_add(s, ((const Part3*)part)[(size_t)p * nt + jj]);
 #pragma unroll
-    for (int off = 32; off >= 64 / T; off >>= 1)
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-            s[c] += __shfl_xor(s[c], off, 64);
+    for (int c = 0; c < 3; ++c)
+        s[c] = lane_sum<64 / T>(s[c]);
     if (j < nt && t == 0)
         sum_epilogue(epi, i0 + j, s);
 }

@@ -12,7 +12,7 @@
 //    with split = w * G + g, G = 64 / TL source groups per wave and SPL =
 //    G * W source splits per workgroup: the TL lanes of a group read the same
 //    LDS record (a broadcast), the G groups consecutive ones;
-//  * the G lanes of a target meet in a butterfly of lane shuffles, the W
+//  * the G lanes of a target meet in registers (lane_sum.h), the W
 //    waves in LDS, in a fixed order (bitwise repeatable), and TW threads run
 //    the integrator epilogue: one launch per step, nothing in HBM between.
 // COMP: sums of up to kSmallBlock sources are Kahan-added per lane (as the
@@ -23,10 +23,12 @@
 // per source shared by the lane's A targets.  Per step, mixed: N = 8192 23.3 us
 // (27.3 with a root per pair), 6001 16.5 (21.2; 18.3 with 32 targets per
 // workgroup instead of 24), 4096 8.9 (9.6); below that the launch and the copy
-// into LDS bound it (N = 1024: 4.0 us either way).
+// into LDS bound it (N = 1024: 4.0 us either way; 3.7 with the lane sums in registers).
 #pragma once
 
 #include <type_traits>
+
+#include "lane_sum.h"
 
 namespace utcnb {
 
@@ -114,7 +116,7 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
         }
     }
 
-    // lanes t, t + TL, ..., t + 64 - TL hold the same targets: butterfly
+    // lanes t, t + TL, ..., t + 64 - TL hold the same targets
 #pragma unroll
     for (int a = 0; a < A; ++a) {
         Acc v[3];
@@ -126,10 +128,8 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
             v[0] = hx[a]; v[1] = hy[a]; v[2] = hz[a];
         }
 #pragma unroll
-        for (int off = TL; off < 64; off <<= 1)
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-                v[c] += __shfl_xor(v[c], off, 64);
+        for (int c = 0; c < 3; ++c)
+            v[c] = lane_sum<TL>(v[c]);
         if (g == 0) {
 #pragma unroll
             for (int c = 0; c < 3; ++c)

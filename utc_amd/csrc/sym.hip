@@ -545,7 +545,7 @@ __global__ __launch_bounds__(256) void sym_react_kernel(const float* __restrict_
 
 // Bodies [start, start + count): their R target-side partials (rows of
 // istride bodies from body ibody0) summed in FP64 by T lanes per body (lane t
-// takes rows t, t + T, ...; a fixed butterfly combines the lanes, as in
+// takes rows t, t + T, ...; lane_sum.h combines the lanes, as in
 // sym_reduce.h), plus react_sum3[j] (the reactions summed over the shares),
 // then the epilogue.
 template <int T, class Epi>
@@ -561,10 +561,8 @@ __global__ __launch_bounds__(256) void sym_share_finish_kernel(const float* __re
     for (int r = t; r < R; r += T)
         part_add(s, ((const Part3*)ipart)[(size_t)r * (size_t)istride + (b - ibody0)]);
 #pragma unroll
-    for (int off = 32; off >= 64 / T; off >>= 1)
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-            s[c] += __shfl_xor(s[c], off, 64);
+    for (int c = 0; c < 3; ++c)
+        s[c] = lane_sum<64 / T>(s[c]);
     if (j < count && t == 0) {
         s[0] += react_sum3[3 * (size_t)j + 0];
         s[1] += react_sum3[3 * (size_t)j + 1];

@@ -6,15 +6,18 @@
 // of n_pad records), q = R + RS d + c the reaction from rotation chunk c of
 // the wave block d + 1 places below (jpart, RS = 2^rsl chunks per sub-unit;
 // RS = 1 for the kernels without a rotation split), absent for the block half
-// way round when the upper half skipped it.  T lanes share a body: lane t adds records t, t + T, t + 2T, ...
-// in that order (in FP64 on the compensated paths, in FP32 on the plain one), then the T partial sums are combined by a butterfly
-// of __shfl_xor over fixed lane offsets.  The order depends only on (T, R,
-// NW), so results are bitwise repeatable; with T = 1 it is the plain
-// sequential order.  Lane layout in a wave: lane = t * (64/T) + j for the
-// wave's j-th body, so the 64/T lanes of one t read 64/T consecutive records.
+// way round when the upper half skipped it.  T lanes share a body: lane t adds
+// records t, t + T, t + 2T, ... in that order (in FP64 on the compensated
+// paths, in FP32 on the plain one), then the T partial sums are combined over
+// the lane bits (lane_sum.h).  The order depends only on (T, R, NW), so results
+// are bitwise repeatable; with T = 1 it is the plain sequential order.  Lane
+// layout in a wave: lane = t * (64/T) + j for the wave's j-th body, so the 64/T
+// lanes of one t read 64/T consecutive records.
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include "lane_sum.h"
 
 namespace utcnb {
 
@@ -82,10 +85,8 @@ __device__ __forceinline__ void sym_split_sum(const P* __restrict__ ipart, const
         part_add(s, *p);
     }
 #pragma unroll
-    for (int off = 32; off >= 64 / T; off >>= 1)
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-            s[c] += __shfl_xor(s[c], off, 64);
+    for (int c = 0; c < C; ++c)
+        s[c] = lane_sum<64 / T>(s[c]);
 }
 
 }  // namespace utcnb
