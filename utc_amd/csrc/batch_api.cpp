@@ -454,7 +454,11 @@ int adj_workspace(utcnb_batch* b, int nck, int seg)
     }
     b->nck = nck;
     b->seg = seg;
-    // the step kernels write real bodies only: pad the work state once
+    // the step kernels write real bodies only: pad the work state and the
+    // segment's positions once (b->pos holds the padding bodies)
+    for (int t = 0; t < seg; ++t)
+        UTCNB_HIP(hipMemcpyAsync(b->segpos + T * (size_t)t, b->pos, T * sizeof(double4), hipMemcpyDeviceToDevice,
+                                 b->stream));
     hipError_t e = launch_batch_pad(b->geom(0), b->nsys, b->wpos, b->wvel, b->wsnap[0], b->wsnap[1],
                                     b->stream);
     if (e != hipSuccess)
@@ -530,11 +534,11 @@ hipError_t for_groups(utcnb_batch* b, F fn)
 }
 
 hipError_t sym_step_group(const utcnb_batch* b, int sk, int g, const float4* so, float4* sn, double4* p,
-                          double4* v, hipStream_t sg)
+                          double4* v, hipStream_t sg, double4* keep = nullptr)
 {
     return launch_batch_sym_step(b->sym_geom(sk, 0, g), b->snwaves[sk][g], b->group_bodies(g), so, sn, p, v,
                                  (float)b->cfg.eps2, b->cfg.dt, b->cfg.damping, b->cfg.kick, b->sipart,
-                                 b->sjpart, sg);
+                                 b->sjpart, sg, keep);
 }
 
 // One run with the symmetric kernels (schedule sk: 0 persistent waves, 1 one
@@ -559,16 +563,20 @@ hipError_t enqueue_run_sym(utcnb_batch* b, int nsteps, int ckpt, bool adj, int s
         ENQ(launch_snapshot(b->pos + b0, b->snap[0] + b0, (int)Tg, sg));
         int c = 0;
         const int nck = (nsteps + k - 1) / k, slast = (nck - 1) * k;
+        // with the adjoint, checkpoints of (x, v) at the segments' first steps,
+        // and the positions of the last segment, kept instead of recomputed
+        // (the steps write them there themselves)
         for (int t = 0; t < nsteps; ++t) {
-            if (adj && t % k == 0) {
+            if (adj && nck > 1 && t % k == 0) {
                 double4* ck = b->ckpt + 2 * T * (size_t)(t / k);
                 ENQ(hipMemcpyAsync(ck + b0, b->pos + b0, sb, hipMemcpyDeviceToDevice, sg));
                 ENQ(hipMemcpyAsync(ck + T + b0, b->vel + b0, sb, hipMemcpyDeviceToDevice, sg));
             }
-            if (adj && t >= slast)  // the last segment's positions, kept instead of recomputed
-                ENQ(hipMemcpyAsync(b->segpos + T * (size_t)(t - slast) + b0, b->pos + b0, sb,
-                                   hipMemcpyDeviceToDevice, sg));
-            ENQ(sym_step_group(b, sk, g, b->snap[c], b->snap[1 - c], b->pos, b->vel, sg));
+            if (adj && t == 0 && slast == 0)
+                ENQ(hipMemcpyAsync(b->segpos + b0, b->pos + b0, sb, hipMemcpyDeviceToDevice, sg));
+            ENQ(sym_step_group(b, sk, g, b->snap[c], b->snap[1 - c], b->pos, b->vel, sg,
+                               adj && t + 1 >= slast && t + 1 < nsteps ? b->segpos + T * (size_t)(t + 1 - slast)
+                                                                      : nullptr));
             c = 1 - c;
         }
         if (!adj)
@@ -584,13 +592,11 @@ hipError_t enqueue_run_sym(utcnb_batch* b, int nsteps, int ckpt, bool adj, int s
                 ENQ(hipMemcpyAsync(b->wvel + b0, ck + T + b0, sb, hipMemcpyDeviceToDevice, sg));
                 ENQ(launch_snapshot(b->wpos + b0, b->wsnap[0] + b0, (int)Tg, sg));
                 int wc = 0;
-                for (int t = s0; t < s1; ++t) {
-                    ENQ(hipMemcpyAsync(b->segpos + T * (size_t)(t - s0) + b0, b->wpos + b0, sb,
-                                       hipMemcpyDeviceToDevice, sg));
-                    if (t + 1 < s1) {
-                        ENQ(sym_step_group(b, sk, g, b->wsnap[wc], b->wsnap[1 - wc], b->wpos, b->wvel, sg));
-                        wc = 1 - wc;
-                    }
+                ENQ(hipMemcpyAsync(b->segpos + b0, b->wpos + b0, sb, hipMemcpyDeviceToDevice, sg));
+                for (int t = s0; t + 1 < s1; ++t) {
+                    ENQ(sym_step_group(b, sk, g, b->wsnap[wc], b->wsnap[1 - wc], b->wpos, b->wvel, sg,
+                                       b->segpos + T * (size_t)(t + 1 - s0)));
+                    wc = 1 - wc;
                 }
             }
             for (int t = s1 - 1; t >= s0; --t) {
@@ -944,13 +950,22 @@ int utcnb_batch_run(utcnb_batch* b, int nsteps, int mode, int ckpt_every, const 
     if (!b->has_state)
         return fail(UTCNB_ESTATE, "utcnb_batch_run: no state set");
     const bool adj = target3 != nullptr;
+    int seg = nsteps;
     if (adj) {
         if (!losses || !dx0 || !dv0 || !dm || ckpt_every < 1)
             return fail(UTCNB_EINVAL, "utcnb_batch_run: adjoint outputs and ckpt_every >= 1 required");
         if (b->cfg.kick != UTCNB_KICK_PHYSICAL)
             return fail(UTCNB_EINVAL, "utcnb_batch_run: the batched adjoint supports the physical kick");
-        const int k = ckpt_every < nsteps ? ckpt_every : nsteps;
-        int rc = adj_workspace(b, (nsteps + k - 1) / k, k);
+        // every step's positions while they fit kAdjointKeepBytes (one segment:
+        // nothing to recompute), else segments of ckpt_every steps
+        seg = ckpt_every < nsteps ? ckpt_every : nsteps;
+        if (seg < nsteps && (size_t)b->total * sizeof(double4) * (size_t)nsteps <= kAdjointKeepBytes) {
+            if (adj_workspace(b, 1, nsteps) == UTCNB_OK)
+                seg = nsteps;
+            else
+                (void)hipGetLastError();  // no memory for that: the segments need less
+        }
+        int rc = adj_workspace(b, (nsteps + seg - 1) / seg, seg);
         if (rc)
             return rc;
         // targets, compact host layout -> padded device layout
@@ -970,14 +985,14 @@ int utcnb_batch_run(utcnb_batch* b, int nsteps, int mode, int ckpt_every, const 
     }
     const int wi = b->wsel < 0 ? 1 : b->wsel;
     if (mode == 0) {
-        if (!b->exec || b->g_nsteps != nsteps || b->g_ckpt != ckpt_every || b->g_adj != adj ||
+        if (!b->exec || b->g_nsteps != nsteps || b->g_ckpt != seg || b->g_adj != adj ||
             b->g_w != wi) {
             if (b->exec)
                 (void)hipGraphExecDestroy(b->exec);
             b->exec = nullptr;
             hipGraph_t graph = nullptr;
             UTCNB_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-            hipError_t e = enqueue_run(b, nsteps, adj ? ckpt_every : nsteps, adj, 0, wi);
+            hipError_t e = enqueue_run(b, nsteps, seg, adj, 0, wi);
             hipError_t e2 = hipStreamEndCapture(b->stream, &graph);
             if (e != hipSuccess || e2 != hipSuccess) {
                 if (graph)
@@ -990,7 +1005,7 @@ int utcnb_batch_run(utcnb_batch* b, int nsteps, int mode, int ckpt_every, const 
             if (e != hipSuccess)
                 return fail(UTCNB_EHIP, std::string("utcnb_batch_run: instantiate: ") + hipGetErrorString(e));
             b->g_nsteps = nsteps;
-            b->g_ckpt = ckpt_every;
+            b->g_ckpt = seg;
             b->g_adj = adj;
             b->g_w = wi;
         }
@@ -1002,7 +1017,7 @@ int utcnb_batch_run(utcnb_batch* b, int nsteps, int mode, int ckpt_every, const 
         if (mode == 1)
             UTCNB_HIP(aux_streams(b));
         UTCNB_HIP(hipEventRecord(b->ev0, b->stream));
-        hipError_t e = enqueue_run(b, nsteps, adj ? ckpt_every : nsteps, adj, mode == 2 ? 0 : 1, wi);
+        hipError_t e = enqueue_run(b, nsteps, seg, adj, mode == 2 ? 0 : 1, wi);
         if (e != hipSuccess)
             return fail(UTCNB_EHIP, std::string("utcnb_batch_run: ") + hipGetErrorString(e));
         UTCNB_HIP(hipEventRecord(b->ev1, b->stream));

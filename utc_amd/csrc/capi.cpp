@@ -627,8 +627,9 @@ int utcnb_get_state(utcnb_system* s, void* pos4, void* vel4, int dtype, int wher
     return UTCNB_OK;
 }
 
-// One step on the current buffers (no bookkeeping of timing).
-static hipError_t step_once(utcnb_system* s)
+// One step on the current buffers (no bookkeeping of timing).  MIXED: the new
+// positions also go to keep (unless null).
+static hipError_t step_once(utcnb_system* s, double4* keep = nullptr)
 {
     hipError_t e = hipSuccess;
     const int c = s->cur;
@@ -647,7 +648,7 @@ static hipError_t step_once(utcnb_system* s)
         s->cur = 1 - c;
         break;
     case UTCNB_PREC_MIXED:
-        e = launch_mixed_step(s->args, s->snap[c], s->snap[1 - c], s->p64[0], s->v64, s->stream);
+        e = launch_mixed_step(s->args, s->snap[c], s->snap[1 - c], s->p64[0], s->v64, s->stream, keep);
         s->cur = 1 - c;
         break;
     case UTCNB_PREC_FP64:
@@ -1046,13 +1047,14 @@ static int adjoint_workspace(utcnb_system* s, int nck, int seg)
     return UTCNB_OK;
 }
 
-// One forward step of the adjoint's work state (wpos/wvel, with wsnap for MIXED).
-static hipError_t work_step(utcnb_system* s, int& wc, hipStream_t st)
+// One forward step of the adjoint's work state (wpos/wvel, with wsnap for
+// MIXED, whose new positions also go to keep unless null).
+static hipError_t work_step(utcnb_system* s, int& wc, hipStream_t st, double4* keep)
 {
     auto& a = s->adj;
     hipError_t e;
     if (s->cfg.precision == UTCNB_PREC_MIXED) {
-        e = launch_mixed_step(s->args, a.wsnap[wc], a.wsnap[1 - wc], a.wpos[0], a.wvel, st);
+        e = launch_mixed_step(s->args, a.wsnap[wc], a.wsnap[1 - wc], a.wpos[0], a.wvel, st, keep);
     } else {
         e = launch_fp64_step(s->args, a.wpos[wc], a.wpos[1 - wc], a.wvel, st);
     }
@@ -1071,7 +1073,15 @@ int utcnb_adjoint(utcnb_system* s, int nsteps, int ckpt_every, const double* tar
         return fail(UTCNB_EINVAL, "utcnb_adjoint: nsteps and ckpt_every must be >= 1");
     if (!s->has_state)
         return fail(UTCNB_ESTATE, "utcnb_adjoint: no state set");
-    const int k = ckpt_every < nsteps ? ckpt_every : nsteps;
+    // every step's positions while they fit kAdjointKeepBytes (one segment:
+    // nothing to recompute), else segments of ckpt_every steps
+    int k = ckpt_every < nsteps ? ckpt_every : nsteps;
+    if (k < nsteps && (size_t)s->n * sizeof(double4) * (size_t)nsteps <= kAdjointKeepBytes) {
+        if (adjoint_workspace(s, 1, nsteps) == UTCNB_OK)
+            k = nsteps;
+        else
+            (void)hipGetLastError();  // no memory for that: the segments need less
+    }
     const int nck = (nsteps + k - 1) / k;
     int rc = adjoint_workspace(s, nck, k);
     if (rc)
@@ -1102,16 +1112,18 @@ int utcnb_adjoint(utcnb_system* s, int nsteps, int ckpt_every, const double* tar
     // segment c's positions live in segbuf(c): two buffers, so that the
     // recompute of segment c - 1 can run beside the VJP steps of segment c
     auto segbuf = [&](int c) { return (c % 2 == 0) ? a.segpos : a.segpos2; };
+    // (the MIXED steps write them there themselves)
     for (int t = 0; t < nsteps; ++t) {
-        if (t % k == 0) {
+        if (nck > 1 && t % k == 0) {
             double4* ck = a.ckpt + 2 * n * (size_t)(t / k);
             ADJ_CHECK(hipMemcpyAsync(ck, cur_p64(s), sb, hipMemcpyDeviceToDevice, st));
             ADJ_CHECK(hipMemcpyAsync(ck + n, s->v64, sb, hipMemcpyDeviceToDevice, st));
         }
-        if (t >= slast)
+        if (t >= slast && (!mixed || t == 0))
             ADJ_CHECK(hipMemcpyAsync(segbuf(nck - 1) + n * (size_t)(t - slast), cur_p64(s), sb,
                                      hipMemcpyDeviceToDevice, st));
-        ADJ_CHECK(step_once(s));
+        ADJ_CHECK(step_once(s, t + 1 >= slast && t + 1 < nsteps ? segbuf(nck - 1) + n * (size_t)(t + 1 - slast)
+                                                               : nullptr));
         ++launches;
     }
     // loss and its seed at the final state
@@ -1138,9 +1150,10 @@ int utcnb_adjoint(utcnb_system* s, int nsteps, int ckpt_every, const double* tar
         int wc = 0;
         for (int t = s0; t < s1 && e == hipSuccess; ++t) {
             const double4* cur = mixed ? a.wpos[0] : a.wpos[wc];
-            e = hipMemcpyAsync(buf + n * (size_t)(t - s0), cur, sb, hipMemcpyDeviceToDevice, rs);
+            if (!mixed || t == s0)
+                e = hipMemcpyAsync(buf + n * (size_t)(t - s0), cur, sb, hipMemcpyDeviceToDevice, rs);
             if (e == hipSuccess && t + 1 < s1) {
-                e = work_step(s, wc, rs);
+                e = work_step(s, wc, rs, buf + n * (size_t)(t + 1 - s0));
                 ++launches;
             }
         }

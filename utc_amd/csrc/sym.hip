@@ -719,7 +719,8 @@ hipError_t launch_batch_counter_reset(int* counter, hipStream_t st)
 
 hipError_t launch_batch_sym_step(const BatchSymGeom& g, int nwaves, int total, const float4* snap_old,
                                  float4* snap_new, double4* pos, double4* vel, float eps2, double dt,
-                                 double damping, int kick, float* ipart, float* jpart, hipStream_t st)
+                                 double damping, int kick, float* ipart, float* jpart, hipStream_t st,
+                                 double4* keep)
 {
     hipError_t e;
     if (g.counter && (e = launch_batch_counter_reset(g.counter, st)) != hipSuccess)
@@ -729,7 +730,7 @@ hipError_t launch_batch_sym_step(const BatchSymGeom& g, int nwaves, int total, c
     e = hipGetLastError();
     if (e != hipSuccess)
         return e;
-    EpiMixed epi{pos, vel, snap_new, dt, damping, kick};
+    EpiMixed epi{pos, vel, snap_new, dt, damping, kick, keep};
     const int T = sym_reduce_lanes(total);
     const dim3 rgrid((unsigned)(((long long)total * T + 255) / 256));
     switch (T) {
