@@ -55,6 +55,8 @@ struct utcnb_system {
     float* jpart = nullptr;
     float* share_ipart = nullptr;  // target-side partials of a share step (utcnb_share_pairs)
     size_t share_ipart_floats = 0;
+    size_t jpart_floats = 0;
+    float* share_jpart = nullptr;  // reactions of a share step, where jpart is smaller than they are
     float* cipart = nullptr;     // chunked symmetric steps: target-side partials,
     float* cjpart = nullptr;     //   one chunk's reaction partials,
     double* react = nullptr;     //   reactions summed per body
@@ -182,6 +184,7 @@ void release(utcnb_system* s)
     dfree(s->jpart);
     dfree(s->share_ipart);
     s->share_ipart_floats = 0;
+    dfree(s->share_jpart);
     dfree(s->cipart);
     dfree(s->cjpart);
     dfree(s->react);
@@ -425,6 +428,7 @@ int utcnb_create(const utcnb_config* cfg, void* stream, utcnb_system** out)
         if (tile_get(t).sym)
             s->args.tile = t;
     }
+    s->args.share_tile = c.tile > 0 ? s->args.tile : sym_share_tile_default(c.n, cus);
     if (fast && c.precision != UTCNB_PREC_FP64 && tile_get(s->args.tile).cap > 0 &&
         s->n_pad > tile_get(s->args.tile).cap) {
         delete s;
@@ -457,21 +461,25 @@ int utcnb_create(const utcnb_config* cfg, void* stream, utcnb_system** out)
         if (np % (size_t)(128 * t.k) != 0) {
             rc = fail(UTCNB_EINVAL, "utcnb_create: symmetric tile needs N padded to 128*K");
         } else {
-            const size_t jf = sym_jpart_floats((int)np, t.k, t.rs),
-                         jif = sym_ipart_floats((int)np, t.k, sym_tile_r(t, (int)np));
+            const size_t jf = sym_jpart_floats((int)np, t);
+            size_t jif = sym_ipart_floats((int)np, t.k, sym_tile_r(t, (int)np));
+            // the slices' tiles take this buffer: 64 rows hold any slice
+            const size_t jif64 = std::max(jif, sym_ipart_floats((int)np, t.k, 64));
+            if ((jf + jif64) * sizeof(float) <= s->partial_budget)
+                jif = jif64;
             const bool full_fits = (jf + jif) * sizeof(float) <= s->partial_budget;
             if (c.precision == UTCNB_PREC_MIXED && (!full_fits || (c.flags & UTCNB_FLAG_SYM_CHUNKS))) {
                 // chunks of wave blocks: the fewest (at least 2) whose partial
                 // sums and per-body reaction sums fit the budget
-                const int NW = (int)(np / (64 * (size_t)t.k));
+                const int K = tile_get(s->args.share_tile).k, NW = (int)(np / (64 * (size_t)K));
                 int G = 2;
                 size_t cif = 0, cjf = 0;
                 int Rs = 0;
                 for (; G <= NW; ++G) {
                     const int nw = (NW + G - 1) / G;
-                    Rs = sym_share_splits(nw, t.s, t.k, NW);
+                    Rs = sym_share_splits(nw, K, NW);
                     cif = (size_t)Rs * np * 3;
-                    cjf = sym_chunk_jpart_floats(nw, NW, t.k);
+                    cjf = sym_chunk_jpart_floats(nw, NW, K);
                     if ((cif + cjf) * sizeof(float) + 3 * n * sizeof(double) <= s->partial_budget)
                         break;
                 }
@@ -493,6 +501,7 @@ int utcnb_create(const utcnb_config* cfg, void* stream, utcnb_system** out)
                                         "(or MIXED, which evaluates the symmetric step in chunks)");
             } else {
                 rc = dalloc(&s->ipart, jif) || dalloc(&s->jpart, jf);
+                s->jpart_floats = jf;
                 s->args.part_ws = s->ipart;
                 s->args.part_ws_floats = jif;
             }
@@ -828,7 +837,7 @@ static int share_geom(const utcnb_system* s, int shares, int share, const char* 
     if (!s->jpart)
         return fail(UTCNB_EINVAL, std::string(who) + ": the system evaluates its symmetric steps in chunks "
                                                      "(no whole-system reaction buffer); use utcnb_step_slice");
-    const Tile& t = tile_get(s->args.tile);
+    const Tile& t = tile_get(s->args.share_tile);
     const int B = 64 * t.k;
     g->NW = s->n_pad / B;
     if (shares < 1 || shares > g->NW || share < 0 || share >= shares)
@@ -839,7 +848,7 @@ static int share_geom(const utcnb_system* s, int shares, int share, const char* 
     g->count = std::min(g->w1 * B, s->n) - g->start;
     // one split count for every share of the partition (from the largest
     // share), so the shares' target-side partials share one layout
-    g->Rs = sym_share_splits((g->NW + shares - 1) / shares, t.s, t.k, g->NW);
+    g->Rs = sym_share_splits((g->NW + shares - 1) / shares, t.k, g->NW);
     return UTCNB_OK;
 }
 
@@ -874,10 +883,19 @@ int utcnb_share_pairs(utcnb_system* s, int shares, int share, double* react3)
             return rc;
         s->share_ipart_floats = need;
     }
+    const Tile& t = tile_get(s->args.share_tile);
+    const size_t jneed = sym_chunk_jpart_floats(g.NW, g.NW, t.k);
+    if (jneed > s->jpart_floats && !s->share_jpart) {
+        if (jneed * sizeof(float) > s->partial_budget)
+            return fail(UTCNB_EINVAL, "utcnb_share_pairs: the share's partial sums exceed the device budget");
+        if (int rc = dalloc(&s->share_jpart, jneed))
+            return rc;
+    }
     UTCNB_HIP(hipEventRecord(s->ev0, s->stream));
-    hipError_t e = launch_sym_share_pairs(tile_get(s->args.tile), s->args.newton, s->snap[s->cur], s->n, s->n_pad,
-                                          s->args.eps2f, shares, share, g.Rs, s->share_ipart, true, s->jpart,
-                                          false, react3, false, s->stream);
+    hipError_t e = launch_sym_share_pairs(t, s->args.newton, s->snap[s->cur], s->n, s->n_pad, s->args.eps2f, shares,
+                                          share, g.Rs, s->share_ipart, true,
+                                          jneed > s->jpart_floats ? s->share_jpart : s->jpart, false, react3, false,
+                                          s->stream);
     if (e != hipSuccess)
         return fail(UTCNB_EHIP, std::string("utcnb_share_pairs: ") + hipGetErrorString(e));
     UTCNB_HIP(hipEventRecord(s->ev1, s->stream));

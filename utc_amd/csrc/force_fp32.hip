@@ -33,6 +33,8 @@ const Tile kTiles[] = {
     {1, 1, "k1p128", false, 1, 0, 0, 128}, {2, 1, "k2p64", false, 1, 0, 0, 64},
     // 24 targets per workgroup
     {3, 16, "sm3t8w16n8k", false, 1, 8, 8192},
+    // symmetric, sub-units shared in chunks; R so that 2048 waves run: symKwWxRS
+    {8, 0, "sym8w2048x8", true, 8, 0, 0, 0, 2048}, {8, 64, "sym8r64x8", true, 8},
 };
 }  // namespace
 
@@ -46,11 +48,15 @@ const Tile& tile_get(int id) { return kTiles[id]; }
 // step, best three; equal masses; log-uniform masses and plain FP32 rank
 // alike):
 //   N = 131072: sym8r64 2.660, sym8r32 2.686, sym8r128 2.714 ms  (sym4r64 2.778)
-//   N =  65536: sym8r64 0.710, sym4r64 0.725, sym4r32 0.726 ms
-//   N =  32768: sym4r64 205.8, sym4r32 205.9, sym8r32 206.4 us   (sym8r64 211.7)
-//   N =  24576: sym4r64 126.8, sym4r32 127.9, sym8r64 129.5 us
-//   N =  16384: sym4r64 65.6, sym4r32 67.5, sym4r64x2 68.3 us    (sym8r128 76)
-//   N =  12288: sym4r64 43.7, sym4r128 43.9, sym2r64 45.1 us
+//   N =  65536: sym8r64x8 0.696, sym8r64 0.717, sym4r64 0.724 ms  (plain FP32: sym8r64 0.701, sym8r64x8 0.716)
+//   N =  49152: sym8r64x8 410, sym8w2048x8 418, sym8r64 429 us
+//   N =  40960: sym8r64x8 290, sym8w2048x8 298, sym4r64x8 305 us  (sym8r64 309)
+//   N =  32768: sym8w2048x8 189.0, sym8r64x8 195.6, sym4r64x8 200.9 us  (sym4r64 205.8)
+//   N =  24576: sym8w2048x8 118.6, sym8r64x8 120.3, sym4r64x8 120.6 us  (sym4r64 126.8)
+//   N =  16384: sym8w2048x8 59.5, sym4r64x2 63.2, sym4r64x8 63.8 us  (sym4r64 65.6)
+//   N =  14336: sym8w2048x8 51.7, sym4r128 52.3, sym8r64x8 54.0 us  (sym4r64 56.1)
+//   N =  12288: sym4r64x2 42.6, sym8w2048x8 42.8, sym4r64x8 43.2 us  (sym4r64 43.7)
+//   N =   9001: sym4w2048x8 32.5, sym8w2048x8 33.3, sym4r128 34.6 us  (sym4r64x2 37.5)
 //   N =   8192: sm2t16w16n8k 23.3, sm1t16w16n8k 26.4, sym4r128 27.9 us
 //   N =   7168: sm2t16w16n8k 20.9, sm4t8w16n8k 23.1, sm1t16w16n8k 23.9 us
 //   N =   6144: sm3t8w16n8k 16.6, sm2t16w16n8k 18.3, sm6t4w16n8k 19.4 us  (sym2r64 20.7)
@@ -58,17 +64,21 @@ const Tile& tile_get(int id) { return kTiles[id]; }
 //   N =   4096: sm1t16w16n8k 8.80, sm1t16w16n4k 8.84, sm1t8w16n8k 11.3 us  (sym2r64 16.4)
 //   N =   2048: sm1t8w16n8k 5.12, sm1t8w8n2k 5.16, sm1t4w8n2k 5.67 us  (sym2r64x2 12.5)
 //   N =   1024: sm1t4w8n2k 4.04, sm1t8w8n2k 4.10, sm1t8w16n8k 4.15 us  (sym2r128x4 12.1)
-// (sym8r48, sym8r24 and several other small-system shapes were swept and are
-// not in the table: 4 to 8 targets per lane, 4 target lanes with 16 waves, 8
-// waves per workgroup.)  Up to 8192 bodies the small-system kernels win:
-// one launch per step against two, and their one-pass pair sums fill the
-// chip where the symmetric kernels' 64-step rotations leave it waiting.  The
-// symmetric tiles need enough wave blocks to fill the chip: K = 4 above 8192
-// bodies, K = 8, which has the less LDS traffic and reaction partials per
-// pair, from 160 bodies per CU.  Their partial sums must fit the device's
-// budget (sym_partial_budget; K = 8 needs half the reaction partials of K =
-// 4); above it the best one-pass tile whose partial sums do is used (N =
-// 262144: k2p64 15.99, k1p128 16.18, k2s8 19.03, k2s16 20.95 ms).
+// (sym8r48, sym8r24, other R and chunk counts for K = 2, 4 and 8 and several
+// other small-system shapes were swept and are not in the table: 4 to 8 targets
+// per lane, 4 target lanes with 16 waves, 8 waves per workgroup.)  Up to 8192
+// bodies the small-system kernels win: one launch per step against two, and
+// their one-pass pair sums fill the chip where the symmetric kernels' 64-step
+// rotations leave it waiting.  Above, K = 8, which has the least LDS traffic
+// and the fewest reaction partials per pair.  Up to 160 bodies per CU the
+// waves' unequal ends weigh most: two waves on every SIMD (2048) that start
+// together and have equal shares of the work but for an eighth of a sub-unit.
+// Longer runs drift apart over the chip and want shorter waves, several in
+// turn; from 256 bodies per CU a sub-unit is small against a wave's work, and
+// whole ones need no second reaction record.  The partial sums must fit the
+// device's budget (sym_partial_budget); above it the best one-pass tile whose
+// partial sums do is used (N = 262144: k2p64 15.99, k1p128 16.18, k2s8 19.03,
+// k2s16 20.95 ms).
 size_t sym_partial_budget(size_t device_bytes)
 {
     if (device_bytes == 0)
@@ -80,9 +90,10 @@ int tile_default(int64_t n, int cu_count, size_t partial_budget)
 {
     const int64_t cus = cu_count > 0 ? cu_count : 256;
     const int64_t n_pad = pad_j(n);
-    const auto fits = [&](int k) {
-        return n_pad <= (1 << 30) && n_pad % (128 * k) == 0 &&
-               (sym_jpart_floats((int)n_pad, k) + sym_ipart_floats((int)n_pad, k, 64)) * sizeof(float) <=
+    const auto fits = [&](int tile) {
+        const Tile& t = kTiles[tile];
+        return n_pad <= (1 << 30) && n_pad % (128 * t.k) == 0 &&
+               (sym_jpart_floats((int)n_pad, t) + sym_ipart_floats((int)n_pad, t.k, sym_tile_r(t, (int)n_pad))) * sizeof(float) <=
                    partial_budget;
     };
     // from the sweeps above: each choice within 2% of the fastest tile at its size
@@ -96,14 +107,12 @@ int tile_default(int64_t n, int cu_count, size_t partial_budget)
         return 39;  // sm3t8w16n8k: 24 targets for each of the 256 CUs at 6144
     if (n <= 8192)
         return 33;  // sm2t16w16n8k
-    if (n >= 160 * cus && fits(8))
+    if (n >= 256 * cus && fits(22))
         return 22;  // sym8r64
-    if (n >= 8 * cus && fits(4))
-        return 18;  // sym4r64
-    if (n >= 96 * cus && fits(8))
-        return 22;
-    if (n >= 8 * cus && fits(2))
-        return 20;  // sym2r32
+    if (n >= 160 * cus && fits(41))
+        return 41;  // sym8r64x8
+    if (n >= 8 * cus && fits(40))
+        return 40;  // sym8w2048x8
     if (part_floats(kTilePart64, n) * sizeof(float) <= partial_budget)
         return kTilePart64;
     if ((n + 127) / 128 * 8 >= cus * 16)
@@ -118,6 +127,15 @@ template <class Epi>
 hipError_t launch_sym_chunked(const Tile& t, bool newton, const float4* src, int n, int n_pad, float eps2,
                               int chunks, int Rs, float* ipart, float* jchunk, double* react3, const Epi& epi,
                               hipStream_t st);
+
+// Shares and chunks of a default system divide it by wave blocks of this
+// tile, whatever tile its whole steps take: at most n_pad / (64 K) shares, so
+// the smaller the system the smaller K.
+int sym_share_tile_default(int64_t n, int cu_count)
+{
+    const int64_t cus = cu_count > 0 ? cu_count : 256;
+    return n >= 96 * cus ? 22 : (n >= 64 * cus ? 18 : 20);  // sym8r64, sym4r64, sym2r32
+}
 
 hipError_t launch_fp32_step(const StepArgs& a, const float4* pos_old, float4* pos_new,
                             float4* vel, hipStream_t st)
@@ -136,7 +154,7 @@ hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* 
 {
     EpiMixed epi{pos, vel, snap_new, a.dt, a.damping, a.kick, keep};
     if (tile_get(a.tile).sym && a.chunks > 0)
-        return launch_sym_chunked(tile_get(a.tile), a.newton, snap_old, a.n, a.n_pad, a.eps2f, a.chunks, a.chunk_r,
+        return launch_sym_chunked(tile_get(a.share_tile), a.newton, snap_old, a.n, a.n_pad, a.eps2f, a.chunks, a.chunk_r,
                                   a.cipart, a.cjpart, a.react, epi, st);
     if (tile_get(a.tile).sym)
         return launch_sym(tile_get(a.tile), a.newton, true, snap_old, a.n, a.n_pad, a.eps2f, a.ipart,
@@ -217,7 +235,7 @@ hipError_t launch_fp32_accel(const StepArgs& a, const float4* src, bool compensa
     if (tile_get(a.tile).sym && a.chunks > 0) {
         if (!compensated)
             return hipErrorInvalidValue;  // the chunked step sums its partials in FP64
-        return launch_sym_chunked(tile_get(a.tile), a.newton, src, a.n, a.n_pad, a.eps2f, a.chunks, a.chunk_r,
+        return launch_sym_chunked(tile_get(a.share_tile), a.newton, src, a.n, a.n_pad, a.eps2f, a.chunks, a.chunk_r,
                                   a.cipart, a.cjpart, a.react, epi, st);
     }
     if (tile_get(a.tile).sym)

@@ -38,10 +38,11 @@ struct Tile {
     int s;       // source split (one-pass tiles) or waves per wave block (symmetric tiles)
     const char* name;
     bool sym;    // evaluates each unordered pair once (sym.hip)
-    int rs = 1;  // symmetric tiles: rotation chunks per sub-unit (1, 2, 4, 8 or 16; K <= 4 when > 1)
+    int rs = 1;  // symmetric tiles: rotation chunks per sub-unit (1, 2, 4, 8 or 16)
     int tl = 0;  // small-system tiles (force_small.h): target lanes per wave; 0 for the other tiles
     int cap = 0; // small-system tiles: the most bodies (padded) their LDS holds
     int parts = 0; // one-pass tiles with the sources split over separate waves (force_part.h): the parts; else 0
+    int waves = 0; // symmetric tiles with s = 0: waves per wave block such that the system has about this many
 };
 int tile_count();
 const Tile& tile_get(int id);
@@ -51,6 +52,7 @@ const Tile& tile_get(int id);
 // device size is unknown).  Larger systems use one-pass kernels.
 size_t sym_partial_budget(size_t device_bytes);
 int tile_default(int64_t n, int cu_count, size_t partial_budget);
+int sym_share_tile_default(int64_t n, int cu_count);
 
 // ---- launchers (force.hip) ------------------------------------------------
 struct StepArgs {
@@ -62,6 +64,7 @@ struct StepArgs {
     int kick;       // UTCNB_KICK_*
     bool newton;
     int tile;       // tile id
+    int share_tile; // symmetric tiles: the tile whose wave blocks shares and chunks divide
     float* ipart;   // symmetric tiles: target-side partials [R][n_pad][3]; tiles
                     // with source parts: [parts][n][3]
     float* jpart;   // symmetric tiles: reaction partials
@@ -78,7 +81,7 @@ struct StepArgs {
 int sym_tile_r(const Tile& t, int n_pad);
 // Workspace of a symmetric tile (floats).
 size_t sym_ipart_floats(int n_pad, int K, int R);
-size_t sym_jpart_floats(int n_pad, int K, int rs = 1);
+size_t sym_jpart_floats(int n_pad, const Tile& t);
 
 // Reference arithmetic, one fused step (pos_new/vel written), T = float/double.
 hipError_t launch_ref_step_f32(const float4* pos_old, float4* pos_new, float4* vel, int n,
@@ -146,8 +149,8 @@ hipError_t launch_fp64_accel_slice(const StepArgs& a, int i0, int nt, const doub
 // Wave blocks [w0, w1) of share `share` of `shares` (the first NW % shares
 // shares take one block more).
 void sym_share_blocks(int NW, int shares, int share, int* w0, int* w1);
-// Waves per wave block for a share of nw_share blocks (R of the tile or more).
-int sym_share_splits(int nw_share, int R, int K, int NW);
+// Waves per wave block for a share of nw_share blocks.
+int sym_share_splits(int nw_share, int K, int NW);
 // The share's pair work (target-side partials into ipart [Rs][n_pad][3],
 // reactions into jpart) and its reactions summed per body into react3 (FP64 [3n]).
 // jpart_share_rows: jpart holds the share's wave blocks' rows only (else all NW);

@@ -118,7 +118,7 @@ extern "C" int utcnb_accel_noalloc(const float* pos4, int n, double eps2, int pr
             ipart_off = need;
             need += round256(sym_ipart_floats((int)n_pad, tl.k, sym_tile_r(tl, (int)n_pad)) * sizeof(float));
             jpart_off = need;
-            need += round256(sym_jpart_floats((int)n_pad, tl.k, tl.rs) * sizeof(float));
+            need += round256(sym_jpart_floats((int)n_pad, tl) * sizeof(float));
         } else if (tl.parts > 0) {
             ipart_off = need;
             need += round256(part_floats(t, n) * sizeof(float));

@@ -31,11 +31,14 @@
 // Q = K (NW/2 + 1).  The waves' target-side partials and the reaction
 // partials go to HBM, and a second kernel adds them per body in a fixed order
 // (deterministic) and applies the integrator epilogue.
-// Small systems have too few sub-units to give every SIMD several waves, and
-// one wave alone on a SIMD waits on its own dependent instructions.  Tiles
-// with a rotation split RS (SPLIT kernels) cut each sub-unit's 64 rotation
-// steps into RS chunks of 64/RS steps, and the R waves of a wave block share
-// its Q * RS chunks, each with a reaction record of its own.
+// Smaller systems have few sub-units per wave: one more or less is a large part
+// of a wave's work, and while the longer waves finish the SIMD's others are
+// gone (a wave alone issues half as fast).  Tiles with a rotation split RS
+// (SPLIT kernels) cut each sub-unit's 64 rotation steps into RS chunks of 64/RS
+// steps, and the R waves of a wave block share its Q * RS chunks in a row;
+// a sub-unit that two waves share has a reaction record from each.  N = 16384
+// 59.5 us per step against 65.6 with whole sub-units, 28672 153 against 163,
+// 9001 33.3 against 37.5 (sweeps at tile_default in force_fp32.hip).
 //
 // What bounds it: FP32 issue and, at large N, the power the FMAs draw.  A step
 // issues one 16-byte and three 4-byte LDS reads and three LDS writes beside
@@ -105,8 +108,11 @@ __device__ __forceinline__ void sym_rotate(SymLds& L, int lane, int t0, int step
     const float4* sp = &L.s[lane + t0];
     float* gp = &L.g[0][lane + t0];
     float4 cur = *sp;
-#pragma unroll 4
-    for (int t = 0; t < steps; ++t) {
+    // a loop with the LDS fences and a run-time trip count is not unrolled
+    // otherwise; steps is a multiple of 4
+    for (int t4 = 0; t4 < steps; t4 += 4)
+#pragma unroll
+    for (int t = t4; t < t4 + 4; ++t) {
         const float4 nxt = sp[t + 1];  // the next step's source: at most L.s[127]
         float gx = 0.f, gy = 0.f, gz = 0.f;
         if constexpr (N2 > 0) {
@@ -221,9 +227,9 @@ __device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane
 // range of bodies only: body b of row r is record r * istride + b - ibody0
 // (istride < 0: n_pad, the whole system).  COMP: the target-side block
 // partials are Kahan-added (the compensated paths); otherwise plain FP32 sums.
-// SPLIT: every sub-unit is cut into rs rotation chunks (rs divides 64); the
-// reactions then take rs records per (wave block, unit): jpart is
-// [NW][NW/2][rs][64K][3].
+// SPLIT: the waves share the sub-units by chunks of 64 / rs rotation steps (rs
+// divides 16) and the reactions take a record per wave and sub-unit: jpart is
+// [NW][R][J][64][3] (SymSplit, sym_reduce.h).
 template <int K, bool NEWTON, bool COMP, bool SPLIT = false>
 __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW, int R, int w, int r,
                                          float eps2, float* __restrict__ ipart,
@@ -247,18 +253,28 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
         tuni = tuni && mi[k] == m0;
     // sub-unit q = (unit u, source block kb): u = 0 is the wave block's own
     // sources, u = 1 + d the wave block d + 1 places round
-    const int Q = (half + 1) * K;
-    const int QS = SPLIT ? Q * rs : Q;  // (sub-unit, chunk) pairs, chunk fastest
-    const int steps = SPLIT ? 64 / rs : 64;
-    const int q0 = (int)((long long)QS * r / R), q1 = (int)((long long)QS * (r + 1) / R);
-    for (int qs = q0; qs < q1; ++qs) {
-        int q = qs, c = 0;
+    int qf, ql, c0 = 0, c1 = 0, J = 0;
+    if constexpr (SPLIT) {
+        const SymSplit sp(NW, w, K, R, rs);
+        c0 = sp.first(r);
+        c1 = sp.first(r + 1);
+        qf = c0 / rs;
+        ql = (c1 + rs - 1) / rs;
+        J = SymSplit::records(NW, K, R, rs);
+    } else {
+        const int Q = (half + 1) * K;
+        qf = (int)((long long)Q * r / R);
+        ql = (int)((long long)Q * (r + 1) / R);
+    }
+    for (int q = qf; q < ql; ++q) {
+        // rotation steps [t0, t0 + steps): all but for the first and last sub-unit
+        int t0 = 0, steps = 64;
         if constexpr (SPLIT) {
-            q = qs / rs;
-            c = qs - q * rs;
+            const int a = q == qf ? c0 - q * rs : 0, e = q + 1 == ql ? c1 - q * rs : rs;
+            t0 = a * (64 / rs);
+            steps = (e - a) * (64 / rs);
         }
         const int u = q / K, kb = q - u * K;
-        const int t0 = c * steps;  // chunk c: rotation steps [t0, t0 + steps)
         if (u == 0) {
             const float4 s = src[w * 64 * K + kb * 64 + lane];
             const bool uni = __ballot(tuni && s.w == m0) == ~0ull;
@@ -290,7 +306,8 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
         else
             sym_block<K, K, K, NEWTON, COMP, false>(L, lane, t0, steps, s, xi, yi, zi, mi, m0, eps2, ax, ay, az, cx,
                                                     cy, cz, g);
-        const size_t o = ((((size_t)(w - jbase) * half + d) * (SPLIT ? rs : 1) + c) * (64 * K) + kb * 64 + lane) * 3;
+        const size_t o = SPLIT ? ((((size_t)w * R + r) * J + (q - qf)) * 64 + lane) * 3
+                               : (((size_t)(w - jbase) * half + d) * (64 * K) + kb * 64 + lane) * 3;
         jpart[o + 0] = g[0];
         jpart[o + 1] = g[1];
         jpart[o + 2] = g[2];
@@ -350,15 +367,15 @@ __global__ void batch_counter_reset_kernel(int* counter)
 
 // Body b's partials summed by T lanes (sym_reduce.h) in FP64 (Acc = double,
 // the compensated paths) or plain FP32 (Acc = float), then the epilogue.
-template <int T, typename Acc, class Epi>
+template <int T, bool SPLIT, typename Acc, class Epi>
 __global__ __launch_bounds__(256) void sym_reduce_kernel(const float* __restrict__ ipart,
                                                          const float* __restrict__ jpart, int n, int NW,
-                                                         int R, int K, int rsl, Epi epi)
+                                                         int R, int K, int rs, Epi epi)
 {
     int b, t;
     sym_reduce_lane<T>(b, t);
     Acc s[3];
-    sym_split_sum<T>((const Part3*)ipart, (const Part3*)jpart, b < n ? b : n - 1, NW, R, K, t, s, rsl);
+    sym_split_sum<T, SPLIT>((const Part3*)ipart, (const Part3*)jpart, b < n ? b : n - 1, NW, R, K, t, s, rs);
     if (b < n && t == 0)
         sum_epilogue(epi, b, s);
 }
@@ -376,7 +393,7 @@ __global__ __launch_bounds__(256) void batch_sym_reduce_kernel(BatchSymGeom g, i
     const int s = g.sys_of_block[bb / kBatchSymAlign];
     const int loc = bb - g.off[s];  // padding bodies are summed too (their records exist)
     double sum[3];
-    sym_split_sum<T>((const Part3*)(ipart + g.ipo[s]), (const Part3*)(jpart + g.jpo[s]), loc, g.nw[s], g.rs[s],
+    sym_split_sum<T, false>((const Part3*)(ipart + g.ipo[s]), (const Part3*)(jpart + g.jpo[s]), loc, g.nw[s], g.rs[s],
                      K, t, sum);
     if (j < total && loc < g.n[s] && t == 0)
         sum_epilogue(epi, b, sum);  // padding bodies keep their far-away zero-mass records
@@ -384,39 +401,34 @@ __global__ __launch_bounds__(256) void batch_sym_reduce_kernel(BatchSymGeom g, i
 
 int sym_tile_r(const Tile& t, int n_pad)
 {
-    (void)n_pad;
-    return t.s;
+    if (t.s > 0)
+        return t.s;
+    const int R = t.waves / (n_pad / (64 * t.k));
+    return R < 1 ? 1 : (R > 128 ? 128 : R);
 }
 
 size_t sym_ipart_floats(int n_pad, int K, int R) { (void)K; return (size_t)R * n_pad * 3; }
-size_t sym_jpart_floats(int n_pad, int K, int rs)
+size_t sym_jpart_floats(int n_pad, const Tile& t)
 {
-    const int NW = n_pad / (64 * K);
-    return (size_t)NW * (NW / 2) * rs * 64 * K * 3;
-}
-
-static int log2_exact(int v)
-{
-    int l = 0;
-    while ((1 << l) < v)
-        ++l;
-    return (1 << l) == v ? l : -1;
+    const int NW = n_pad / (64 * t.k);
+    if (t.rs == 1)
+        return (size_t)NW * (NW / 2) * 64 * t.k * 3;
+    const int R = sym_tile_r(t, n_pad);
+    return (size_t)NW * R * SymSplit::records(NW, t.k, R, t.rs) * 64 * 3;
 }
 
 template <int K, bool COMP>
 static void launch_sym_pairs(bool newton, int rs, dim3 grid, const float4* src, int NW, int R, float eps2,
                              float* ipart, float* jpart, hipStream_t st)
 {
-    if constexpr (K <= 4) {
-        if (rs > 1) {
-            if (newton)
-                hipLaunchKernelGGL((sym_force_kernel<K, true, COMP, true>), grid, dim3(256), 0, st, src, NW, R, eps2,
-                                   ipart, jpart, rs);
-            else
-                hipLaunchKernelGGL((sym_force_kernel<K, false, COMP, true>), grid, dim3(256), 0, st, src, NW, R, eps2,
-                                   ipart, jpart, rs);
-            return;
-        }
+    if (rs > 1) {
+        if (newton)
+            hipLaunchKernelGGL((sym_force_kernel<K, true, COMP, true>), grid, dim3(256), 0, st, src, NW, R, eps2,
+                               ipart, jpart, rs);
+        else
+            hipLaunchKernelGGL((sym_force_kernel<K, false, COMP, true>), grid, dim3(256), 0, st, src, NW, R, eps2,
+                               ipart, jpart, rs);
+        return;
     }
     if (newton)
         hipLaunchKernelGGL((sym_force_kernel<K, true, COMP, false>), grid, dim3(256), 0, st, src, NW, R, eps2,
@@ -426,13 +438,14 @@ static void launch_sym_pairs(bool newton, int rs, dim3 grid, const float4* src, 
                            ipart, jpart, 1);
 }
 
-template <typename Acc, class Epi>
-static void launch_sym_reduce(int T, const float* ipart, const float* jpart, int n, int NW, int R, int K, int rsl,
+template <bool SPLIT, typename Acc, class Epi>
+static void launch_sym_reduce(int T, const float* ipart, const float* jpart, int n, int NW, int R, int K, int rs,
                               const Epi& epi, hipStream_t st)
 {
     const dim3 rgrid((unsigned)(((long long)n * T + 255) / 256));
 #define SYM_REDUCE(TT) \
-    hipLaunchKernelGGL((sym_reduce_kernel<TT, Acc, Epi>), rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, K, rsl, epi)
+    hipLaunchKernelGGL((sym_reduce_kernel<TT, SPLIT, Acc, Epi>), rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, K, rs, \
+                       epi)
     switch (T) {
     case 1: SYM_REDUCE(1); break;
     case 2: SYM_REDUCE(2); break;
@@ -450,8 +463,8 @@ template <class Epi>
 hipError_t launch_sym(const Tile& t, bool newton, bool comp, const float4* src, int n, int n_pad, float eps2,
                       float* ipart, float* jpart, const Epi& epi, hipStream_t st)
 {
-    const int K = t.k, R = sym_tile_r(t, n_pad), rs = t.rs, rsl = log2_exact(rs);
-    if (n_pad % (128 * K) != 0 || !ipart || !jpart || rsl < 0 || rs > 16 || (rs > 1 && K > 4))
+    const int K = t.k, R = sym_tile_r(t, n_pad), rs = t.rs;
+    if (n_pad % (128 * K) != 0 || !ipart || !jpart || rs < 1 || 16 % rs != 0)
         return hipErrorInvalidValue;
     const int NW = n_pad / (64 * K);
     const int waves = NW * R;
@@ -471,10 +484,14 @@ hipError_t launch_sym(const Tile& t, bool newton, bool comp, const float4* src, 
     if (e != hipSuccess)
         return e;
     const int T = sym_reduce_lanes(n);
-    if (comp)
-        launch_sym_reduce<double>(T, ipart, jpart, n, NW, R, K, rsl, epi, st);
+    if (rs > 1 && comp)
+        launch_sym_reduce<true, double>(T, ipart, jpart, n, NW, R, K, rs, epi, st);
+    else if (rs > 1)
+        launch_sym_reduce<true, float>(T, ipart, jpart, n, NW, R, K, rs, epi, st);
+    else if (comp)
+        launch_sym_reduce<false, double>(T, ipart, jpart, n, NW, R, K, rs, epi, st);
     else
-        launch_sym_reduce<float>(T, ipart, jpart, n, NW, R, K, rsl, epi, st);
+        launch_sym_reduce<false, float>(T, ipart, jpart, n, NW, R, K, rs, epi, st);
     return hipGetLastError();
 }
 
@@ -578,13 +595,12 @@ void sym_share_blocks(int NW, int shares, int share, int* w0, int* w1)
     *w1 = *w0 + (share < extra ? per + 1 : per);
 }
 
-int sym_share_splits(int nw_share, int R, int K, int NW)
+int sym_share_splits(int nw_share, int K, int NW)
 {
     // about 32768 waves (ten rounds of the chip's 256 CUs x 4 SIMDs x 3 waves
     // of this kernel), every wave with the same number u of the Q sub-units
     // of its wave block (the last one of a block fewer): u = Q nw / 32768,
     // R_share = ceil(Q / u)
-    (void)R;
     const long long Q = (long long)K * (NW / 2 + 1);
     long long u = Q * nw_share / 32768;
     if (u < 1)
@@ -699,7 +715,7 @@ hipError_t launch_sym_share_finish_mixed(const StepArgs& a, int shares, int shar
                                          const float* ipart, const double* react_sum3, float4* snap_new,
                                          double4* pos, double4* vel, hipStream_t st)
 {
-    const Tile& t = tile_get(a.tile);
+    const Tile& t = tile_get(a.share_tile);
     const int NW = a.n_pad / (64 * t.k);
     int w0, w1;
     sym_share_blocks(NW, shares, share, &w0, &w1);

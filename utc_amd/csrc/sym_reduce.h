@@ -1,16 +1,18 @@
 // sym_reduce.h -- per-body sums of the symmetric kernels' partials (device
 // code only), shared by the force (sym.hip) and VJP (sym_vjp.hip) reductions.
 //
-// Body b of a system with NW wave blocks of 64K bodies has Q = R + RS NW/2
-// partial records: q < R is wave r = q's target-side partial (ipart, R rows
-// of n_pad records), q = R + RS d + c the reaction from rotation chunk c of
-// the wave block d + 1 places below (jpart, RS = 2^rsl chunks per sub-unit;
-// RS = 1 for the kernels without a rotation split), absent for the block half
-// way round when the upper half skipped it.  T lanes share a body: lane t adds
-// records t, t + T, t + 2T, ... in that order (in FP64 on the compensated
-// paths, in FP32 on the plain one), then the T partial sums are combined over
-// the lane bits (lane_sum.h).  The order depends only on (T, R, NW), so results
-// are bitwise repeatable; with T = 1 it is the plain sequential order.  Lane
+// Body b of a system with NW wave blocks of 64K bodies has R target-side
+// partials, row r of ipart (n_pad records) from wave r of its wave block, and
+// the reactions from the NW/2 wave blocks before its own, d + 1 = 1 .. NW/2
+// places below, the one half way round only where the upper half did not skip
+// it.  Undivided sub-units (RS = 1): one record per wave block and d, jpart
+// [NW][NW/2][64K].  Divided ones (SymSplit below): each of the waves that share
+// a sub-unit left a record of 64 bodies, jpart [NW][R][J][64].
+// T lanes share a body: lane t adds rows t, t + T, ... of ipart, then the
+// reactions from d = t, t + T, ..., in that order (in FP64 on the compensated
+// paths, in FP32 on the plain one), then the T sums are combined over the lane
+// bits (lane_sum.h).  The order depends only on (T, R, RS, NW), so results are
+// bitwise repeatable; with T = 1 it is the plain sequential order.  Lane
 // layout in a wave: lane = t * (64/T) + j for the wave's j-th body, so the 64/T
 // lanes of one t read 64/T consecutive records.
 #pragma once
@@ -56,33 +58,71 @@ __device__ __forceinline__ void sym_reduce_lane(int& body, int& t)
     body = (g >> 6) * (64 / T) + lane % (64 / T);
 }
 
-// All 64 lanes of the wave must call this (it shuffles); b must be a valid
-// body of the system for every lane.
-template <int T, typename P, typename Acc, int C>
+// How the R waves of wave block w of NW share its sub-units when each is cut
+// into RS chunks (K sub-units for the own unit and each of the NW/2 after it,
+// one less in the upper half, which skips the block half way round): wave r
+// takes chunks [first(r), first(r + 1)) in a row, whole sub-units but for the
+// first and the last, and leaves one reaction record for each of the at most
+// J sub-units it touches.  Waves past the last chunk take none.
+struct SymSplit {
+    int chunks, R, rs;
+    __host__ __device__ SymSplit(int NW, int w, int K, int R_, int rs_)
+        : chunks((NW / 2 + (w < NW / 2)) * K * rs_), R(R_ < chunks ? R_ : chunks), rs(rs_)
+    {
+    }
+    __host__ __device__ int first(int r) const { return r < R ? (int)((long long)chunks * r / R) : chunks; }
+    // the wave that takes chunk x: the last r with first(r) <= x
+    __host__ __device__ int wave(int x) const { return (int)(((long long)(x + 1) * R - 1) / chunks); }
+    __host__ __device__ int records() const { return ((chunks + R - 1) / R + rs - 2) / rs + 1; }
+    // J: the lower half's waves touch the most
+    __host__ __device__ static int records(int NW, int K, int R, int rs) { return SymSplit(NW, 0, K, R, rs).records(); }
+};
+
+// All 64 lanes of the wave must call this (it exchanges lanes); b must be a
+// valid body of the system for every lane.
+template <int T, bool SPLIT, typename P, typename Acc, int C>
 __device__ __forceinline__ void sym_split_sum(const P* __restrict__ ipart, const P* __restrict__ jpart, int b,
-                                              int NW, int R, int K, int t, Acc (&s)[C], int rsl = 0)
+                                              int NW, int R, int K, int t, Acc (&s)[C], int rs = 1)
 {
     const int n_pad = NW * 64 * K;
     const int half = NW / 2, v = b / (64 * K), loc = b - v * (64 * K);
 #pragma unroll
     for (int c = 0; c < C; ++c)
         s[c] = Acc(0);
-    const int Q = R + (half << rsl);
+    if constexpr (!SPLIT) {
+        const int Q = R + half;
 #pragma unroll 4
-    for (int q = t; q < Q; q += T) {
-        const P* p;
-        if (q < R) {
-            p = ipart + (size_t)q * n_pad + b;
-        } else {
-            const int dc = q - R, d = dc >> rsl;
+        for (int q = t; q < Q; q += T) {
+            const P* p;
+            if (q < R) {
+                p = ipart + (size_t)q * n_pad + b;
+            } else {
+                const int d = q - R;
+                int w = v - 1 - d;
+                if (w < 0)
+                    w += NW;
+                if (2 * (d + 1) == NW && w >= half)
+                    continue;
+                p = jpart + ((size_t)w * half + d) * (64 * K) + loc;
+            }
+            part_add(s, *p);
+        }
+    } else {
+#pragma unroll 4
+        for (int r = t; r < R; r += T)
+            part_add(s, ipart[(size_t)r * n_pad + b]);
+        const int J = SymSplit::records(NW, K, R, rs), kb = loc >> 6, lane = loc & 63;
+        for (int d = t; d < half; d += T) {
             int w = v - 1 - d;
             if (w < 0)
                 w += NW;
             if (2 * (d + 1) == NW && w >= half)
                 continue;
-            p = jpart + ((((size_t)w * half + d) << rsl) + (dc - (d << rsl))) * (64 * K) + loc;
+            const SymSplit sp(NW, w, K, R, rs);
+            const int q = (d + 1) * K + kb, r1 = sp.wave((q + 1) * rs - 1);
+            for (int r = sp.wave(q * rs); r <= r1; ++r)
+                part_add(s, jpart[(((size_t)w * R + r) * J + (q - sp.first(r) / rs)) * 64 + lane]);
         }
-        part_add(s, *p);
     }
 #pragma unroll
     for (int c = 0; c < C; ++c)

@@ -317,7 +317,7 @@ __global__ __launch_bounds__(256) void sym_vjp_reduce_kernel(const float4* __res
     int b, t;
     sym_reduce_lane<T>(b, t);
     double s[4];
-    sym_split_sum<T>(ipart, jpart, b < n ? b : n - 1, NW, R, K, t, s);
+    sym_split_sum<T, false>(ipart, jpart, b < n ? b : n - 1, NW, R, K, t, s);
     if (b < n && t == 0) {
         xbar3[3 * (size_t)b + 0] += s[0];
         xbar3[3 * (size_t)b + 1] += s[1];
@@ -340,7 +340,7 @@ __global__ __launch_bounds__(256) void batch_sym_vjp_reduce_kernel(BatchSymGeom 
     const int s = g.sys_of_block[bb / kBatchSymAlign];
     const int loc = bb - g.off[s];
     double sum[4];
-    sym_split_sum<T>(ipart + g.vipo[s], jpart + g.vjpo[s], loc, g.nw[s], g.rs[s], K, t, sum);
+    sym_split_sum<T, false>(ipart + g.vipo[s], jpart + g.vjpo[s], loc, g.nw[s], g.rs[s], K, t, sum);
     if (j < total && loc < g.n[s] && t == 0) {
         xbar3[3 * (size_t)b + 0] += sum[0];
         xbar3[3 * (size_t)b + 1] += sum[1];
