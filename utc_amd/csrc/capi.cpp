@@ -1019,14 +1019,14 @@ static int adjoint_workspace(utcnb_system* s, int nck, int seg)
     const int Rv = sym_vjp_splits((int)np, s->cu_count);
     const Tile& ft = tile_get(s->args.tile);
     if (!rc && f32 && (ft.sym || ft.cap > 0) && sym_vjp_applies((int)np) &&
-        (sym_vjp_jpart_float4s((int)np) + sym_vjp_ipart_float4s((int)np, Rv)) * sizeof(float4) <=
+        (sym_vjp_jpart_float4s((int)np, Rv) + sym_vjp_ipart_float4s((int)np, Rv)) * sizeof(float4) <=
             s->partial_budget) {
         // a symmetric force tile (or a small-system one, whose sizes the
         // symmetric VJP also serves best) evaluates the adjoint pair sum
         // symmetrically
         const int R = Rv;
         rc = dalloc(&a.vjp_ipart, sym_vjp_ipart_float4s((int)np, R)) ||
-             dalloc(&a.vjp_jpart, sym_vjp_jpart_float4s((int)np));
+             dalloc(&a.vjp_jpart, sym_vjp_jpart_float4s((int)np, Rv));
         a.vjp_r = R;
     }
     if (!rc) {

@@ -186,7 +186,7 @@ hipError_t launch_jrec_pad(bool fp32_records, void* jrec, int n, int n_pad, hipS
 bool sym_vjp_applies(int n_pad);                 // n_pad a multiple of 512
 int sym_vjp_splits(int n_pad, int cu_count);     // waves per wave block
 size_t sym_vjp_ipart_float4s(int n_pad, int R);
-size_t sym_vjp_jpart_float4s(int n_pad);
+size_t sym_vjp_jpart_float4s(int n_pad, int R);
 // xbar3 / mbar (first n bodies) += the pair sums; ipart / jpart are workspace.
 hipError_t launch_sym_vjp(const float4* jrec, int n, int n_pad, float eps2, int R, float4* ipart,
                           float4* jpart, double* xbar3, double* mbar, hipStream_t st);

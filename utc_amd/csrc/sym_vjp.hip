@@ -23,14 +23,15 @@
 // round the wave in 10 DPP moves per step and one root at a time), N = 16384
 // with log-uniform masses 162 us (200); 96 systems of 256 to 8192 bodies, 20
 // steps forward and adjoint 16.7 ms (20.9).  Roots 2 at a time, an unroll of 4
-// and 128 VGPRs (four waves per SIMD, for 143 and three) are the same within
+// and 128 VGPRs (four waves per SIMD, for three) are the same within
 // 1%; without unrolling it is 8% slower at N = 65536.
 //
 // The mapping is the symmetric force kernel's (sym.hip): wave blocks of 64*K
 // bodies, unit 0 = own blocks (source block kb two-sided against target slots
 // k < kb, one-sided against slot kb), unit 1 + d = the wave block d + 1 places
 // round (both sides), R waves per wave block split the K (NW/2+1) (unit,
-// source block) sub-units.
+// source block) sub-units: in chunks of 4 rotation steps (SymSplit,
+// sym_reduce.h), or whole ones in batches.
 // Partials go to HBM (float4 per body: x, y, z, m) and a second kernel adds
 // them per body in FP64, in a fixed order, into xbar and mbar.
 #include "internal.h"
@@ -67,14 +68,14 @@ __device__ __forceinline__ void vjp_lds_fence()
 }
 
 // A block of 64 sources (lane l's source: position/mass sp, alpha sa; wave
-// private LDS L) against target slots 0 .. N-1 of each lane: at step t lane l
-// meets source (l + t) mod 64.  Slots k < N2 are two-sided; slot N2 < N is the
+// private LDS L) against target slots 0 .. N-1 of each lane: at step t in
+// [t0, t0 + steps) lane l meets source (l + t) mod 64.  Slots k < N2 are two-sided; slot N2 < N is the
 // block with itself (self pairs included, so w is exact: vjp_pair.h), target
 // side only.  The target-side block partials are Kahan-added into (g, c); the
 // reaction sums of lane l's own source come back in h (N2 > 0).
 // UNI: every target mass mi[k] and source mass equals m (two-sided slots).
 template <int K, int N, int N2, bool UNI>
-__device__ __forceinline__ void sym_vjp_block(SymVjpLds& L, int lane, float4 sp, float4 sa, const float (&xi)[K],
+__device__ __forceinline__ void sym_vjp_block(SymVjpLds& L, int lane, int t0, int steps, float4 sp, float4 sa, const float (&xi)[K],
                                               const float (&yi)[K], const float (&zi)[K], const float (&mi)[K],
                                               const float (&bx)[K], const float (&by)[K], const float (&bz)[K],
                                               float m, float eps2, float (&g)[K][4], float (&c)[K][4], float4& h)
@@ -95,9 +96,12 @@ __device__ __forceinline__ void sym_vjp_block(SymVjpLds& L, int lane, float4 sp,
     const float4* pp = &L.p[lane];
     const float4* pa = &L.a[lane];
     float* ph = &L.h[0][lane];
-    float4 cp = *pp, ca = *pa;
-#pragma unroll 2
-    for (int t = 0; t < 64; ++t) {
+    float4 cp = pp[t0], ca = pa[t0];
+    // a loop with the LDS fences and a run-time trip count is not unrolled
+    // otherwise; steps is even
+    for (int t2 = t0; t2 < t0 + steps; t2 += 2)
+#pragma unroll
+    for (int t = t2; t < t2 + 2; ++t) {
         const float4 np = pp[t + 1], na = pa[t + 1];  // the next step's source: at most slot 127
         float hx = 0.f, hy = 0.f, hz = 0.f, hm = 0.f;
         if constexpr (N2 > 0) {
@@ -181,7 +185,7 @@ __device__ __forceinline__ void sym_vjp_block(SymVjpLds& L, int lane, float4 sp,
 // slots k > KB take these sources when their own block is the source.  The
 // reaction sums belong to slot KB.
 template <int K, int KB = 0>
-__device__ __forceinline__ void sym_vjp_own_at(int kb, bool uni, SymVjpLds& L, int lane, float4 sp, float4 sa,
+__device__ __forceinline__ void sym_vjp_own_at(int kb, bool uni, SymVjpLds& L, int lane, int t0, int steps, float4 sp, float4 sa,
                                                const float (&xi)[K], const float (&yi)[K], const float (&zi)[K],
                                                const float (&mi)[K], const float (&bx)[K], const float (&by)[K],
                                                const float (&bz)[K], float m, float eps2, float (&g)[K][4],
@@ -190,9 +194,9 @@ __device__ __forceinline__ void sym_vjp_own_at(int kb, bool uni, SymVjpLds& L, i
     if (kb == KB) {
         float4 h;
         if (uni)
-            sym_vjp_block<K, KB + 1, KB, true>(L, lane, sp, sa, xi, yi, zi, mi, bx, by, bz, m, eps2, g, c, h);
+            sym_vjp_block<K, KB + 1, KB, true>(L, lane, t0, steps, sp, sa, xi, yi, zi, mi, bx, by, bz, m, eps2, g, c, h);
         else
-            sym_vjp_block<K, KB + 1, KB, false>(L, lane, sp, sa, xi, yi, zi, mi, bx, by, bz, m, eps2, g, c, h);
+            sym_vjp_block<K, KB + 1, KB, false>(L, lane, t0, steps, sp, sa, xi, yi, zi, mi, bx, by, bz, m, eps2, g, c, h);
         if constexpr (KB > 0) {
             kahan1(g[KB][0], c[KB][0], h.x);
             kahan1(g[KB][1], c[KB][1], h.y);
@@ -203,17 +207,17 @@ __device__ __forceinline__ void sym_vjp_own_at(int kb, bool uni, SymVjpLds& L, i
         // through a pointer to slot KB, which would put the sums in memory
         asm volatile("; own block %0" : : "n"(KB));
     } else if constexpr (KB + 1 < K) {
-        sym_vjp_own_at<K, KB + 1>(kb, uni, L, lane, sp, sa, xi, yi, zi, mi, bx, by, bz, m, eps2, g, c);
+        sym_vjp_own_at<K, KB + 1>(kb, uni, L, lane, t0, steps, sp, sa, xi, yi, zi, mi, bx, by, bz, m, eps2, g, c);
     }
 }
 
 // The work of wave r of wave block w of one system.  jrec: two float4 per
 // body {x,y,z,m} {ax,ay,az,0}, n_pad = NW*64*K bodies; ipart: [R][n_pad]
-// float4; jpart: [NW][NW/2][64K] float4.
-template <int K>
+// float4; jpart: [NW][NW/2][64K] float4, SPLIT: [NW][R][J][64] (SymSplit).
+template <int K, bool SPLIT>
 __device__ __forceinline__ void sym_vjp_wave(const float4* __restrict__ jrec, int NW, int R, int w, int r,
                                              float eps2, float4* __restrict__ ipart,
-                                             float4* __restrict__ jpart, SymVjpLds& L, int lane)
+                                             float4* __restrict__ jpart, SymVjpLds& L, int lane, int rs = 1)
 {
     const int half = NW / 2;
     const int n_pad = NW * 64 * K;
@@ -237,16 +241,34 @@ __device__ __forceinline__ void sym_vjp_wave(const float4* __restrict__ jrec, in
         tuni = tuni && mi[k] == m0;
     // sub-unit su = (unit u, source block kb): u = 0 is the wave block's own
     // sources, u = 1 + d the wave block d + 1 places round
-    const int Q = (half + 1) * K;
-    const int q0 = (int)((long long)Q * r / R), q1 = (int)((long long)Q * (r + 1) / R);
-    for (int su = q0; su < q1; ++su) {
+    int qf, ql, c0 = 0, c1 = 0, J = 0;
+    if constexpr (SPLIT) {
+        const SymSplit split(NW, w, K, R, rs);
+        c0 = split.first(r);
+        c1 = split.first(r + 1);
+        qf = c0 / rs;
+        ql = (c1 + rs - 1) / rs;
+        J = SymSplit::records(NW, K, R, rs);
+    } else {
+        const int Q = (half + 1) * K;
+        qf = (int)((long long)Q * r / R);
+        ql = (int)((long long)Q * (r + 1) / R);
+    }
+    for (int su = qf; su < ql; ++su) {
+        // rotation steps [t0, t0 + steps): all but for the first and last sub-unit
+        int t0 = 0, steps = 64;
+        if constexpr (SPLIT) {
+            const int a = su == qf ? c0 - su * rs : 0, e = su + 1 == ql ? c1 - su * rs : rs;
+            t0 = a * (64 / rs);
+            steps = (e - a) * (64 / rs);
+        }
         const int u = su / K, kb = su - u * K;
         if (u == 0) {
             // own block kb: two-sided against the lower target slots
             const int b = w * 64 * K + kb * 64 + lane;
             const float4 sp = jrec[2 * b], sa = jrec[2 * b + 1];
             const bool uni = __ballot(tuni && sp.w == m0) == ~0ull;
-            sym_vjp_own_at<K>(kb, uni, L, lane, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c);
+            sym_vjp_own_at<K>(kb, uni, L, lane, t0, steps, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c);
             continue;
         }
         const int d = u - 1;
@@ -259,10 +281,11 @@ __device__ __forceinline__ void sym_vjp_wave(const float4* __restrict__ jrec, in
         const float4 sp = jrec[2 * b], sa = jrec[2 * b + 1];
         float4 h;
         if (__ballot(tuni && sp.w == m0) == ~0ull)
-            sym_vjp_block<K, K, K, true>(L, lane, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c, h);
+            sym_vjp_block<K, K, K, true>(L, lane, t0, steps, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c, h);
         else
-            sym_vjp_block<K, K, K, false>(L, lane, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c, h);
-        jpart[((size_t)w * half + d) * (64 * K) + kb * 64 + lane] = h;
+            sym_vjp_block<K, K, K, false>(L, lane, t0, steps, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c, h);
+        jpart[SPLIT ? (((size_t)w * R + r) * J + (su - qf)) * 64 + lane
+                    : ((size_t)w * half + d) * (64 * K) + kb * 64 + lane] = h;
     }
 #pragma unroll
     for (int k = 0; k < K; ++k)
@@ -274,13 +297,14 @@ __device__ __forceinline__ void sym_vjp_wave(const float4* __restrict__ jrec, in
 template <int K>
 __global__ __launch_bounds__(256, 2) void sym_vjp_kernel(const float4* __restrict__ jrec, int NW, int R,
                                                       float eps2, float4* __restrict__ ipart,
-                                                      float4* __restrict__ jpart)
+                                                      float4* __restrict__ jpart, int rs)
 {
     __shared__ SymVjpLds lds[4];
     const int gw = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     if (gw >= NW * R)
         return;  // whole waves only
-    sym_vjp_wave<K>(jrec, NW, R, gw / R, gw % R, eps2, ipart, jpart, lds[threadIdx.x >> 6], threadIdx.x & 63);
+    sym_vjp_wave<K, true>(jrec, NW, R, gw / R, gw % R, eps2, ipart, jpart, lds[threadIdx.x >> 6], threadIdx.x & 63,
+                          rs);
 }
 
 // Batched systems: each wave runs items in the schedule of batch_next_item
@@ -300,7 +324,7 @@ __global__ __launch_bounds__(256, 2) void batch_sym_vjp_kernel(BatchSymGeom g, i
     for (int it = batch_next_item(g, gw, pos, lane); it >= 0; it = batch_next_item(g, gw, pos, lane)) {
         const int4 item = g.items[it];  // (system, wave block, split, splits)
         const int s = item.x;
-        sym_vjp_wave<K>(jrec + 2 * (size_t)g.off[s], g.nw[s], item.w, item.y, item.z, eps2,
+        sym_vjp_wave<K, false>(jrec + 2 * (size_t)g.off[s], g.nw[s], item.w, item.y, item.z, eps2,
                         ipart + g.vipo[s], jpart + g.vjpo[s], lds[threadIdx.x >> 6], lane);
     }
 }
@@ -310,14 +334,14 @@ __global__ __launch_bounds__(256, 2) void batch_sym_vjp_kernel(BatchSymGeom g, i
 template <int T>
 __global__ __launch_bounds__(256) void sym_vjp_reduce_kernel(const float4* __restrict__ ipart,
                                                              const float4* __restrict__ jpart, int n,
-                                                             int NW, int R, int K,
+                                                             int NW, int R, int K, int rs,
                                                              double* __restrict__ xbar3,
                                                              double* __restrict__ mbar)
 {
     int b, t;
     sym_reduce_lane<T>(b, t);
     double s[4];
-    sym_split_sum<T, false>(ipart, jpart, b < n ? b : n - 1, NW, R, K, t, s);
+    sym_split_sum<T, true>(ipart, jpart, b < n ? b : n - 1, NW, R, K, t, s, rs);
     if (b < n && t == 0) {
         xbar3[3 * (size_t)b + 0] += s[0];
         xbar3[3 * (size_t)b + 1] += s[1];
@@ -350,30 +374,32 @@ __global__ __launch_bounds__(256) void batch_sym_vjp_reduce_kernel(BatchSymGeom 
 }
 
 constexpr int kSymVjpK = 4;
+constexpr int kSymVjpRs = 16;  // rotation chunks per sub-unit, single systems
 
 int sym_vjp_splits(int n_pad, int cu_count)
 {
-    // ~16 waves per SIMD, at least one source block per wave, at most 32
-    // splits (sweeps of R on MI355X: for the adjoint at N = 16384, 50 steps,
-    // checkpoint every 10, with the segment recomputes beside the VJP steps,
-    // 32 is 2.6% faster than 48 and 0.6% faster than 64; at 65536 16..64 are
-    // the same within noise; N = 262144 takes R = 16 either way)
+    // Two waves for every SIMD, that start together and end together but for a
+    // chunk of 4 steps (a third wave on a SIMD runs unpaired); at most
+    // 128, whose target-side records the reduction reads for each body, and at
+    // least 3 chunks each.  From 40960 bodies 32: there the waves drift apart
+    // over the chip and shorter ones, several in turn, fill its end.  Adjoint
+    // of 20 steps, ms, against 32 waves of whole sub-units: N = 4096 0.79
+    // (1.22), 8192 1.40 (1.93), 16384 3.48 (3.85), 32768 11.55 (12.37); 10
+    // steps at 65536 21.75 (21.85; with R = 16 22.4).  Chunks of 8 steps are
+    // the same within 2%, 4096 and 6144 waves up to 10% slower at 8192.
     const int NW = n_pad / (64 * kSymVjpK);
-    const int want = (cu_count > 0 ? cu_count : 256) * 4 * 16;
-    int R = (want + NW - 1) / NW;
-    const int sub = (NW / 2 + 1) * kSymVjpK;
-    if (R > sub)
-        R = sub;
-    if (R > 32)
+    int R = (cu_count > 0 ? cu_count : 256) * 8 / NW;
+    if (R < 16)
         R = 32;
-    return R < 1 ? 1 : R;
+    const int most = SymSplit(NW, 0, kSymVjpK, 1, kSymVjpRs).chunks / 3;
+    return R < most ? (R < 128 ? R : 128) : (most < 128 ? most : 128);
 }
 
 size_t sym_vjp_ipart_float4s(int n_pad, int R) { return (size_t)R * n_pad; }
-size_t sym_vjp_jpart_float4s(int n_pad)
+size_t sym_vjp_jpart_float4s(int n_pad, int R)
 {
     const int NW = n_pad / (64 * kSymVjpK);
-    return (size_t)NW * (NW / 2) * 64 * kSymVjpK;
+    return (size_t)NW * R * SymSplit::records(NW, kSymVjpK, R, kSymVjpRs) * 64;
 }
 bool sym_vjp_applies(int n_pad) { return n_pad % (128 * kSymVjpK) == 0; }
 
@@ -385,18 +411,18 @@ hipError_t launch_sym_vjp(const float4* jrec, int n, int n_pad, float eps2, int 
     const int NW = n_pad / (64 * kSymVjpK);
     const int waves = NW * R;
     hipLaunchKernelGGL((sym_vjp_kernel<kSymVjpK>), dim3((waves + 3) / 4), dim3(256), 0, st, jrec, NW, R,
-                       eps2, ipart, jpart);
+                       eps2, ipart, jpart, kSymVjpRs);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return e;
     const int T = sym_reduce_lanes(n);
     const dim3 rgrid((unsigned)(((long long)n * T + 255) / 256));
     switch (T) {
-    case 1: hipLaunchKernelGGL(sym_vjp_reduce_kernel<1>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, xbar3, mbar); break;
-    case 2: hipLaunchKernelGGL(sym_vjp_reduce_kernel<2>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, xbar3, mbar); break;
-    case 4: hipLaunchKernelGGL(sym_vjp_reduce_kernel<4>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, xbar3, mbar); break;
-    case 8: hipLaunchKernelGGL(sym_vjp_reduce_kernel<8>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, xbar3, mbar); break;
-    default: hipLaunchKernelGGL(sym_vjp_reduce_kernel<16>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, xbar3, mbar); break;
+    case 1: hipLaunchKernelGGL(sym_vjp_reduce_kernel<1>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar); break;
+    case 2: hipLaunchKernelGGL(sym_vjp_reduce_kernel<2>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar); break;
+    case 4: hipLaunchKernelGGL(sym_vjp_reduce_kernel<4>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar); break;
+    case 8: hipLaunchKernelGGL(sym_vjp_reduce_kernel<8>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar); break;
+    default: hipLaunchKernelGGL(sym_vjp_reduce_kernel<16>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar); break;
     }
     return hipGetLastError();
 }
