@@ -30,11 +30,24 @@ constexpr int kWs[3] = {4, 8, 16};  // waves per work item of the one-pass kerne
 // waves through an atomic work counter (4), or one wave per item for the
 // hardware dispatcher to place (5).
 constexpr int kSymPersist = 3, kSymFlat = 4, kSels = 5;
-// Work units (K source blocks of 64) per symmetric item.  With the two
-// concurrent system groups, 3 ran the 256-system graph 1.2% faster forward
-// and 2.5% faster forward + adjoint than 2 (MI355X, tile 5; 1 and 4 in
-// between).
-constexpr int kSymUnitsPerItem = 3;
+// Sub-units (64 sources against a wave block) per symmetric item: the fewest
+// that give a chip's worth of items, since a target-side record of each item is
+// written and read.  20 steps forward and adjoint, tile 5, ms, systems of 256
+// to 8192 bodies (mean 2300), by sub-units per item:
+//   systems     1      2      3      4      6      8     12     16
+//         8   1.46   2.01   2.62   3.23   4.50   5.60   8.03   9.10
+//        20   3.75   3.72   3.74   4.12   4.83   6.07   8.56  11.11
+//        48   6.39   6.31   6.16   6.20   6.56   6.88   8.93  11.26
+//        96  14.25  13.72  13.71  13.91  13.61  13.76  14.64  14.61
+//       160  20.63  19.36  19.30  19.28  19.19  19.01  19.36  19.89
+//       256  31.52  29.22  28.85  28.79  28.36  28.28  28.19  28.31
+// Up to 131072 bodies in all the split is the system's alone (1, or a 8192nd
+// of a larger system's sub-units), and so are its bits.
+int sym_item_subunits(long long total_bodies, long long system_subunits)
+{
+    const long long least = total_bodies < (1 << 17) ? 1 : (total_bodies < (1 << 18) ? 6 : 8);
+    return (int)std::max(least, system_subunits / 8192);
+}
 // The per-system baseline (mode 1) spreads its launches over this many streams,
 // as the reference runs one task with its own stream per system; 4 is the
 // number of hardware queues a process gets by default.
@@ -43,10 +56,13 @@ constexpr int kAuxStreams = 4;
 // of about equal pair count, each run on a stream of its own inside the
 // captured graph, so that one group's work fills the tail of the other's
 // steps (a step ends with the last long items, then the reduction).  On
-// MI355X, 256 systems of 256..8192 bodies: two groups ran the 20-step graph
-// 6.6% faster forward and 7.7% faster forward + adjoint than one; three or
-// four groups were within 1.3% of two.
+// MI355X, 20 steps forward and adjoint of systems of 256..8192 bodies, one
+// group against two: 256 systems 30.5 to 29.2 ms, 96 14.3 to 13.7, but 20
+// systems 3.64 to 3.75 and 8 1.25 to 1.46, where twice the launches cost more
+// than the tails; three groups are within 2% of two.  Below kOneGroup bodies
+// in all there is one.
 constexpr int kGroups = 2;
+constexpr long long kOneGroup = 1 << 16;
 
 template <typename T>
 int dalloc(T** p, size_t count)
@@ -277,8 +293,8 @@ void schedule(const utcnb_batch* b, int W, int blocks, std::vector<int2>& items,
 }
 
 // Symmetric kernels: per system NW = npad / kBatchSymAlign wave blocks, each
-// with K (NW/2 + 1) (unit, source block) sub-units split over R waves (about
-// kSymUnitsPerItem units each); an item's cost is its number of sub-units.
+// with K (NW/2 + 1) (unit, source block) sub-units split over R waves
+// (sym_item_subunits each); an item's cost is its number of sub-units.
 // Items (system, wave block, split, R) are listed longest first; persistent
 // waves take them in that order through an atomic work counter, or each item
 // gets a wave of its own.
@@ -304,7 +320,7 @@ void plan_sym(const utcnb_batch* b, int persistent_waves, SymPlan& P)
             ++grp;
         const int NW = b->npad[s] / kBatchSymAlign;
         const int sub = (NW / 2 + 1) * kBatchSymK;  // (unit, source block) sub-units per wave block
-        const int per = kSymUnitsPerItem * kBatchSymK;
+        const int per = sym_item_subunits(b->total, (long long)NW * sub);
         const int R = std::max(1, (sub + per - 1) / per);
         P.nw.push_back(NW);
         P.rs.push_back(R);
@@ -350,13 +366,13 @@ void plan_sym(const utcnb_batch* b, int persistent_waves, SymPlan& P)
     }
 }
 
-// Splits the systems into ngroups = min(kGroups, nsys) contiguous groups of
+// Splits the systems into ngroups (at most kGroups and nsys) contiguous groups of
 // about equal pair count: group g ends at the first system where the running
 // sum of n_pad^2 reaches (g+1)/ngroups of the total, or just before it,
 // whichever is nearer, keeping every group non-empty.
 void split_groups(utcnb_batch* b)
 {
-    b->ngroups = std::min(kGroups, b->nsys);
+    b->ngroups = b->total < kOneGroup ? 1 : std::min(kGroups, b->nsys);
     std::vector<double> pre(b->nsys + 1, 0.0);
     for (int s = 0; s < b->nsys; ++s)
         pre[s + 1] = pre[s] + (double)b->npad[s] * b->npad[s];
