@@ -597,12 +597,18 @@ void sym_share_blocks(int NW, int shares, int share, int* w0, int* w1)
 
 int sym_share_splits(int nw_share, int K, int NW)
 {
-    // about 32768 waves (ten rounds of the chip's 256 CUs x 4 SIMDs x 3 waves
+    // about 12288 waves (four rounds of the chip's 256 CUs x 4 SIMDs x 3 waves
     // of this kernel), every wave with the same number u of the Q sub-units
-    // of its wave block (the last one of a block fewer): u = Q nw / 32768,
-    // R_share = ceil(Q / u)
+    // of its wave block (the last one of a block fewer): u = Q nw / 12288,
+    // R_share = ceil(Q / u).  Fewer waves leave a longer end, more leave more
+    // target-side records for the finish to read.  Pairs and finish, us, by
+    // waves:         4096   6144   8192  12288  16384  32768
+    //   131072, 1/8   459    420    425    412    415    432
+    //   131072, 1/2  1729   1587   1545   1406   1457   1446
+    //   262144, 1/8  1712   1579   1532   1393   1444   1437
+    //    65536, 1/4   251    235    235    236    237    239
     const long long Q = (long long)K * (NW / 2 + 1);
-    long long u = Q * nw_share / 32768;
+    long long u = Q * nw_share / 12288;
     if (u < 1)
         u = 1;
     return (int)((Q + u - 1) / u);
