@@ -20,10 +20,13 @@
 // combined in FP64; otherwise plain FP32 throughout (the plain FP32 path).
 // Pair arithmetic as in stream_sources: 12 VALU instructions and a root per
 // ordered pair, the roots of 8 pairs together (rsq_group.h), plus one LDS read
-// per source shared by the lane's A targets.  Per step, mixed: N = 8192 23.3 us
-// (27.3 with a root per pair), 6001 16.5 (21.2; 18.3 with 32 targets per
-// workgroup instead of 24), 4096 8.9 (9.6); below that the launch and the copy
-// into LDS bound it (N = 1024: 4.0 us either way; 3.7 with the lane sums in registers).
+// per source shared by the lane's A targets.  Per step, mixed: N = 8192 22.1 us
+// (27.3 with a root per pair), 6001 15.1 (21.2; 18.3 with 32 targets per
+// workgroup instead of 24), 4096 8.2 (9.6), 2000 4.7, 1000 3.4.  Up to 2048
+// bodies the launch, the copy into LDS and the ends of the sums bound it: lane
+// sums by shuffles took 4.0 at 1000, and the copy through registers, a load and
+// its store in turn, 3.7 at 1000, 8.8 at 4096 and 23.3 at 8192 (all loads into
+// registers first, in a run-time number, went through scratch: 4.7, 13.0, 32.3).
 #pragma once
 
 #include <type_traits>
@@ -42,7 +45,7 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
     using Acc = typename std::conditional<COMP, double, float>::type;
     __shared__ float4 sh[CAP];
     __shared__ Acc red[W][TW][3];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int t = lane % TL, g = lane / TL;
     const int tgt0 = blockIdx.x * TW;
     // the epilogue's state loads, issued before the pair work (thread j < TW
@@ -59,8 +62,12 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
         px[a] = p.x; py[a] = p.y; pz[a] = p.z;
         hx[a] = hy[a] = hz[a] = cx[a] = cy[a] = cz[a] = 0.f;
     }
-    for (int k = threadIdx.x; k < n_pad; k += 64 * W)
-        sh[k] = src[k];
+    // every load of the copy in flight at once, past the registers: a wave
+    // fills 64 consecutive LDS slots with one load
+    for (int k = wave * 64; k < n_pad; k += 64 * W)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + k + lane),
+                                         (__attribute__((address_space(3))) void*)&sh[k], 16, 0, 0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
 
     const int split = wave * G + g;
