@@ -145,8 +145,8 @@ hipError_t launch_fp32_step(const StepArgs& a, const float4* pos_old, float4* po
         return launch_sym(tile_get(a.tile), a.newton, false, pos_old, a.n, a.n_pad, a.eps2f, a.ipart,
                           a.jpart, epi, st);
     if (a.newton)
-        return launch_force<false, true>(a.tile, pos_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
-    return launch_force<false, false>(a.tile, pos_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+        return launch_force<false, true>(a.tile, pos_old, a.n, a.n_pad, a.n_pad, a.eps2f, a.ipart, epi, st);
+    return launch_force<false, false>(a.tile, pos_old, a.n, a.n_pad, a.n_pad, a.eps2f, a.ipart, epi, st);
 }
 
 hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* snap_new,
@@ -160,8 +160,8 @@ hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* 
         return launch_sym(tile_get(a.tile), a.newton, true, snap_old, a.n, a.n_pad, a.eps2f, a.ipart,
                           a.jpart, epi, st);
     if (a.newton)
-        return launch_force<true, true>(a.tile, snap_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
-    return launch_force<true, false>(a.tile, snap_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+        return launch_force<true, true>(a.tile, snap_old, a.n, a.n_pad, a.n_pad, a.eps2f, a.ipart, epi, st);
+    return launch_force<true, false>(a.tile, snap_old, a.n, a.n_pad, a.n_pad, a.eps2f, a.ipart, epi, st);
 }
 
 // One-pass tile for a slice of nt targets against all sources (the
@@ -200,8 +200,8 @@ hipError_t launch_fp32_step_slice(const StepArgs& a, int tile, int i0, int nt, c
         return hipErrorInvalidValue;
     EpiFP32 epi{pos_old, pos_new, vel, (float)a.dt, (float)a.damping, a.kick};
     if (a.newton)
-        return launch_force_range<false, true>(tile, pos_old, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st);
-    return launch_force_range<false, false>(tile, pos_old, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st);
+        return launch_force_range<false, true>(tile, pos_old, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st);
+    return launch_force_range<false, false>(tile, pos_old, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st);
 }
 
 hipError_t launch_mixed_step_slice(const StepArgs& a, int tile, int i0, int nt, const float4* snap_old,
@@ -211,8 +211,8 @@ hipError_t launch_mixed_step_slice(const StepArgs& a, int tile, int i0, int nt, 
         return hipErrorInvalidValue;
     EpiMixed epi{pos, vel, snap_new, a.dt, a.damping, a.kick};
     if (a.newton)
-        return launch_force_range<true, true>(tile, snap_old, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st);
-    return launch_force_range<true, false>(tile, snap_old, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st);
+        return launch_force_range<true, true>(tile, snap_old, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st);
+    return launch_force_range<true, false>(tile, snap_old, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st);
 }
 
 hipError_t launch_fp32_accel_slice(const StepArgs& a, int tile, int i0, int nt, const float4* src,
@@ -222,16 +222,17 @@ hipError_t launch_fp32_accel_slice(const StepArgs& a, int tile, int i0, int nt, 
         return hipErrorInvalidValue;
     EpiAccel epi{acc3, i0};
     if (compensated)
-        return a.newton ? launch_force_range<true, true>(tile, src, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st)
-                        : launch_force_range<true, false>(tile, src, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st);
-    return a.newton ? launch_force_range<false, true>(tile, src, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st)
-                    : launch_force_range<false, false>(tile, src, i0, nt, a.n_pad, a.eps2f, a.part_ws, epi, st);
+        return a.newton ? launch_force_range<true, true>(tile, src, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st)
+                        : launch_force_range<true, false>(tile, src, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st);
+    return a.newton ? launch_force_range<false, true>(tile, src, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st)
+                    : launch_force_range<false, false>(tile, src, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st);
 }
 
 hipError_t launch_fp32_accel(const StepArgs& a, const float4* src, bool compensated,
                              double* acc3, hipStream_t st)
 {
     EpiAccel epi{acc3};
+    const int nsrc = a.nsrc > 0 ? a.nsrc : a.n_pad;
     if (tile_get(a.tile).sym && a.chunks > 0) {
         if (!compensated)
             return hipErrorInvalidValue;  // the chunked step sums its partials in FP64
@@ -243,12 +244,12 @@ hipError_t launch_fp32_accel(const StepArgs& a, const float4* src, bool compensa
                           a.jpart, epi, st);
     if (compensated) {
         if (a.newton)
-            return launch_force<true, true>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
-        return launch_force<true, false>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+            return launch_force<true, true>(a.tile, src, a.n, a.n_pad, nsrc, a.eps2f, a.ipart, epi, st);
+        return launch_force<true, false>(a.tile, src, a.n, a.n_pad, nsrc, a.eps2f, a.ipart, epi, st);
     }
     if (a.newton)
-        return launch_force<false, true>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
-    return launch_force<false, false>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+        return launch_force<false, true>(a.tile, src, a.n, a.n_pad, nsrc, a.eps2f, a.ipart, epi, st);
+    return launch_force<false, false>(a.tile, src, a.n, a.n_pad, nsrc, a.eps2f, a.ipart, epi, st);
 }
 
 }  // namespace utcnb

@@ -6,7 +6,8 @@
 // one-pass kernels give every wave 64 targets, so a small system has too few
 // waves to fill the chip and each wave waits on its scalar source loads.
 // Here a workgroup of W waves owns TW = TL * A targets and all sources:
-//  * the workgroup copies every source body (n_pad <= CAP) into LDS once;
+//  * the workgroup copies every source body (n_pad <= CAP) into LDS once, or
+//    the nsrc that src holds and padding bodies after them;
 //  * lane l = t + TL * g of wave w holds targets t, t + TL, ..., t + (A-1) TL
 //    of the workgroup and sums sources split, split + SPL, split + 2 SPL, ...
 //    with split = w * G + g, G = 64 / TL source groups per wave and SPL =
@@ -39,7 +40,7 @@ constexpr int kSmallBlock = 32;  // sources per plain partial of a lane (COMP)
 
 template <int A, int TL, int W, int CAP, bool COMP, bool NEWTON, class Epi>
 __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __restrict__ src, int i0, int nt,
-                                                             int n_pad, float eps2, Epi epi)
+                                                             int n_pad, int nsrc, float eps2, Epi epi)
 {
     constexpr int G = 64 / TL, TW = TL * A, SPL = G * W;
     using Acc = typename std::conditional<COMP, double, float>::type;
@@ -64,9 +65,13 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
     }
     // every load of the copy in flight at once, past the registers: a wave
     // fills 64 consecutive LDS slots with one load
-    for (int k = wave * 64; k < n_pad; k += 64 * W)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + k + lane),
-                                         (__attribute__((address_space(3))) void*)&sh[k], 16, 0, 0);
+    for (int k = wave * 64; k < n_pad; k += 64 * W) {
+        if (k + lane < nsrc)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + k + lane),
+                                             (__attribute__((address_space(3))) void*)&sh[k], 16, 0, 0);
+        else
+            sh[k + lane] = make_float4(kPadCoord, kPadCoord, kPadCoord, 0.f);
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
 
@@ -168,7 +173,7 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
 // Targets [i0, i0 + nt) of a system whose n_pad sources fit the tile's LDS
 // capacity CAP.
 template <int A, int TL, int W, int CAP, bool COMP, bool NEWTON, class Epi>
-hipError_t launch_small_tile(const float4* src, int i0, int nt, int n_pad, float eps2, const Epi& epi,
+hipError_t launch_small_tile(const float4* src, int i0, int nt, int n_pad, int nsrc, float eps2, const Epi& epi,
                              hipStream_t st)
 {
     static_assert(A <= 3 && 64 % TL == 0 && kPadJ / 8 % ((64 / TL) * W) == 0,
@@ -179,7 +184,7 @@ hipError_t launch_small_tile(const float4* src, int i0, int nt, int n_pad, float
     constexpr int TW = TL * A;
     const int blocks = (nt + TW - 1) / TW;
     hipLaunchKernelGGL((small_force_kernel<A, TL, W, CAP, COMP, NEWTON, Epi>), dim3(blocks), dim3(64 * W), 0, st,
-                       src, i0, nt, n_pad, eps2, epi);
+                       src, i0, nt, n_pad, nsrc, eps2, epi);
     return hipGetLastError();
 }
 
