@@ -57,13 +57,13 @@ const Tile& tile_get(int id) { return kTiles[id]; }
 //   N =  14336: sym8w2048x8 51.7, sym4r128 52.3, sym8r64x8 54.0 us  (sym4r64 56.1)
 //   N =  12288: sym4r64x2 42.6, sym8w2048x8 42.8, sym4r64x8 43.2 us  (sym4r64 43.7)
 //   N =   9001: sym4w2048x8 32.5, sym8w2048x8 33.3, sym4r128 34.6 us  (sym4r64x2 37.5)
-//   N =   8192: sm2t16w16n8k 23.3, sm1t16w16n8k 26.4, sym4r128 27.9 us
-//   N =   7168: sm2t16w16n8k 20.9, sm4t8w16n8k 23.1, sm1t16w16n8k 23.9 us
-//   N =   6144: sm3t8w16n8k 16.6, sm2t16w16n8k 18.3, sm6t4w16n8k 19.4 us  (sym2r64 20.7)
-//   N =   5120: sm3t8w16n8k 14.5, sm5t4w16n8k 15.3, sm2t16w16n8k 15.8 us
-//   N =   4096: sm1t16w16n8k 8.80, sm1t16w16n4k 8.84, sm1t8w16n8k 11.3 us  (sym2r64 16.4)
-//   N =   2048: sm1t8w16n8k 5.12, sm1t8w8n2k 5.16, sm1t4w8n2k 5.67 us  (sym2r64x2 12.5)
-//   N =   1024: sm1t4w8n2k 4.04, sm1t8w8n2k 4.10, sm1t8w16n8k 4.15 us  (sym2r128x4 12.1)
+//   N =   8192: sm2t16w16n8k 22.1, sm1t16w16n8k 25.1, sm1t8w16n8k 30.1 us  (sym4r64x16 24.2)
+//   N =   7168: sm2t16w16n8k 19.8, sm1t16w16n8k 22.5, sm1t8w16n8k 27.3 us
+//   N =   6144: sm3t8w16n8k 15.2, sm2t16w16n8k 17.4, sm1t8w16n8k 19.3 us  (sym2r64 20.7)
+//   N =   5120: sm3t8w16n8k 13.4, sm2t16w16n8k 15.1, sm1t8w16n8k 17.1 us
+//   N =   4096: sm1t16w16n4k 8.2, sm1t16w16n8k 8.2, sm1t8w16n8k 10.4 us  (sym2r64 16.4)
+//   N =   2048: sm1t8w8n2k 4.4, sm1t8w16n8k 4.7, sm1t4w8n2k 4.9 us  (sym2r64x2 12.5)
+//   N =   1024: sm1t4w8n2k 3.5, sm1t8w8n2k 3.7, sm1t8w16n8k 3.9 us  (sym2r128x4 12.1)
 // (sym8r48, sym8r24, other R and chunk counts for K = 2, 4 and 8 and several
 // other small-system shapes were swept and are not in the table: 4 to 8 targets
 // per lane, 4 target lanes with 16 waves, 8 waves per workgroup.)  Up to 8192
@@ -100,7 +100,7 @@ int tile_default(int64_t n, int cu_count, size_t partial_budget)
     if (n <= 1024)
         return 28;  // sm1t4w8n2k
     if (n <= 2048)
-        return 30;  // sm1t8w16n8k
+        return 29;  // sm1t8w8n2k
     if (n <= 4096)
         return 31;  // sm1t16w16n4k
     if (n <= 6144)
@@ -145,8 +145,8 @@ hipError_t launch_fp32_step(const StepArgs& a, const float4* pos_old, float4* po
         return launch_sym(tile_get(a.tile), a.newton, false, pos_old, a.n, a.n_pad, a.eps2f, a.ipart,
                           a.jpart, epi, st);
     if (a.newton)
-        return launch_force<false, true>(a.tile, pos_old, a.n, a.n_pad, a.n_pad, a.eps2f, a.ipart, epi, st);
-    return launch_force<false, false>(a.tile, pos_old, a.n, a.n_pad, a.n_pad, a.eps2f, a.ipart, epi, st);
+        return launch_force<false, true>(a.tile, pos_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+    return launch_force<false, false>(a.tile, pos_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
 }
 
 hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* snap_new,
@@ -160,8 +160,8 @@ hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* 
         return launch_sym(tile_get(a.tile), a.newton, true, snap_old, a.n, a.n_pad, a.eps2f, a.ipart,
                           a.jpart, epi, st);
     if (a.newton)
-        return launch_force<true, true>(a.tile, snap_old, a.n, a.n_pad, a.n_pad, a.eps2f, a.ipart, epi, st);
-    return launch_force<true, false>(a.tile, snap_old, a.n, a.n_pad, a.n_pad, a.eps2f, a.ipart, epi, st);
+        return launch_force<true, true>(a.tile, snap_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+    return launch_force<true, false>(a.tile, snap_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
 }
 
 // One-pass tile for a slice of nt targets against all sources (the
@@ -200,8 +200,8 @@ hipError_t launch_fp32_step_slice(const StepArgs& a, int tile, int i0, int nt, c
         return hipErrorInvalidValue;
     EpiFP32 epi{pos_old, pos_new, vel, (float)a.dt, (float)a.damping, a.kick};
     if (a.newton)
-        return launch_force_range<false, true>(tile, pos_old, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st);
-    return launch_force_range<false, false>(tile, pos_old, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st);
+        return launch_force_range<false, true>(tile, pos_old, i0, nt, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
+    return launch_force_range<false, false>(tile, pos_old, i0, nt, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
 }
 
 hipError_t launch_mixed_step_slice(const StepArgs& a, int tile, int i0, int nt, const float4* snap_old,
@@ -211,8 +211,8 @@ hipError_t launch_mixed_step_slice(const StepArgs& a, int tile, int i0, int nt, 
         return hipErrorInvalidValue;
     EpiMixed epi{pos, vel, snap_new, a.dt, a.damping, a.kick};
     if (a.newton)
-        return launch_force_range<true, true>(tile, snap_old, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st);
-    return launch_force_range<true, false>(tile, snap_old, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st);
+        return launch_force_range<true, true>(tile, snap_old, i0, nt, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
+    return launch_force_range<true, false>(tile, snap_old, i0, nt, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
 }
 
 hipError_t launch_fp32_accel_slice(const StepArgs& a, int tile, int i0, int nt, const float4* src,
@@ -222,17 +222,16 @@ hipError_t launch_fp32_accel_slice(const StepArgs& a, int tile, int i0, int nt, 
         return hipErrorInvalidValue;
     EpiAccel epi{acc3, i0};
     if (compensated)
-        return a.newton ? launch_force_range<true, true>(tile, src, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st)
-                        : launch_force_range<true, false>(tile, src, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st);
-    return a.newton ? launch_force_range<false, true>(tile, src, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st)
-                    : launch_force_range<false, false>(tile, src, i0, nt, a.n_pad, a.n_pad, a.eps2f, a.part_ws, epi, st);
+        return a.newton ? launch_force_range<true, true>(tile, src, i0, nt, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st)
+                        : launch_force_range<true, false>(tile, src, i0, nt, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
+    return a.newton ? launch_force_range<false, true>(tile, src, i0, nt, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st)
+                    : launch_force_range<false, false>(tile, src, i0, nt, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
 }
 
 hipError_t launch_fp32_accel(const StepArgs& a, const float4* src, bool compensated,
                              double* acc3, hipStream_t st)
 {
     EpiAccel epi{acc3};
-    const int nsrc = a.nsrc > 0 ? a.nsrc : a.n_pad;
     if (tile_get(a.tile).sym && a.chunks > 0) {
         if (!compensated)
             return hipErrorInvalidValue;  // the chunked step sums its partials in FP64
@@ -244,12 +243,12 @@ hipError_t launch_fp32_accel(const StepArgs& a, const float4* src, bool compensa
                           a.jpart, epi, st);
     if (compensated) {
         if (a.newton)
-            return launch_force<true, true>(a.tile, src, a.n, a.n_pad, nsrc, a.eps2f, a.ipart, epi, st);
-        return launch_force<true, false>(a.tile, src, a.n, a.n_pad, nsrc, a.eps2f, a.ipart, epi, st);
+            return launch_force<true, true>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+        return launch_force<true, false>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
     }
     if (a.newton)
-        return launch_force<false, true>(a.tile, src, a.n, a.n_pad, nsrc, a.eps2f, a.ipart, epi, st);
-    return launch_force<false, false>(a.tile, src, a.n, a.n_pad, nsrc, a.eps2f, a.ipart, epi, st);
+        return launch_force<false, true>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+    return launch_force<false, false>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
 }
 
 }  // namespace utcnb

@@ -6,8 +6,9 @@
 // one-pass kernels give every wave 64 targets, so a small system has too few
 // waves to fill the chip and each wave waits on its scalar source loads.
 // Here a workgroup of W waves owns TW = TL * A targets and all sources:
-//  * the workgroup copies every source body (n_pad <= CAP) into LDS once, or
-//    the nsrc that src holds and padding bodies after them;
+//  * the workgroup copies the n source bodies into LDS once, with padding
+//    after them to a whole number of the splits' root groups (256 to 1024
+//    bodies; at most CAP);
 //  * lane l = t + TL * g of wave w holds targets t, t + TL, ..., t + (A-1) TL
 //    of the workgroup and sums sources split, split + SPL, split + 2 SPL, ...
 //    with split = w * G + g, G = 64 / TL source groups per wave and SPL =
@@ -28,6 +29,8 @@
 // sums by shuffles took 4.0 at 1000, and the copy through registers, a load and
 // its store in turn, 3.7 at 1000, 8.8 at 4096 and 23.3 at 8192 (all loads into
 // registers first, in a run-time number, went through scratch: 4.7, 13.0, 32.3).
+// Padding to whole root groups instead of to 1024 bodies: 1100 4.6 to 4.0, 4200
+// 13.3 to 12.1, 7200 22.0 to 20.5.
 #pragma once
 
 #include <type_traits>
@@ -40,9 +43,12 @@ constexpr int kSmallBlock = 32;  // sources per plain partial of a lane (COMP)
 
 template <int A, int TL, int W, int CAP, bool COMP, bool NEWTON, class Epi>
 __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __restrict__ src, int i0, int nt,
-                                                             int n_pad, int nsrc, float eps2, Epi epi)
+                                                             int n, float eps2, Epi epi)
 {
     constexpr int G = 64 / TL, TW = TL * A, SPL = G * W;
+    constexpr int J = A == 1 ? 8 : A == 2 ? 4 : 2;  // sources per group of reciprocal roots
+    // the same number of sources for every split, whole groups: padding after n
+    const int iters = (n + SPL * J - 1) / (SPL * J) * J, fill = iters * SPL;
     using Acc = typename std::conditional<COMP, double, float>::type;
     __shared__ float4 sh[CAP];
     __shared__ Acc red[W][TW][3];
@@ -65,8 +71,8 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
     }
     // every load of the copy in flight at once, past the registers: a wave
     // fills 64 consecutive LDS slots with one load
-    for (int k = wave * 64; k < n_pad; k += 64 * W) {
-        if (k + lane < nsrc)
+    for (int k = wave * 64; k < fill; k += 64 * W) {
+        if (k + lane < n)
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + k + lane),
                                              (__attribute__((address_space(3))) void*)&sh[k], 16, 0, 0);
         else
@@ -76,7 +82,6 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
     __syncthreads();
 
     const int split = wave * G + g;
-    const int iters = n_pad / SPL;  // n_pad is a multiple of 1024 and SPL divides 128: a multiple of 8
     for (int b0 = 0; b0 < iters; b0 += kSmallBlock) {
         const int b1 = b0 + kSmallBlock < iters ? b0 + kSmallBlock : iters;
         float ax[A], ay[A], az[A];
@@ -88,7 +93,6 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
                 ax[a] = hx[a]; ay[a] = hy[a]; az[a] = hz[a];
             }
         }
-        constexpr int J = A == 1 ? 8 : A == 2 ? 4 : 2;  // sources per group of reciprocal roots
 #pragma unroll 1
         for (int i = b0; i < b1; i += J) {
             float rx[J * A], ry[J * A], rz[J * A], d2[J * A], y[J * A], m[J];
@@ -170,21 +174,21 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
     }
 }
 
-// Targets [i0, i0 + nt) of a system whose n_pad sources fit the tile's LDS
-// capacity CAP.
+// Targets [i0, i0 + nt) of a system whose n sources, padded, fit the tile's
+// LDS capacity CAP.
 template <int A, int TL, int W, int CAP, bool COMP, bool NEWTON, class Epi>
-hipError_t launch_small_tile(const float4* src, int i0, int nt, int n_pad, int nsrc, float eps2, const Epi& epi,
+hipError_t launch_small_tile(const float4* src, int i0, int nt, int n, float eps2, const Epi& epi,
                              hipStream_t st)
 {
     static_assert(A <= 3 && 64 % TL == 0 && kPadJ / 8 % ((64 / TL) * W) == 0,
                   "each split takes a multiple of 8 sources, in groups of 8 / A");
 
-    if (n_pad > CAP || n_pad % kPadJ != 0)
+    if (n < 1 || pad_j(n) > CAP)
         return hipErrorInvalidValue;
     constexpr int TW = TL * A;
     const int blocks = (nt + TW - 1) / TW;
     hipLaunchKernelGGL((small_force_kernel<A, TL, W, CAP, COMP, NEWTON, Epi>), dim3(blocks), dim3(64 * W), 0, st,
-                       src, i0, nt, n_pad, nsrc, eps2, epi);
+                       src, i0, nt, n, eps2, epi);
     return hipGetLastError();
 }
 

@@ -327,13 +327,13 @@ hipError_t launch_force_tile(const float4* src, int i0, int nt, int n_pad, float
 
 // Dispatch over the tile table (must match tile_get()); targets [i0, i0 + nt).
 // part: workspace of the tiles with source parts ([parts][nt][3] floats).
-// nsrc: bodies that src holds, if fewer than n_pad (small-system tiles only:
-// the others read n_pad).
+// n: the system's bodies (the small-system tiles read no more of src, the
+// others the n_pad padded ones).
 template <bool COMP, bool NEWTON, class Epi>
-hipError_t launch_force_range(int tile, const float4* src, int i0, int nt, int n_pad, int nsrc, float eps2, float* part,
+hipError_t launch_force_range(int tile, const float4* src, int i0, int nt, int n, int n_pad, float eps2, float* part,
                               const Epi& epi, hipStream_t st)
 {
-    if (nt < 1 || nsrc < 1 || (nsrc < n_pad && tile_get(tile).cap == 0))
+    if (nt < 1)
         return hipErrorInvalidValue;
     if (const int P = tile_get(tile).parts) {
         if (tile_get(tile).k == 1)
@@ -351,26 +351,26 @@ hipError_t launch_force_range(int tile, const float4* src, int i0, int nt, int n
     case 7: return launch_force_tile<1, 8, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
     case 8: return launch_force_tile<2, 8, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
     case 9: return launch_force_tile<1, 16, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
-    case 28: return launch_small_tile<1, 4, 8, 2048, COMP, NEWTON>(src, i0, nt, n_pad, nsrc, eps2, epi, st);
-    case 29: return launch_small_tile<1, 8, 8, 2048, COMP, NEWTON>(src, i0, nt, n_pad, nsrc, eps2, epi, st);
-    case 30: return launch_small_tile<1, 8, 16, 8192, COMP, NEWTON>(src, i0, nt, n_pad, nsrc, eps2, epi, st);
-    case 31: return launch_small_tile<1, 16, 16, 4096, COMP, NEWTON>(src, i0, nt, n_pad, nsrc, eps2, epi, st);
-    case 32: return launch_small_tile<1, 16, 16, 8192, COMP, NEWTON>(src, i0, nt, n_pad, nsrc, eps2, epi, st);
-    case 33: return launch_small_tile<2, 16, 16, 8192, COMP, NEWTON>(src, i0, nt, n_pad, nsrc, eps2, epi, st);
+    case 28: return launch_small_tile<1, 4, 8, 2048, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
+    case 29: return launch_small_tile<1, 8, 8, 2048, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
+    case 30: return launch_small_tile<1, 8, 16, 8192, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
+    case 31: return launch_small_tile<1, 16, 16, 4096, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
+    case 32: return launch_small_tile<1, 16, 16, 8192, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
+    case 33: return launch_small_tile<2, 16, 16, 8192, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
     case 34: return launch_force_tile<2, 16, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
     case 35: return launch_force_tile<4, 8, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
     case 36: return launch_force_tile<4, 16, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
-    case 39: return launch_small_tile<3, 8, 16, 8192, COMP, NEWTON>(src, i0, nt, n_pad, nsrc, eps2, epi, st);
+    case 39: return launch_small_tile<3, 8, 16, 8192, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
     default: return hipErrorInvalidValue;
     }
 }
 
 // All n bodies as targets.
 template <bool COMP, bool NEWTON, class Epi>
-hipError_t launch_force(int tile, const float4* src, int n, int n_pad, int nsrc, float eps2, float* part,
+hipError_t launch_force(int tile, const float4* src, int n, int n_pad, float eps2, float* part,
                         const Epi& epi, hipStream_t st)
 {
-    return launch_force_range<COMP, NEWTON>(tile, src, 0, n, n_pad, nsrc, eps2, part, epi, st);
+    return launch_force_range<COMP, NEWTON>(tile, src, 0, n, n, n_pad, eps2, part, epi, st);
 }
 
 }  // namespace utcnb

@@ -58,7 +58,6 @@ int sym_share_tile_default(int64_t n, int cu_count);
 struct StepArgs {
     int n;          // bodies
     int n_pad;      // padded j length (fast kernels)
-    int nsrc;       // field on a small-system tile: bodies the source array holds, if not n_pad (else 0)
     float eps2f;
     double eps2;
     double dt, damping;

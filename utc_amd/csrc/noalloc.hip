@@ -152,7 +152,6 @@ extern "C" int utcnb_accel_noalloc(const float* pos4, int n, double eps2, int pr
     const bool apart = pb + (size_t)n * sizeof(float4) <= ab || ab + (size_t)n * 3 * sizeof(double) <= pb;
     if (tl.cap > 0 && apart && pb % sizeof(float4) == 0) {
         src = (const float4*)pos4;
-        a.nsrc = n;
     } else {
         hipLaunchKernelGGL(copy_pad_kernel, dim3((unsigned)((n_pad + 255) / 256)), dim3(256), 0, st,
                            (const float4*)pos4, (float4*)base, n, (int)n_pad);
