@@ -261,6 +261,30 @@ int download4(utcnb_system* s, const T4* src, void* dst, int dtype, int where)
     return UTCNB_OK;
 }
 
+// Whether a kernel on the handle's device may read and write the n records of
+// 4 `dtype` values at p as vectors: memory of that device, on 16 bytes.  (The
+// runtime's copies also take other devices' memory and any alignment.)
+bool on_device(const utcnb_system* s, const void* p)
+{
+    hipPointerAttribute_t at;
+    if ((uintptr_t)p % 16 != 0)
+        return false;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice && at.device == s->device;
+}
+
+// Whether the n-record arrays a and b (of `ab` and `bb` bytes per record) overlap.
+bool overlap(const utcnb_system* s, const void* a, int ab, const void* b, int bb)
+{
+    if (!a || !b)
+        return false;
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return x < y + (size_t)s->n * bb && y < x + (size_t)s->n * ab;
+}
+
 }  // namespace
 
 extern "C" {
@@ -582,7 +606,18 @@ int utcnb_set_state(utcnb_system* s, const void* pos4, const void* vel4, int dty
     }
     s->cur = 0;
     int rc;
-    if (is_f32_state(s)) {
+    const bool f32 = is_f32_state(s);
+    void *p = f32 ? (void*)s->p32[0] : (void*)s->p64[0], *v = f32 ? (void*)s->v32 : (void*)s->v64;
+    float4* snap = s->cfg.precision == UTCNB_PREC_MIXED ? s->snap[0] : nullptr;
+    const int ib = dtype == UTCNB_F32 ? 16 : 32, sb = f32 ? 16 : 32;
+    if (where == UTCNB_DEVICE && vwhere == UTCNB_DEVICE && on_device(s, pos4) && on_device(s, vel4) &&
+        !overlap(s, pos4, ib, p, sb) && !overlap(s, pos4, ib, v, sb) && !overlap(s, pos4, ib, snap, 16) &&
+        !overlap(s, vel4, ib, p, sb) && !overlap(s, vel4, ib, v, sb) && !overlap(s, vel4, ib, snap, 16)) {
+        UTCNB_HIP(launch_state_copy(pos4, vel4, dtype == UTCNB_F32, p, v, f32, snap, s->n, s->stream));
+        s->has_state = true;
+        return UTCNB_OK;
+    }
+    if (f32) {
         rc = upload4(s, pos4, dtype, where, s->p32[0]);
         if (!rc)
             rc = upload4(s, vel4, vdtype, vwhere, s->v32);
@@ -612,7 +647,16 @@ int utcnb_get_state(utcnb_system* s, void* pos4, void* vel4, int dtype, int wher
     if ((dtype != UTCNB_F32 && dtype != UTCNB_F64) || (where != UTCNB_HOST && where != UTCNB_DEVICE))
         return fail(UTCNB_EINVAL, "utcnb_get_state: bad dtype or location");
     int rc = UTCNB_OK;
-    if (is_f32_state(s)) {
+    const bool f32 = is_f32_state(s);
+    const void *p = f32 ? (void*)s->p32[s->cur] : (void*)cur_p64(s), *v = f32 ? (void*)s->v32 : (void*)s->v64;
+    const int ob = dtype == UTCNB_F32 ? 16 : 32, sb = f32 ? 16 : 32;
+    if (where == UTCNB_DEVICE && pos4 && vel4 && on_device(s, pos4) && on_device(s, vel4) &&
+        !overlap(s, pos4, ob, vel4, ob) && !overlap(s, pos4, ob, p, sb) && !overlap(s, pos4, ob, v, sb) &&
+        !overlap(s, vel4, ob, p, sb) && !overlap(s, vel4, ob, v, sb)) {
+        UTCNB_HIP(launch_state_copy(p, v, f32, pos4, vel4, dtype == UTCNB_F32, nullptr, s->n, s->stream));
+        return UTCNB_OK;
+    }
+    if (f32) {
         if (pos4)
             rc = download4(s, s->p32[s->cur], pos4, dtype, where);
         if (!rc && vel4) {

@@ -248,6 +248,11 @@ hipError_t launch_snapshot(const double4* pos, float4* snap, int n, hipStream_t 
 // Type conversions between state arrays.
 hipError_t launch_f32_to_f64(const float4* src, double4* dst, int n, hipStream_t st);
 hipError_t launch_f64_to_f32(const double4* src, float4* dst, int n, hipStream_t st);
+// n records of 4 values, positions and velocities (vel null: positions only),
+// between FP32 and FP64 arrays on 16 bytes that do not overlap; the positions
+// also to snap (FP32) unless null.
+hipError_t launch_state_copy(const void* pos, const void* vel, bool from_f32, void* p, void* v, bool to_f32,
+                             float4* snap, int n, hipStream_t st);
 // FP64 diagnostics: kinetic, potential (pairs i<j) and momentum, accumulated
 // into out[5] = {K, W, Px, Py, Pz} (device, zeroed by the launcher).
 hipError_t launch_energy(const double4* pos, const double4* vel, int n, double eps2,
