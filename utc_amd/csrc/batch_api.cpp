@@ -616,11 +616,16 @@ hipError_t enqueue_run_sym(utcnb_batch* b, int nsteps, int ckpt, bool adj, int s
                 }
             }
             for (int t = s1 - 1; t >= s0; --t) {
-                ENQ(launch_adjoint_pre(true, b->segpos + T * (size_t)(t - s0) + b0, nullptr, (int)Tg, dt, damp,
-                                       kick, b->xbar + 3 * b0, b->vbar + 3 * b0, b->mbar + b0,
-                                       b->jrec + 2 * b0, sg));
+                // the first of a segment; the others' is done by the VJP's reduction
+                if (t == s1 - 1)
+                    ENQ(launch_adjoint_pre(true, b->segpos + T * (size_t)(t - s0) + b0, nullptr, (int)Tg, dt, damp,
+                                           kick, b->xbar + 3 * b0, b->vbar + 3 * b0, b->mbar + b0,
+                                           b->jrec + 2 * b0, sg));
+                AdjointNext next;
+                if (t > s0)
+                    next = {b->segpos + T * (size_t)(t - 1 - s0), dt, damp, kick, b->vbar, b->jrec};
                 ENQ(launch_batch_sym_vjp(b->sym_geom(sk, 1, g), b->snwaves[sk][g], (int)Tg, b->jrec,
-                                         (float)b->cfg.eps2, b->svipart, b->svjpart, b->xbar, b->mbar, sg));
+                                         (float)b->cfg.eps2, b->svipart, b->svjpart, b->xbar, b->mbar, next, sg));
             }
         }
 #undef ENQ

@@ -1234,6 +1234,7 @@ int utcnb_adjoint(utcnb_system* s, int nsteps, int ckpt_every, const double* tar
         const int s1 = (s0 + k < nsteps) ? s0 + k : nsteps;
         if (overlap && c < nck - 1)
             ADJ_CHECK(hipStreamWaitEvent(st, a.evrec[c % 2], 0));
+        bool pre_done = false;
         for (int t = s1 - 1; t >= s0; --t) {
             const double4* xs = segbuf(c) + n * (size_t)(t - s0);
             const double* acc = nullptr;
@@ -1248,12 +1249,19 @@ int utcnb_adjoint(utcnb_system* s, int nsteps, int ckpt_every, const double* tar
                 acc = s->scratch;
                 ++launches;
             }
-            ADJ_CHECK(launch_adjoint_pre(mixed, xs, acc, s->n, s->cfg.dt, s->cfg.damping,
-                                         s->cfg.kick, a.xbar, a.vbar, a.mbar, a.jrec, st));
-            if (mixed && a.vjp_r > 0)
+            if (!pre_done)
+                ADJ_CHECK(launch_adjoint_pre(mixed, xs, acc, s->n, s->cfg.dt, s->cfg.damping,
+                                             s->cfg.kick, a.xbar, a.vbar, a.mbar, a.jrec, st));
+            pre_done = false;
+            if (mixed && a.vjp_r > 0) {
+                AdjointNext next;
+                if (!refkick && t > s0) {  // the segment's step before, whose positions are there
+                    next = {xs - n, s->cfg.dt, s->cfg.damping, s->cfg.kick, a.vbar, (float4*)a.jrec};
+                    pre_done = true;
+                }
                 ADJ_CHECK(launch_sym_vjp((const float4*)a.jrec, s->n, s->n_pad, s->args.eps2f, a.vjp_r,
-                                         a.vjp_ipart, a.vjp_jpart, a.xbar, a.mbar, st));
-            else if (mixed)
+                                         a.vjp_ipart, a.vjp_jpart, a.xbar, a.mbar, next, st));
+            } else if (mixed)
                 ADJ_CHECK(launch_vjp_f32((const float4*)a.jrec, s->n, s->n_pad, s->cfg.eps2,
                                          a.xbar, a.mbar, s->cu_count, st));
             else

@@ -187,9 +187,19 @@ bool sym_vjp_applies(int n_pad);                 // n_pad a multiple of 512
 int sym_vjp_splits(int n_pad, int cu_count);     // waves per wave block
 size_t sym_vjp_ipart_float4s(int n_pad, int R);
 size_t sym_vjp_jpart_float4s(int n_pad, int R);
+// The per-body adjoint of the step before (launch_adjoint_pre without a field,
+// FP32 records), done by the reduction of a VJP: pos null = not.  The records
+// are those the VJP read.
+struct AdjointNext {
+    const double4* pos = nullptr;
+    double dt = 0.0, damping = 1.0;
+    int kick = 0;
+    double* vbar3 = nullptr;
+    float4* jrec = nullptr;
+};
 // xbar3 / mbar (first n bodies) += the pair sums; ipart / jpart are workspace.
 hipError_t launch_sym_vjp(const float4* jrec, int n, int n_pad, float eps2, int R, float4* ipart,
-                          float4* jpart, double* xbar3, double* mbar, hipStream_t st);
+                          float4* jpart, double* xbar3, double* mbar, const AdjointNext& next, hipStream_t st);
 
 // ---- batched systems (batch.hip) ---------------------------------------------
 struct BatchGeom {
@@ -232,7 +242,7 @@ hipError_t launch_batch_sym_step(const BatchSymGeom& g, int nwaves, int total, c
                                  double4* keep = nullptr);
 hipError_t launch_batch_sym_vjp(const BatchSymGeom& g, int nwaves, int total, const float4* jrec,
                                 float eps2, float4* ipart, float4* jpart, double* xbar3, double* mbar,
-                                hipStream_t st);
+                                const AdjointNext& next, hipStream_t st);
 hipError_t launch_batch_loss(const BatchGeom& g, int nsys, const double4* pos, const double* tgt3,
                              double* xbar3, double* vbar3, double* mbar, double* loss,
                              hipStream_t st);

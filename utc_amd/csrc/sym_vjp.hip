@@ -329,25 +329,50 @@ __global__ __launch_bounds__(256, 2) void batch_sym_vjp_kernel(BatchSymGeom g, i
     }
 }
 
+// Body b's position adjoint after the VJP, and the record of the step before:
+// the work of adjoint_pre_kernel (adjoint.hip), the same operations, on values
+// still in registers.  Adjoint of 20 steps, ms: N = 1000 0.51 (0.55 with a
+// launch of its own), 4096 0.70 (0.73), 16384 3.62 (3.71).
+__device__ __forceinline__ void adjoint_next(const AdjointNext& next, size_t b, const double (&s)[4],
+                                             double* __restrict__ xbar3, double* __restrict__ mbar)
+{
+    double x[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        x[k] = xbar3[3 * b + k] + s[k];
+        xbar3[3 * b + k] = x[k];
+    }
+    mbar[b] += s[3];
+    if (!next.pos)
+        return;
+    const double4 p = next.pos[b];
+    const double ki = next.kick == UTCNB_KICK_REFERENCE ? p.w : 1.0;
+    double al[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const double ub = next.vbar3[3 * b + k] + x[k] * next.dt;
+        next.vbar3[3 * b + k] = next.damping * ub;
+        al[k] = next.damping * ki * next.dt * ub;
+    }
+    next.jrec[2 * b] = make_float4((float)p.x, (float)p.y, (float)p.z, (float)p.w);
+    next.jrec[2 * b + 1] = make_float4((float)al[0], (float)al[1], (float)al[2], 0.f);
+}
+
 // xbar_b += the sum of body b's partials, mbar_b likewise (T lanes per body,
-// sym_reduce.h).
+// sym_reduce.h), then adjoint_next.
 template <int T>
 __global__ __launch_bounds__(256) void sym_vjp_reduce_kernel(const float4* __restrict__ ipart,
                                                              const float4* __restrict__ jpart, int n,
                                                              int NW, int R, int K, int rs,
                                                              double* __restrict__ xbar3,
-                                                             double* __restrict__ mbar)
+                                                             double* __restrict__ mbar, AdjointNext next)
 {
     int b, t;
     sym_reduce_lane<T>(b, t);
     double s[4];
     sym_split_sum<T, true>(ipart, jpart, b < n ? b : n - 1, NW, R, K, t, s, rs);
-    if (b < n && t == 0) {
-        xbar3[3 * (size_t)b + 0] += s[0];
-        xbar3[3 * (size_t)b + 1] += s[1];
-        xbar3[3 * (size_t)b + 2] += s[2];
-        mbar[b] += s[3];
-    }
+    if (b < n && t == 0)
+        adjoint_next(next, b, s, xbar3, mbar);
 }
 
 // Batched systems: body b of the concatenated padded layout.
@@ -356,7 +381,7 @@ __global__ __launch_bounds__(256) void batch_sym_vjp_reduce_kernel(BatchSymGeom 
                                                                    const float4* __restrict__ ipart,
                                                                    const float4* __restrict__ jpart,
                                                                    double* __restrict__ xbar3,
-                                                                   double* __restrict__ mbar)
+                                                                   double* __restrict__ mbar, AdjointNext next)
 {
     int j, t;
     sym_reduce_lane<T>(j, t);
@@ -365,12 +390,8 @@ __global__ __launch_bounds__(256) void batch_sym_vjp_reduce_kernel(BatchSymGeom 
     const int loc = bb - g.off[s];
     double sum[4];
     sym_split_sum<T, false>(ipart + g.vipo[s], jpart + g.vjpo[s], loc, g.nw[s], g.rs[s], K, t, sum);
-    if (j < total && loc < g.n[s] && t == 0) {
-        xbar3[3 * (size_t)b + 0] += sum[0];
-        xbar3[3 * (size_t)b + 1] += sum[1];
-        xbar3[3 * (size_t)b + 2] += sum[2];
-        mbar[b] += sum[3];
-    }
+    if (j < total && loc < g.n[s] && t == 0)
+        adjoint_next(next, b, sum, xbar3, mbar);
 }
 
 constexpr int kSymVjpK = 4;
@@ -404,7 +425,7 @@ size_t sym_vjp_jpart_float4s(int n_pad, int R)
 bool sym_vjp_applies(int n_pad) { return n_pad % (128 * kSymVjpK) == 0; }
 
 hipError_t launch_sym_vjp(const float4* jrec, int n, int n_pad, float eps2, int R, float4* ipart,
-                          float4* jpart, double* xbar3, double* mbar, hipStream_t st)
+                          float4* jpart, double* xbar3, double* mbar, const AdjointNext& next, hipStream_t st)
 {
     if (!sym_vjp_applies(n_pad) || R < 1 || !ipart || !jpart)
         return hipErrorInvalidValue;
@@ -418,18 +439,18 @@ hipError_t launch_sym_vjp(const float4* jrec, int n, int n_pad, float eps2, int 
     const int T = sym_reduce_lanes(n);
     const dim3 rgrid((unsigned)(((long long)n * T + 255) / 256));
     switch (T) {
-    case 1: hipLaunchKernelGGL(sym_vjp_reduce_kernel<1>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar); break;
-    case 2: hipLaunchKernelGGL(sym_vjp_reduce_kernel<2>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar); break;
-    case 4: hipLaunchKernelGGL(sym_vjp_reduce_kernel<4>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar); break;
-    case 8: hipLaunchKernelGGL(sym_vjp_reduce_kernel<8>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar); break;
-    default: hipLaunchKernelGGL(sym_vjp_reduce_kernel<16>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar); break;
+    case 1: hipLaunchKernelGGL(sym_vjp_reduce_kernel<1>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar, next); break;
+    case 2: hipLaunchKernelGGL(sym_vjp_reduce_kernel<2>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar, next); break;
+    case 4: hipLaunchKernelGGL(sym_vjp_reduce_kernel<4>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar, next); break;
+    case 8: hipLaunchKernelGGL(sym_vjp_reduce_kernel<8>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar, next); break;
+    default: hipLaunchKernelGGL(sym_vjp_reduce_kernel<16>, rgrid, dim3(256), 0, st, ipart, jpart, n, NW, R, kSymVjpK, kSymVjpRs, xbar3, mbar, next); break;
     }
     return hipGetLastError();
 }
 
 hipError_t launch_batch_sym_vjp(const BatchSymGeom& g, int nwaves, int total, const float4* jrec,
                                 float eps2, float4* ipart, float4* jpart, double* xbar3, double* mbar,
-                                hipStream_t st)
+                                const AdjointNext& next, hipStream_t st)
 {
     static_assert(kBatchSymK == kSymVjpK, "batched and single-system symmetric VJP share K");
     hipError_t e;
@@ -443,11 +464,11 @@ hipError_t launch_batch_sym_vjp(const BatchSymGeom& g, int nwaves, int total, co
     const int T = sym_reduce_lanes(total);
     const dim3 rgrid((unsigned)(((long long)total * T + 255) / 256));
     switch (T) {
-    case 1: hipLaunchKernelGGL(batch_sym_vjp_reduce_kernel<1>, rgrid, dim3(256), 0, st, g, total, kBatchSymK, ipart, jpart, xbar3, mbar); break;
-    case 2: hipLaunchKernelGGL(batch_sym_vjp_reduce_kernel<2>, rgrid, dim3(256), 0, st, g, total, kBatchSymK, ipart, jpart, xbar3, mbar); break;
-    case 4: hipLaunchKernelGGL(batch_sym_vjp_reduce_kernel<4>, rgrid, dim3(256), 0, st, g, total, kBatchSymK, ipart, jpart, xbar3, mbar); break;
-    case 8: hipLaunchKernelGGL(batch_sym_vjp_reduce_kernel<8>, rgrid, dim3(256), 0, st, g, total, kBatchSymK, ipart, jpart, xbar3, mbar); break;
-    default: hipLaunchKernelGGL(batch_sym_vjp_reduce_kernel<16>, rgrid, dim3(256), 0, st, g, total, kBatchSymK, ipart, jpart, xbar3, mbar); break;
+    case 1: hipLaunchKernelGGL(batch_sym_vjp_reduce_kernel<1>, rgrid, dim3(256), 0, st, g, total, kBatchSymK, ipart, jpart, xbar3, mbar, next); break;
+    case 2: hipLaunchKernelGGL(batch_sym_vjp_reduce_kernel<2>, rgrid, dim3(256), 0, st, g, total, kBatchSymK, ipart, jpart, xbar3, mbar, next); break;
+    case 4: hipLaunchKernelGGL(batch_sym_vjp_reduce_kernel<4>, rgrid, dim3(256), 0, st, g, total, kBatchSymK, ipart, jpart, xbar3, mbar, next); break;
+    case 8: hipLaunchKernelGGL(batch_sym_vjp_reduce_kernel<8>, rgrid, dim3(256), 0, st, g, total, kBatchSymK, ipart, jpart, xbar3, mbar, next); break;
+    default: hipLaunchKernelGGL(batch_sym_vjp_reduce_kernel<16>, rgrid, dim3(256), 0, st, g, total, kBatchSymK, ipart, jpart, xbar3, mbar, next); break;
     }
     return hipGetLastError();
 }
