@@ -300,7 +300,7 @@ __global__ __launch_bounds__(256, 2) void sym_vjp_kernel(const float4* __restric
                                                       float4* __restrict__ jpart, int rs)
 {
     __shared__ SymVjpLds lds[4];
-    const int gw = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    const int gw = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
     if (gw >= NW * R)
         return;  // whole waves only
     sym_vjp_wave<K, true>(jrec, NW, R, gw / R, gw % R, eps2, ipart, jpart, lds[threadIdx.x >> 6], threadIdx.x & 63,
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(256, 2) void batch_sym_vjp_kernel(BatchSymGeom g, i
                                                             float4* __restrict__ jpart)
 {
     __shared__ SymVjpLds lds[4];
-    const int gw = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    const int gw = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
     if (gw >= nwaves)
         return;  // whole waves only
     const int lane = threadIdx.x & 63;
