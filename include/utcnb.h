@@ -170,7 +170,9 @@ int utcnb_sync(utcnb_system* sys);
  * the configured tile when it is one, else a default by count; REFERENCE and
  * FP64 run their only kernels.  Per body the arithmetic does not depend on the
  * slicing: slices covering [0, n) then a commit give bitwise the same state as
- * utcnb_step(sys, 1) with that one-pass tile.  Asynchronous on the handle's
+ * utcnb_step(sys, 1) with that one-pass tile.  (A symmetric system's slices
+ * default to tiles that only slices run, with ids above utcnb_tile_count():
+ * k1p128 for up to half the bodies, else k2p64.)  Asynchronous on the handle's
  * stream; utcnb_last_kernel_ms times the slice.
  */
 int utcnb_step_slice(utcnb_system* sys, int start, int count);
@@ -332,7 +334,8 @@ int utcnb_batch_get_tile(const utcnb_batch* b, int* tile);
  */
 int utcnb_autotune(int n, int precision, const char* cache_path, int* best_tile,
                    double* best_ms);
-/* Number of tiles and a description of tile id t (static string). */
+/* Number of tiles a system can be given and a description of tile id t (static
+ * string; also of the ids above it that utcnb_slice_tile may return). */
 int utcnb_tile_count(void);
 const char* utcnb_tile_name(int tile);
 

@@ -27,7 +27,7 @@ def test_field(n):
 
 
 @pytest.mark.parametrize("n,name", [(1024, "sm1t4w8n2k"), (1025, "sm1t8w8n2k"), (2048, "sm1t8w8n2k"),
-                                    (2049, "sm1t16w16n4k"), (4097, "sm3t8w16n8k"), (6145, "sm2t16w16n8k")])
+                                    (2049, "sm1t16w16n4k"), (4097, "sm1t8w16n8k"), (6144, "sm1t8w16n8k"), (6145, "sm2t16w16n8k")])
 def test_default_tile(n, name):
     with U.System(n, U.PREC_MIXED, 1e-4, 1e-3) as s:
         assert s.tile()[1] == name

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("prec", [U.PREC_MIXED, U.PREC_FP32])
 @pytest.mark.parametrize("n", [2, 513, 1024, 1025, 3000, 8193, 9001])
-@pytest.mark.parametrize("name", ["sym8w2048x8", "sym8r64x8", "sym4r128x4", "sym2r64x2"])
+@pytest.mark.parametrize("name", ["sym8r128", "sym8r64", "sym4r128x4", "sym2r64x2"])
 def test_field(name, n, prec):
     c = plummer(n, eps=0.005)
     print(f"case: split tile {name} n={n} prec={prec}", flush=True)
@@ -29,9 +29,9 @@ def test_field(name, n, prec):
                 assert relnorm(s.accel(), O.accel_f64(pos, c["eps"] ** 2)) <= 2e-6
 
 
-@pytest.mark.parametrize("n,name", [(8193, "sym8w2048x8"), (40959, "sym8w2048x8"), (40960, "sym8r64x8"),
-                                    (65535, "sym8r64x8"), (65536, "sym8r64")])
+@pytest.mark.parametrize("n,name", [(8193, "sym8r128"), (39936, "sym8r128"), (39937, "sym8r64"), (65536, "sym8r64")])
 def test_default_tile(n, name):
+    """sym8r128 is divided below 40960 bodies (padded), sym8r64 below 65536."""
     for prec in (U.PREC_MIXED, U.PREC_FP32):
         with U.System(n, prec, 1e-4, 1e-3) as s:
             assert s.tile()[1] == name

@@ -254,7 +254,7 @@ class System:
         """(tile id, name) that the slice calls run for `count` targets."""
         t = C.c_int()
         check(lib().utcnb_slice_tile(self.h, count, C.byref(t)), "utcnb_slice_tile")
-        return t.value, (tiles()[t.value - 1] if t.value > 0 else "")
+        return t.value, lib().utcnb_tile_name(t.value).decode()
 
     def last_kernel_ms(self):
         ms, cnt = C.c_double(), C.c_int()

@@ -385,7 +385,7 @@ int utcnb_tile_count(void) { return tile_count(); }
 
 const char* utcnb_tile_name(int tile)
 {
-    if (tile < 1 || tile > tile_count())
+    if (tile < 1 || tile > tile_total())
         return "";
     return tile_get(tile - 1).name;
 }
@@ -532,17 +532,6 @@ int utcnb_create(const utcnb_config* cfg, void* stream, utcnb_system** out)
         }
         s->args.ipart = s->ipart;
         s->args.jpart = s->jpart;
-    }
-    if (!rc && (c.precision == UTCNB_PREC_FP32 || c.precision == UTCNB_PREC_MIXED) &&
-        tile_get(s->args.tile).parts > 0) {
-        const size_t pf = part_floats(s->args.tile, c.n);
-        if (pf * sizeof(float) > s->partial_budget)
-            rc = fail(UTCNB_EINVAL, "utcnb_create: N too large for a tile with source parts (partial sums above a "
-                                    "quarter of the device, at most 64 GiB); use another one-pass tile");
-        else
-            rc = dalloc(&s->ipart, pf);
-        s->args.ipart = s->args.part_ws = s->ipart;
-        s->args.part_ws_floats = pf;
     }
     if (!rc) {
         s->scratch_bytes = sizeof(double) * (3 * n + 5 + 5 * ((n + 255) / 256));

@@ -29,38 +29,36 @@ const Tile kTiles[] = {
     {1, 16, "sm1t16w16n8k", false, 1, 16, 8192}, {2, 16, "sm2t16w16n8k", false, 1, 16, 8192},
     // more one-pass tiles (appended: ids are stable)
     {2, 16, "k2s16", false}, {4, 8, "k4s8", false}, {4, 16, "k4s16", false},
-    // one-pass, the sources in P parts over separate waves (force_part.h): kKpP
+    // past the tiles a system can be given (tile_count): one-pass, the sources
+    // in P parts over separate waves (force_part.h), for slices and the
+    // handle-free field: kKpP
     {1, 1, "k1p128", false, 1, 0, 0, 128}, {2, 1, "k2p64", false, 1, 0, 0, 64},
-    // 24 targets per workgroup
-    {3, 16, "sm3t8w16n8k", false, 1, 8, 8192},
-    // symmetric, sub-units shared in chunks; R so that 2048 waves run: symKwWxRS
-    {8, 0, "sym8w2048x8", true, 8, 0, 0, 0, 2048}, {8, 64, "sym8r64x8", true, 8},
 };
 }  // namespace
 
-constexpr int kTilePart128 = 37, kTilePart64 = 38;  // k1p128, k2p64
 size_t part_floats(int tile, int64_t nt) { return (size_t)kTiles[tile].parts * nt * 3; }
 
-int tile_count() { return (int)(sizeof(kTiles) / sizeof(kTiles[0])); }
+int tile_count() { return kTilePart128; }
+int tile_total() { return (int)(sizeof(kTiles) / sizeof(kTiles[0])); }
 const Tile& tile_get(int id) { return kTiles[id]; }
 
 // Default tile, from sweeps of every tile on MI355X (mixed precision, time per
 // step, best three; equal masses; log-uniform masses and plain FP32 rank
 // alike):
 //   N = 131072: sym8r64 2.660, sym8r32 2.686, sym8r128 2.714 ms  (sym4r64 2.778)
-//   N =  65536: sym8r64x8 0.696, sym8r64 0.717, sym4r64 0.724 ms  (plain FP32: sym8r64 0.701, sym8r64x8 0.716)
-//   N =  49152: sym8r64x8 410, sym8w2048x8 418, sym8r64 429 us
-//   N =  40960: sym8r64x8 290, sym8w2048x8 298, sym4r64x8 305 us  (sym8r64 309)
-//   N =  32768: sym8w2048x8 189.0, sym8r64x8 195.6, sym4r64x8 200.9 us  (sym4r64 205.8)
-//   N =  24576: sym8w2048x8 118.6, sym8r64x8 120.3, sym4r64x8 120.6 us  (sym4r64 126.8)
-//   N =  16384: sym8w2048x8 59.5, sym4r64x2 63.2, sym4r64x8 63.8 us  (sym4r64 65.6)
-//   N =  14336: sym8w2048x8 51.7, sym4r128 52.3, sym8r64x8 54.0 us  (sym4r64 56.1)
-//   N =  12288: sym4r64x2 42.6, sym8w2048x8 42.8, sym4r64x8 43.2 us  (sym4r64 43.7)
-//   N =   9001: sym4w2048x8 32.5, sym8w2048x8 33.3, sym4r128 34.6 us  (sym4r64x2 37.5)
-//   N =   8192: sm2t16w16n8k 22.1, sm1t16w16n8k 25.1, sm1t8w16n8k 30.1 us  (sym4r64x16 24.2)
+//   N =  65536: sym8r64 0.717, sym4r64 0.724 ms  (its sub-units divided 0.696, but 0.716 for 0.701 in plain FP32)
+//   N =  49152: sym8r64 410, sym8r128 418 us  (undivided sym8r64 429)
+//   N =  40960: sym8r64 290, sym8r128 298 us  (sym4r64 307, undivided sym8r64 309)
+//   N =  32768: sym8r128 189.0, sym8r64 195.6, sym4r64x2 202 us  (sym4r64 205.8)
+//   N =  24576: sym8r128 118.6, sym8r64 120.3, sym4r64x2 120.7 us  (sym4r64 126.8)
+//   N =  16384: sym8r128 59.5, sym8r64 59.5, sym4r64x2 63.2 us  (sym4r64 65.6)
+//   N =  14336: sym8r128 51.7, sym4r128 52.3, sym8r64 54.0 us  (sym4r64 56.1)
+//   N =  12288: sym4r64x2 42.6, sym8r128 42.8, sym4r64 43.7 us
+//   N =   9001: sym8r128 33.3, sym4r128 34.6, sym2r64 35.7 us  (sym4r64x2 37.5)
+//   N =   8192: sm2t16w16n8k 22.1, sm1t16w16n8k 25.1, sm1t8w16n8k 30.1 us  (sym4r64x2 26.0)
 //   N =   7168: sm2t16w16n8k 19.8, sm1t16w16n8k 22.5, sm1t8w16n8k 27.3 us
-//   N =   6144: sm3t8w16n8k 15.2, sm2t16w16n8k 17.4, sm1t8w16n8k 19.3 us  (sym2r64 20.7)
-//   N =   5120: sm3t8w16n8k 13.4, sm2t16w16n8k 15.1, sm1t8w16n8k 17.1 us
+//   N =   6144: sm1t8w16n8k 15.2, sm2t16w16n8k 17.4, sm1t16w16n8k 19.8 us  (sym2r64 20.7)
+//   N =   5120: sm1t8w16n8k 13.4, sm2t16w16n8k 15.1, sm1t16w16n8k 17.3 us
 //   N =   4096: sm1t16w16n4k 8.2, sm1t16w16n8k 8.2, sm1t8w16n8k 10.4 us  (sym2r64 16.4)
 //   N =   2048: sm1t8w8n2k 4.4, sm1t8w16n8k 4.7, sm1t4w8n2k 4.9 us  (sym2r64x2 12.5)
 //   N =   1024: sm1t4w8n2k 3.5, sm1t8w8n2k 3.7, sm1t8w16n8k 3.9 us  (sym2r128x4 12.1)
@@ -77,8 +75,7 @@ const Tile& tile_get(int id) { return kTiles[id]; }
 // turn; from 256 bodies per CU a sub-unit is small against a wave's work, and
 // whole ones need no second reaction record.  The partial sums must fit the
 // device's budget (sym_partial_budget); above it the best one-pass tile whose
-// partial sums do is used (N = 262144: k2p64 15.99, k1p128 16.18, k2s8 19.03,
-// k2s16 20.95 ms).
+// partial sums do is used (N = 262144: k2s8 19.03, k2s16 20.95 ms).
 size_t sym_partial_budget(size_t device_bytes)
 {
     if (device_bytes == 0)
@@ -104,17 +101,13 @@ int tile_default(int64_t n, int cu_count, size_t partial_budget)
     if (n <= 4096)
         return 31;  // sm1t16w16n4k
     if (n <= 6144)
-        return 39;  // sm3t8w16n8k: 24 targets for each of the 256 CUs at 6144
+        return 30;  // sm1t8w16n8k, with 3 targets per lane: 24 for each of the 256 CUs at 6144
     if (n <= 8192)
         return 33;  // sm2t16w16n8k
-    if (n >= 256 * cus && fits(22))
+    if (n_pad >= 160 * cus && fits(22))
         return 22;  // sym8r64
-    if (n >= 160 * cus && fits(41))
-        return 41;  // sym8r64x8
-    if (n >= 8 * cus && fits(40))
-        return 40;  // sym8w2048x8
-    if (part_floats(kTilePart64, n) * sizeof(float) <= partial_budget)
-        return kTilePart64;
+    if (n >= 8 * cus && fits(23))
+        return 23;  // sym8r128
     if ((n + 127) / 128 * 8 >= cus * 16)
         return 8;   // k2s8
     return 9;       // k1s16

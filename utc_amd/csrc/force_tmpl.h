@@ -353,14 +353,18 @@ hipError_t launch_force_range(int tile, const float4* src, int i0, int nt, int n
     case 9: return launch_force_tile<1, 16, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
     case 28: return launch_small_tile<1, 4, 8, 2048, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
     case 29: return launch_small_tile<1, 8, 8, 2048, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
-    case 30: return launch_small_tile<1, 8, 16, 8192, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
+    // 8 targets per workgroup, 24 where 8 would take 3 rounds of the 256 CUs
+    // and 24 one: 4097 to 6144 bodies (6001: 15.1 us for 19.2; 6500: 31.7 for 27.1)
+    case 30:
+        if (n > 4096 && n <= 6144)
+            return launch_small_tile<3, 8, 16, 8192, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
+        return launch_small_tile<1, 8, 16, 8192, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
     case 31: return launch_small_tile<1, 16, 16, 4096, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
     case 32: return launch_small_tile<1, 16, 16, 8192, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
     case 33: return launch_small_tile<2, 16, 16, 8192, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
     case 34: return launch_force_tile<2, 16, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
     case 35: return launch_force_tile<4, 8, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
     case 36: return launch_force_tile<4, 16, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
-    case 39: return launch_small_tile<3, 8, 16, 8192, COMP, NEWTON>(src, i0, nt, n, eps2, epi, st);
     default: return hipErrorInvalidValue;
     }
 }

@@ -42,9 +42,10 @@ struct Tile {
     int tl = 0;  // small-system tiles (force_small.h): target lanes per wave; 0 for the other tiles
     int cap = 0; // small-system tiles: the most bodies (padded) their LDS holds
     int parts = 0; // one-pass tiles with the sources split over separate waves (force_part.h): the parts; else 0
-    int waves = 0; // symmetric tiles with s = 0: waves per wave block such that the system has about this many
 };
-int tile_count();
+int tile_count();  // tiles a system can be given
+constexpr int kTilePart128 = 37, kTilePart64 = 38;  // k1p128, k2p64: slices and the handle-free field
+int tile_total();  // those and the ones of slices only
 const Tile& tile_get(int id);
 // Heuristic default: enough waves to cover the chip (256 CUs x 8 waves).
 // Device memory the symmetric kernels may take for their partial sums (force
@@ -77,8 +78,10 @@ struct StepArgs {
     float* cjpart;  // reaction partials of one chunk's wave blocks
     double* react;  // reactions summed per body over the chunks, FP64 [3n]
 };
-// Waves per wave block of a symmetric tile for a system of n_pad bodies.
+// Waves per wave block of a symmetric tile for a system of n_pad bodies, and
+// the chunks it divides each sub-unit into (1: undivided).
 int sym_tile_r(const Tile& t, int n_pad);
+int sym_tile_rs(const Tile& t, int n_pad);
 // Workspace of a symmetric tile (floats).
 size_t sym_ipart_floats(int n_pad, int K, int R);
 size_t sym_jpart_floats(int n_pad, const Tile& t);

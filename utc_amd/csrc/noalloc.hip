@@ -128,6 +128,9 @@ extern "C" int utcnb_accel_noalloc(const float* pos4, int n, double eps2, int pr
     int t = tile > 0 ? tile - 1 : tile_default(n, ds.cus, kScratchBytes - src_bytes);
     if (tile == 0 && need_of(t) > kScratchBytes)
         t = tile_default(n, ds.cus, 0);  // the best one-pass tile: no partial sums
+    // ... with the sources in parts where their sums fit (N = 50000 0.69 ms for 1.51 of k2s8, 65536 1.05 for 1.41)
+    if (tile == 0 && !tile_get(t).sym && tile_get(t).cap == 0 && need_of(kTilePart64) <= kScratchBytes)
+        t = kTilePart64;
     const Tile& tl = tile_get(t);
     if (tl.sym && n_pad % (128 * tl.k) != 0)
         return fail(UTCNB_EINVAL, "utcnb_accel_noalloc: symmetric tile needs N padded to 128*K");

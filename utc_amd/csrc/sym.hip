@@ -403,22 +403,32 @@ __global__ __launch_bounds__(256) void batch_sym_reduce_kernel(BatchSymGeom g, i
         sum_epilogue(epi, b, sum);  // padding bodies keep their far-away zero-mass records
 }
 
+// K = 8 tiles divide the sub-units of smaller systems: below 65536 bodies
+// sym8r64, below 40960 sym8r128, there with the waves that make 2048 in all
+// (sweeps at tile_default, force_fp32.hip; undivided sym8r128 at 28672 161 us for
+// 153, sym8r64 at 49152 429 for 410).
 int sym_tile_r(const Tile& t, int n_pad)
 {
-    if (t.s > 0)
+    if (t.k != 8 || t.s != 128 || n_pad >= 40960)
         return t.s;
-    const int R = t.waves / (n_pad / (64 * t.k));
-    return R < 1 ? 1 : (R > 128 ? 128 : R);
+    const int R = 2048 / (n_pad / (64 * t.k));
+    return R < t.s ? R : t.s;
+}
+
+int sym_tile_rs(const Tile& t, int n_pad)
+{
+    return t.k == 8 && ((t.s == 64 && n_pad < 65536) || (t.s == 128 && n_pad < 40960)) ? 8 : t.rs;
 }
 
 size_t sym_ipart_floats(int n_pad, int K, int R) { (void)K; return (size_t)R * n_pad * 3; }
 size_t sym_jpart_floats(int n_pad, const Tile& t)
 {
     const int NW = n_pad / (64 * t.k);
-    if (t.rs == 1)
+    const int rs = sym_tile_rs(t, n_pad);
+    if (rs == 1)
         return (size_t)NW * (NW / 2) * 64 * t.k * 3;
     const int R = sym_tile_r(t, n_pad);
-    return (size_t)NW * R * SymSplit::records(NW, t.k, R, t.rs) * 64 * 3;
+    return (size_t)NW * R * SymSplit::records(NW, t.k, R, rs) * 64 * 3;
 }
 
 template <int K, bool COMP>
@@ -467,7 +477,7 @@ template <class Epi>
 hipError_t launch_sym(const Tile& t, bool newton, bool comp, const float4* src, int n, int n_pad, float eps2,
                       float* ipart, float* jpart, const Epi& epi, hipStream_t st)
 {
-    const int K = t.k, R = sym_tile_r(t, n_pad), rs = t.rs;
+    const int K = t.k, R = sym_tile_r(t, n_pad), rs = sym_tile_rs(t, n_pad);
     if (n_pad % (128 * K) != 0 || !ipart || !jpart || rs < 1 || 16 % rs != 0)
         return hipErrorInvalidValue;
     const int NW = n_pad / (64 * K);
