@@ -262,12 +262,14 @@ int download4(utcnb_system* s, const T4* src, void* dst, int dtype, int where)
 }
 
 // Whether a kernel on the handle's device may read and write the n records of
-// 4 `dtype` values at p as vectors: memory of that device, on 16 bytes.  (The
-// runtime's copies also take other devices' memory and any alignment.)
+// 4 values at p as vectors: memory of that device, which is current, on 16
+// bytes.  (The runtime's copies also take other devices' memory, any alignment
+// and any current device.)
 bool on_device(const utcnb_system* s, const void* p)
 {
     hipPointerAttribute_t at;
-    if ((uintptr_t)p % 16 != 0)
+    int dev = -1;
+    if ((uintptr_t)p % 16 != 0 || hipGetDevice(&dev) != hipSuccess || dev != s->device)
         return false;
     if (hipPointerGetAttributes(&at, p) != hipSuccess) {
         (void)hipGetLastError();

@@ -12,7 +12,8 @@ const Tile kTiles[] = {
     {1, 2, "k1s2", false},  {2, 2, "k2s2", false},  {1, 4, "k1s4", false},
     {2, 4, "k2s4", false},  {1, 8, "k1s8", false},  {2, 8, "k2s8", false},
     {1, 16, "k1s16", false},
-    // symmetric (sym.hip): K targets per lane, R waves per wave block
+    // symmetric (sym.hip): K targets per lane, R waves per wave block (sym8r64 and
+    // sym8r128 are divided below 65536 and 40960 bodies: sym_tile_r, sym_tile_rs)
     {4, 4, "sym4r4", true}, {4, 8, "sym4r8", true}, {8, 4, "sym8r4", true},
     {8, 8, "sym8r8", true}, {8, 16, "sym8r16", true}, {4, 16, "sym4r16", true},
     {4, 32, "sym4r32", true}, {8, 32, "sym8r32", true}, {4, 64, "sym4r64", true},
@@ -23,7 +24,7 @@ const Tile kTiles[] = {
     {4, 128, "sym4r128x4", true, 4},
     // one kernel per step for small systems (force_small.h): A targets per
     // lane, TL target lanes per wave, W waves, at most CAP bodies:
-    // smAtTLwWnCAPk; k = A, s = W
+    // smAtTLwWnCAPk; k = A, s = W (sm1t8w16n8k has A = 3 from 4097 to 6144 bodies)
     {1, 8, "sm1t4w8n2k", false, 1, 4, 2048}, {1, 8, "sm1t8w8n2k", false, 1, 8, 2048},
     {1, 16, "sm1t8w16n8k", false, 1, 8, 8192}, {1, 16, "sm1t16w16n4k", false, 1, 16, 4096},
     {1, 16, "sm1t16w16n8k", false, 1, 16, 8192}, {2, 16, "sm2t16w16n8k", false, 1, 16, 8192},

@@ -47,11 +47,12 @@ int tile_count();  // tiles a system can be given
 constexpr int kTilePart128 = 37, kTilePart64 = 38;  // k1p128, k2p64: slices and the handle-free field
 int tile_total();  // those and the ones of slices only
 const Tile& tile_get(int id);
-// Heuristic default: enough waves to cover the chip (256 CUs x 8 waves).
 // Device memory the symmetric kernels may take for their partial sums (force
 // and VJP each): a quarter of the device, at most 64 GiB (16 GiB when the
 // device size is unknown).  Larger systems use one-pass kernels.
 size_t sym_partial_budget(size_t device_bytes);
+// The default tile by size (sweeps in force_fp32.hip), and the one whose wave
+// blocks a default system's shares and chunks divide.
 int tile_default(int64_t n, int cu_count, size_t partial_budget);
 int sym_share_tile_default(int64_t n, int cu_count);
 
