@@ -17,9 +17,13 @@
 //  * the G lanes of a target meet in registers (lane_sum.h), the W
 //    waves in LDS, in a fixed order (bitwise repeatable), and TW threads run
 //    the integrator epilogue: one launch per step, nothing in HBM between.
-// COMP: sums of up to kSmallBlock sources are Kahan-added per lane (as the
-// 64-source partials of the other kernels) and the lanes and waves are
-// combined in FP64; otherwise plain FP32 throughout (the plain FP32 path).
+// COMP: sums of up to BLOCK sources are Kahan-added per lane (as the 64-source
+// partials of the other kernels) and the lanes and waves are combined in FP64;
+// otherwise plain FP32 throughout (the plain FP32 path).  BLOCK is 32, but 8 for
+// the 64 splits of TL = 8, W = 8: they serve 1025 to 2048 bodies in place of
+// 128 splits, whose sums are half as long (the field's error there, 2048
+// bodies in a cube, Newton: 4.1e-8 with 128 splits, 5.0e-8 with 64 and blocks of
+// 32, 3.7e-8 with blocks of 8, which take 4.6 us per step for 4.5).
 // Pair arithmetic as in stream_sources: 12 VALU instructions and a root per
 // ordered pair, the roots of 8 pairs together (rsq_group.h), plus one LDS read
 // per source shared by the lane's A targets.  Per step, mixed: N = 8192 22.1 us
@@ -39,14 +43,13 @@
 
 namespace utcnb {
 
-constexpr int kSmallBlock = 32;  // sources per plain partial of a lane (COMP)
-
 template <int A, int TL, int W, int CAP, bool COMP, bool NEWTON, class Epi>
 __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __restrict__ src, int i0, int nt,
                                                              int n, float eps2, Epi epi)
 {
     constexpr int G = 64 / TL, TW = TL * A, SPL = G * W;
     constexpr int J = A == 1 ? 8 : A == 2 ? 4 : 2;  // sources per group of reciprocal roots
+    constexpr int BLOCK = TL == 8 && W == 8 ? 8 : 32;  // sources per plain partial of a lane
     // the same number of sources for every split, whole groups: padding after n
     const int iters = (n + SPL * J - 1) / (SPL * J) * J, fill = iters * SPL;
     using Acc = typename std::conditional<COMP, double, float>::type;
@@ -82,8 +85,8 @@ __global__ __launch_bounds__(64 * W) void small_force_kernel(const float4* __res
     __syncthreads();
 
     const int split = wave * G + g;
-    for (int b0 = 0; b0 < iters; b0 += kSmallBlock) {
-        const int b1 = b0 + kSmallBlock < iters ? b0 + kSmallBlock : iters;
+    for (int b0 = 0; b0 < iters; b0 += BLOCK) {
+        const int b1 = b0 + BLOCK < iters ? b0 + BLOCK : iters;
         float ax[A], ay[A], az[A];
 #pragma unroll
         for (int a = 0; a < A; ++a) {
