@@ -1,5 +1,6 @@
 """The default tiles' field is no further from FP64 than that of tiles with
-shorter chains of plain FP32 additions: 128 source splits up to 2048 bodies.
+shorter chains of plain FP32 additions: 128 source splits up to 2048 bodies,
+2 and 4 targets per lane from 8193 to 24575.
 
 The bound: both errors are root mean squares over the 3 components of at least
 1025 bodies in 5 systems, nearly independent, each good to
@@ -15,7 +16,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("prec", [U.PREC_MIXED, U.PREC_FP32])
-@pytest.mark.parametrize("n,tile", [(1025, "sm1t8w16n8k"), (1500, "sm1t8w16n8k"), (2048, "sm1t8w16n8k")])
+@pytest.mark.parametrize("n,tile", [(1025, "sm1t8w16n8k"), (1500, "sm1t8w16n8k"), (2048, "sm1t8w16n8k"),
+                                    (8193, "sym2r32"), (12288, "sym2r32"), (16384, "sym4r64x2"),
+                                    (24575, "sym4r64x2")])
 def test_default_against_shorter_chains(n, tile, prec):
     err = {"default": 0.0, tile: 0.0}
     for seed in range(5):

@@ -37,8 +37,8 @@
 // (SPLIT kernels) cut each sub-unit's 64 rotation steps into RS chunks of 64/RS
 // steps, and the R waves of a wave block share its Q * RS chunks in a row;
 // a sub-unit that two waves share has a reaction record from each.  N = 16384
-// 59.5 us per step against 65.6 with whole sub-units, 28672 153 against 163,
-// 9001 33.3 against 37.5 (sweeps at tile_default in force_fp32.hip).
+// 61.1 us per step against 65.6 with whole sub-units, 28672 153 against 163,
+// 9001 33.9 against 37.5 (sweeps at tile_default in force_fp32.hip).
 //
 // What bounds it: FP32 issue and, at large N, the power the FMAs draw.  A step
 // issues one 16-byte and three 4-byte LDS reads and three LDS writes beside
@@ -84,17 +84,10 @@ __device__ __forceinline__ void wave_lds_fence()
     __builtin_amdgcn_wave_barrier();
 }
 
-// Rotation steps [t0, t0 + steps) of a block of 64 sources (lane l's source
-// s; wave private LDS L) against target slots 0 .. N-1 of each lane: at step
-// t lane l meets source (l + t) mod 64.  Slots k < N2 are two-sided; the
-// others collect the target side only.  Target-side sums are added to p; the
-// reaction sums of lane l's own source come back in g (N2 > 0).
-// UNI: every target mass mi[k] and source mass is the same, and p and g lack
-// that factor.
-template <int K, int N, int N2, bool NEWTON, bool UNI>
-__device__ __forceinline__ void sym_rotate(SymLds& L, int lane, int t0, int steps, float4 s, const float (&xi)[K],
-                                           const float (&yi)[K], const float (&zi)[K], const float (&mi)[K],
-                                           float eps2, float (&px)[N], float (&py)[N], float (&pz)[N], float (&g)[3])
+// A block of 64 sources (lane l's source s) into the wave's LDS, its reaction
+// sums zeroed (N2 > 0).
+template <int N2>
+__device__ __forceinline__ void sym_fill(SymLds& L, int lane, float4 s)
 {
     wave_lds_fence();
     L.s[lane] = s;
@@ -105,6 +98,20 @@ __device__ __forceinline__ void sym_rotate(SymLds& L, int lane, int t0, int step
             L.g[c][lane] = L.g[c][lane + 64] = 0.f;
     }
     wave_lds_fence();
+}
+
+// Rotation steps [t0, t0 + steps) of the block in L against target slots
+// 0 .. N-1 of each lane: at step t lane l meets source (l + t) mod 64.  Slots
+// k < N2 are two-sided; the others collect the target side only.  Target-side
+// sums are added to p, the reactions to the sources' sums in L.
+// UNI: every target mass mi[k] and source mass is the same, and the sums lack
+// that factor.  STEPSUM: a step's N2 reactions on a source are summed by
+// themselves before they meet its sum, which so takes 64 additions, not 64 N2.
+template <int K, int N, int N2, bool NEWTON, bool UNI, bool STEPSUM>
+__device__ __forceinline__ void sym_rotate(SymLds& L, int lane, int t0, int steps, const float (&xi)[K],
+                                           const float (&yi)[K], const float (&zi)[K], const float (&mi)[K],
+                                           float eps2, float (&px)[N], float (&py)[N], float (&pz)[N])
+{
     const float4* sp = &L.s[lane + t0];
     float* gp = &L.g[0][lane + t0];
     float4 cur = *sp;
@@ -114,10 +121,11 @@ __device__ __forceinline__ void sym_rotate(SymLds& L, int lane, int t0, int step
 #pragma unroll
     for (int t = t4; t < t4 + 4; ++t) {
         const float4 nxt = sp[t + 1];  // the next step's source: at most L.s[127]
-        float gx = 0.f, gy = 0.f, gz = 0.f;
+        float ox = 0.f, oy = 0.f, oz = 0.f;
         if constexpr (N2 > 0) {
-            gx = gp[t]; gy = gp[128 + t]; gz = gp[256 + t];
+            ox = gp[t]; oy = gp[128 + t]; oz = gp[256 + t];
         }
+        float gx = STEPSUM ? 0.f : ox, gy = STEPSUM ? 0.f : oy, gz = STEPSUM ? 0.f : oz;
         constexpr int GK = N < 4 ? N : 4;  // pairs per group of reciprocal roots
 #pragma unroll
         for (int k0 = 0; k0 < N; k0 += GK) {
@@ -146,39 +154,69 @@ __device__ __forceinline__ void sym_rotate(SymLds& L, int lane, int t0, int step
             }
         }
         if constexpr (N2 > 0) {
-            gp[t] = gx; gp[128 + t] = gy; gp[256 + t] = gz;
+            gp[t] = STEPSUM ? ox + gx : gx;
+            gp[128 + t] = STEPSUM ? oy + gy : gy;
+            gp[256 + t] = STEPSUM ? oz + gz : gz;
         }
         wave_lds_fence();
         cur = nxt;
     }
-    if constexpr (N2 > 0) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-            g[c] = L.g[c][lane] + L.g[c][lane + 64];
-    }
 }
 
-// sym_rotate with the block's target-side partials added into (a, c) by
-// block_add<COMP> and everything scaled by the mass m (UNI).
-template <int K, int N, int N2, bool NEWTON, bool COMP, bool UNI>
-__device__ __forceinline__ void sym_block(SymLds& L, int lane, int t0, int steps, float4 s, const float (&xi)[K],
-                                          const float (&yi)[K], const float (&zi)[K], const float (&mi)[K], float m,
-                                          float eps2, float (&ax)[K], float (&ay)[K], float (&az)[K], float (&cx)[K],
-                                          float (&cy)[K], float (&cz)[K], float (&g)[3])
+// Rotation steps [t0, t0 + steps) of a block of 64 sources against the lanes'
+// target slots (sym_rotate): target-side partials are added into (a, c) by
+// block_add<COMP>, the reaction sums of lane l's own source come back in g
+// (N2 > 0), all of it scaled by the mass m (UNI).
+// SPLIT 1, K <= 4: partials and reaction sums are taken up after every len
+// steps, a chunk, so that no chain of plain FP32 additions is longer than a
+// chunk's pairs.  SPLIT 2: STEPSUM (K = 8, for the sizes whose K = 2 and 4 tiles
+// had chains a quarter as long).  Field's error against 64 bits, N = 16384 in a
+// cube, Newton: sym4r64x2 3.71e-8 without and 3.00e-8 with, sym8r128 5.04e-8
+// without and 2.80e-8 with (59.3 and 61.1 us per step; 24575 4.18e-8 and
+// 2.34e-8).
+template <int K, int N, int N2, bool NEWTON, bool COMP, bool UNI, int SPLIT>
+__device__ __forceinline__ void sym_block(SymLds& L, int lane, int t0, int steps, int len, float4 s,
+                                          const float (&xi)[K], const float (&yi)[K], const float (&zi)[K],
+                                          const float (&mi)[K], float m, float eps2, float (&ax)[K], float (&ay)[K],
+                                          float (&az)[K], float (&cx)[K], float (&cy)[K], float (&cz)[K], float (&g)[3])
 {
-    float px[N], py[N], pz[N];
+    constexpr bool CHUNKS = SPLIT == 1 && K <= 4;
+    sym_fill<N2>(L, lane, s);
+    for (int t = t0;;) {
+        float px[N], py[N], pz[N];
 #pragma unroll
-    for (int k = 0; k < N; ++k)
-        px[k] = py[k] = pz[k] = 0.f;
-    sym_rotate<K, N, N2, NEWTON, UNI>(L, lane, t0, steps, s, xi, yi, zi, mi, eps2, px, py, pz, g);
+        for (int k = 0; k < N; ++k)
+            px[k] = py[k] = pz[k] = 0.f;
+        sym_rotate<K, N, N2, NEWTON, UNI, SPLIT == 2>(L, lane, t, CHUNKS ? len : steps, xi, yi, zi, mi, eps2, px,
+                                                            py, pz);
 #pragma unroll
-    for (int k = 0; k < N; ++k) {
-        if constexpr (UNI) {
-            px[k] *= m; py[k] *= m; pz[k] *= m;
+        for (int k = 0; k < N; ++k) {
+            if constexpr (UNI) {
+                px[k] *= m; py[k] *= m; pz[k] *= m;
+            }
+            block_add<COMP>(ax[k], cx[k], px[k]);
+            block_add<COMP>(ay[k], cy[k], py[k]);
+            block_add<COMP>(az[k], cz[k], pz[k]);
         }
-        block_add<COMP>(ax[k], cx[k], px[k]);
-        block_add<COMP>(ay[k], cy[k], py[k]);
-        block_add<COMP>(az[k], cz[k], pz[k]);
+        if constexpr (N2 > 0) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const float r = L.g[c][lane] + L.g[c][lane + 64];
+                g[c] = t == t0 ? r : g[c] + r;
+            }
+        }
+        if constexpr (!CHUNKS)
+            break;
+        t += len;
+        if (t >= t0 + steps)
+            break;
+        if constexpr (N2 > 0) {
+            wave_lds_fence();
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                L.g[c][lane] = L.g[c][lane + 64] = 0.f;
+            wave_lds_fence();
+        }
     }
     if constexpr (UNI && N2 > 0) {
 #pragma unroll
@@ -192,8 +230,8 @@ __device__ __forceinline__ void sym_block(SymLds& L, int lane, int t0, int steps
 // KB one-sided (the block with itself: each ordered pair once, the self pair
 // adds r = 0); slots k > KB take these sources when their own block is the
 // source.  The reaction sums belong to slot KB.
-template <int K, bool NEWTON, bool COMP, int KB = 0>
-__device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane, int t0, int steps, float4 s,
+template <int K, bool NEWTON, bool COMP, int SPLIT, int KB = 0>
+__device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane, int t0, int steps, int len, float4 s,
                                            const float (&xi)[K], const float (&yi)[K], const float (&zi)[K],
                                            const float (&mi)[K], float m, float eps2, float (&ax)[K], float (&ay)[K],
                                            float (&az)[K], float (&cx)[K], float (&cy)[K], float (&cz)[K])
@@ -201,11 +239,11 @@ __device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane
     if (kb == KB) {
         float g[3];
         if (uni)
-            sym_block<K, KB + 1, KB, NEWTON, COMP, true>(L, lane, t0, steps, s, xi, yi, zi, mi, m, eps2, ax, ay, az,
-                                                         cx, cy, cz, g);
+            sym_block<K, KB + 1, KB, NEWTON, COMP, true, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m, eps2, ax,
+                                                                ay, az, cx, cy, cz, g);
         else
-            sym_block<K, KB + 1, KB, NEWTON, COMP, false>(L, lane, t0, steps, s, xi, yi, zi, mi, m, eps2, ax, ay, az,
-                                                          cx, cy, cz, g);
+            sym_block<K, KB + 1, KB, NEWTON, COMP, false, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m, eps2, ax,
+                                                                 ay, az, cx, cy, cz, g);
         if constexpr (KB > 0) {
             block_add<COMP>(ax[KB], cx[KB], g[0]);
             block_add<COMP>(ay[KB], cy[KB], g[1]);
@@ -215,8 +253,8 @@ __device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane
             asm volatile("; own block %0" : : "n"(KB));
         }
     } else if constexpr (KB + 1 < K) {
-        sym_own_at<K, NEWTON, COMP, KB + 1>(kb, uni, L, lane, t0, steps, s, xi, yi, zi, mi, m, eps2, ax, ay, az, cx,
-                                            cy, cz);
+        sym_own_at<K, NEWTON, COMP, SPLIT, KB + 1>(kb, uni, L, lane, t0, steps, len, s, xi, yi, zi, mi, m, eps2, ax, ay,
+                                                   az, cx, cy, cz);
     }
 }
 
@@ -227,10 +265,10 @@ __device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane
 // range of bodies only: body b of row r is record r * istride + b - ibody0
 // (istride < 0: n_pad, the whole system).  COMP: the target-side block
 // partials are Kahan-added (the compensated paths); otherwise plain FP32 sums.
-// SPLIT: the waves share the sub-units by chunks of 64 / rs rotation steps (rs
-// divides 16) and the reactions take a record per wave and sub-unit: jpart is
+// SPLIT (1 or 2, sym_block): the waves share the sub-units by chunks of 64 / rs
+// rotation steps (rs divides 16) and the reactions take a record per wave and sub-unit: jpart is
 // [NW][R][J][64][3] (SymSplit, sym_reduce.h).
-template <int K, bool NEWTON, bool COMP, bool SPLIT = false>
+template <int K, bool NEWTON, bool COMP, int SPLIT = 0>
 __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW, int R, int w, int r,
                                          float eps2, float* __restrict__ ipart,
                                          float* __restrict__ jpart, SymLds& L, int lane, int jbase = 0,
@@ -254,7 +292,8 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
     // sub-unit q = (unit u, source block kb): u = 0 is the wave block's own
     // sources, u = 1 + d the wave block d + 1 places round
     int qf, ql, c0 = 0, c1 = 0, J = 0;
-    if constexpr (SPLIT) {
+    const int len = SPLIT != 0 ? 64 / rs : 64;
+    if constexpr (SPLIT != 0) {
         const SymSplit sp(NW, w, K, R, rs);
         c0 = sp.first(r);
         c1 = sp.first(r + 1);
@@ -269,10 +308,10 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
     for (int q = qf; q < ql; ++q) {
         // rotation steps [t0, t0 + steps): all but for the first and last sub-unit
         int t0 = 0, steps = 64;
-        if constexpr (SPLIT) {
+        if constexpr (SPLIT != 0) {
             const int a = q == qf ? c0 - q * rs : 0, e = q + 1 == ql ? c1 - q * rs : rs;
-            t0 = a * (64 / rs);
-            steps = (e - a) * (64 / rs);
+            t0 = a * len;
+            steps = (e - a) * len;
         }
         const int u = q / K, kb = q - u * K;
         if (u == 0) {
@@ -280,15 +319,15 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
             const bool uni = __ballot(tuni && s.w == m0) == ~0ull;
             if constexpr (K <= 4) {
                 // own block kb: two-sided against the lower target slots
-                sym_own_at<K, NEWTON, COMP>(kb, uni, L, lane, t0, steps, s, xi, yi, zi, mi, m0, eps2, ax, ay, az, cx,
-                                            cy, cz);
+                sym_own_at<K, NEWTON, COMP, SPLIT>(kb, uni, L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
+                                                   az, cx, cy, cz);
             } else {
                 // own block kb (K = 8, where own blocks are a small share and
                 // eight variants of sym_own_at would crowd the instruction cache):
                 // target side only (each ordered pair once, self pair gives 0)
                 float g[3];
-                sym_block<K, K, 0, NEWTON, COMP, false>(L, lane, t0, steps, s, xi, yi, zi, mi, m0, eps2, ax, ay, az,
-                                                        cx, cy, cz, g);
+                sym_block<K, K, 0, NEWTON, COMP, false, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax,
+                                                               ay, az, cx, cy, cz, g);
             }
             continue;
         }
@@ -301,12 +340,12 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
         const float4 s = src[v * 64 * K + kb * 64 + lane];
         float g[3];
         if (__ballot(tuni && s.w == m0) == ~0ull)
-            sym_block<K, K, K, NEWTON, COMP, true>(L, lane, t0, steps, s, xi, yi, zi, mi, m0, eps2, ax, ay, az, cx,
-                                                   cy, cz, g);
+            sym_block<K, K, K, NEWTON, COMP, true, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
+                                                          az, cx, cy, cz, g);
         else
-            sym_block<K, K, K, NEWTON, COMP, false>(L, lane, t0, steps, s, xi, yi, zi, mi, m0, eps2, ax, ay, az, cx,
-                                                    cy, cz, g);
-        const size_t o = SPLIT ? ((((size_t)w * R + r) * J + (q - qf)) * 64 + lane) * 3
+            sym_block<K, K, K, NEWTON, COMP, false, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
+                                                           az, cx, cy, cz, g);
+        const size_t o = SPLIT != 0 ? ((((size_t)w * R + r) * J + (q - qf)) * 64 + lane) * 3
                                : (((size_t)(w - jbase) * half + d) * (64 * K) + kb * 64 + lane) * 3;
         jpart[o + 0] = g[0];
         jpart[o + 1] = g[1];
@@ -323,7 +362,7 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
 }
 
 // One system: wave gw = w * R + r.  SPLIT: rs rotation chunks per sub-unit.
-template <int K, bool NEWTON, bool COMP, bool SPLIT>
+template <int K, bool NEWTON, bool COMP, int SPLIT>
 __global__ __launch_bounds__(256, 2) void sym_force_kernel(const float4* __restrict__ src, int NW, int R,
                                                         float eps2, float* __restrict__ ipart,
                                                         float* __restrict__ jpart, int rs)
@@ -332,7 +371,7 @@ __global__ __launch_bounds__(256, 2) void sym_force_kernel(const float4* __restr
     int gw = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     // whole sub-units: the schedule in scalar registers, 1 to 3% from 65536
     // bodies (717 to 704 us); split, the same within 0.7% either way
-    if constexpr (!SPLIT)
+    if constexpr (SPLIT == 0)
         gw = __builtin_amdgcn_readfirstlane(gw);
     if (gw >= NW * R)
         return;  // whole waves only
@@ -431,25 +470,41 @@ size_t sym_jpart_floats(int n_pad, const Tile& t)
     return (size_t)NW * R * SymSplit::records(NW, t.k, R, rs) * 64 * 3;
 }
 
+// The form of the divided kernels (sym_block): below 24576 bodies K = 8 serves
+// sizes that K = 2 and 4 did; above it has no longer chains than undivided, and
+// summing by steps takes 3.7% at 32768.
+static int sym_split_form(const Tile& t, int n_pad)
+{
+    if (sym_tile_rs(t, n_pad) == 1)
+        return 0;
+    return t.k == 8 && n_pad < 24576 ? 2 : 1;
+}
+
 template <int K, bool COMP>
-static void launch_sym_pairs(bool newton, int rs, dim3 grid, const float4* src, int NW, int R, float eps2,
+static void launch_sym_pairs(bool newton, int split, int rs, dim3 grid, const float4* src, int NW, int R, float eps2,
                              float* ipart, float* jpart, hipStream_t st)
 {
-    if (rs > 1) {
-        if (newton)
-            hipLaunchKernelGGL((sym_force_kernel<K, true, COMP, true>), grid, dim3(256), 0, st, src, NW, R, eps2,
-                               ipart, jpart, rs);
-        else
-            hipLaunchKernelGGL((sym_force_kernel<K, false, COMP, true>), grid, dim3(256), 0, st, src, NW, R, eps2,
-                               ipart, jpart, rs);
-        return;
+#define SYM_PAIRS(NEWTON, SPLIT)                                                                                \
+    hipLaunchKernelGGL((sym_force_kernel<K, NEWTON, COMP, SPLIT>), grid, dim3(256), 0, st, src, NW, R, eps2, ipart, \
+                       jpart, rs)
+    if constexpr (K == 8) {
+        if (split == 2) {
+            if (newton)
+                SYM_PAIRS(true, 2);
+            else
+                SYM_PAIRS(false, 2);
+            return;
+        }
     }
-    if (newton)
-        hipLaunchKernelGGL((sym_force_kernel<K, true, COMP, false>), grid, dim3(256), 0, st, src, NW, R, eps2,
-                           ipart, jpart, 1);
+    if (split != 0 && newton)
+        SYM_PAIRS(true, 1);
+    else if (split != 0)
+        SYM_PAIRS(false, 1);
+    else if (newton)
+        SYM_PAIRS(true, 0);
     else
-        hipLaunchKernelGGL((sym_force_kernel<K, false, COMP, false>), grid, dim3(256), 0, st, src, NW, R, eps2,
-                           ipart, jpart, 1);
+        SYM_PAIRS(false, 0);
+#undef SYM_PAIRS
 }
 
 template <bool SPLIT, typename Acc, class Epi>
@@ -477,21 +532,21 @@ template <class Epi>
 hipError_t launch_sym(const Tile& t, bool newton, bool comp, const float4* src, int n, int n_pad, float eps2,
                       float* ipart, float* jpart, const Epi& epi, hipStream_t st)
 {
-    const int K = t.k, R = sym_tile_r(t, n_pad), rs = sym_tile_rs(t, n_pad);
+    const int K = t.k, R = sym_tile_r(t, n_pad), rs = sym_tile_rs(t, n_pad), split = sym_split_form(t, n_pad);
     if (n_pad % (128 * K) != 0 || !ipart || !jpart || rs < 1 || 16 % rs != 0)
         return hipErrorInvalidValue;
     const int NW = n_pad / (64 * K);
     const int waves = NW * R;
     const dim3 grid((waves + 3) / 4);
     if (K == 2)
-        comp ? launch_sym_pairs<2, true>(newton, rs, grid, src, NW, R, eps2, ipart, jpart, st)
-             : launch_sym_pairs<2, false>(newton, rs, grid, src, NW, R, eps2, ipart, jpart, st);
+        comp ? launch_sym_pairs<2, true>(newton, split, rs, grid, src, NW, R, eps2, ipart, jpart, st)
+             : launch_sym_pairs<2, false>(newton, split, rs, grid, src, NW, R, eps2, ipart, jpart, st);
     else if (K == 4)
-        comp ? launch_sym_pairs<4, true>(newton, rs, grid, src, NW, R, eps2, ipart, jpart, st)
-             : launch_sym_pairs<4, false>(newton, rs, grid, src, NW, R, eps2, ipart, jpart, st);
+        comp ? launch_sym_pairs<4, true>(newton, split, rs, grid, src, NW, R, eps2, ipart, jpart, st)
+             : launch_sym_pairs<4, false>(newton, split, rs, grid, src, NW, R, eps2, ipart, jpart, st);
     else if (K == 8)
-        comp ? launch_sym_pairs<8, true>(newton, rs, grid, src, NW, R, eps2, ipart, jpart, st)
-             : launch_sym_pairs<8, false>(newton, rs, grid, src, NW, R, eps2, ipart, jpart, st);
+        comp ? launch_sym_pairs<8, true>(newton, split, rs, grid, src, NW, R, eps2, ipart, jpart, st)
+             : launch_sym_pairs<8, false>(newton, split, rs, grid, src, NW, R, eps2, ipart, jpart, st);
     else
         return hipErrorInvalidValue;
     hipError_t e = hipGetLastError();
