@@ -13,7 +13,7 @@ const Tile kTiles[] = {
     {2, 4, "k2s4", false},  {1, 8, "k1s8", false},  {2, 8, "k2s8", false},
     {1, 16, "k1s16", false},
     // symmetric (sym.hip): K targets per lane, R waves per wave block (sym8r64 and
-    // sym8r128 are divided below 65536 and 40960 bodies: sym_tile_r, sym_tile_rs)
+    // sym8r128 are divided up to 46080 and 39936 bodies: sym_tile_r, sym_tile_rs)
     {4, 4, "sym4r4", true}, {4, 8, "sym4r8", true}, {8, 4, "sym8r4", true},
     {8, 8, "sym8r8", true}, {8, 16, "sym8r16", true}, {4, 16, "sym4r16", true},
     {4, 32, "sym4r32", true}, {8, 32, "sym8r32", true}, {4, 64, "sym4r64", true},
@@ -47,8 +47,8 @@ const Tile& tile_get(int id) { return kTiles[id]; }
 // step, best three; equal masses; log-uniform masses and plain FP32 rank
 // alike):
 //   N = 131072: sym8r64 2.660, sym8r32 2.686, sym8r128 2.714 ms  (sym4r64 2.778)
-//   N =  65536: sym8r64 0.717, sym4r64 0.724 ms  (its sub-units divided 0.696, but 0.716 for 0.701 in plain FP32)
-//   N =  49152: sym8r64 410, sym8r128 418 us  (undivided sym8r64 429)
+//   N =  65536: sym8r64 0.717, sym4r64 0.724 ms  (its sub-units divided 0.696)
+//   N =  49152: sym8r64 427, sym8r128 439 us  (divided sym8r64 406: sym_tile_rs)
 //   N =  40960: sym8r64 290, sym8r128 298 us  (sym4r64 307, undivided sym8r64 309)
 //   N =  32768: sym8r128 189.0, sym8r64 195.6, sym4r64x2 202 us  (sym4r64 205.8)
 //   N =  24576: sym8r128 118.6, sym8r64 120.3, sym4r64x2 120.7 us  (sym4r64 126.8)

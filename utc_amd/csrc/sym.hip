@@ -442,10 +442,13 @@ __global__ __launch_bounds__(256) void batch_sym_reduce_kernel(BatchSymGeom g, i
         sum_epilogue(epi, b, sum);  // padding bodies keep their far-away zero-mass records
 }
 
-// K = 8 tiles divide the sub-units of smaller systems: below 65536 bodies
+// K = 8 tiles divide the sub-units of smaller systems: up to 46080 bodies
 // sym8r64, below 40960 sym8r128, there with the waves that make 2048 in all
 // (sweeps at tile_default, force_fp32.hip; undivided sym8r128 at 28672 161 us for
-// 153, sym8r64 at 49152 429 for 410).
+// 153).  Divided sym8r64 would be faster up to 65535 bodies (49152 406 us for
+// 427), but its reaction records, one more per wave, no longer fit the 64 MiB
+// of utcnb_accel_noalloc from 46081, where the undivided ones do up to 49152, and
+// a tile's bits are the same with a handle and without.
 int sym_tile_r(const Tile& t, int n_pad)
 {
     if (t.k != 8 || t.s != 128 || n_pad >= 40960)
@@ -456,7 +459,7 @@ int sym_tile_r(const Tile& t, int n_pad)
 
 int sym_tile_rs(const Tile& t, int n_pad)
 {
-    return t.k == 8 && ((t.s == 64 && n_pad < 65536) || (t.s == 128 && n_pad < 40960)) ? 8 : t.rs;
+    return t.k == 8 && ((t.s == 64 && n_pad <= 46080) || (t.s == 128 && n_pad < 40960)) ? 8 : t.rs;
 }
 
 size_t sym_ipart_floats(int n_pad, int K, int R) { (void)K; return (size_t)R * n_pad * 3; }
