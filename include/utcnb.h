@@ -167,13 +167,15 @@ int utcnb_sync(utcnb_system* sys);
  * further utcnb_step_slice calls, or the peers' slices received into
  * utcnb_position_buffer(sys, 1, ...) by an all-gather), then calls
  * utcnb_commit_step.  FP32 and MIXED run a one-pass tile (utcnb_slice_tile):
- * the configured tile when it is one, else a default by count; REFERENCE and
+ * the configured tile when it is one, else a default; REFERENCE and
  * FP64 run their only kernels.  Per body the arithmetic does not depend on the
- * slicing: slices covering [0, n) then a commit give bitwise the same state as
- * utcnb_step(sys, 1) with that one-pass tile.  (A symmetric system's slices
- * default to tiles that only slices run, with ids above utcnb_tile_count():
- * k1p128 for up to half the bodies, else k2p64.)  Asynchronous on the handle's
- * stream; utcnb_last_kernel_ms times the slice.
+ * slicing: slices covering [0, n) then a commit give bitwise the same state
+ * however many they are, and the state of utcnb_step(sys, 1) where the system's
+ * tile is one-pass.  A symmetric system's slices default to tiles that only
+ * slices run, with ids above utcnb_tile_count(): k1p128, and k2p64 for more
+ * targets than its workspace holds, which give the same bits; one slice of all
+ * bodies is then what any slicing is to be compared with.  Asynchronous on the
+ * handle's stream; utcnb_last_kernel_ms times the slice.
  */
 int utcnb_step_slice(utcnb_system* sys, int start, int count);
 /* Make the next position buffer current (after the slices of a step). */

@@ -32,7 +32,7 @@ const Tile kTiles[] = {
     {2, 16, "k2s16", false}, {4, 8, "k4s8", false}, {4, 16, "k4s16", false},
     // past the tiles a system can be given (tile_count): one-pass, the sources
     // in P parts over separate waves (force_part.h), for slices and the
-    // handle-free field: kKpP
+    // handle-free field: kKpP, whose bits are the same
     {1, 1, "k1p128", false, 1, 0, 0, 128}, {2, 1, "k2p64", false, 1, 0, 0, 64},
 };
 }  // namespace
@@ -170,7 +170,8 @@ hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* 
 //   N =  32768: nt =   4096 k1p128 0.051, k2p64 0.056               (k1s16 0.237)
 // Many small waves fill the chip whatever the number of targets; 256 parts
 // gain at most 3% more and take twice the workspace, K = 4 (k4p32 ... k4p128)
-// is slower throughout.
+// is slower throughout.  Which of the two it is does not change a bit of the
+// result, nor does the slicing.
 int slice_tile_default(int64_t nt, int cu_count, size_t part_ws)
 {
     if (part_floats(kTilePart128, nt) <= part_ws)

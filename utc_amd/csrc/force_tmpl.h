@@ -335,12 +335,9 @@ hipError_t launch_force_range(int tile, const float4* src, int i0, int nt, int n
 {
     if (nt < 1)
         return hipErrorInvalidValue;
-    if (const int P = tile_get(tile).parts) {
-        if (tile_get(tile).k == 1)
-            return launch_part_tile<1, COMP, NEWTON>(P, src, i0, nt, n_pad, eps2, part, epi, st);
-        return launch_part_tile<2, COMP, NEWTON>(P, src, i0, nt, n_pad, eps2, part, epi, st);
-    }
     switch (tile) {
+    case kTilePart128: return launch_part_tile<1, 1, COMP, NEWTON>(src, i0, nt, n_pad, eps2, part, epi, st);
+    case kTilePart64: return launch_part_tile<2, 2, COMP, NEWTON>(src, i0, nt, n_pad, eps2, part, epi, st);
     case 0: return launch_force_tile<1, 1, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
     case 1: return launch_force_tile<2, 1, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
     case 2: return launch_force_tile<4, 1, COMP, NEWTON>(src, i0, nt, n_pad, eps2, epi, st);
