@@ -139,8 +139,8 @@ hipError_t launch_fp32_step(const StepArgs& a, const float4* pos_old, float4* po
         return launch_sym(tile_get(a.tile), a.newton, false, pos_old, a.n, a.n_pad, a.eps2f, a.ipart,
                           a.jpart, epi, st);
     if (a.newton)
-        return launch_force<false, true>(a.tile, pos_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
-    return launch_force<false, false>(a.tile, pos_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+        return launch_force<false, true>(a.tile, pos_old, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
+    return launch_force<false, false>(a.tile, pos_old, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
 }
 
 hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* snap_new,
@@ -154,8 +154,8 @@ hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* 
         return launch_sym(tile_get(a.tile), a.newton, true, snap_old, a.n, a.n_pad, a.eps2f, a.ipart,
                           a.jpart, epi, st);
     if (a.newton)
-        return launch_force<true, true>(a.tile, snap_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
-    return launch_force<true, false>(a.tile, snap_old, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+        return launch_force<true, true>(a.tile, snap_old, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
+    return launch_force<true, false>(a.tile, snap_old, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
 }
 
 // One-pass tile for a slice of nt targets against all sources (the
@@ -171,21 +171,11 @@ hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* 
 // Many small waves fill the chip whatever the number of targets; 256 parts
 // gain at most 3% more and take twice the workspace, K = 4 (k4p32 ... k4p128)
 // is slower throughout.  Which of the two it is does not change a bit of the
-// result, nor does the slicing.
-int slice_tile_default(int64_t nt, int cu_count, size_t part_ws)
+// result, nor does the slicing: where the workspace holds fewer targets than
+// the slice has, it is evaluated in several launches (launch_part_tile).
+int slice_tile_default(int64_t nt, size_t part_ws)
 {
-    if (part_floats(kTilePart128, nt) <= part_ws)
-        return kTilePart128;
-    if (part_floats(kTilePart64, nt) <= part_ws)
-        return kTilePart64;
-    // without the workspace: the fewer the targets per CU, the more source
-    // splits keep the waves busy
-    const int64_t cus = cu_count > 0 ? cu_count : 256;
-    if (nt <= 64 * cus)
-        return 9;   // k1s16
-    if (nt <= 128 * cus)
-        return 34;  // k2s16
-    return 8;       // k2s8
+    return part_floats(kTilePart128, nt) <= part_ws ? kTilePart128 : kTilePart64;
 }
 
 hipError_t launch_fp32_step_slice(const StepArgs& a, int tile, int i0, int nt, const float4* pos_old,
@@ -238,12 +228,12 @@ hipError_t launch_fp32_accel(const StepArgs& a, const float4* src, bool compensa
                           a.jpart, epi, st);
     if (compensated) {
         if (a.newton)
-            return launch_force<true, true>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
-        return launch_force<true, false>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+            return launch_force<true, true>(a.tile, src, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
+        return launch_force<true, false>(a.tile, src, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
     }
     if (a.newton)
-        return launch_force<false, true>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
-    return launch_force<false, false>(a.tile, src, a.n, a.n_pad, a.eps2f, a.ipart, epi, st);
+        return launch_force<false, true>(a.tile, src, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
+    return launch_force<false, false>(a.tile, src, a.n, a.n_pad, a.eps2f, a.part_ws, epi, st);
 }
 
 }  // namespace utcnb

@@ -98,22 +98,32 @@ __global__ __launch_bounds__(256) void part_reduce_kernel(const float* __restric
         sum_epilogue(epi, i0 + j, s);
 }
 
+// Targets [i0, i0 + nt), as many per launch as the workspace holds.
 template <int K, int H, bool COMP, bool NEWTON, class Epi>
-hipError_t launch_part_tile(const float4* src, int i0, int nt, int n_pad, float eps2, float* part, const Epi& epi,
+hipError_t launch_part_tile(const float4* src, int i0, int nt, int n_pad, float eps2, const PartWs& ws, const Epi& epi,
                             hipStream_t st)
 {
-    if (!part)
-        return hipErrorInvalidValue;
-    const int tiles = (nt + 64 * K - 1) / (64 * K);
-    hipLaunchKernelGGL((part_force_kernel<K, H, COMP, NEWTON>), dim3((tiles + 3) / 4, kSourceParts / H), dim3(256), 0,
-                       st, src, i0, nt, n_pad, eps2, part);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess)
-        return e;
+    constexpr int P = kSourceParts / H;
     using Acc = typename std::conditional<COMP, double, float>::type;
-    const dim3 grid((unsigned)(((long long)nt * kPartLanes + 255) / 256));
-    hipLaunchKernelGGL((part_reduce_kernel<H, Acc, Epi>), grid, dim3(256), 0, st, part, i0, nt, epi);
-    return hipGetLastError();
+    const size_t most = ws.p ? ws.floats / (3 * P) : 0;
+    if (most < 1)
+        return hipErrorInvalidValue;
+    for (int a = 0; a < nt;) {
+        const int c = most < (size_t)(nt - a) ? (int)most : nt - a;
+        const int tiles = (c + 64 * K - 1) / (64 * K);
+        hipLaunchKernelGGL((part_force_kernel<K, H, COMP, NEWTON>), dim3((tiles + 3) / 4, P), dim3(256), 0, st, src,
+                           i0 + a, c, n_pad, eps2, ws.p);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess)
+            return e;
+        const dim3 grid((unsigned)(((long long)c * kPartLanes + 255) / 256));
+        hipLaunchKernelGGL((part_reduce_kernel<H, Acc, Epi>), grid, dim3(256), 0, st, ws.p, i0 + a, c, epi);
+        e = hipGetLastError();
+        if (e != hipSuccess)
+            return e;
+        a += c;
+    }
+    return hipSuccess;
 }
 
 }  // namespace utcnb

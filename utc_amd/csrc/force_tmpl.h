@@ -326,12 +326,12 @@ hipError_t launch_force_tile(const float4* src, int i0, int nt, int n_pad, float
 }
 
 // Dispatch over the tile table (must match tile_get()); targets [i0, i0 + nt).
-// part: workspace of the tiles with source parts ([parts][nt][3] floats).
+// part: workspace of the tiles with source parts.
 // n: the system's bodies (the small-system tiles read no more of src, the
 // others the n_pad padded ones).
 template <bool COMP, bool NEWTON, class Epi>
-hipError_t launch_force_range(int tile, const float4* src, int i0, int nt, int n, int n_pad, float eps2, float* part,
-                              const Epi& epi, hipStream_t st)
+hipError_t launch_force_range(int tile, const float4* src, int i0, int nt, int n, int n_pad, float eps2,
+                              const PartWs& part, const Epi& epi, hipStream_t st)
 {
     if (nt < 1)
         return hipErrorInvalidValue;
@@ -368,7 +368,7 @@ hipError_t launch_force_range(int tile, const float4* src, int i0, int nt, int n
 
 // All n bodies as targets.
 template <bool COMP, bool NEWTON, class Epi>
-hipError_t launch_force(int tile, const float4* src, int n, int n_pad, float eps2, float* part,
+hipError_t launch_force(int tile, const float4* src, int n, int n_pad, float eps2, const PartWs& part,
                         const Epi& epi, hipStream_t st)
 {
     return launch_force_range<COMP, NEWTON>(tile, src, 0, n, n, n_pad, eps2, part, epi, st);

@@ -57,6 +57,12 @@ int tile_default(int64_t n, int cu_count, size_t partial_budget);
 int sym_share_tile_default(int64_t n, int cu_count);
 
 // ---- launchers (force.hip) ------------------------------------------------
+// Workspace of the tiles with source parts, [parts][targets][3].
+struct PartWs {
+    float* p = nullptr;
+    size_t floats = 0;
+};
+
 struct StepArgs {
     int n;          // bodies
     int n_pad;      // padded j length (fast kernels)
@@ -67,11 +73,9 @@ struct StepArgs {
     bool newton;
     int tile;       // tile id
     int share_tile; // symmetric tiles: the tile whose wave blocks shares and chunks divide
-    float* ipart;   // symmetric tiles: target-side partials [R][n_pad][3]; tiles
-                    // with source parts: [parts][n][3]
+    float* ipart;   // symmetric tiles: target-side partials [R][n_pad][3]
     float* jpart;   // symmetric tiles: reaction partials
-    float* part_ws;        // slices: workspace of the tiles with source parts
-    size_t part_ws_floats; //   and its size
+    PartWs part_ws; // tiles with source parts
     // symmetric tiles evaluated in chunks of wave blocks (0: one launch)
     int chunks;
     int chunk_r;    // waves per wave block in a chunk
@@ -134,7 +138,7 @@ hipError_t launch_ref_accel_slice_f64(const double4* src, int n, int i0, int nt,
                                       hipStream_t st);
 // Fast paths on one-pass tiles (`tile`; the symmetric ones do not split by
 // target): full-size state arrays, updated for the slice only.
-int slice_tile_default(int64_t nt, int cu_count, size_t part_ws);
+int slice_tile_default(int64_t nt, size_t part_ws);
 // Workspace of a tile with source parts for nt targets (floats; 0 for others).
 size_t part_floats(int tile, int64_t nt);
 hipError_t launch_fp32_step_slice(const StepArgs& a, int tile, int i0, int nt, const float4* pos_old,

@@ -168,8 +168,9 @@ extern "C" int utcnb_accel_noalloc(const float* pos4, int n, double eps2, int pr
     a.eps2f = (float)eps2;
     a.newton = (flags & UTCNB_FLAG_NO_NEWTON) == 0;
     a.tile = t;
-    a.ipart = tl.sym || tl.parts > 0 ? (float*)(base + ipart_off) : nullptr;
+    a.ipart = tl.sym ? (float*)(base + ipart_off) : nullptr;
     a.jpart = tl.sym ? (float*)(base + jpart_off) : nullptr;
+    a.part_ws = {(float*)(base + ipart_off), part_floats(t, n)};
     e = launch_fp32_accel(a, src, precision == UTCNB_PREC_MIXED, acc3, st);
     if (e != hipSuccess)
         return fail(UTCNB_EHIP, std::string("utcnb_accel_noalloc: field kernel: ") + hipGetErrorString(e));
