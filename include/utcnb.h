@@ -236,11 +236,13 @@ int utcnb_accel(utcnb_system* sys, double* acc3);
  * the null stream).  precision FP32 (plain sums) or MIXED (compensated), tile
  * and flags (UTCNB_FLAG_NO_NEWTON) as in utcnb_config; the result is bitwise
  * the utcnb_accel field of a handle of that precision, tile and flags whose
- * FP32 source positions equal pos4.  Work memory (padded sources, partial
+ * FP32 source positions equal pos4 -- with tile 0 where a handle's default tile
+ * fits the work memory; beyond, it is the utcnb_accel_slice field of all n
+ * bodies (tile k2p64) up to about 85000 bodies, then that of tile k2s8.  Work memory (padded sources, partial
  * sums) comes from a 64 MiB device array that the library holds on each
  * device it runs on until the process ends; sizes whose work memory exceeds
- * it are refused with UTCNB_EINVAL (with the default tile, n up to about
- * 32768 on the symmetric tiles and about 4M on the one-pass ones).  Calls on
+ * it are refused with UTCNB_EINVAL (with the default tile, n up to 49152 on the
+ * symmetric tiles and about 4M on the one-pass ones).  Calls on
  * one device share that array: calls that overlap on one device race.
  */
 int utcnb_accel_noalloc(const float* pos4, int n, double eps2, int precision, int tile, int flags,
