@@ -254,15 +254,17 @@ int utcnb_diagnostics(utcnb_system* sys, double* kinetic, double* potential,
 
 /*
  * Forward `nsteps` steps from the current state, then the adjoint for
- * L = (1/n) sum_i |x_i(T) - t_i|^2 back to that state.  The positions of every
- * step are kept on the device while they take at most 1 GiB (32 n nsteps
- * bytes); else FP64 checkpoints of (x, v) are kept every `ckpt_every` steps and
- * the steps in between are recomputed during the reverse sweep, except those
- * of the last segment, whose positions the forward sweep leaves in the segment
- * buffer (the same bits a recompute gives).  With more than one segment the
- * recomputes run on an internal stream, one segment ahead of the VJP steps on
- * the handle's stream (the reference kick keeps them on the handle's stream); the call
- * returns after both.  Precision MIXED (FP32 pair VJP) or
+ * L = (1/n) sum_i |x_i(T) - t_i|^2 back to that state.  FP64 checkpoints of
+ * (x, v) are kept every `ckpt_every` steps and the steps in between are
+ * recomputed during the reverse sweep, except those of the last segment, whose
+ * positions the forward sweep leaves in the segment buffer (the same bits a
+ * recompute gives).  `ckpt_every` bounds the device memory: 64 bytes a body for
+ * each checkpoint and 32 for each step of two segments.  Where the positions of
+ * all steps (16 bytes a body and step for MIXED, 32 for FP64) take no more than
+ * that, they are kept instead and nothing is recomputed.  With more than one
+ * segment the recomputes run on an internal stream, one segment ahead of the VJP
+ * steps on the handle's stream (the reference kick keeps them on the handle's
+ * stream); the call returns after both.  Precision MIXED (FP32 pair VJP) or
  * FP64.  target3: host FP64 [3n].  Outputs (host, FP64): *loss, dx0[3n],
  * dv0[3n], dm[n].  The system ends in the final (step nsteps) state.
  */
@@ -316,8 +318,8 @@ int utcnb_batch_get_state(utcnb_batch* b, double* pos4, double* vel4);
  * tile 0, 4 or 5 every system is padded to a multiple of 256 bodies, else 64.
  * The batched adjoint supports the physical kick only.
  * When target3 is non-NULL the adjoint of the same loss as utcnb_adjoint runs
- * after the forward steps (checkpoint every ckpt_every, or every step's
- * positions kept, as there) and losses[nsys],
+ * after the forward steps (checkpoint every ckpt_every, or all positions kept
+ * where they take no more than the checkpoints and one segment) and losses[nsys],
  * dx0/dv0 [3 * sum(sizes)], dm [sum(sizes)] receive per-system results.
  * *ms receives the wall time of the call measured with HIP events.
  */

@@ -251,10 +251,12 @@ __global__ __launch_bounds__(64) void loss_finish_kernel(const double* __restric
         *loss = v / n;
 }
 
-// One step's per-body adjoint and the source records for the VJP.
-// acc3 (nullable) is the field at this step's positions (reference kick only).
+// One step's per-body adjoint and the source records for the VJP, whose
+// positions are pos.  Reference kick only: mass[i].w is body i's mass in FP64,
+// and acc3 (nullable) the field at this step's positions.
 template <typename T4, typename E>
-__global__ __launch_bounds__(256) void adjoint_pre_kernel(const double4* __restrict__ pos,
+__global__ __launch_bounds__(256) void adjoint_pre_kernel(const T4* __restrict__ pos,
+                                                          const double4* __restrict__ mass,
                                                           const double* __restrict__ acc3,
                                                           int n, double dt, double damping,
                                                           int kick, double* __restrict__ xbar3,
@@ -265,8 +267,7 @@ __global__ __launch_bounds__(256) void adjoint_pre_kernel(const double4* __restr
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n)
         return;
-    const double4 p = pos[i];
-    const double ki = kick == UTCNB_KICK_REFERENCE ? p.w : 1.0;
+    const double ki = kick == UTCNB_KICK_REFERENCE ? mass[i].w : 1.0;
     double al[3], dota = 0.0;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -278,7 +279,7 @@ __global__ __launch_bounds__(256) void adjoint_pre_kernel(const double4* __restr
     }
     if (acc3)
         mbar[i] += damping * dt * dota;
-    jrec[2 * (size_t)i] = T4((E)p.x, (E)p.y, (E)p.z, (E)p.w);
+    jrec[2 * (size_t)i] = pos[i];
     jrec[2 * (size_t)i + 1] = T4((E)al[0], (E)al[1], (E)al[2], (E)0);
 }
 
@@ -306,17 +307,17 @@ hipError_t launch_loss_seed(const double4* pos, const double* tgt3, int n, doubl
     return hipGetLastError();
 }
 
-hipError_t launch_adjoint_pre(bool fp32_records, const double4* pos, const double* acc3, int n,
+hipError_t launch_adjoint_pre(bool fp32_records, const void* pos, const double4* mass, const double* acc3, int n,
                               double dt, double damping, int kick, double* xbar3, double* vbar3,
                               double* mbar, void* jrec, hipStream_t st)
 {
     const int blocks = (n + 255) / 256;
     if (fp32_records)
-        hipLaunchKernelGGL((adjoint_pre_kernel<float4, float>), dim3(blocks), dim3(256), 0, st, pos,
-                           acc3, n, dt, damping, kick, xbar3, vbar3, mbar, (float4*)jrec);
+        hipLaunchKernelGGL((adjoint_pre_kernel<float4, float>), dim3(blocks), dim3(256), 0, st,
+                           (const float4*)pos, mass, acc3, n, dt, damping, kick, xbar3, vbar3, mbar, (float4*)jrec);
     else
-        hipLaunchKernelGGL((adjoint_pre_kernel<double4, double>), dim3(blocks), dim3(256), 0, st, pos,
-                           acc3, n, dt, damping, kick, xbar3, vbar3, mbar, (double4*)jrec);
+        hipLaunchKernelGGL((adjoint_pre_kernel<double4, double>), dim3(blocks), dim3(256), 0, st,
+                           (const double4*)pos, mass, acc3, n, dt, damping, kick, xbar3, vbar3, mbar, (double4*)jrec);
     return hipGetLastError();
 }
 

@@ -134,9 +134,10 @@ struct utcnb_batch {
     float4* svjpart = nullptr;
     bool has_state = false;
     // adjoint workspace
-    int nck = 0, seg = 0;
+    int nck = 0;  // checkpoints ckpt holds (several segments only)
+    int seg = 0;  // steps segpos holds
     double4* ckpt = nullptr;
-    double4* segpos = nullptr;
+    float4* segpos = nullptr;
     double4* wpos = nullptr;
     double4* wvel = nullptr;
     float4* wsnap[2] = {nullptr, nullptr};
@@ -168,15 +169,20 @@ struct utcnb_batch {
 
 namespace {
 
-void release_adj(utcnb_batch* b)
+// A captured graph holds the addresses of the adjoint's buffers: it is dropped
+// before one of them is freed, so the next mode 0 run captures again instead of
+// replaying launches on freed memory.
+void drop_graph(utcnb_batch* b)
 {
-    // a captured graph holds the addresses of the buffers freed below: drop
-    // it, so the next mode 0 run captures again instead of replaying launches
-    // on freed memory
     if (b->exec)
         (void)hipGraphExecDestroy(b->exec);
     b->exec = nullptr;
     b->g_nsteps = -1;
+}
+
+void release_adj(utcnb_batch* b)
+{
+    drop_graph(b);
     dfree(b->ckpt);
     dfree(b->segpos);
     dfree(b->wpos);
@@ -451,34 +457,47 @@ hipError_t setup_sym(utcnb_batch* b)
     return e;
 }
 
+// The adjoint's workspace for nck segments of up to seg steps: buffers that are
+// too small are replaced, the others stay.
 int adj_workspace(utcnb_batch* b, int nck, int seg)
 {
-    if (b->xbar && b->nck >= nck && b->seg >= seg)
-        return UTCNB_OK;
-    release_adj(b);
     const size_t T = (size_t)b->total;
-    int rc = dalloc(&b->ckpt, 2 * T * (size_t)nck) || dalloc(&b->segpos, T * (size_t)seg) ||
-             dalloc(&b->wpos, T) || dalloc(&b->wvel, T) || dalloc(&b->wsnap[0], T) ||
-             dalloc(&b->wsnap[1], T) || dalloc(&b->jrec, 2 * T) || dalloc(&b->xbar, 3 * T) ||
-             dalloc(&b->vbar, 3 * T) || dalloc(&b->mbar, T) || dalloc(&b->tgt, 3 * T) ||
-             dalloc(&b->loss, (size_t)b->nsys);
-    if (!rc && b->has_sym())
-        rc = dalloc(&b->svipart, b->svi_count) || dalloc(&b->svjpart, b->svj_count);
-    if (rc) {
-        release_adj(b);
-        return fail(UTCNB_ENOMEM, "utcnb_batch_run: adjoint workspace allocation failed");
+    if (!b->xbar) {
+        int rc = dalloc(&b->wpos, T) || dalloc(&b->wvel, T) || dalloc(&b->wsnap[0], T) ||
+                 dalloc(&b->wsnap[1], T) || dalloc(&b->jrec, 2 * T) || dalloc(&b->xbar, 3 * T) ||
+                 dalloc(&b->vbar, 3 * T) || dalloc(&b->mbar, T) || dalloc(&b->tgt, 3 * T) ||
+                 dalloc(&b->loss, (size_t)b->nsys);
+        if (!rc && b->has_sym())
+            rc = dalloc(&b->svipart, b->svi_count) || dalloc(&b->svjpart, b->svj_count);
+        if (rc) {
+            release_adj(b);
+            return fail(UTCNB_ENOMEM, "utcnb_batch_run: adjoint workspace allocation failed");
+        }
+        // the step kernels write real bodies only: pad the work state once
+        hipError_t e = launch_batch_pad(b->geom(0), b->nsys, b->wpos, b->wvel, b->wsnap[0], b->wsnap[1],
+                                        b->stream);
+        if (e != hipSuccess)
+            return fail(UTCNB_EHIP, std::string("utcnb_batch_run: padding: ") + hipGetErrorString(e));
     }
-    b->nck = nck;
-    b->seg = seg;
-    // the step kernels write real bodies only: pad the work state and the
-    // segment's positions once (b->pos holds the padding bodies)
-    for (int t = 0; t < seg; ++t)
-        UTCNB_HIP(hipMemcpyAsync(b->segpos + T * (size_t)t, b->pos, T * sizeof(double4), hipMemcpyDeviceToDevice,
-                                 b->stream));
-    hipError_t e = launch_batch_pad(b->geom(0), b->nsys, b->wpos, b->wvel, b->wsnap[0], b->wsnap[1],
-                                    b->stream);
-    if (e != hipSuccess)
-        return fail(UTCNB_EHIP, std::string("utcnb_batch_run: padding: ") + hipGetErrorString(e));
+    if (nck > 1 && b->nck < nck) {
+        drop_graph(b);
+        b->nck = 0;
+        dfree(b->ckpt);
+        if (dalloc(&b->ckpt, 2 * T * (size_t)nck))
+            return fail(UTCNB_ENOMEM, "utcnb_batch_run: adjoint workspace allocation failed");
+        b->nck = nck;
+    }
+    if (b->seg < seg) {
+        drop_graph(b);
+        b->seg = 0;
+        dfree(b->segpos);
+        if (dalloc(&b->segpos, T * (size_t)seg))
+            return fail(UTCNB_ENOMEM, "utcnb_batch_run: adjoint workspace allocation failed");
+        // and the segment's positions (b->pos holds the padding bodies)
+        for (int t = 0; t < seg; ++t)
+            UTCNB_HIP(launch_snapshot(b->pos, b->segpos + T * (size_t)t, (int)T, b->stream));
+        b->seg = seg;
+    }
     return UTCNB_OK;
 }
 
@@ -550,7 +569,7 @@ hipError_t for_groups(utcnb_batch* b, F fn)
 }
 
 hipError_t sym_step_group(const utcnb_batch* b, int sk, int g, const float4* so, float4* sn, double4* p,
-                          double4* v, hipStream_t sg, double4* keep = nullptr)
+                          double4* v, hipStream_t sg, float4* keep = nullptr)
 {
     return launch_batch_sym_step(b->sym_geom(sk, 0, g), b->snwaves[sk][g], b->group_bodies(g), so, sn, p, v,
                                  (float)b->cfg.eps2, b->cfg.dt, b->cfg.damping, b->cfg.kick, b->sipart,
@@ -589,7 +608,7 @@ hipError_t enqueue_run_sym(utcnb_batch* b, int nsteps, int ckpt, bool adj, int s
                 ENQ(hipMemcpyAsync(ck + T + b0, b->vel + b0, sb, hipMemcpyDeviceToDevice, sg));
             }
             if (adj && t == 0 && slast == 0)
-                ENQ(hipMemcpyAsync(b->segpos + b0, b->pos + b0, sb, hipMemcpyDeviceToDevice, sg));
+                ENQ(launch_snapshot(b->pos + b0, b->segpos + b0, (int)Tg, sg));
             ENQ(sym_step_group(b, sk, g, b->snap[c], b->snap[1 - c], b->pos, b->vel, sg,
                                adj && t + 1 >= slast && t + 1 < nsteps ? b->segpos + T * (size_t)(t + 1 - slast)
                                                                       : nullptr));
@@ -608,7 +627,7 @@ hipError_t enqueue_run_sym(utcnb_batch* b, int nsteps, int ckpt, bool adj, int s
                 ENQ(hipMemcpyAsync(b->wvel + b0, ck + T + b0, sb, hipMemcpyDeviceToDevice, sg));
                 ENQ(launch_snapshot(b->wpos + b0, b->wsnap[0] + b0, (int)Tg, sg));
                 int wc = 0;
-                ENQ(hipMemcpyAsync(b->segpos + b0, b->wpos + b0, sb, hipMemcpyDeviceToDevice, sg));
+                ENQ(launch_snapshot(b->wpos + b0, b->segpos + b0, (int)Tg, sg));
                 for (int t = s0; t + 1 < s1; ++t) {
                     ENQ(sym_step_group(b, sk, g, b->wsnap[wc], b->wsnap[1 - wc], b->wpos, b->wvel, sg,
                                        b->segpos + T * (size_t)(t + 1 - s0)));
@@ -618,12 +637,12 @@ hipError_t enqueue_run_sym(utcnb_batch* b, int nsteps, int ckpt, bool adj, int s
             for (int t = s1 - 1; t >= s0; --t) {
                 // the first of a segment; the others' is done by the VJP's reduction
                 if (t == s1 - 1)
-                    ENQ(launch_adjoint_pre(true, b->segpos + T * (size_t)(t - s0) + b0, nullptr, (int)Tg, dt, damp,
-                                           kick, b->xbar + 3 * b0, b->vbar + 3 * b0, b->mbar + b0,
+                    ENQ(launch_adjoint_pre(true, b->segpos + T * (size_t)(t - s0) + b0, nullptr, nullptr, (int)Tg, dt,
+                                           damp, kick, b->xbar + 3 * b0, b->vbar + 3 * b0, b->mbar + b0,
                                            b->jrec + 2 * b0, sg));
                 AdjointNext next;
                 if (t > s0)
-                    next = {b->segpos + T * (size_t)(t - 1 - s0), dt, damp, kick, b->vbar, b->jrec};
+                    next = {b->segpos + T * (size_t)(t - 1 - s0), dt, damp, b->vbar, b->jrec};
                 ENQ(launch_batch_sym_vjp(b->sym_geom(sk, 1, g), b->snwaves[sk][g], (int)Tg, b->jrec,
                                          (float)b->cfg.eps2, b->svipart, b->svjpart, b->xbar, b->mbar, next, sg));
             }
@@ -689,13 +708,13 @@ hipError_t enqueue_run(utcnb_batch* b, int nsteps, int ckpt, bool adj, int mode,
     const int k = ckpt < nsteps ? ckpt : nsteps;
     const int nck = (nsteps + k - 1) / k, slast = (nck - 1) * k;
     for (int t = 0; t < nsteps; ++t) {
-        if (adj && t % k == 0) {
+        if (adj && nck > 1 && t % k == 0) {
             double4* ck = b->ckpt + 2 * T * (size_t)(t / k);
             ENQ(hipMemcpyAsync(ck, b->pos, sb, hipMemcpyDeviceToDevice, st));
             ENQ(hipMemcpyAsync(ck + T, b->vel, sb, hipMemcpyDeviceToDevice, st));
         }
         if (adj && t >= slast)  // the last segment's positions, kept instead of recomputed
-            ENQ(hipMemcpyAsync(b->segpos + T * (size_t)(t - slast), b->pos, sb, hipMemcpyDeviceToDevice, st));
+            ENQ(launch_snapshot(b->pos, b->segpos + T * (size_t)(t - slast), (int)T, st));
         ENQ(step(b->snap[c], b->snap[1 - c], b->pos, b->vel));
         c = 1 - c;
     }
@@ -711,8 +730,7 @@ hipError_t enqueue_run(utcnb_batch* b, int nsteps, int ckpt, bool adj, int mode,
             ENQ(launch_snapshot(b->wpos, b->wsnap[0], (int)T, st));
             int wc = 0;
             for (int t = s0; t < s1; ++t) {
-                ENQ(hipMemcpyAsync(b->segpos + T * (size_t)(t - s0), b->wpos, sb,
-                                   hipMemcpyDeviceToDevice, st));
+                ENQ(launch_snapshot(b->wpos, b->segpos + T * (size_t)(t - s0), (int)T, st));
                 if (t + 1 < s1) {
                     ENQ(step(b->wsnap[wc], b->wsnap[1 - wc], b->wpos, b->wvel));
                     wc = 1 - wc;
@@ -720,7 +738,7 @@ hipError_t enqueue_run(utcnb_batch* b, int nsteps, int ckpt, bool adj, int mode,
             }
         }
         for (int t = s1 - 1; t >= s0; --t) {
-            ENQ(launch_adjoint_pre(true, b->segpos + T * (size_t)(t - s0), nullptr, (int)T, dt, damp,
+            ENQ(launch_adjoint_pre(true, b->segpos + T * (size_t)(t - s0), nullptr, nullptr, (int)T, dt, damp,
                                    kick, b->xbar, b->vbar, b->mbar, b->jrec, st));
             ENQ(vjp());
         }
@@ -977,15 +995,7 @@ int utcnb_batch_run(utcnb_batch* b, int nsteps, int mode, int ckpt_every, const 
             return fail(UTCNB_EINVAL, "utcnb_batch_run: adjoint outputs and ckpt_every >= 1 required");
         if (b->cfg.kick != UTCNB_KICK_PHYSICAL)
             return fail(UTCNB_EINVAL, "utcnb_batch_run: the batched adjoint supports the physical kick");
-        // every step's positions while they fit kAdjointKeepBytes (one segment:
-        // nothing to recompute), else segments of ckpt_every steps
-        seg = ckpt_every < nsteps ? ckpt_every : nsteps;
-        if (seg < nsteps && (size_t)b->total * sizeof(double4) * (size_t)nsteps <= kAdjointKeepBytes) {
-            if (adj_workspace(b, 1, nsteps) == UTCNB_OK)
-                seg = nsteps;
-            else
-                (void)hipGetLastError();  // no memory for that: the segments need less
-        }
+        seg = adjoint_segment(nsteps, ckpt_every, 1, sizeof(float4));
         int rc = adj_workspace(b, (nsteps + seg - 1) / seg, seg);
         if (rc)
             return rc;

@@ -66,10 +66,10 @@ struct utcnb_system {
     int last_launches = 0;
     // adjoint workspace (allocated on first use, grown on demand)
     struct Adj {
-        int nck = 0, seg = 0;
+        int nck = 0;                 // checkpoints ckpt holds (several segments only)
         double4* ckpt = nullptr;     // nck * 2n (pos, vel)
-        double4* segpos = nullptr;   // seg * n
-        double4* segpos2 = nullptr;  // seg * n, second segment buffer (nck > 1)
+        int seg[2] = {0, 0};         // steps segpos[b] holds (the second: several segments only)
+        char* segpos[2] = {nullptr, nullptr};  // seg[b] * n positions (MIXED float4, FP64 double4)
         hipStream_t rstream = nullptr;  // segment recomputes beside the VJP steps
         hipEvent_t evfwd = nullptr, evrec[2] = {nullptr, nullptr}, evvjp = nullptr;
         double4* wpos[2] = {nullptr, nullptr};  // n_pad (FP64 work positions)
@@ -138,8 +138,8 @@ void release_adjoint(utcnb_system* s)
 {
     auto& a = s->adj;
     dfree(a.ckpt);
-    dfree(a.segpos);
-    dfree(a.segpos2);
+    dfree(a.segpos[0]);
+    dfree(a.segpos[1]);
     for (hipEvent_t* ev : {&a.evfwd, &a.evrec[0], &a.evrec[1], &a.evvjp}) {
         if (*ev)
             (void)hipEventDestroy(*ev);
@@ -165,7 +165,7 @@ void release_adjoint(utcnb_system* s)
     dfree(a.part);
     dfree(a.vjp_ipart);
     dfree(a.vjp_jpart);
-    a.nck = a.seg = a.vjp_r = 0;
+    a.nck = a.seg[0] = a.seg[1] = a.vjp_r = 0;
 }
 
 void release(utcnb_system* s)
@@ -673,8 +673,8 @@ int utcnb_get_state(utcnb_system* s, void* pos4, void* vel4, int dtype, int wher
 }
 
 // One step on the current buffers (no bookkeeping of timing).  MIXED: the new
-// positions also go to keep (unless null).
-static hipError_t step_once(utcnb_system* s, double4* keep = nullptr)
+// snapshot also goes to keep (unless null).
+static hipError_t step_once(utcnb_system* s, float4* keep = nullptr)
 {
     hipError_t e = hipSuccess;
     const int c = s->cur;
@@ -1037,17 +1037,21 @@ int utcnb_accel(utcnb_system* s, double* acc3)
 
 
 // ---- adjoint -------------------------------------------------------------------
-static int adjoint_workspace(utcnb_system* s, int nck, int seg)
+// Bytes of one body's positions in the segments' buffers.
+static int adjoint_row_bytes(const utcnb_system* s)
+{
+    return s->cfg.precision == UTCNB_PREC_MIXED ? sizeof(float4) : sizeof(double4);
+}
+
+// What does not depend on the number of steps.
+static int adjoint_base(utcnb_system* s)
 {
     auto& a = s->adj;
     const size_t n = (size_t)s->n, np = (size_t)s->n_pad;
     const bool f32 = s->cfg.precision == UTCNB_PREC_MIXED;
-    if (a.xbar && a.nck >= nck && a.seg >= seg)
+    if (a.xbar)
         return UTCNB_OK;
-    release_adjoint(s);
-    int rc = dalloc(&a.ckpt, 2 * n * (size_t)nck) || dalloc(&a.segpos, n * (size_t)seg) ||
-             (nck > 1 && dalloc(&a.segpos2, n * (size_t)seg)) ||
-             dalloc(&a.wpos[0], np) || dalloc(&a.wpos[1], np) || dalloc(&a.wvel, n) ||
+    int rc = dalloc(&a.wpos[0], np) || dalloc(&a.wpos[1], np) || dalloc(&a.wvel, n) ||
              dalloc(&a.xbar, 3 * n) || dalloc(&a.vbar, 3 * n) || dalloc(&a.mbar, n) ||
              dalloc(&a.tgt, 3 * n) || dalloc(&a.part, (n + 255) / 256 + 1);
     if (!rc && f32)
@@ -1070,19 +1074,10 @@ static int adjoint_workspace(utcnb_system* s, int nck, int seg)
         if (hipMalloc(&a.jrec, 2 * np * rb) != hipSuccess || hipMalloc(&a.fsrc, np * rb) != hipSuccess)
             rc = 1;
     }
-    if (!rc && nck > 1) {
-        if (hipStreamCreateWithFlags(&a.rstream, hipStreamNonBlocking) != hipSuccess)
-            rc = 1;
-        for (hipEvent_t* ev : {&a.evfwd, &a.evrec[0], &a.evrec[1], &a.evvjp})
-            if (!rc && hipEventCreateWithFlags(ev, hipEventDisableTiming) != hipSuccess)
-                rc = 1;
-    }
     if (rc) {
         release_adjoint(s);
         return fail(UTCNB_ENOMEM, "utcnb_adjoint: workspace allocation failed");
     }
-    a.nck = nck;
-    a.seg = seg;
     hipError_t e = launch_jrec_pad(f32, a.jrec, s->n, s->n_pad, s->stream);
     if (e == hipSuccess && f32)
         e = launch_pad_f32((float4*)a.fsrc, s->n, s->n_pad, s->stream);
@@ -1101,9 +1096,43 @@ static int adjoint_workspace(utcnb_system* s, int nck, int seg)
     return UTCNB_OK;
 }
 
+// The workspace of nck segments of up to seg steps: buffers that are too small
+// are replaced, the others stay.
+static int adjoint_workspace(utcnb_system* s, int nck, int seg)
+{
+    if (int rc = adjoint_base(s))
+        return rc;
+    auto& a = s->adj;
+    const size_t n = (size_t)s->n;
+    for (int b = 0; b < (nck > 1 ? 2 : 1); ++b) {
+        if (a.seg[b] >= seg)
+            continue;
+        a.seg[b] = 0;
+        dfree(a.segpos[b]);
+        if (int rc = dalloc(&a.segpos[b], n * (size_t)seg * adjoint_row_bytes(s)))
+            return rc;
+        a.seg[b] = seg;
+    }
+    if (nck == 1)
+        return UTCNB_OK;
+    if (a.nck < nck) {
+        a.nck = 0;
+        dfree(a.ckpt);
+        if (int rc = dalloc(&a.ckpt, 2 * n * (size_t)nck))
+            return rc;
+        a.nck = nck;
+    }
+    if (!a.rstream)
+        UTCNB_HIP(hipStreamCreateWithFlags(&a.rstream, hipStreamNonBlocking));
+    for (hipEvent_t* ev : {&a.evfwd, &a.evrec[0], &a.evrec[1], &a.evvjp})
+        if (!*ev)
+            UTCNB_HIP(hipEventCreateWithFlags(ev, hipEventDisableTiming));
+    return UTCNB_OK;
+}
+
 // One forward step of the adjoint's work state (wpos/wvel, with wsnap for
-// MIXED, whose new positions also go to keep unless null).
-static hipError_t work_step(utcnb_system* s, int& wc, hipStream_t st, double4* keep)
+// MIXED, whose new snapshot also goes to keep unless null).
+static hipError_t work_step(utcnb_system* s, int& wc, hipStream_t st, float4* keep)
 {
     auto& a = s->adj;
     hipError_t e;
@@ -1127,15 +1156,8 @@ int utcnb_adjoint(utcnb_system* s, int nsteps, int ckpt_every, const double* tar
         return fail(UTCNB_EINVAL, "utcnb_adjoint: nsteps and ckpt_every must be >= 1");
     if (!s->has_state)
         return fail(UTCNB_ESTATE, "utcnb_adjoint: no state set");
-    // every step's positions while they fit kAdjointKeepBytes (one segment:
-    // nothing to recompute), else segments of ckpt_every steps
-    int k = ckpt_every < nsteps ? ckpt_every : nsteps;
-    if (k < nsteps && (size_t)s->n * sizeof(double4) * (size_t)nsteps <= kAdjointKeepBytes) {
-        if (adjoint_workspace(s, 1, nsteps) == UTCNB_OK)
-            k = nsteps;
-        else
-            (void)hipGetLastError();  // no memory for that: the segments need less
-    }
+    const int rb = adjoint_row_bytes(s);
+    const int k = adjoint_segment(nsteps, ckpt_every, 2, rb);
     const int nck = (nsteps + k - 1) / k;
     int rc = adjoint_workspace(s, nck, k);
     if (rc)
@@ -1163,21 +1185,24 @@ int utcnb_adjoint(utcnb_system* s, int nsteps, int ckpt_every, const double* tar
     // recompute runs the same kernels on the same state, so the positions are
     // the same bits)
     const int slast = (nck - 1) * k;
-    // segment c's positions live in segbuf(c): two buffers, so that the
+    // segment c's positions live in segpos[c % 2]: two buffers, so that the
     // recompute of segment c - 1 can run beside the VJP steps of segment c
-    auto segbuf = [&](int c) { return (c % 2 == 0) ? a.segpos : a.segpos2; };
-    // (the MIXED steps write them there themselves)
+    auto row = [&](int t) { return a.segpos[t / k % 2] + n * rb * (size_t)(t % k); };
+    // step t's positions from the FP64 state (the MIXED steps write all but a
+    // segment's first there themselves)
+    auto store = [&](int t, const double4* pos, hipStream_t q) {
+        return mixed ? launch_snapshot(pos, (float4*)row(t), s->n, q)
+                     : hipMemcpyAsync(row(t), pos, sb, hipMemcpyDeviceToDevice, q);
+    };
     for (int t = 0; t < nsteps; ++t) {
         if (nck > 1 && t % k == 0) {
             double4* ck = a.ckpt + 2 * n * (size_t)(t / k);
             ADJ_CHECK(hipMemcpyAsync(ck, cur_p64(s), sb, hipMemcpyDeviceToDevice, st));
             ADJ_CHECK(hipMemcpyAsync(ck + n, s->v64, sb, hipMemcpyDeviceToDevice, st));
         }
-        if (t >= slast && (!mixed || t == 0))
-            ADJ_CHECK(hipMemcpyAsync(segbuf(nck - 1) + n * (size_t)(t - slast), cur_p64(s), sb,
-                                     hipMemcpyDeviceToDevice, st));
-        ADJ_CHECK(step_once(s, t + 1 >= slast && t + 1 < nsteps ? segbuf(nck - 1) + n * (size_t)(t + 1 - slast)
-                                                               : nullptr));
+        if (t >= slast && (!mixed || t == slast))
+            ADJ_CHECK(store(t, cur_p64(s), st));
+        ADJ_CHECK(step_once(s, t >= slast && t + 1 < nsteps ? (float4*)row(t + 1) : nullptr));
         ++launches;
     }
     // loss and its seed at the final state
@@ -1195,7 +1220,6 @@ int utcnb_adjoint(utcnb_system* s, int nsteps, int ckpt_every, const double* tar
     auto recompute = [&](int c) -> hipError_t {
         const int s0 = c * k, s1 = (s0 + k < nsteps) ? s0 + k : nsteps;
         const double4* ck = a.ckpt + 2 * n * (size_t)c;
-        double4* buf = segbuf(c);
         hipError_t e = hipMemcpyAsync(a.wpos[0], ck, sb, hipMemcpyDeviceToDevice, rs);
         if (e == hipSuccess)
             e = hipMemcpyAsync(a.wvel, ck + n, sb, hipMemcpyDeviceToDevice, rs);
@@ -1205,9 +1229,9 @@ int utcnb_adjoint(utcnb_system* s, int nsteps, int ckpt_every, const double* tar
         for (int t = s0; t < s1 && e == hipSuccess; ++t) {
             const double4* cur = mixed ? a.wpos[0] : a.wpos[wc];
             if (!mixed || t == s0)
-                e = hipMemcpyAsync(buf + n * (size_t)(t - s0), cur, sb, hipMemcpyDeviceToDevice, rs);
+                e = store(t, cur, rs);
             if (e == hipSuccess && t + 1 < s1) {
-                e = work_step(s, wc, rs, buf + n * (size_t)(t + 1 - s0));
+                e = work_step(s, wc, rs, (float4*)row(t + 1));
                 ++launches;
             }
         }
@@ -1228,27 +1252,25 @@ int utcnb_adjoint(utcnb_system* s, int nsteps, int ckpt_every, const double* tar
             ADJ_CHECK(hipStreamWaitEvent(st, a.evrec[c % 2], 0));
         bool pre_done = false;
         for (int t = s1 - 1; t >= s0; --t) {
-            const double4* xs = segbuf(c) + n * (size_t)(t - s0);
+            const char* xs = row(t);
             const double* acc = nullptr;
             if (refkick) {
-                if (mixed) {
-                    ADJ_CHECK(launch_snapshot(xs, (float4*)a.fsrc, s->n, st));
+                ADJ_CHECK(hipMemcpyAsync(a.fsrc, xs, n * rb, hipMemcpyDeviceToDevice, st));
+                if (mixed)
                     ADJ_CHECK(launch_fp32_accel(s->args, (const float4*)a.fsrc, true, s->scratch, st));
-                } else {
-                    ADJ_CHECK(hipMemcpyAsync(a.fsrc, xs, sb, hipMemcpyDeviceToDevice, st));
+                else
                     ADJ_CHECK(launch_fp64_accel(s->args, (const double4*)a.fsrc, s->scratch, st));
-                }
                 acc = s->scratch;
                 ++launches;
             }
             if (!pre_done)
-                ADJ_CHECK(launch_adjoint_pre(mixed, xs, acc, s->n, s->cfg.dt, s->cfg.damping,
-                                             s->cfg.kick, a.xbar, a.vbar, a.mbar, a.jrec, st));
+                ADJ_CHECK(launch_adjoint_pre(mixed, xs, cur_p64(s), acc, s->n, s->cfg.dt, s->cfg.damping, s->cfg.kick,
+                                             a.xbar, a.vbar, a.mbar, a.jrec, st));
             pre_done = false;
             if (mixed && a.vjp_r > 0) {
                 AdjointNext next;
                 if (!refkick && t > s0) {  // the segment's step before, whose positions are there
-                    next = {xs - n, s->cfg.dt, s->cfg.damping, s->cfg.kick, a.vbar, (float4*)a.jrec};
+                    next = {(const float4*)row(t - 1), s->cfg.dt, s->cfg.damping, a.vbar, (float4*)a.jrec};
                     pre_done = true;
                 }
                 ADJ_CHECK(launch_sym_vjp((const float4*)a.jrec, s->n, s->n_pad, s->args.eps2f, a.vjp_r,

@@ -144,7 +144,7 @@ hipError_t launch_fp32_step(const StepArgs& a, const float4* pos_old, float4* po
 }
 
 hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* snap_new,
-                             double4* pos, double4* vel, hipStream_t st, double4* keep)
+                             double4* pos, double4* vel, hipStream_t st, float4* keep)
 {
     EpiMixed epi{pos, vel, snap_new, a.dt, a.damping, a.kick, keep};
     if (tile_get(a.tile).sym && a.chunks > 0)

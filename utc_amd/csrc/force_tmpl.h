@@ -155,15 +155,15 @@ struct EpiFP32 {
     }
 };
 
-// FP64 state updated in place, new FP32 snapshot written for the next step;
-// keep (or null): the new positions once more (the adjoint's trajectory).
+// FP64 state updated in place, new FP32 snapshot written for the next step and
+// once more to keep (or null; the adjoint's trajectory).
 struct EpiMixed {
     double4* pos;
     double4* vel;
     float4* snap_new;
     double dt, damping;
     int kick;
-    double4* keep = nullptr;
+    float4* keep = nullptr;
     struct State {
         double4 p, v;
     };
@@ -186,9 +186,10 @@ struct EpiMixed {
         p.z += v.z * dt;
         pos[i] = p;
         vel[i] = v;
-        snap_new[i] = make_float4((float)p.x, (float)p.y, (float)p.z, (float)p.w);
+        const float4 s = make_float4((float)p.x, (float)p.y, (float)p.z, (float)p.w);
+        snap_new[i] = s;
         if (keep)
-            keep[i] = p;
+            keep[i] = s;
     }
     __device__ __forceinline__ void operator()(int i, float hx, float hy, float hz, float cx, float cy,
                                                float cz) const

@@ -103,15 +103,24 @@ hipError_t launch_ref_step_f64(const double4* pos_old, double4* pos_new, double4
 hipError_t launch_fp32_step(const StepArgs& a, const float4* pos_old, float4* pos_new,
                             float4* vel, hipStream_t st);
 // Mixed: forces from snap_old (padded float4), FP64 state updated in place,
-// new snapshot written to snap_new; the new positions also to keep unless null.
+// new snapshot written to snap_new, and once more to keep unless null.
 hipError_t launch_mixed_step(const StepArgs& a, const float4* snap_old, float4* snap_new,
-                             double4* pos, double4* vel, hipStream_t st, double4* keep = nullptr);
-// Device memory (bytes) the adjoint takes to keep the positions of every step
-// instead of recomputing all segments but the last (utcnb_adjoint,
-// utcnb_batch_run).  N = 16384, 50 steps, checkpoint every 10 (26 MB): 11.6 ms
-// with four segments recomputed beside the VJP steps, 10.2 without; 96 systems
-// of 256 to 8192 bodies, 20 steps, checkpoint every 10: 16.7 and 14.5 ms.
-constexpr size_t kAdjointKeepBytes = (size_t)1 << 30;
+                             double4* pos, double4* vel, hipStream_t st, float4* keep = nullptr);
+// Steps per segment of an adjoint of nsteps steps with a checkpoint every
+// ckpt_every (utcnb_adjoint, utcnb_batch_run).  The reverse sweep reads each
+// step's positions as FP32 records (MIXED, row_bytes 16 a body) or FP64 ones
+// (32).  What ckpt_every asks for is 64 bytes a body for each checkpoint and 32
+// for each step of the segments' buffers; where the positions of all steps take
+// no more than that they are all kept, in one segment, and nothing is
+// recomputed.  100 steps, all kept against segments of 10: N = 16384 17.8 and
+// 21.5 ms (recomputed beside the VJP steps), 40 systems of 256 to 4096 bodies
+// 12.5 and 16.4.
+inline int adjoint_segment(int nsteps, int ckpt_every, int buffers, int row_bytes)
+{
+    const long long k = ckpt_every < nsteps ? ckpt_every : nsteps, nck = (nsteps + k - 1) / k;
+    const long long asked = 64 * nck + 32 * k * (nck > 1 ? buffers : 1);
+    return (long long)row_bytes * nsteps <= asked ? nsteps : (int)k;
+}
 // FP64: forces from pos_old (padded double4) into pos_new / vel.
 hipError_t launch_fp64_step(const StepArgs& a, const double4* pos_old, double4* pos_new,
                             double4* vel, hipStream_t st);
@@ -185,7 +194,9 @@ hipError_t launch_vjp_f64(const double4* jrec, int n, int n_pad, double eps2, do
 hipError_t launch_loss_seed(const double4* pos, const double* tgt3, int n, double* xbar3,
                             double* vbar3, double* mbar, double* part, double* loss,
                             hipStream_t st);
-hipError_t launch_adjoint_pre(bool fp32_records, const double4* pos, const double* acc3, int n,
+// pos: n records of four values, FP32 or FP64; mass: FP64 records whose w is the
+// mass (reference kick only).
+hipError_t launch_adjoint_pre(bool fp32_records, const void* pos, const double4* mass, const double* acc3, int n,
                               double dt, double damping, int kick, double* xbar3, double* vbar3,
                               double* mbar, void* jrec, hipStream_t st);
 hipError_t launch_jrec_pad(bool fp32_records, void* jrec, int n, int n_pad, hipStream_t st);
@@ -196,12 +207,11 @@ int sym_vjp_splits(int n_pad, int cu_count);     // waves per wave block
 size_t sym_vjp_ipart_float4s(int n_pad, int R);
 size_t sym_vjp_jpart_float4s(int n_pad, int R);
 // The per-body adjoint of the step before (launch_adjoint_pre without a field,
-// FP32 records), done by the reduction of a VJP: pos null = not.  The records
-// are those the VJP read.
+// FP32 records, physical kick), done by the reduction of a VJP: pos null = not.
+// The records are those the VJP read.
 struct AdjointNext {
-    const double4* pos = nullptr;
+    const float4* pos = nullptr;
     double dt = 0.0, damping = 1.0;
-    int kick = 0;
     double* vbar3 = nullptr;
     float4* jrec = nullptr;
 };
@@ -247,7 +257,7 @@ hipError_t launch_batch_counter_reset(int* counter, hipStream_t st);
 hipError_t launch_batch_sym_step(const BatchSymGeom& g, int nwaves, int total, const float4* snap_old,
                                  float4* snap_new, double4* pos, double4* vel, float eps2, double dt,
                                  double damping, int kick, float* ipart, float* jpart, hipStream_t st,
-                                 double4* keep = nullptr);
+                                 float4* keep = nullptr);
 hipError_t launch_batch_sym_vjp(const BatchSymGeom& g, int nwaves, int total, const float4* jrec,
                                 float eps2, float4* ipart, float4* jpart, double* xbar3, double* mbar,
                                 const AdjointNext& next, hipStream_t st);

@@ -818,7 +818,7 @@ hipError_t launch_batch_counter_reset(int* counter, hipStream_t st)
 hipError_t launch_batch_sym_step(const BatchSymGeom& g, int nwaves, int total, const float4* snap_old,
                                  float4* snap_new, double4* pos, double4* vel, float eps2, double dt,
                                  double damping, int kick, float* ipart, float* jpart, hipStream_t st,
-                                 double4* keep)
+                                 float4* keep)
 {
     hipError_t e;
     if (g.counter && (e = launch_batch_counter_reset(g.counter, st)) != hipSuccess)

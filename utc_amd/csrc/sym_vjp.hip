@@ -345,16 +345,14 @@ __device__ __forceinline__ void adjoint_next(const AdjointNext& next, size_t b, 
     mbar[b] += s[3];
     if (!next.pos)
         return;
-    const double4 p = next.pos[b];
-    const double ki = next.kick == UTCNB_KICK_REFERENCE ? p.w : 1.0;
     double al[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const double ub = next.vbar3[3 * b + k] + x[k] * next.dt;
         next.vbar3[3 * b + k] = next.damping * ub;
-        al[k] = next.damping * ki * next.dt * ub;
+        al[k] = next.damping * next.dt * ub;
     }
-    next.jrec[2 * b] = make_float4((float)p.x, (float)p.y, (float)p.z, (float)p.w);
+    next.jrec[2 * b] = next.pos[b];
     next.jrec[2 * b + 1] = make_float4((float)al[0], (float)al[1], (float)al[2], 0.f);
 }
 
