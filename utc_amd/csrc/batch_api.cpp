@@ -30,10 +30,17 @@ constexpr int kWs[3] = {4, 8, 16};  // waves per work item of the one-pass kerne
 // waves through an atomic work counter (4), or one wave per item for the
 // hardware dispatcher to place (5).
 constexpr int kSymPersist = 3, kSymFlat = 4, kSels = 5;
-// Sub-units (64 sources against a wave block) per symmetric item: the fewest
-// that give a chip's worth of items, since a target-side record of each item is
-// written and read.  20 steps forward and adjoint, tile 5, ms, systems of 256
-// to 8192 bodies (mean 2300), by sub-units per item:
+// Sub-units (64 sources against a wave block) per split, that is per target-side
+// record, from the system alone, as are its bits then: one for systems of up to
+// 2048 bodies, two for others, a 8192nd of a larger system's.
+int sym_split_subunits(long long system_subunits)
+{
+    return (int)std::max(system_subunits <= 160 ? 1LL : 2LL, system_subunits / 8192);
+}
+// Sub-units per symmetric item, which takes whole splits: the fewest that give a
+// chip's worth of items, as an item loads its targets.  20 steps forward and
+// adjoint, tile 5, ms, systems of 256 to 8192 bodies (mean 2300), where each item
+// was one split, by sub-units of both:
 //   systems     1      2      3      4      6      8     12     16
 //         8   1.46   2.01   2.62   3.23   4.50   5.60   8.03   9.10
 //        20   3.75   3.72   3.74   4.12   4.83   6.07   8.56  11.11
@@ -41,12 +48,11 @@ constexpr int kSymPersist = 3, kSymFlat = 4, kSels = 5;
 //        96  14.25  13.72  13.71  13.91  13.61  13.76  14.64  14.61
 //       160  20.63  19.36  19.30  19.28  19.19  19.01  19.36  19.89
 //       256  31.52  29.22  28.85  28.79  28.36  28.28  28.19  28.31
-// Up to 131072 bodies in all the split is the system's alone (1, or a 8192nd
-// of a larger system's sub-units), and so are its bits.
-int sym_item_subunits(long long total_bodies, long long system_subunits)
+// With the splits of sym_split_subunits, against items of one split each chosen by
+// the batch: 8 systems 1.76 ms for 1.61, 96 12.7 for 12.4, 256 30.5 for 29.1.
+int sym_item_subunits(long long total_bodies)
 {
-    const long long least = total_bodies < (1 << 17) ? 1 : (total_bodies < (1 << 18) ? 6 : 8);
-    return (int)std::max(least, system_subunits / 8192);
+    return total_bodies < (1 << 17) ? 1 : (total_bodies < (1 << 18) ? 6 : 8);
 }
 // The per-system baseline (mode 1) spreads its launches over this many streams,
 // as the reference runs one task with its own stream per system; 4 is the
@@ -299,9 +305,9 @@ void schedule(const utcnb_batch* b, int W, int blocks, std::vector<int2>& items,
 }
 
 // Symmetric kernels: per system NW = npad / kBatchSymAlign wave blocks, each
-// with K (NW/2 + 1) (unit, source block) sub-units split over R waves
-// (sym_item_subunits each); an item's cost is its number of sub-units.
-// Items (system, wave block, split, R) are listed longest first; persistent
+// with K (NW/2 + 1) (unit, source block) sub-units in R splits
+// (sym_split_subunits each); an item's cost is its number of sub-units.
+// Items (system, wave block, splits, R) are listed longest first; persistent
 // waves take them in that order through an atomic work counter, or each item
 // gets a wave of its own.
 struct SymPlan {
@@ -326,8 +332,10 @@ void plan_sym(const utcnb_batch* b, int persistent_waves, SymPlan& P)
             ++grp;
         const int NW = b->npad[s] / kBatchSymAlign;
         const int sub = (NW / 2 + 1) * kBatchSymK;  // (unit, source block) sub-units per wave block
-        const int per = sym_item_subunits(b->total, (long long)NW * sub);
-        const int R = std::max(1, (sub + per - 1) / per);
+        const int per = sym_split_subunits((long long)NW * sub);
+        const int R = (sub + per - 1) / per;
+        // items per wave block, of as equal numbers of splits as can be
+        const int m = std::max(1, sym_item_subunits(b->total) / per), I = (R + m - 1) / m;
         P.nw.push_back(NW);
         P.rs.push_back(R);
         P.ipo.push_back(P.ifloats);
@@ -341,9 +349,10 @@ void plan_sym(const utcnb_batch* b, int persistent_waves, SymPlan& P)
         for (int blk = 0; blk < NW; ++blk)
             P.sysblk.push_back(s);
         for (int w = 0; w < NW; ++w)
-            for (int r = 0; r < R; ++r) {
-                const int q0 = (int)((long long)sub * r / R), q1 = (int)((long long)sub * (r + 1) / R);
-                all[grp].push_back({q1 - q0, make_int4(s, w, r, R)});
+            for (int i = 0; i < I; ++i) {
+                const int r0 = (int)((long long)R * i / I), r1 = (int)((long long)R * (i + 1) / I);
+                const int q0 = (int)((long long)sub * r0 / R), q1 = (int)((long long)sub * r1 / R);
+                all[grp].push_back({q1 - q0, make_int4(s, w, r0 + ((r1 - r0) << 16), R)});
             }
     }
     for (int k = 0; k < 2; ++k) {

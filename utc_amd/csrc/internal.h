@@ -238,7 +238,7 @@ hipError_t launch_batch_vjp(int W, const BatchGeom& g, int nblocks, const float4
 constexpr int kBatchSymK = 4;
 constexpr int kBatchSymAlign = 64 * kBatchSymK;
 struct BatchSymGeom {
-    const int4* items;        // (system, wave block, split, splits of the system)
+    const int4* items;        // (system, wave block, first split + 65536 * number of splits, splits of the system)
     const int* start;         // items of wave g: [start[g], start[g+1])
     const int* off;           // first body of each system (padded layout)
     const int* n;             // bodies per system

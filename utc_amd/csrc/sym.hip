@@ -265,6 +265,7 @@ __device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane
 // range of bodies only: body b of row r is record r * istride + b - ibody0
 // (istride < 0: n_pad, the whole system).  COMP: the target-side block
 // partials are Kahan-added (the compensated paths); otherwise plain FP32 sums.
+// nr: the wave does the work of waves r .. r + nr - 1 in turn (not SPLIT).
 // SPLIT (1 or 2, sym_block): the waves share the sub-units by chunks of 64 / rs
 // rotation steps (rs divides 16) and the reactions take a record per wave and sub-unit: jpart is
 // [NW][R][J][64][3] (SymSplit, sym_reduce.h).
@@ -272,7 +273,7 @@ template <int K, bool NEWTON, bool COMP, int SPLIT = 0>
 __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW, int R, int w, int r,
                                          float eps2, float* __restrict__ ipart,
                                          float* __restrict__ jpart, SymLds& L, int lane, int jbase = 0,
-                                         long long istride = -1, int ibody0 = 0, int rs = 1)
+                                         long long istride = -1, int ibody0 = 0, int rs = 1, int nr = 1)
 {
     const int half = NW / 2;
     const int n_pad = NW * 64 * K;
@@ -281,7 +282,6 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
     for (int k = 0; k < K; ++k) {
         const float4 p = src[w * 64 * K + k * 64 + lane];
         xi[k] = p.x; yi[k] = p.y; zi[k] = p.z; mi[k] = p.w;
-        ax[k] = ay[k] = az[k] = cx[k] = cy[k] = cz[k] = 0.f;
     }
     // one mass for every target of the wave?
     const float m0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(mi[0])));
@@ -289,75 +289,80 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
 #pragma unroll
     for (int k = 0; k < K; ++k)
         tuni = tuni && mi[k] == m0;
-    // sub-unit q = (unit u, source block kb): u = 0 is the wave block's own
-    // sources, u = 1 + d the wave block d + 1 places round
-    int qf, ql, c0 = 0, c1 = 0, J = 0;
-    const int len = SPLIT != 0 ? 64 / rs : 64;
-    if constexpr (SPLIT != 0) {
-        const SymSplit sp(NW, w, K, R, rs);
-        c0 = sp.first(r);
-        c1 = sp.first(r + 1);
-        qf = c0 / rs;
-        ql = (c1 + rs - 1) / rs;
-        J = SymSplit::records(NW, K, R, rs);
-    } else {
-        const int Q = (half + 1) * K;
-        qf = (int)((long long)Q * r / R);
-        ql = (int)((long long)Q * (r + 1) / R);
-    }
-    for (int q = qf; q < ql; ++q) {
-        // rotation steps [t0, t0 + steps): all but for the first and last sub-unit
-        int t0 = 0, steps = 64;
-        if constexpr (SPLIT != 0) {
-            const int a = q == qf ? c0 - q * rs : 0, e = q + 1 == ql ? c1 - q * rs : rs;
-            t0 = a * len;
-            steps = (e - a) * len;
-        }
-        const int u = q / K, kb = q - u * K;
-        if (u == 0) {
-            const float4 s = src[w * 64 * K + kb * 64 + lane];
-            const bool uni = __ballot(tuni && s.w == m0) == ~0ull;
-            if constexpr (K <= 4) {
-                // own block kb: two-sided against the lower target slots
-                sym_own_at<K, NEWTON, COMP, SPLIT>(kb, uni, L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
-                                                   az, cx, cy, cz);
-            } else {
-                // own block kb (K = 8, where own blocks are a small share and
-                // eight variants of sym_own_at would crowd the instruction cache):
-                // target side only (each ordered pair once, self pair gives 0)
-                float g[3];
-                sym_block<K, K, 0, NEWTON, COMP, false, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax,
-                                                               ay, az, cx, cy, cz, g);
-            }
-            continue;
-        }
-        const int d = u - 1;
-        if (2 * (d + 1) == NW && w >= half)
-            continue;  // the block half way round: taken by the lower half
-        int v = w + 1 + d;
-        if (v >= NW)
-            v -= NW;
-        const float4 s = src[v * 64 * K + kb * 64 + lane];
-        float g[3];
-        if (__ballot(tuni && s.w == m0) == ~0ull)
-            sym_block<K, K, K, NEWTON, COMP, true, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
-                                                          az, cx, cy, cz, g);
-        else
-            sym_block<K, K, K, NEWTON, COMP, false, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
-                                                           az, cx, cy, cz, g);
-        const size_t o = SPLIT != 0 ? ((((size_t)w * R + r) * J + (q - qf)) * 64 + lane) * 3
-                               : (((size_t)(w - jbase) * half + d) * (64 * K) + kb * 64 + lane) * 3;
-        jpart[o + 0] = g[0];
-        jpart[o + 1] = g[1];
-        jpart[o + 2] = g[2];
-    }
+    for (const int r1 = r + nr; r < r1; ++r) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const size_t o = ((size_t)r * (size_t)(istride < 0 ? n_pad : istride) + (w * 64 * K - ibody0) + k * 64 +
-                          lane) * 3;
-        ipart[o + 0] = ax[k] - cx[k];
-        ipart[o + 1] = ay[k] - cy[k];
-        ipart[o + 2] = az[k] - cz[k];
+        for (int k = 0; k < K; ++k)
+            ax[k] = ay[k] = az[k] = cx[k] = cy[k] = cz[k] = 0.f;
+        // sub-unit q = (unit u, source block kb): u = 0 is the wave block's own
+        // sources, u = 1 + d the wave block d + 1 places round
+        int qf, ql, c0 = 0, c1 = 0, J = 0;
+        const int len = SPLIT != 0 ? 64 / rs : 64;
+        if constexpr (SPLIT != 0) {
+            const SymSplit sp(NW, w, K, R, rs);
+            c0 = sp.first(r);
+            c1 = sp.first(r + 1);
+            qf = c0 / rs;
+            ql = (c1 + rs - 1) / rs;
+            J = SymSplit::records(NW, K, R, rs);
+        } else {
+            const int Q = (half + 1) * K;
+            qf = (int)((long long)Q * r / R);
+            ql = (int)((long long)Q * (r + 1) / R);
+        }
+        for (int q = qf; q < ql; ++q) {
+            // rotation steps [t0, t0 + steps): all but for the first and last sub-unit
+            int t0 = 0, steps = 64;
+            if constexpr (SPLIT != 0) {
+                const int a = q == qf ? c0 - q * rs : 0, e = q + 1 == ql ? c1 - q * rs : rs;
+                t0 = a * len;
+                steps = (e - a) * len;
+            }
+            const int u = q / K, kb = q - u * K;
+            if (u == 0) {
+                const float4 s = src[w * 64 * K + kb * 64 + lane];
+                const bool uni = __ballot(tuni && s.w == m0) == ~0ull;
+                if constexpr (K <= 4) {
+                    // own block kb: two-sided against the lower target slots
+                    sym_own_at<K, NEWTON, COMP, SPLIT>(kb, uni, L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
+                                                       az, cx, cy, cz);
+                } else {
+                    // own block kb (K = 8, where own blocks are a small share and
+                    // eight variants of sym_own_at would crowd the instruction cache):
+                    // target side only (each ordered pair once, self pair gives 0)
+                    float g[3];
+                    sym_block<K, K, 0, NEWTON, COMP, false, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax,
+                                                                   ay, az, cx, cy, cz, g);
+                }
+                continue;
+            }
+            const int d = u - 1;
+            if (2 * (d + 1) == NW && w >= half)
+                continue;  // the block half way round: taken by the lower half
+            int v = w + 1 + d;
+            if (v >= NW)
+                v -= NW;
+            const float4 s = src[v * 64 * K + kb * 64 + lane];
+            float g[3];
+            if (__ballot(tuni && s.w == m0) == ~0ull)
+                sym_block<K, K, K, NEWTON, COMP, true, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
+                                                              az, cx, cy, cz, g);
+            else
+                sym_block<K, K, K, NEWTON, COMP, false, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
+                                                               az, cx, cy, cz, g);
+            const size_t o = SPLIT != 0 ? ((((size_t)w * R + r) * J + (q - qf)) * 64 + lane) * 3
+                                   : (((size_t)(w - jbase) * half + d) * (64 * K) + kb * 64 + lane) * 3;
+            jpart[o + 0] = g[0];
+            jpart[o + 1] = g[1];
+            jpart[o + 2] = g[2];
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const size_t o = ((size_t)r * (size_t)(istride < 0 ? n_pad : istride) + (w * 64 * K - ibody0) + k * 64 +
+                              lane) * 3;
+            ipart[o + 0] = ax[k] - cx[k];
+            ipart[o + 1] = ay[k] - cy[k];
+            ipart[o + 2] = az[k] - cz[k];
+        }
     }
 }
 
@@ -393,10 +398,10 @@ __global__ __launch_bounds__(256) void batch_sym_kernel(BatchSymGeom g, int nwav
     const int lane = threadIdx.x & 63;
     int pos = 0;
     for (int it = batch_next_item(g, gw, pos, lane); it >= 0; it = batch_next_item(g, gw, pos, lane)) {
-        const int4 item = g.items[it];  // (system, wave block, split, splits)
+        const int4 item = g.items[it];  // (system, wave block, splits)
         const int s = item.x;
-        sym_wave<K, false, true>(snap + g.off[s], g.nw[s], item.w, item.y, item.z, eps2, ipart + g.ipo[s],
-                           jpart + g.jpo[s], lds[threadIdx.x >> 6], lane);
+        sym_wave<K, false, true>(snap + g.off[s], g.nw[s], item.w, item.y, item.z & 0xffff, eps2, ipart + g.ipo[s],
+                                 jpart + g.jpo[s], lds[threadIdx.x >> 6], lane, 0, -1, 0, 1, item.z >> 16);
     }
 }
 
@@ -436,8 +441,8 @@ __global__ __launch_bounds__(256) void batch_sym_reduce_kernel(BatchSymGeom g, i
     const int s = g.sys_of_block[bb / kBatchSymAlign];
     const int loc = bb - g.off[s];  // padding bodies are summed too (their records exist)
     double sum[3];
-    sym_split_sum<T, false>((const Part3*)(ipart + g.ipo[s]), (const Part3*)(jpart + g.jpo[s]), loc, g.nw[s], g.rs[s],
-                     K, t, sum);
+    sym_batch_sum<T>((const Part3*)(ipart + g.ipo[s]), (const Part3*)(jpart + g.jpo[s]), loc, g.nw[s], g.rs[s], K, t,
+                     sum);
     if (j < total && loc < g.n[s] && t == 0)
         sum_epilogue(epi, b, sum);  // padding bodies keep their far-away zero-mass records
 }

@@ -11,8 +11,8 @@
 // T lanes share a body: lane t adds rows t, t + T, ... of ipart, then the
 // reactions from d = t, t + T, ..., in that order (in FP64 on the compensated
 // paths, in FP32 on the plain one), then the T sums are combined over the lane
-// bits (lane_sum.h).  The order depends only on (T, R, RS, NW), so results are
-// bitwise repeatable; with T = 1 it is the plain sequential order.  Lane
+// bits (lane_sum.h).  The order depends only on (T, R, RS, NW), in batches on
+// (R, NW) (sym_batch_sum), so results are bitwise repeatable; with T = 1 it is the plain sequential order.  Lane
 // layout in a wave: lane = t * (64/T) + j for the wave's j-th body, so the 64/T
 // lanes of one t read 64/T consecutive records.
 #pragma once
@@ -144,6 +144,54 @@ __device__ __forceinline__ void sym_split_sum(const P* __restrict__ ipart, const
 #pragma unroll
     for (int c = 0; c < C; ++c)
         s[c] = lane_sum<64 / T>(s[c]);
+}
+
+// The same sums of undivided sub-units in batches, in an order that does not
+// depend on T, which follows the batch's size, so that a system's bits are its
+// own: always 16 interleaved sums, 16 / T to a lane, which meet in the order of
+// lane_sum's levels for T = 16.
+template <int T, typename P, int C>
+__device__ __forceinline__ void sym_batch_sum(const P* __restrict__ ipart, const P* __restrict__ jpart, int b, int NW,
+                                              int R, int K, int t, double (&s)[C])
+{
+    constexpr int U = 16 / T;
+    const int n_pad = NW * 64 * K, half = NW / 2, v = b / (64 * K), loc = b - v * (64 * K);
+    // the last record is the block half way round's, which a lower half's body
+    // does not have: the upper half skipped it
+    const int Q = R + half - (NW % 2 == 0 && v < half);
+    const auto record = [&](int q) {
+        const int d = q - R;
+        int w = v - 1 - d;
+        if (w < 0)
+            w += NW;
+        return *(q < R ? ipart + (size_t)q * n_pad + b : jpart + ((size_t)w * half + d) * (64 * K) + loc);
+    };
+    double a[U][C];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+            a[u][c] = 0.0;
+    int q = t;
+#pragma unroll(U >= 4 ? 1 : 4 / U)
+    for (; q + T * (U - 1) < Q; q += 16)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            part_add(a[u], record(q + T * u));
+#pragma unroll
+    for (int u = 0; u < U - 1; ++u)
+        if (q + T * u < Q)
+            part_add(a[u], record(q + T * u));
+#pragma unroll
+    for (int m = U / 2; m >= 1; m /= 2)
+#pragma unroll
+        for (int u = 0; u < m; ++u)
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+                a[u][c] += a[u + m][c];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+        s[c] = lane_sum<64 / T>(a[0][c]);
 }
 
 }  // namespace utcnb

@@ -212,12 +212,14 @@ __device__ __forceinline__ void sym_vjp_own_at(int kb, bool uni, SymVjpLds& L, i
 }
 
 // The work of wave r of wave block w of one system.  jrec: two float4 per
-// body {x,y,z,m} {ax,ay,az,0}, n_pad = NW*64*K bodies; ipart: [R][n_pad]
+// body {x,y,z,m} {ax,ay,az,0}, n_pad = NW*64*K bodies; nr: it does that of
+// waves r .. r + nr - 1 in turn (not SPLIT); ipart: [R][n_pad]
 // float4; jpart: [NW][NW/2][64K] float4, SPLIT: [NW][R][J][64] (SymSplit).
 template <int K, bool SPLIT>
 __device__ __forceinline__ void sym_vjp_wave(const float4* __restrict__ jrec, int NW, int R, int w, int r,
                                              float eps2, float4* __restrict__ ipart,
-                                             float4* __restrict__ jpart, SymVjpLds& L, int lane, int rs = 1)
+                                             float4* __restrict__ jpart, SymVjpLds& L, int lane, int rs = 1,
+                                             int nr = 1)
 {
     const int half = NW / 2;
     const int n_pad = NW * 64 * K;
@@ -229,9 +231,6 @@ __device__ __forceinline__ void sym_vjp_wave(const float4* __restrict__ jrec, in
         const float4 p = jrec[2 * b], a = jrec[2 * b + 1];
         xi[k] = p.x; yi[k] = p.y; zi[k] = p.z; mi[k] = p.w;
         bx[k] = a.x; by[k] = a.y; bz[k] = a.z;
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            g[k][q] = c[k][q] = 0.f;
     }
     // one mass m0 for every target of the wave?
     const float m0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(mi[0])));
@@ -239,58 +238,65 @@ __device__ __forceinline__ void sym_vjp_wave(const float4* __restrict__ jrec, in
 #pragma unroll
     for (int k = 0; k < K; ++k)
         tuni = tuni && mi[k] == m0;
-    // sub-unit su = (unit u, source block kb): u = 0 is the wave block's own
-    // sources, u = 1 + d the wave block d + 1 places round
-    int qf, ql, c0 = 0, c1 = 0, J = 0;
-    if constexpr (SPLIT) {
-        const SymSplit split(NW, w, K, R, rs);
-        c0 = split.first(r);
-        c1 = split.first(r + 1);
-        qf = c0 / rs;
-        ql = (c1 + rs - 1) / rs;
-        J = SymSplit::records(NW, K, R, rs);
-    } else {
-        const int Q = (half + 1) * K;
-        qf = (int)((long long)Q * r / R);
-        ql = (int)((long long)Q * (r + 1) / R);
-    }
-    for (int su = qf; su < ql; ++su) {
-        // rotation steps [t0, t0 + steps): all but for the first and last sub-unit
-        int t0 = 0, steps = 64;
-        if constexpr (SPLIT) {
-            const int a = su == qf ? c0 - su * rs : 0, e = su + 1 == ql ? c1 - su * rs : rs;
-            t0 = a * (64 / rs);
-            steps = (e - a) * (64 / rs);
-        }
-        const int u = su / K, kb = su - u * K;
-        if (u == 0) {
-            // own block kb: two-sided against the lower target slots
-            const int b = w * 64 * K + kb * 64 + lane;
-            const float4 sp = jrec[2 * b], sa = jrec[2 * b + 1];
-            const bool uni = __ballot(tuni && sp.w == m0) == ~0ull;
-            sym_vjp_own_at<K>(kb, uni, L, lane, t0, steps, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c);
-            continue;
-        }
-        const int d = u - 1;
-        if (2 * (d + 1) == NW && w >= half)
-            continue;  // the block half way round: taken by the lower half
-        int v = w + 1 + d;
-        if (v >= NW)
-            v -= NW;
-        const int b = v * 64 * K + kb * 64 + lane;
-        const float4 sp = jrec[2 * b], sa = jrec[2 * b + 1];
-        float4 h;
-        if (__ballot(tuni && sp.w == m0) == ~0ull)
-            sym_vjp_block<K, K, K, true>(L, lane, t0, steps, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c, h);
-        else
-            sym_vjp_block<K, K, K, false>(L, lane, t0, steps, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c, h);
-        jpart[SPLIT ? (((size_t)w * R + r) * J + (su - qf)) * 64 + lane
-                    : ((size_t)w * half + d) * (64 * K) + kb * 64 + lane] = h;
-    }
+    for (const int r1 = r + nr; r < r1; ++r) {
 #pragma unroll
-    for (int k = 0; k < K; ++k)
-        ipart[(size_t)r * n_pad + w * 64 * K + k * 64 + lane] =
-            make_float4(g[k][0] - c[k][0], g[k][1] - c[k][1], g[k][2] - c[k][2], g[k][3] - c[k][3]);
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                g[k][q] = c[k][q] = 0.f;
+        // sub-unit su = (unit u, source block kb): u = 0 is the wave block's own
+        // sources, u = 1 + d the wave block d + 1 places round
+        int qf, ql, c0 = 0, c1 = 0, J = 0;
+        if constexpr (SPLIT) {
+            const SymSplit split(NW, w, K, R, rs);
+            c0 = split.first(r);
+            c1 = split.first(r + 1);
+            qf = c0 / rs;
+            ql = (c1 + rs - 1) / rs;
+            J = SymSplit::records(NW, K, R, rs);
+        } else {
+            const int Q = (half + 1) * K;
+            qf = (int)((long long)Q * r / R);
+            ql = (int)((long long)Q * (r + 1) / R);
+        }
+        for (int su = qf; su < ql; ++su) {
+            // rotation steps [t0, t0 + steps): all but for the first and last sub-unit
+            int t0 = 0, steps = 64;
+            if constexpr (SPLIT) {
+                const int a = su == qf ? c0 - su * rs : 0, e = su + 1 == ql ? c1 - su * rs : rs;
+                t0 = a * (64 / rs);
+                steps = (e - a) * (64 / rs);
+            }
+            const int u = su / K, kb = su - u * K;
+            if (u == 0) {
+                // own block kb: two-sided against the lower target slots
+                const int b = w * 64 * K + kb * 64 + lane;
+                const float4 sp = jrec[2 * b], sa = jrec[2 * b + 1];
+                const bool uni = __ballot(tuni && sp.w == m0) == ~0ull;
+                sym_vjp_own_at<K>(kb, uni, L, lane, t0, steps, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c);
+                continue;
+            }
+            const int d = u - 1;
+            if (2 * (d + 1) == NW && w >= half)
+                continue;  // the block half way round: taken by the lower half
+            int v = w + 1 + d;
+            if (v >= NW)
+                v -= NW;
+            const int b = v * 64 * K + kb * 64 + lane;
+            const float4 sp = jrec[2 * b], sa = jrec[2 * b + 1];
+            float4 h;
+            if (__ballot(tuni && sp.w == m0) == ~0ull)
+                sym_vjp_block<K, K, K, true>(L, lane, t0, steps, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c, h);
+            else
+                sym_vjp_block<K, K, K, false>(L, lane, t0, steps, sp, sa, xi, yi, zi, mi, bx, by, bz, m0, eps2, g, c, h);
+            jpart[SPLIT ? (((size_t)w * R + r) * J + (su - qf)) * 64 + lane
+                        : ((size_t)w * half + d) * (64 * K) + kb * 64 + lane] = h;
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            ipart[(size_t)r * n_pad + w * 64 * K + k * 64 + lane] =
+                make_float4(g[k][0] - c[k][0], g[k][1] - c[k][1], g[k][2] - c[k][2], g[k][3] - c[k][3]);
+    }
 }
 
 // One system: wave gw = w * R + r.
@@ -322,10 +328,10 @@ __global__ __launch_bounds__(256, 2) void batch_sym_vjp_kernel(BatchSymGeom g, i
     const int lane = threadIdx.x & 63;
     int pos = 0;
     for (int it = batch_next_item(g, gw, pos, lane); it >= 0; it = batch_next_item(g, gw, pos, lane)) {
-        const int4 item = g.items[it];  // (system, wave block, split, splits)
+        const int4 item = g.items[it];  // (system, wave block, splits)
         const int s = item.x;
-        sym_vjp_wave<K, false>(jrec + 2 * (size_t)g.off[s], g.nw[s], item.w, item.y, item.z, eps2,
-                        ipart + g.vipo[s], jpart + g.vjpo[s], lds[threadIdx.x >> 6], lane);
+        sym_vjp_wave<K, false>(jrec + 2 * (size_t)g.off[s], g.nw[s], item.w, item.y, item.z & 0xffff, eps2,
+                               ipart + g.vipo[s], jpart + g.vjpo[s], lds[threadIdx.x >> 6], lane, 1, item.z >> 16);
     }
 }
 
@@ -387,7 +393,7 @@ __global__ __launch_bounds__(256) void batch_sym_vjp_reduce_kernel(BatchSymGeom 
     const int s = g.sys_of_block[bb / kBatchSymAlign];
     const int loc = bb - g.off[s];
     double sum[4];
-    sym_split_sum<T, false>(ipart + g.vipo[s], jpart + g.vjpo[s], loc, g.nw[s], g.rs[s], K, t, sum);
+    sym_batch_sum<T>(ipart + g.vipo[s], jpart + g.vjpo[s], loc, g.nw[s], g.rs[s], K, t, sum);
     if (j < total && loc < g.n[s] && t == 0)
         adjoint_next(next, b, sum, xbar3, mbar);
 }
