@@ -2,10 +2,11 @@
 //
 // Mapping.  A wavefront owns K target bodies per lane (64*K targets) and
 // streams a contiguous range of source bodies.  The source index is uniform
-// across the wave, so the compiler loads source bodies with scalar loads
-// (s_load_dwordx16 = four float4 bodies) into SGPRs, and every VALU op takes
-// its source operand straight from an SGPR: no LDS traffic and no broadcast
-// instructions in the inner loop.  S waves of a workgroup split the source
+// across the wave: with K = 1 or S = 1 source bodies come through scalar loads
+// (s_load_dwordx16 = four float4 bodies) into SGPRs and every VALU op takes
+// its source operand straight from an SGPR, else through vector loads of one
+// address (at the kernel): no LDS traffic and no broadcast instructions in the
+// inner loop.  S waves of a workgroup split the source
 // range of one target tile; their partial sums meet in LDS at the end.
 //
 // Arithmetic per pair (the reference's pair, benchapps/nbody/seq/bodysystem.h:70-96,
@@ -253,7 +254,13 @@ __global__ __launch_bounds__(64 * W) void force_kernel(const float4* __restrict_
 {
     constexpr int T = W / S;  // target tiles per workgroup
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    // K = 1: in a scalar register, so that the sources come through scalar loads;
+    // 16 waves of vector loads, 1 KiB each, were bound by the L1 with a source for
+    // one pair per lane (N = 16384: k1s16 143 us, now 87, k1s8 124 and 114; 131072:
+    // k1s4 8.9 and 4.5 ms).  With K = 2 and 4 the vector loads are faster up to
+    // 40000 bodies, as scalar ones leave one group of them in flight (k2s2 at 16384
+    // 736 us, scalar 879; k2s8 196 and 215).
+    const int w0 = threadIdx.x >> 6, wave = K == 1 ? __builtin_amdgcn_readfirstlane(w0) : w0;
     const int tile = blockIdx.x * T + wave / S;
     const int part = wave % S;
 
