@@ -478,14 +478,14 @@ size_t sym_jpart_floats(int n_pad, const Tile& t)
     return (size_t)NW * R * SymSplit::records(NW, t.k, R, rs) * 64 * 3;
 }
 
-// The form of the divided kernels (sym_block): below 24576 bodies K = 8 serves
+// The form of the divided kernels (sym_block): to 24576 bodies K = 8 serves
 // sizes that K = 2 and 4 did; above it has no longer chains than undivided, and
 // summing by steps takes 3.7% at 32768.
 static int sym_split_form(const Tile& t, int n_pad)
 {
     if (sym_tile_rs(t, n_pad) == 1)
         return 0;
-    return t.k == 8 && n_pad < 24576 ? 2 : 1;
+    return t.k == 8 && n_pad <= 24576 ? 2 : 1;
 }
 
 template <int K, bool COMP>
