@@ -43,10 +43,11 @@
 // What bounds it: FP32 issue and, at large N, the power the FMAs draw.  A step
 // issues one 16-byte and three 4-byte LDS reads and three LDS writes beside
 // its K pairs; carrying the source and its sums round the wave in registers
-// instead (7 DPP moves per step, which pair with nothing) and taking each
-// root as it comes cost 55 cycles per pair and wave where this takes 44
-// (N = 262144, equal masses: 23.2e6 clocks for 28.9e6; the clock drops from
-// 2383 to 2113 MHz meanwhile, so the time falls less).  Per step, mixed, same
+// instead (7 DPP moves per step, which pair with nothing), as launches of few
+// waves do (sym_block_reg), and taking each root as it comes cost 55 cycles per
+// pair and wave where this takes 44 (N = 262144, equal masses: 23.2e6 clocks for
+// 28.9e6; the clock drops from 2383 to 2113 MHz meanwhile, so the time falls
+// less).  Per step, mixed, same
 // device: N = 262144 10.7-10.9 ms (12.3 before), log-uniform masses 11.8
 // (14.0), N = 65536 0.716 ms (0.829), plain FP32 0.700 (0.819), N = 16384
 // (sym4r64) 68 us (75).  The roots are taken 4 at a time: with 8 the K = 8
@@ -163,6 +164,108 @@ __device__ __forceinline__ void sym_rotate(SymLds& L, int lane, int t0, int step
     }
 }
 
+// Lane l receives lane l-1's value (lane 0 lane 63's).  Every lane has a source
+// under wave_ror:1, so the "old" operand is never used; passing v rotates in
+// place (K = 2, 7.7% faster there), 0 writes a new register (K = 8, 3%).
+template <int K>
+__device__ __forceinline__ float wave_ror1(float v)
+{
+    const int x = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(K <= 2 ? x : 0, x, 0x13C /* wave_ror:1 */, 0xF, 0xF, false));
+}
+
+// sym_block (below) with the block and its reaction sums carried round the wave
+// in registers: at step t lane l meets source (l - t) mod 64.  The DPP moves pair
+// with nothing, but a wave that has a SIMD to itself waits longer for the LDS of
+// sym_rotate than it issues them.
+template <int K, int N, int N2, bool NEWTON, bool COMP, bool UNI, int SPLIT>
+__device__ __forceinline__ void sym_block_reg(int lane, int t0, int steps, int len, float4 s, const float (&xi)[K],
+                                              const float (&yi)[K], const float (&zi)[K], const float (&mi)[K],
+                                              float m, float eps2, float (&ax)[K], float (&ay)[K], float (&az)[K],
+                                              float (&cx)[K], float (&cy)[K], float (&cz)[K], float (&g)[3])
+{
+    float sx = s.x, sy = s.y, sz = s.z, sm = s.w;
+    if (SPLIT != 0 && t0 != 0) {  // wave-uniform
+        const int from = (lane - t0) & 63;
+        sx = __shfl(sx, from, 64); sy = __shfl(sy, from, 64); sz = __shfl(sz, from, 64); sm = __shfl(sm, from, 64);
+    }
+    for (int t = t0;;) {
+        float px[N], py[N], pz[N], gx = 0.f, gy = 0.f, gz = 0.f;
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            px[k] = py[k] = pz[k] = 0.f;
+        const int n = SPLIT != 0 ? len : 64;  // a multiple of 4
+        for (int i4 = 0; i4 < n; i4 += 4)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                constexpr int GK = N < 4 ? N : 4;  // pairs per group of reciprocal roots
+#pragma unroll
+                for (int k0 = 0; k0 < N; k0 += GK) {
+                    float rx[GK], ry[GK], rz[GK], d2[GK], y[GK];
+#pragma unroll
+                    for (int q = 0; q < GK; ++q) {
+                        const int k = k0 + q;
+                        rx[q] = sx - xi[k]; ry[q] = sy - yi[k]; rz[q] = sz - zi[k];
+                        d2[q] = __builtin_fmaf(rx[q], rx[q],
+                                               __builtin_fmaf(ry[q], ry[q], __builtin_fmaf(rz[q], rz[q], eps2)));
+                        if constexpr (K == 2)
+                            y[q] = __builtin_amdgcn_rsqf(d2[q]);
+                    }
+                    if constexpr (K != 2)
+                        rsq_group<GK>(d2, y);
+#pragma unroll
+                    for (int q = 0; q < GK; ++q) {
+                        const int k = k0 + q;
+                        const float y3 = pair_scale<NEWTON>(d2[q], y[q], 1.0f);
+                        const float si = UNI ? y3 : sm * y3;
+                        px[k] = __builtin_fmaf(rx[q], si, px[k]);
+                        py[k] = __builtin_fmaf(ry[q], si, py[k]);
+                        pz[k] = __builtin_fmaf(rz[q], si, pz[k]);
+                        if (k < N2) {
+                            const float cj = UNI ? y3 : mi[k] * y3;
+                            gx = __builtin_fmaf(-rx[q], cj, gx);
+                            gy = __builtin_fmaf(-ry[q], cj, gy);
+                            gz = __builtin_fmaf(-rz[q], cj, gz);
+                        }
+                    }
+                }
+                sx = wave_ror1<K>(sx); sy = wave_ror1<K>(sy); sz = wave_ror1<K>(sz);
+                if constexpr (!UNI)
+                    sm = wave_ror1<K>(sm);
+                if constexpr (N2 > 0) {
+                    gx = wave_ror1<K>(gx); gy = wave_ror1<K>(gy); gz = wave_ror1<K>(gz);
+                }
+            }
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            if constexpr (UNI) {
+                px[k] *= m; py[k] *= m; pz[k] *= m;
+            }
+            block_add<COMP>(ax[k], cx[k], px[k]);
+            block_add<COMP>(ay[k], cy[k], py[k]);
+            block_add<COMP>(az[k], cz[k], pz[k]);
+        }
+        if constexpr (N2 > 0) {
+            const int home = (t + n) & 63;  // lane l holds the sums of source l - home
+            if (SPLIT != 0 && home != 0) {
+                const int from = (lane + home) & 63;
+                gx = __shfl(gx, from, 64); gy = __shfl(gy, from, 64); gz = __shfl(gz, from, 64);
+            }
+            g[0] = t == t0 ? gx : g[0] + gx;
+            g[1] = t == t0 ? gy : g[1] + gy;
+            g[2] = t == t0 ? gz : g[2] + gz;
+        }
+        t += n;
+        if (SPLIT == 0 || t >= t0 + steps)
+            break;
+    }
+    if constexpr (UNI && N2 > 0) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            g[c] *= m;
+    }
+}
+
 // Rotation steps [t0, t0 + steps) of a block of 64 sources against the lanes'
 // target slots (sym_rotate): target-side partials are added into (a, c) by
 // block_add<COMP>, the reaction sums of lane l's own source come back in g
@@ -174,12 +277,17 @@ __device__ __forceinline__ void sym_rotate(SymLds& L, int lane, int t0, int step
 // cube, Newton: sym4r64x2 3.71e-8 without and 3.00e-8 with, sym8r128 5.04e-8
 // without and 2.80e-8 with (59.3 and 61.1 us per step; 24575 4.18e-8 and
 // 2.34e-8).
-template <int K, int N, int N2, bool NEWTON, bool COMP, bool UNI, int SPLIT>
+template <int K, int N, int N2, bool NEWTON, bool COMP, bool UNI, int SPLIT, bool REG>
 __device__ __forceinline__ void sym_block(SymLds& L, int lane, int t0, int steps, int len, float4 s,
                                           const float (&xi)[K], const float (&yi)[K], const float (&zi)[K],
                                           const float (&mi)[K], float m, float eps2, float (&ax)[K], float (&ay)[K],
                                           float (&az)[K], float (&cx)[K], float (&cy)[K], float (&cz)[K], float (&g)[3])
 {
+    if constexpr (REG) {
+        sym_block_reg<K, N, N2, NEWTON, COMP, UNI, SPLIT>(lane, t0, steps, len, s, xi, yi, zi, mi, m, eps2, ax, ay, az,
+                                                          cx, cy, cz, g);
+        return;
+    }
     constexpr bool CHUNKS = SPLIT == 1 && K <= 4;
     sym_fill<N2>(L, lane, s);
     for (int t = t0;;) {
@@ -230,7 +338,7 @@ __device__ __forceinline__ void sym_block(SymLds& L, int lane, int t0, int steps
 // KB one-sided (the block with itself: each ordered pair once, the self pair
 // adds r = 0); slots k > KB take these sources when their own block is the
 // source.  The reaction sums belong to slot KB.
-template <int K, bool NEWTON, bool COMP, int SPLIT, int KB = 0>
+template <int K, bool NEWTON, bool COMP, int SPLIT, bool REG, int KB = 0>
 __device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane, int t0, int steps, int len, float4 s,
                                            const float (&xi)[K], const float (&yi)[K], const float (&zi)[K],
                                            const float (&mi)[K], float m, float eps2, float (&ax)[K], float (&ay)[K],
@@ -239,10 +347,10 @@ __device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane
     if (kb == KB) {
         float g[3];
         if (uni)
-            sym_block<K, KB + 1, KB, NEWTON, COMP, true, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m, eps2, ax,
+            sym_block<K, KB + 1, KB, NEWTON, COMP, true, SPLIT, REG>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m, eps2, ax,
                                                                 ay, az, cx, cy, cz, g);
         else
-            sym_block<K, KB + 1, KB, NEWTON, COMP, false, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m, eps2, ax,
+            sym_block<K, KB + 1, KB, NEWTON, COMP, false, SPLIT, REG>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m, eps2, ax,
                                                                  ay, az, cx, cy, cz, g);
         if constexpr (KB > 0) {
             block_add<COMP>(ax[KB], cx[KB], g[0]);
@@ -253,7 +361,7 @@ __device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane
             asm volatile("; own block %0" : : "n"(KB));
         }
     } else if constexpr (KB + 1 < K) {
-        sym_own_at<K, NEWTON, COMP, SPLIT, KB + 1>(kb, uni, L, lane, t0, steps, len, s, xi, yi, zi, mi, m, eps2, ax, ay,
+        sym_own_at<K, NEWTON, COMP, SPLIT, REG, KB + 1>(kb, uni, L, lane, t0, steps, len, s, xi, yi, zi, mi, m, eps2, ax, ay,
                                                    az, cx, cy, cz);
     }
 }
@@ -269,7 +377,7 @@ __device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane
 // SPLIT (1 or 2, sym_block): the waves share the sub-units by chunks of 64 / rs
 // rotation steps (rs divides 16) and the reactions take a record per wave and sub-unit: jpart is
 // [NW][R][J][64][3] (SymSplit, sym_reduce.h).
-template <int K, bool NEWTON, bool COMP, int SPLIT = 0>
+template <int K, bool NEWTON, bool COMP, int SPLIT = 0, bool REG = false>
 __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW, int R, int w, int r,
                                          float eps2, float* __restrict__ ipart,
                                          float* __restrict__ jpart, SymLds& L, int lane, int jbase = 0,
@@ -323,14 +431,14 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
                 const bool uni = __ballot(tuni && s.w == m0) == ~0ull;
                 if constexpr (K <= 4) {
                     // own block kb: two-sided against the lower target slots
-                    sym_own_at<K, NEWTON, COMP, SPLIT>(kb, uni, L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
+                    sym_own_at<K, NEWTON, COMP, SPLIT, REG>(kb, uni, L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
                                                        az, cx, cy, cz);
                 } else {
                     // own block kb (K = 8, where own blocks are a small share and
                     // eight variants of sym_own_at would crowd the instruction cache):
                     // target side only (each ordered pair once, self pair gives 0)
                     float g[3];
-                    sym_block<K, K, 0, NEWTON, COMP, false, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax,
+                    sym_block<K, K, 0, NEWTON, COMP, false, SPLIT, REG>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax,
                                                                    ay, az, cx, cy, cz, g);
                 }
                 continue;
@@ -344,10 +452,10 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
             const float4 s = src[v * 64 * K + kb * 64 + lane];
             float g[3];
             if (__ballot(tuni && s.w == m0) == ~0ull)
-                sym_block<K, K, K, NEWTON, COMP, true, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
+                sym_block<K, K, K, NEWTON, COMP, true, SPLIT, REG>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
                                                               az, cx, cy, cz, g);
             else
-                sym_block<K, K, K, NEWTON, COMP, false, SPLIT>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
+                sym_block<K, K, K, NEWTON, COMP, false, SPLIT, REG>(L, lane, t0, steps, len, s, xi, yi, zi, mi, m0, eps2, ax, ay,
                                                                az, cx, cy, cz, g);
             const size_t o = SPLIT != 0 ? ((((size_t)w * R + r) * J + (q - qf)) * 64 + lane) * 3
                                    : (((size_t)(w - jbase) * half + d) * (64 * K) + kb * 64 + lane) * 3;
@@ -367,12 +475,12 @@ __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW,
 }
 
 // One system: wave gw = w * R + r.  SPLIT: rs rotation chunks per sub-unit.
-template <int K, bool NEWTON, bool COMP, int SPLIT>
+template <int K, bool NEWTON, bool COMP, int SPLIT, bool REG>
 __global__ __launch_bounds__(256, 2) void sym_force_kernel(const float4* __restrict__ src, int NW, int R,
                                                         float eps2, float* __restrict__ ipart,
                                                         float* __restrict__ jpart, int rs)
 {
-    __shared__ SymLds lds[4];
+    __shared__ SymLds lds[REG ? 1 : 4];
     int gw = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     // whole sub-units: the schedule in scalar registers, 1 to 3% from 65536
     // bodies (717 to 704 us); split, the same within 0.7% either way
@@ -380,8 +488,8 @@ __global__ __launch_bounds__(256, 2) void sym_force_kernel(const float4* __restr
         gw = __builtin_amdgcn_readfirstlane(gw);
     if (gw >= NW * R)
         return;  // whole waves only
-    sym_wave<K, NEWTON, COMP, SPLIT>(src, NW, R, gw / R, gw % R, eps2, ipart, jpart, lds[threadIdx.x >> 6],
-                                     threadIdx.x & 63, 0, -1, 0, rs);
+    sym_wave<K, NEWTON, COMP, SPLIT, REG>(src, NW, R, gw / R, gw % R, eps2, ipart, jpart,
+                                          lds[REG ? 0 : threadIdx.x >> 6], threadIdx.x & 63, 0, -1, 0, rs);
 }
 
 // Batched systems: each wave runs items (system, wave block, split), a system
@@ -488,30 +596,50 @@ static int sym_split_form(const Tile& t, int n_pad)
     return t.k == 8 && n_pad <= 24576 ? 2 : 1;
 }
 
+// Launches of at most this many waves carry the sources in registers
+// (sym_block_reg): a wave to a SIMD, for K = 2 two.  Per step, mixed, us,
+// registers and LDS: sym2r32 at 1024 bodies (256 waves) 10.8 and 13.8, 4096 (1024)
+// 15.8 and 21.2, 8192 (2048) 29.4 and 31.2, 9001 (2304) 41.3 and 37.7; sym4r4 at
+// 8192 (128) 165 and 186, sym4r64 at 4096 (1024) 17.7 and 18.9, sym4r16 at 20480
+// (1280) 182 and 143; sym8r4 at 8192 (64) 309 and 327, sym8r32 at 20480 (1280) 170
+// and 135; divided, sym2r64x2 at 2048 (1024) 9.8 and 11.5, sym4r64x2 at 4096 (1024)
+// 16.9 and 18.3, at 8192 (2048) 26.8 and 26.0.  Shares: 3 of 8 of 9001 bodies (666)
+// 30.1 and 32.8, of 12288 (1176) 35.2 and 34.3, of 16384 (1056) 42.6 and 39.1.
+constexpr int kRegWaves = 1024, kRegWavesK2 = 2048;
+
+template <int K, bool COMP, int SPLIT, bool REG>
+static void launch_sym_pairs_as(bool newton, int rs, dim3 grid, const float4* src, int NW, int R, float eps2,
+                                float* ipart, float* jpart, hipStream_t st)
+{
+    if (newton)
+        hipLaunchKernelGGL((sym_force_kernel<K, true, COMP, SPLIT, REG>), grid, dim3(256), 0, st, src, NW, R, eps2,
+                           ipart, jpart, rs);
+    else
+        hipLaunchKernelGGL((sym_force_kernel<K, false, COMP, SPLIT, REG>), grid, dim3(256), 0, st, src, NW, R, eps2,
+                           ipart, jpart, rs);
+}
+
 template <int K, bool COMP>
 static void launch_sym_pairs(bool newton, int split, int rs, dim3 grid, const float4* src, int NW, int R, float eps2,
                              float* ipart, float* jpart, hipStream_t st)
 {
-#define SYM_PAIRS(NEWTON, SPLIT)                                                                                \
-    hipLaunchKernelGGL((sym_force_kernel<K, NEWTON, COMP, SPLIT>), grid, dim3(256), 0, st, src, NW, R, eps2, ipart, \
-                       jpart, rs)
+#define SYM_PAIRS(SPLIT, REG) launch_sym_pairs_as<K, COMP, SPLIT, REG>(newton, rs, grid, src, NW, R, eps2, ipart, jpart, st)
+    const bool reg = NW * R <= (K == 2 ? kRegWavesK2 : kRegWaves);
     if constexpr (K == 8) {
-        if (split == 2) {
-            if (newton)
-                SYM_PAIRS(true, 2);
-            else
-                SYM_PAIRS(false, 2);
-            return;
-        }
+        if (split == 2)
+            return SYM_PAIRS(2, false);
+        if (split == 1)
+            return SYM_PAIRS(1, false);
+    } else {
+        if (split == 1 && reg)
+            return SYM_PAIRS(1, true);
+        if (split == 1)
+            return SYM_PAIRS(1, false);
     }
-    if (split != 0 && newton)
-        SYM_PAIRS(true, 1);
-    else if (split != 0)
-        SYM_PAIRS(false, 1);
-    else if (newton)
-        SYM_PAIRS(true, 0);
+    if (reg)
+        SYM_PAIRS(0, true);
     else
-        SYM_PAIRS(false, 0);
+        SYM_PAIRS(0, false);
 #undef SYM_PAIRS
 }
 
@@ -587,18 +715,18 @@ hipError_t launch_sym(const Tile& t, bool newton, bool comp, const float4* src, 
 // jbase: the first wave block whose reaction rows jpart holds (0 for a
 // whole-system buffer, w0 for a buffer of the share's rows only).
 // ipart: rows of istride bodies starting at body ibody0 (see sym_wave).
-template <int K, bool NEWTON>
+template <int K, bool NEWTON, bool REG>
 __global__ __launch_bounds__(256) void sym_share_kernel(const float4* __restrict__ src, int NW, int R, int w0,
                                                         int nwaves, float eps2, float* __restrict__ ipart,
                                                         float* __restrict__ jpart, int jbase, long long istride,
                                                         int ibody0)
 {
-    __shared__ SymLds lds[4];
+    __shared__ SymLds lds[REG ? 1 : 4];
     const int gw = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
     if (gw >= nwaves)
         return;  // whole waves only
-    sym_wave<K, NEWTON, true>(src, NW, R, w0 + gw / R, gw % R, eps2, ipart, jpart, lds[threadIdx.x >> 6],
-                              threadIdx.x & 63, jbase, istride, ibody0);
+    sym_wave<K, NEWTON, true, 0, REG>(src, NW, R, w0 + gw / R, gw % R, eps2, ipart, jpart,
+                                      lds[REG ? 0 : threadIdx.x >> 6], threadIdx.x & 63, jbase, istride, ibody0);
 }
 
 // react3[b] (FP64, bodies b < n) = the reactions on body b from the wave
@@ -727,13 +855,19 @@ hipError_t launch_sym_share_pairs(const Tile& t, bool newton, const float4* src,
     share_ipart_layout(n_pad, K, Rs, w0, w1, compact_ipart, &ibase, &istride, &ibody0);
     if (nwaves > 0) {
         const dim3 grid((nwaves + 3) / 4), block(256);
-#define SHARE_LAUNCH(KK)                                                                                  \
-    if (newton)                                                                                           \
-        hipLaunchKernelGGL((sym_share_kernel<KK, true>), grid, block, 0, st, src, NW, Rs, w0, nwaves, eps2, \
-                           ipart + ibase, jpart, jbase, istride, ibody0);                                 \
-    else                                                                                                  \
-        hipLaunchKernelGGL((sym_share_kernel<KK, false>), grid, block, 0, st, src, NW, Rs, w0, nwaves, eps2, \
-                           ipart + ibase, jpart, jbase, istride, ibody0);
+        const bool reg = nwaves <= kRegWaves;
+#define SHARE_AS(KK, NEWTON, REG)                                                                                \
+    hipLaunchKernelGGL((sym_share_kernel<KK, NEWTON, REG>), grid, block, 0, st, src, NW, Rs, w0, nwaves, eps2, \
+                       ipart + ibase, jpart, jbase, istride, ibody0)
+#define SHARE_LAUNCH(KK)              \
+    if (newton && reg)                \
+        SHARE_AS(KK, true, true);     \
+    else if (newton)                  \
+        SHARE_AS(KK, true, false);    \
+    else if (reg)                     \
+        SHARE_AS(KK, false, true);    \
+    else                              \
+        SHARE_AS(KK, false, false);
         if (K == 2) {
             SHARE_LAUNCH(2)
         } else if (K == 4) {
@@ -743,6 +877,7 @@ hipError_t launch_sym_share_pairs(const Tile& t, bool newton, const float4* src,
         } else {
             return hipErrorInvalidValue;
         }
+#undef SHARE_AS
 #undef SHARE_LAUNCH
         hipError_t e = hipGetLastError();
         if (e != hipSuccess)
