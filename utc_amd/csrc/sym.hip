@@ -376,7 +376,7 @@ __device__ __forceinline__ void sym_own_at(int kb, bool uni, SymLds& L, int lane
 // nr: the wave does the work of waves r .. r + nr - 1 in turn (not SPLIT).
 // SPLIT (1 or 2, sym_block): the waves share the sub-units by chunks of 64 / rs
 // rotation steps (rs divides 16) and the reactions take a record per wave and sub-unit: jpart is
-// [NW][R][J][64][3] (SymSplit, sym_reduce.h).
+// [NW][R][J][64][3] (SymSplit, sym_split.h).
 template <int K, bool NEWTON, bool COMP, int SPLIT = 0, bool REG = false>
 __device__ __forceinline__ void sym_wave(const float4* __restrict__ src, int NW, int R, int w, int r,
                                          float eps2, float* __restrict__ ipart,

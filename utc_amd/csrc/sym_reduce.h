@@ -6,13 +6,14 @@
 // the reactions from the NW/2 wave blocks before its own, d + 1 = 1 .. NW/2
 // places below, the one half way round only where the upper half did not skip
 // it.  Undivided sub-units (RS = 1): one record per wave block and d, jpart
-// [NW][NW/2][64K].  Divided ones (SymSplit below): each of the waves that share
+// [NW][NW/2][64K].  Divided ones (sym_split.h): each of the waves that share
 // a sub-unit left a record of 64 bodies, jpart [NW][R][J][64].
 // T lanes share a body: lane t adds rows t, t + T, ... of ipart, then the
 // reactions from d = t, t + T, ..., in that order (in FP64 on the compensated
 // paths, in FP32 on the plain one), then the T sums are combined over the lane
 // bits (lane_sum.h).  The order depends only on (T, R, RS, NW), in batches on
-// (R, NW) (sym_batch_sum), so results are bitwise repeatable; with T = 1 it is the plain sequential order.  Lane
+// (R, NW) (sym_batch_sum), so results are bitwise repeatable; with T = 1 it is the
+// plain sequential order.  Lane
 // layout in a wave: lane = t * (64/T) + j for the wave's j-th body, so the 64/T
 // lanes of one t read 64/T consecutive records.
 #pragma once
@@ -20,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include "lane_sum.h"
+#include "sym_split.h"
 
 namespace utcnb {
 
@@ -57,28 +59,6 @@ __device__ __forceinline__ void sym_reduce_lane(int& body, int& t)
     t = lane / (64 / T);
     body = (g >> 6) * (64 / T) + lane % (64 / T);
 }
-
-// How the R waves of wave block w of NW share its sub-units when each is cut
-// into RS chunks (K sub-units for the own unit and each of the NW/2 after it,
-// one less in the upper half, which skips the block half way round): wave r
-// takes chunks [first(r), first(r + 1)) in a row, whole sub-units but for the
-// first and the last, and leaves one reaction record for each of the at most
-// J sub-units it touches.  Waves past the last chunk take none.  The products
-// stay below 2^31: partial sums of at most 64 GiB hold some 150000 chunks per
-// wave block, and R <= 128.
-struct SymSplit {
-    int chunks, R, rs;
-    __host__ __device__ SymSplit(int NW, int w, int K, int R_, int rs_)
-        : chunks((NW / 2 + (w < NW / 2)) * K * rs_), R(R_ < chunks ? R_ : chunks), rs(rs_)
-    {
-    }
-    __host__ __device__ int first(int r) const { return r < R ? (int)((unsigned)(chunks * r) / (unsigned)R) : chunks; }
-    // the wave that takes chunk x: the last r with first(r) <= x
-    __host__ __device__ int wave(int x) const { return (int)((unsigned)((x + 1) * R - 1) / (unsigned)chunks); }
-    __host__ __device__ int records() const { return ((chunks + R - 1) / R + rs - 2) / rs + 1; }
-    // J: the lower half's waves touch the most
-    __host__ __device__ static int records(int NW, int K, int R, int rs) { return SymSplit(NW, 0, K, R, rs).records(); }
-};
 
 // All 64 lanes of the wave must call this (it exchanges lanes); b must be a
 // valid body of the system for every lane.

@@ -31,7 +31,7 @@
 // k < kb, one-sided against slot kb), unit 1 + d = the wave block d + 1 places
 // round (both sides), R waves per wave block split the K (NW/2+1) (unit,
 // source block) sub-units: in chunks of 4 rotation steps (SymSplit,
-// sym_reduce.h), or whole ones in batches.
+// sym_split.h), or whole ones in batches.
 // Partials go to HBM (float4 per body: x, y, z, m) and a second kernel adds
 // them per body in FP64, in a fixed order, into xbar and mbar.
 #include "internal.h"
