@@ -37,8 +37,8 @@
 // (SPLIT kernels) cut each sub-unit's 64 rotation steps into RS chunks of 64/RS
 // steps, and the R waves of a wave block share its Q * RS chunks in a row;
 // a sub-unit that two waves share has a reaction record from each.  N = 16384
-// 61.1 us per step against 65.6 with whole sub-units, 28672 153 against 163,
-// 9001 33.9 against 37.5 (sweeps at tile_default in force_fp32.hip).
+// 61.5 us per step against 67.5 with whole sub-units of K = 4, 32768 195 against
+// 211, 9001 33.2 against 38.7 (sweeps at tile_default in force_fp32.hip).
 //
 // What bounds it: FP32 issue and, at large N, the power the FMAs draw.  A step
 // issues one 16-byte and three 4-byte LDS reads and three LDS writes beside
