@@ -74,8 +74,9 @@ extern "C" {
  * benchapps/nbody/utc/sgpu/body_task_sgpu.cu:117-154 (kernels:
  * benchapps/nbody/cuda/bodysystem_kernel.cu:87-138,186-243), with the same
  * argument meaning.  `blocksize` is the workgroup size (64..1024, multiple of
- * 64; 0 = 256).  Unlike the reference, numBodies need not be a multiple of
- * blocksize.  Results are bit-identical to the reference's CPU path; the
+ * 64; 0 = 256) from 98305 targets on (f64: 49153); fewer are served by kernels
+ * of fixed workgroups, with the same bits.  Unlike the reference, numBodies
+ * need not be a multiple of blocksize.  Results are bit-identical to the reference's CPU path; the
  * reference's split-j "Small" variant changes the summation order and is not
  * reproduced.  pos_old and pos_new must not alias.
  */
@@ -208,8 +209,10 @@ int utcnb_position_buffer(utcnb_system* sys, int which, void** pos4, int* dtype)
  *      the next position buffer;
  *   4. the caller gathers the other shares' positions into that buffer and
  *      calls utcnb_commit_step.
- * Every share's partial sums are those of utcnb_step with the same tile; only
- * the FP64 order of the final per-body sums differs.  No reference
+ * Every share's pair terms are those of utcnb_step with wave blocks of the
+ * share's size (128 bodies below 16384, 256 below 24576, else 512, or the
+ * configured tile's); where its waves cut the partial sums differs, so a step's
+ * kicks agree to the FP32 rounding of those sums (some 1e-9 to 4e-8).  No reference
  * counterpart (the reference's multi-GPU kernel evaluates every ordered pair,
  * benchapps/nbody/utc-snode-mgpu/mgpu/bodysystem_kernel.cu:88-140).
  * 1 <= shares <= the number of wave blocks; asynchronous on the handle's stream.

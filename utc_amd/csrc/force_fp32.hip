@@ -73,8 +73,8 @@ const Tile& tile_get(int id) { return kTiles[id]; }
 // waves' unequal ends weigh most: two waves on every SIMD (2048) that start
 // together and have equal shares of the work but for an eighth of a sub-unit.
 // Longer runs drift apart over the chip and want shorter waves, several in
-// turn; from 256 bodies per CU a sub-unit is small against a wave's work, and
-// whole ones need no second reaction record.  The partial sums must fit the
+// turn; from 46081 bodies whole ones, without a second reaction record
+// (sym_tile_rs).  The partial sums must fit the
 // device's budget (sym_partial_budget); above it a one-pass tile is used (N =
 // 262144: k2s8 19.1 ms, k2s16 21.1).
 size_t sym_partial_budget(size_t device_bytes)
